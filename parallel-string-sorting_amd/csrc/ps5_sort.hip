@@ -3647,6 +3647,9 @@ int ps5_ctx_create(ps5_ctx** out, int device)
     if (e == hipSuccess)
         e = hipHostMalloc(reinterpret_cast<void**>(&c->h_stage), kStageHead + kPeek * sizeof(Item),
                           hipHostMallocMapped | hipHostMallocCoherent);
+    // recycled pinned memory may hold an older context's sequence number: the
+    // wait for this context's first staged copies must not see it
+    if (e == hipSuccess) memset(c->h_stage, 0, kStageHead);
     if (e == hipSuccess) e = hipHostGetDevicePointer(reinterpret_cast<void**>(&c->h_stage_dev), c->h_stage, 0);
     if (e == hipSuccess) e = hipMalloc(&c->d_sums, S_NUM * sizeof(unsigned long long));
     if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&c->h_sums), S_NUM * sizeof(unsigned long long));
