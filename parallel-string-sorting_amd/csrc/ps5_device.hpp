@@ -104,6 +104,102 @@ __device__ __forceinline__ uint32_t key_depth(key64 a)
     return a ? 8u - ((uint32_t)__builtin_ctzll(a) >> 3) : 0u;
 }
 
+// the same for keys of format F
+__device__ __forceinline__ uint32_t lcp_key(key64 a, key64 b, KeyFmt F)
+{
+    const key64 x = a ^ b;
+    return x ? ((uint32_t)__clzll((long long)x) * F.mul) >> 8 : F.cpk;
+}
+__device__ __forceinline__ uint32_t key_depth(key64 a, KeyFmt F)
+{
+    return a ? F.cpk - ((((uint32_t)__builtin_ctzll(a) - F.pad) * F.mul) >> 8) : 0u;
+}
+__device__ __forceinline__ bool key_ends(key64 a, KeyFmt F) { return ((uint32_t)a & F.last) == 0; }
+
+// The 24 characters from byte offset off as three little-endian words
+// (zeros past the arena's end).
+struct Chars24 { uint64_t w[3]; };
+__device__ __forceinline__ Chars24 load_chars24(const uint8_t* arena, uint64_t alen, uint64_t off)
+{
+    const uint64_t a8 = off & ~7ull;
+    uint64_t v[4];
+    if (a8 + 32 <= alen) {
+        const g_u64* p = (const g_u64*)(arena + a8);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = p[i];
+    } else {
+        const g_u8* b = (const g_u8*)arena;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = 0;
+        for (uint64_t q = a8; q < alen; ++q) {     // (fewer than 32 bytes are left)
+            const uint64_t c = (uint64_t)b[q] << (8 * (q & 7));
+            const uint32_t j = (uint32_t)(q - a8) >> 3;
+            v[0] |= j == 0 ? c : 0ull;
+            v[1] |= j == 1 ? c : 0ull;
+            v[2] |= j == 2 ? c : 0ull;
+            v[3] |= j == 3 ? c : 0ull;
+        }
+    }
+    const uint32_t sh = (uint32_t)(off & 7) * 8;
+    Chars24 r;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) r.w[i] = sh ? ((v[i] >> sh) | (v[i + 1] << (64 - sh))) : v[i];
+    return r;
+}
+
+// characters of c before its first NUL (24 if there is none)
+__device__ __forceinline__ uint32_t chars_before_nul(const Chars24& c)
+{
+    uint32_t n = 24;
+#pragma unroll
+    for (int i = 2; i >= 0; --i) {
+        const uint64_t t = ((c.w[i] & 0x7F7F7F7F7F7F7F7Full) + 0x7F7F7F7F7F7F7F7Full) | c.w[i];
+        const uint64_t z = ~t & 0x8080808080808080ull;
+        if (z) n = 8 * i + ((uint32_t)__builtin_ctzll(z) >> 3);
+    }
+    return n;
+}
+
+// The packed key of c under the code table lut (LDS: 0 for the NUL, 1.. for
+// the alphabet, 0x81 for anything else).  *bad is set when a character of
+// the key is outside the alphabet.  BITS code bits, BITS * 7 or more of them
+// per 32-bit word, so that a character costs a byte extract, a table read
+// and a shift-or.
+template <int BITS>
+__device__ __forceinline__ key64 pack_key(const Chars24& c, const uint8_t* lut, bool* bad)
+{
+    constexpr int kPerWord = BITS == 3 ? 10 : BITS == 4 ? 8 : 6;
+    constexpr int kChars = BITS == 3 ? 21 : BITS == 4 ? 16 : 12;
+    constexpr int kPad = 64 - kChars * BITS;
+    uint32_t acc[3] = { 0, 0, 0 }, any = 0;
+#pragma unroll
+    for (int i = 0; i < kChars; ++i) {
+        const uint32_t word = (uint32_t)(c.w[i / 8] >> (32 * ((i / 4) & 1)));
+        const uint32_t code = lut[(word >> (8 * (i & 3))) & 0xFFu];
+        any |= code;
+        acc[i / kPerWord] = (acc[i / kPerWord] << BITS) | code;
+    }
+    key64 k = ((key64)acc[0] << (64 - kPerWord * BITS)) | ((key64)acc[1] << (64 - 2 * kPerWord * BITS));
+    if (kChars > 2 * kPerWord) k |= (key64)acc[2] << kPad;
+    const uint32_t len = chars_before_nul(c);
+    if (any & 0x80u) {     // rare: an unknown character in the key or in what follows the string
+        k = 0;
+        for (int i = 0; i < kChars && i < (int)len; ++i) {
+            const uint64_t w = i < 8 ? c.w[0] : i < 16 ? c.w[1] : c.w[2];
+            const uint32_t code = lut[(uint32_t)(w >> (8 * (i & 7))) & 0xFFu];
+            if (code & 0x80u) *bad = true;
+            k |= (key64)(code & 0x1Fu) << (64 - (i + 1) * BITS);
+        }
+        return k;
+    }
+    if (len < (uint32_t)kChars) k = len ? k & (~0ull << (64 - len * BITS)) : 0ull;
+    return k;
+}
+__device__ __forceinline__ key64 pack_key_fmt(const Chars24& c, uint32_t fmt, const uint8_t* lut, bool* bad)
+{
+    return fmt == 1 ? pack_key<3>(c, lut, bad) : fmt == 2 ? pack_key<4>(c, lut, bad) : pack_key<5>(c, lut, bad);
+}
+
 // tid_x() through an opaque move: values derived from it are recomputed
 // where they are used, instead of being hoisted out of the persistent loops
 // of the kernels and holding registers across every iteration
@@ -181,6 +277,12 @@ __device__ __forceinline__ uint64_t match_bucket_lds(uint32_t b, uint64_t* tab, 
 }
 
 __device__ __forceinline__ void flag_error(uint32_t* cnt, uint32_t e) { atomicOr(&cnt[C_ERR], e); }
+
+// characters the strings of the round segment that starts at rbeg share
+__device__ __forceinline__ uint32_t seg_depth(const Bufs& B, uint32_t rbeg)
+{
+    return B.sdepth_in ? B.sdepth_in[rbeg] : 0u;
+}
 
 // byte offset of input string i in the arena
 __device__ __forceinline__ uint64_t str_off(const Bufs& B, uint32_t i)

@@ -8,11 +8,14 @@
 //   idx[2][n]  uint32 ping-pong: input index of the string at a position
 //   bktrank[n] uint32 scratch: (bucket << 21) | rank inside its wave chunk
 //   bkey[n]    uint64 scratch: depth key of the first/last position of a leaf
+//   sdepth[2][n] uint32 by round parity: characters the strings of the round
+//              segment starting at a position are known to share
 //   perm[n], lcp[n]  results (caller memory)
 //
-// A sort proceeds in rounds; round r compares the 8 characters at depth 8r.
+// A sort proceeds in rounds; a round compares one key (8 characters, or up to
+// 21 in round 0, see KeyFmt) of every string at the depth of its segment.
 // Inside a round, segments (contiguous position ranges whose strings share
-// their first 8r characters) are split by multi-workgroup splitter-tree steps
+// the characters before that depth) are split by multi-workgroup splitter-tree steps
 // until every piece is a leaf: a block (at most kBlkT strings, sorted
 // completely in LDS by one workgroup), a tiny leaf (at most 64 strings, one
 // wave) or an equal-key bucket.  Leaves finish their strings at this depth
@@ -70,6 +73,8 @@ struct Item {            // a segment or a leaf
 constexpr uint32_t F_BUFB = 1u;              // data lives in key[1]/idx[1]
 constexpr uint32_t F_SORTED = 2u;            // all keys equal (equal bucket)
 constexpr uint32_t F_IDENT = 4u;             // a root: idx[p] = p, not stored
+constexpr uint32_t kFmtShift = 3;            // (flags >> kFmtShift) & 3: format of the segment's keys (KeyFmt)
+constexpr uint32_t kFmtMask = 3u << kFmtShift;
 constexpr uint32_t kFlagShift = 8;           // flags >> kFlagShift: chunk index of an equal-key chunk
 
 // device counters
@@ -86,6 +91,25 @@ enum : int {
 };
 constexpr uint32_t ERR_CAP = 1u, ERR_LCP = 2u, ERR_BOUNDS = 4u;
 constexpr uint32_t ERR_LEVELS = 8u;          // a captured round had more levels than it was built with
+constexpr uint32_t ERR_ALPHA = 16u;          // a packed root holds a character outside the alphabet its samples showed
+constexpr uint32_t kLutBytes = 256;          // code table of one packed root
+
+// Formats of a key.  Format 0: 8 characters of 8 bits.  Formats 1..3: codes
+// of 3, 4 or 5 bits, 21, 16 or 12 characters (code 0 is the NUL, the
+// characters of the alphabet count up from 1 in byte order), left-aligned
+// with `pad` zero bits below.  All formats order like the strings.
+struct KeyFmt {
+    uint32_t mul;        // (bit index * mul) >> 8 = bit index / code bits, for bit indices below 64
+    uint32_t cpk;        // characters per key
+    uint32_t pad;        // unused low bits
+    uint32_t last;       // mask of the last character's code: zero there = the key holds a NUL
+};
+__host__ __device__ constexpr KeyFmt key_fmt(uint32_t flags)
+{
+    const uint32_t f = (flags & kFmtMask) >> kFmtShift;
+    return f == 0 ? KeyFmt{ 32, 8, 0, 0xFFu } : f == 1 ? KeyFmt{ 86, 21, 1, 7u << 1 }
+         : f == 2 ? KeyFmt{ 64, 16, 0, 15u } : KeyFmt{ 52, 12, 4, 31u << 4 };
+}
 
 struct LargeDesc {       // one segment of the multi-workgroup sample-sort step
     Item seg;
@@ -115,7 +139,7 @@ struct LevelHdr {        // totals of one level's multi-workgroup step
 // no pointer arithmetic on the host).
 struct Plan {
     const LevelHdr* hdr;
-    const LargeDesc* desc;
+    LargeDesc* desc;     // (k_tree records a root's key format in it)
     const TileRef* tiles;
 };
 
@@ -143,6 +167,9 @@ struct Bufs {
     uint32_t* bktrank;
     const uint32_t* pending;   // non-null and non-zero: large segments remain, the round's leaves wait
     uint32_t pending_err;      // ... and that is an error (ERR_LEVELS: a captured graph cannot continue the round)
+    const uint32_t* sdepth_in; // depths of this round's segments (null in round 0: depth 0)
+    uint32_t* sdepth_out;      // depths of the next round's segments
+    uint8_t* lut;              // code tables of packed roots, kLutBytes per large segment; null: every key has format 0
     uint32_t leaf_keys;        // keys (8 characters each) a leaf pass fetches per string at a time, 1..8
 };
 

@@ -268,13 +268,65 @@ __global__ __launch_bounds__(kBigWG) void k_plan(PlanArgs A, uint32_t* cnt)
 // oversample/2 + oversample*i (the reference's choice for oversample factor 2,
 // bingmann-sample_sort_tree_builder.hpp:44-58) and the tree is stored in
 // level order: trees[seg*2048 + t], t = 1..nspl, followed by the splitters in
-// sorted order at trees[seg*2048 + 1024 + i], i < nspl.  With from_arena (the root
-// of a sort whose keys are not extracted yet) the samples are read from the
+// sorted order at trees[seg*2048 + 1024 + i], i < nspl.  ROOT: the roots
+// of a sort, whose keys are not extracted yet; the samples are read from the
 // arena directly.
-__device__ __forceinline__ void tree_of_segment(const LargeDesc D, const Bufs& B, uint64_t seed, key64* tree,
-                                                int from_arena, key64* s_samp)
+//
+// A root's samples also choose the format of its keys (KeyFmt).  Eight
+// characters of a small alphabet leave many strings equal: 20 M windows of
+// ACGT text have 65536 different keys, and every equal run then gathers its
+// strings again.  When the samples say that a key would be shared by
+// kPackRun strings or more beside its own (d equal neighbours among s sorted
+// samples of n strings: 2 d n / s^2 strings for each key, one of them the
+// string itself, drawn twice) and the
+// characters of a second sample form an alphabet of at most 31, the root's
+// keys hold 21, 16 or 12 packed characters instead.  A character the sample
+// missed is found by the extraction (ERR_ALPHA) and the sort starts over
+// unpacked.
+// what a kernel of a level knows of its segments: no roots, roots with plain
+// keys, or roots that may pack theirs
+constexpr int kNoRoot = 0, kRootPlain = 1, kRootPack = 2;
+
+struct TreeLds {
+    key64 samp[kMaxSamples + 1];      // + 1: a merge step reads the slot after the one it takes
+    uint32_t alpha[8];                // characters of the sample
+    uint32_t dups;                    // equal neighbours among the sorted samples
+    uint8_t lut[kLutBytes];           // code table
+};
+constexpr float kPackRun = 1.0f;
+
+constexpr uint32_t kAlphaSamples = 256;
+
+// the alphabet of one string per thread, as a bitmap in S.alpha (cleared by the caller)
+__device__ __forceinline__ void sample_alphabet(const Item& seg, const Bufs& B, uint64_t seed, uint32_t* alpha)
 {
+    const uint64_t h = mix64(seed ^ 0xA1FABE7ull ^ ((uint64_t)seg.begin << 21) ^ ((uint64_t)tid_x() << 40));
+    const uint32_t pos = seg.begin + (uint32_t)(((h >> 32) * (uint64_t)seg.size) >> 32);
+    const Chars24 c = load_chars24(B.arena, B.alen, str_off(B, pos));
+    const uint32_t len = chars_before_nul(c);
+    uint32_t m[8] = {};
+#pragma unroll
+    for (int i = 0; i < 24; ++i) {
+        const uint32_t ch = (uint32_t)(c.w[i / 8] >> (8 * (i & 7))) & 0xFFu;
+        const uint32_t bit = (uint32_t)i < len ? 1u << (ch & 31) : 0u;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) m[j] |= (ch >> 5) == (uint32_t)j ? bit : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) m[j] |= (uint32_t)__shfl_xor((int)m[j], d, 64);
+        if (lane_id() == 0 && m[j]) atomicOr(&alpha[j], m[j]);
+    }
+}
+
+template <int ROOT>
+__device__ __forceinline__ void tree_of_segment(LargeDesc* Dp, uint32_t si, const Bufs& B, uint64_t seed, key64* tree,
+                                                TreeLds& S)
+{
+    const LargeDesc D = *Dp;
     const Item seg = D.seg;
+    key64* s_samp = S.samp;
     if (!item_ok(seg, B)) {
         if (tid_x() == 0) flag_error(B.cnt, ERR_BOUNDS);
         return;
@@ -296,79 +348,127 @@ __device__ __forceinline__ void tree_of_segment(const LargeDesc D, const Bufs& B
     constexpr int kPer = kMaxSamples / kBigWG;
     static_assert(kMaxSamples % kBigWG == 0 && kPer == 4, "four samples per thread");
     const uint32_t o = tid_x() * kPer;
+    const bool act = o < P;
+    constexpr bool may_pack = ROOT == kRootPack;
+    if (may_pack) {     // (cleared before the merge rounds' barriers)
+        if (tid_x() < 8) S.alpha[tid_x()] = 0;
+        if (tid_x() == 8) S.dups = 0;
+    }
+    auto sample = [&](uint32_t j) {
+        const uint64_t h = mix64(seed ^ ((uint64_t)seg.begin << 21) ^ (uint64_t)j);
+        return seg.begin + (uint32_t)(((h >> 32) * (uint64_t)seg.size) >> 32);
+    };
     key64 v[kPer];
 #pragma unroll
     for (int e = 0; e < kPer; ++e) {
-        const uint32_t j = o + e;
         v[e] = ~0ull;
-        if (j < ss) {
-            const uint64_t h = mix64(seed ^ ((uint64_t)seg.begin << 21) ^ (uint64_t)j);
-            const uint32_t pos = seg.begin + (uint32_t)(((h >> 32) * (uint64_t)seg.size) >> 32);
-            v[e] = from_arena ? load_key(B.arena, B.alen, str_off(B, pos)) : K[pos];
-        }
+        if (o + e < ss) v[e] = ROOT ? load_key(B.arena, B.alen, str_off(B, sample(o + e))) : K[sample(o + e)];
     }
-    const bool act = o < P;
-    if (act) {
-        constexpr int net[][2] = { { 0, 1 }, { 2, 3 }, { 0, 2 }, { 1, 3 }, { 1, 2 } };
-#pragma unroll
-        for (int c = 0; c < 5; ++c) {
-            const key64 x = v[net[c][0]], y = v[net[c][1]];
-            v[net[c][0]] = min(x, y);
-            v[net[c][1]] = max(x, y);
-        }
-#pragma unroll
-        for (int e = 0; e < kPer; ++e) s_samp[o + e] = v[e];
-    }
-    __syncthreads();
-    key64* sa = s_samp;
-    for (uint32_t L = kPer; L < P; L <<= 1) {
+    uint32_t fmt = 0;
+    for (;;) {
         if (act) {
-            const uint32_t a0 = (o / (2 * L)) * (2 * L), b0 = a0 + L, diag = o - a0;
-            uint32_t lo = diag > L ? diag - L : 0u, hi = min(diag, L);
-            while (lo < hi) {
-                const uint32_t mid = (lo + hi) >> 1;
-                if (sa[a0 + mid] <= sa[b0 + diag - 1 - mid]) lo = mid + 1;
-                else hi = mid;
-            }
-            // branch-free steps on byte offsets, as in the block sort: one
-            // read of the consumed run's next head (unused past the run's
-            // end; s_samp has one spare slot)
-            const unsigned char* sbase = reinterpret_cast<const unsigned char*>(sa);
-            uint32_t pa = (a0 + lo) * 8u, pb = (b0 + diag - lo) * 8u;
-            const uint32_t ea = (a0 + L) * 8u, eb = (b0 + L) * 8u;
-            key64 ka = pa < ea ? *reinterpret_cast<const key64*>(sbase + pa) : 0ull;
-            key64 kb = pb < eb ? *reinterpret_cast<const key64*>(sbase + pb) : 0ull;
+            constexpr int net[][2] = { { 0, 1 }, { 2, 3 }, { 0, 2 }, { 1, 3 }, { 1, 2 } };
 #pragma unroll
-            for (int e = 0; e < kPer; ++e) {
-                const bool take_a = pb >= eb || (pa < ea && ka <= kb);
-                const uint32_t src = take_a ? pa : pb;
-                v[e] = take_a ? ka : kb;
-                const key64 nx = *reinterpret_cast<const key64*>(sbase + src + 8u);
-                pa += take_a ? 8u : 0u;
-                pb += take_a ? 0u : 8u;
-                ka = take_a ? nx : ka;
-                kb = take_a ? kb : nx;
+            for (int c = 0; c < 5; ++c) {
+                const key64 x = v[net[c][0]], y = v[net[c][1]];
+                v[net[c][0]] = min(x, y);
+                v[net[c][1]] = max(x, y);
             }
+#pragma unroll
+            for (int e = 0; e < kPer; ++e) s_samp[o + e] = v[e];
         }
         __syncthreads();
-        if (act) {
+        for (uint32_t L = kPer; L < P; L <<= 1) {
+            if (act) {
+                const uint32_t a0 = (o / (2 * L)) * (2 * L), b0 = a0 + L, diag = o - a0;
+                uint32_t lo = diag > L ? diag - L : 0u, hi = min(diag, L);
+                while (lo < hi) {
+                    const uint32_t mid = (lo + hi) >> 1;
+                    if (s_samp[a0 + mid] <= s_samp[b0 + diag - 1 - mid]) lo = mid + 1;
+                    else hi = mid;
+                }
+                // branch-free steps on byte offsets, as in the block sort: one
+                // read of the consumed run's next head (unused past the run's
+                // end; s_samp has one spare slot)
+                const unsigned char* sbase = reinterpret_cast<const unsigned char*>(s_samp);
+                uint32_t pa = (a0 + lo) * 8u, pb = (b0 + diag - lo) * 8u;
+                const uint32_t ea = (a0 + L) * 8u, eb = (b0 + L) * 8u;
+                key64 ka = pa < ea ? *reinterpret_cast<const key64*>(sbase + pa) : 0ull;
+                key64 kb = pb < eb ? *reinterpret_cast<const key64*>(sbase + pb) : 0ull;
 #pragma unroll
-            for (int e = 0; e < kPer; ++e) sa[o + e] = v[e];
+                for (int e = 0; e < kPer; ++e) {
+                    const bool take_a = pb >= eb || (pa < ea && ka <= kb);
+                    const uint32_t src = take_a ? pa : pb;
+                    v[e] = take_a ? ka : kb;
+                    const key64 nx = *reinterpret_cast<const key64*>(sbase + src + 8u);
+                    pa += take_a ? 8u : 0u;
+                    pb += take_a ? 0u : 8u;
+                    ka = take_a ? nx : ka;
+                    kb = take_a ? kb : nx;
+                }
+            }
+            __syncthreads();
+            if (act) {
+#pragma unroll
+                for (int e = 0; e < kPer; ++e) s_samp[o + e] = v[e];
+            }
+            __syncthreads();
+        }
+        if (!may_pack || fmt) break;
+        uint32_t d = 0;
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) {
+            const uint32_t j = o + e;
+            if (j + 1 < ss) d += s_samp[j] == s_samp[j + 1] && (s_samp[j] & 0xFFull) != 0 ? 1u : 0u;
+        }
+        if (d) atomicAdd(&S.dups, d);
+        __syncthreads();
+        const uint32_t dups = S.dups;
+        if (dups < 16 || 2.0f * (float)dups * (float)seg.size < (1.0f + kPackRun) * (float)ss * (float)ss) break;     // (uniform)
+        if (tid_x() < kAlphaSamples) sample_alphabet(seg, B, seed, S.alpha);     // (whole waves)
+        __syncthreads();
+        uint32_t sigma = 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sigma += (uint32_t)__popc(S.alpha[j]);
+        fmt = sigma <= 7 ? 1u : sigma <= 15 ? 2u : sigma <= 31 ? 3u : 0u;
+        if (fmt == 0) break;     // (uniform)
+        if (tid_x() < kLutBytes) {
+            const uint32_t c = tid_x();
+            uint32_t rank = 1;
+            for (uint32_t j = 0; j < c / 32; ++j) rank += (uint32_t)__popc(S.alpha[j]);
+            rank += (uint32_t)__popc(S.alpha[c / 32] & ((1u << (c & 31)) - 1));
+            const uint32_t code = c == 0 ? 0u : (S.alpha[c / 32] >> (c & 31)) & 1u ? rank : 0x81u;
+            S.lut[c] = (uint8_t)code;
+            B.lut[(uint64_t)si * kLutBytes + c] = (uint8_t)code;
         }
         __syncthreads();
+        // the same samples with packed keys (a rolled loop: this code runs in
+        // few workgroups, where its size would cost more than its latency)
+        if (act) {
+#pragma unroll 1
+            for (uint32_t j = o; j < o + kPer; ++j) {
+                bool bad = false;     // (the extraction flags it; any splitters do)
+                s_samp[j] = j < ss ? pack_key_fmt(load_chars24(B.arena, B.alen, str_off(B, sample(j))), fmt, S.lut, &bad)
+                                   : ~0ull;
+            }
+#pragma unroll
+            for (int e = 0; e < kPer; ++e) v[e] = s_samp[o + e];
+        }
     }
-    const key64* sorted = sa;
+    if (fmt && tid_x() == 0) Dp->seg.flags = seg.flags | (fmt << kFmtShift);
+    const key64* sorted = s_samp;
     for (int t = tid_x() + 1; t <= nspl; t += kBigWG) tree[t] = sorted[a / 2 + a * inorder_of(t, k)];
     for (int i = tid_x(); i < nspl; i += kBigWG) tree[1024 + i] = sorted[a / 2 + a * i];
 }
 
-__global__ __launch_bounds__(kBigWG) void k_tree(Plan P, Bufs B, uint64_t seed, key64* trees, int from_arena)
+template <int ROOT>
+__global__ __launch_bounds__(kBigWG) void k_tree(Plan P, Bufs B, uint64_t seed, key64* trees)
 {
-    __shared__ key64 s_samp[kMaxSamples + 1];     // + 1: a merge step reads the slot after the one it takes
+    __shared__ TreeLds S;
     const uint32_t nlarge = P.hdr->nlarge;
     for (uint32_t si = blockIdx.x; si < nlarge; si += gridDim.x) {
         __syncthreads();     // the previous segment's samples are consumed
-        tree_of_segment(P.desc[si], B, seed, trees + (uint64_t)si * kTreeSlots, from_arena, s_samp);
+        tree_of_segment<ROOT>(P.desc + si, si, B, seed, trees + (uint64_t)si * kTreeSlots, S);
     }
 }
 
@@ -378,16 +478,18 @@ __global__ __launch_bounds__(kBigWG) void k_tree(Plan P, Bufs B, uint64_t seed, 
 // then tile, then wave -- the order of the reference's prefix sum
 // (.hpp:1437-1460) with wave chunks as the parts -- so an exclusive scan of
 // hist gives every chunk's base offset per bucket.  bktrank gets bucket and
-// rank inside the chunk.  With from_arena (the root of a sort, positions =
+// rank inside the chunk.  ROOT (the roots of a sort, positions =
 // input indices) the keys are extracted from the arena here and stored: this
 // replaces the separate extraction pass and saves reading the keys back.
 // The tree and the sorted splitters sit in static LDS (their addresses are
 // constants, so a descent step needs no address arithmetic); the per-wave
 // 16-bit counts[kWaves][2^(kmax+1)] in dynamic LDS, sized by the largest
-// tree of the level (kmax treebits).
+// tree of the level (kmax treebits); a packed root's code table takes their
+// place while its keys are extracted.
 __host__ __device__ constexpr uint32_t count_lds_bytes(int kmax)
 {
-    return kWaves * (2u << kmax) * 2u;
+    const uint32_t counts = kWaves * (2u << kmax) * 2u;
+    return counts > kLutBytes ? counts : kLutBytes;
 }
 
 // Load a read-only value that every lane of the wave reads at the same
@@ -414,9 +516,9 @@ __device__ __forceinline__ T load_uniform(const T* p)
 template <int NB>
 constexpr int kPeerBits = NB <= 10 ? (NB < 8 ? NB : 8) : 0;
 
-template <int NB>
+template <int NB, int ROOT>
 __device__ __forceinline__ void count_tile(uint32_t ti, const Plan& P, const Bufs& B, const key64* trees,
-                                           uint32_t* hist, int from_arena, int kmax, key64* s_tree, key64* s_sorted,
+                                           uint32_t* hist, int kmax, key64* s_tree, key64* s_sorted,
                                            uint16_t* s_hist_base, uint64_t* s_peer)
 {
     constexpr uint32_t kNoBkt = (1u << NB) - 1;   // id of inactive lanes, above every bucket of the launch
@@ -434,8 +536,6 @@ __device__ __forceinline__ void count_tile(uint32_t ti, const Plan& P, const Buf
     const int nspl = (1 << k) - 1;
     for (int i = tid_x(); i <= nspl; i += kWG) s_tree[i] = tree[i];
     for (int i = tid_x(); i < nspl; i += kWG) s_sorted[i] = tree[1024 + i];
-    for (uint32_t i = tid_x(); i < kWaves * nb2; i += kWG) s_hist_base[i] = 0;
-    __syncthreads();
     const key64* K = (seg.flags & F_BUFB) ? B.key1 : B.key0;
     const uint32_t t = tr.t;
     const uint32_t w = wave_id(), lane = lane_id();
@@ -445,13 +545,33 @@ __device__ __forceinline__ void count_tile(uint32_t ti, const Plan& P, const Buf
     const uint32_t cb = (t * kWaves + w) * D.chunk;
     const uint32_t cmax = (seg.flags & F_IDENT) ? kChunkMaxIdent : kChunkMax;
     const uint32_t ce = (item_ok(seg, B) && t < D.T && D.chunk <= cmax) ? min(seg.size, cb + D.chunk) : 0u;
+    const uint32_t fmt = ROOT == kRootPack ? (seg.flags & kFmtMask) >> kFmtShift : 0u;
+    const bool plain = ROOT && fmt == 0;     // (uniform)
+    if (fmt) {
+        // a packed root's keys are extracted first, in a loop of their own, and
+        // read back from the cache below: extracting them inside the main loop
+        // takes 116 registers instead of 72 (4 instead of 7 waves per SIMD)
+        uint8_t* s_lut = reinterpret_cast<uint8_t*>(s_hist_base);
+        static_assert(kLutBytes == kWG, "a table byte per thread");
+        s_lut[tid_x()] = B.lut[(uint64_t)tr.seg * kLutBytes + tid_x()];
+        __syncthreads();
+        bool bad = false;
+#pragma unroll 2
+        for (uint32_t p = cb + lane; p < ce; p += 64)
+            B.key0[seg.begin + p] =
+                pack_key_fmt(load_chars24(B.arena, B.alen, str_off(B, seg.begin + p)), fmt, s_lut, &bad);
+        if (bad) flag_error(B.cnt, ERR_ALPHA);
+        __syncthreads();     // the table is no longer read
+    }
+    for (uint32_t i = tid_x(); i < kWaves * nb2; i += kWG) s_hist_base[i] = 0;
+    __syncthreads();
     // kGroups 64-key groups per iteration: all loads are in flight before the
     // tree descents, then the groups are ranked in order (stable)
     constexpr int kGroups = 8;
     // extracting at the root, the string offsets of the next iteration are
     // loaded one iteration ahead (the first link of offset -> characters)
     uint64_t off_next[kGroups];
-    if (from_arena) {
+    if (plain) {
 #pragma unroll
         for (int j = 0; j < kGroups; ++j) {
             const uint32_t p = cb + 64 * j + lane;
@@ -460,7 +580,7 @@ __device__ __forceinline__ void count_tile(uint32_t ti, const Plan& P, const Buf
     }
     for (uint32_t g = cb; g < ce; g += 64 * kGroups) {
         key64 kv[kGroups];
-        if (from_arena) {
+        if (plain) {
             uint64_t off[kGroups];
 #pragma unroll
             for (int j = 0; j < kGroups; ++j) off[j] = off_next[j];
@@ -501,7 +621,7 @@ __device__ __forceinline__ void count_tile(uint32_t ti, const Plan& P, const Buf
                 B.bktrank[seg.begin + p] = (bv[j] << kRankBits) | (old + r);
             }
         }
-        if (from_arena) {     // the extracted keys, for the scatter
+        if (plain) {     // the extracted keys, for the scatter
 #pragma unroll
             for (int j = 0; j < kGroups; ++j) {
                 const uint32_t p = g + 64 * j + lane;
@@ -521,9 +641,8 @@ __device__ __forceinline__ void count_tile(uint32_t ti, const Plan& P, const Buf
 // multiple of kXcds), and XCD x takes the tiles [N x / kXcds, N (x+1) /
 // kXcds): one per workgroup, or with LOOP (levels planned on the device)
 // each workgroup loops over its XCD's share.
-template <int NB, bool LOOP>
-__global__ __launch_bounds__(kWG) void k_count(Plan P, Bufs B, const key64* trees, uint32_t* hist, int from_arena,
-                                                int kmax)
+template <int NB, bool LOOP, int ROOT>
+__global__ __launch_bounds__(kWG) void k_count(Plan P, Bufs B, const key64* trees, uint32_t* hist, int kmax)
 {
     static_assert(NB >= 2 && NB <= kMaxTreebits + 1, "bucket ids of up to 2047 buckets");
     static_assert(kChunkMax <= 65535 && kChunkMaxIdent <= 65535, "per-wave bucket counts must fit 16 bits");
@@ -538,12 +657,12 @@ __global__ __launch_bounds__(kWG) void k_count(Plan P, Bufs B, const key64* tree
     const uint32_t thi = (uint32_t)((uint64_t)N * (xcd + 1) / kXcds);
     uint32_t ti = (uint32_t)((uint64_t)N * xcd / kXcds) + blockIdx.x / kXcds;
     if (!LOOP) {
-        if (ti < thi) count_tile<NB>(ti, P, B, trees, hist, from_arena, kmax, s_tree, s_sorted, s_hist_base, s_peer);
+        if (ti < thi) count_tile<NB, ROOT>(ti, P, B, trees, hist, kmax, s_tree, s_sorted, s_hist_base, s_peer);
         return;
     }
     for (; ti < thi; ti += per) {
         __syncthreads();     // the previous tile's counts are written out
-        count_tile<NB>(ti, P, B, trees, hist, from_arena, kmax, s_tree, s_sorted, s_hist_base, s_peer);
+        count_tile<NB, ROOT>(ti, P, B, trees, hist, kmax, s_tree, s_sorted, s_hist_base, s_peer);
     }
 }
 
@@ -870,7 +989,8 @@ __device__ void emit_children(const Item& seg, int nbkt, const uint32_t* bstart,
                               const key64* spl, const Sink& s, uint32_t* s_tmp)
 {
     constexpr int kPer = (kMaxBkt + kWG - 1) / kWG;   // 8
-    const uint32_t dstbuf = (seg.flags & F_BUFB) ^ F_BUFB;
+    const uint32_t dstbuf = ((seg.flags & F_BUFB) ^ F_BUFB) | (seg.flags & kFmtMask);
+    const KeyFmt F = key_fmt(seg.flags);
     uint32_t c_t = 0, c_l = 0, c_r = 0, c_b[kBlkClasses] = {}, c_cont = 0;
     uint32_t st[kPer], sz[kPer];
 #pragma unroll
@@ -887,7 +1007,7 @@ __device__ void emit_children(const Item& seg, int nbkt, const uint32_t* bstart,
             if (m <= kTinyT) c_t++;
             else if (b & 1) {
                 c_r += (m + kRunChunk - 1) / kRunChunk;
-                if ((spl[b >> 1] & 0xFFull) != 0) c_cont++;
+                if (!key_ends(spl[b >> 1], F)) c_cont++;
             }
             else if (m <= kBlkT) c_b[block_class(m)]++;
             else c_l++;
@@ -965,19 +1085,19 @@ __global__ __launch_bounds__(kWG) void k_children(Plan P, const uint32_t* hscan,
 // Finish one sorted position at depth d: LCP with the predecessor when the
 // keys differ; inside a run of equal keys the LCP is known when the key holds
 // a NUL (fill_lcp with lcpKeyDepth, .hpp:1546-1547), otherwise the run moves
-// on to depth d+8 and the string's next key is gathered for round r+1.
+// on to the next depth and the string's next key is gathered for round r+1.
 __device__ __forceinline__ void finish_position(const Bufs& B, uint32_t pos, uint32_t id, key64 k, bool has_prev,
-                                                key64 pk, bool run_single, uint32_t depth)
+                                                key64 pk, bool run_single, uint32_t depth, KeyFmt F)
 {
     const bool eqp = has_prev && pk == k;
-    if (has_prev && !eqp && B.lcp) B.lcp[pos] = depth + lcp_key(pk, k);
-    const bool term = (k & 0xFFull) == 0;
+    if (has_prev && !eqp && B.lcp) B.lcp[pos] = depth + lcp_key(pk, k, F);
+    const bool term = key_ends(k, F);
     if (run_single || term) {
         B.perm[pos] = id;
-        if (eqp && B.lcp) B.lcp[pos] = depth + key_depth(k);
+        if (eqp && B.lcp) B.lcp[pos] = depth + key_depth(k, F);
     } else {
         B.idx0[pos] = id;
-        if (id < B.n) B.key0[pos] = load_key(B.arena, B.alen, str_off(B, id) + depth + 8);
+        if (id < B.n) B.key0[pos] = load_key(B.arena, B.alen, str_off(B, id) + depth + F.cpk);
         else flag_error(B.cnt, ERR_BOUNDS);
     }
 }
@@ -992,7 +1112,8 @@ __device__ __forceinline__ void wave_lds_sync()
 
 // One wave finishes a leaf of m <= 64 strings at positions [begin, begin+m)
 // completely: a rank sort by broadcast compares (the slot each string takes
-// in an LCP insertion sort, lcp_inssort.hpp:36-187) at depth `cur`, then,
+// in an LCP insertion sort, lcp_inssort.hpp:36-187) at depth `cur` (keys of
+// format F), then,
 // while runs of equal keys without a NUL remain, their strings fetch their
 // next 8 characters and every such run is re-sorted in place.  Runs never
 // leave the wave, so deep shared prefixes cost one gather per string per 8
@@ -1010,7 +1131,7 @@ __device__ __forceinline__ void wave_lds_sync()
 // NK: keys fetched per string at a time (1..8), or 0 for B.leaf_keys.
 template <int NK>
 __device__ void wave_finish_leaf(const Bufs& B, uint32_t pos, uint32_t m, key64 k, uint32_t id, uint32_t cur,
-                                 bool write_bkey, uint32_t run0, key64* s_k, uint32_t* s_i, uint32_t* s_r)
+                                 KeyFmt F, bool write_bkey, uint32_t run0, key64* s_k, uint32_t* s_i, uint32_t* s_r)
 {
     const uint32_t lane = lane_id();
     const bool act = lane < m;
@@ -1062,11 +1183,11 @@ __device__ void wave_finish_leaf(const Bufs& B, uint32_t pos, uint32_t m, key64 
             eqp = same_prev && pk == k;
             eqn = lane + 1 < m && s_r[lane + 1] == run && s_k[lane + 1] == k;
         }
-        const bool term = (k & 0xFFull) == 0;
+        const bool term = key_ends(k, F);
         if (act && live) {
             if (first_pass && (lane == 0 || lane == m - 1)) B.bkey[pos] = k;
-            if (same_prev && !eqp && B.lcp) B.lcp[pos] = cur + lcp_key(pk, k);
-            if (eqp && term && B.lcp) B.lcp[pos] = cur + key_depth(k);
+            if (same_prev && !eqp && B.lcp) B.lcp[pos] = cur + lcp_key(pk, k, F);
+            if (eqp && term && B.lcp) B.lcp[pos] = cur + key_depth(k, F);
             if ((!eqp && !eqn) || term) {
                 B.perm[pos] = id;     // decided: a single string or identical strings
                 live = false;
@@ -1088,7 +1209,8 @@ __device__ void wave_finish_leaf(const Bufs& B, uint32_t pos, uint32_t m, key64 
         // to the string it was loaded for (bid); when a re-sort moved any
         // string to another lane, the wave loads afresh.
         first_pass = false;
-        cur += 8;
+        cur += F.cpk;
+        F = key_fmt(0);      // (what is fetched here is plain characters)
         if (nbuf == 0 || __ballot(live && id != bid) != 0) {     // (uniform)
             if (live) {
                 if (id < B.n) load_keys<kLeafKeys>(B.arena, B.alen, str_off(B, id) + cur, kbuf, nk);
@@ -1126,7 +1248,7 @@ __device__ void wave_finish_leaf(const Bufs& B, uint32_t pos, uint32_t m, key64 
 // One wave per tiny leaf (at most 64 strings), finished completely.
 template <int NK>
 __global__ __launch_bounds__(kWG) void k_leaf_tiny(const Item* items, const uint32_t* cnt_items, uint32_t cap,
-                                                   Bufs B, uint32_t depth)
+                                                   Bufs B)
 {
     __shared__ key64 s_k[kWaves][64];
     __shared__ uint32_t s_i[kWaves][64];
@@ -1143,6 +1265,7 @@ __global__ __launch_bounds__(kWG) void k_leaf_tiny(const Item* items, const uint
         L.begin = (uint32_t)__builtin_amdgcn_readfirstlane((int)L.begin);
         L.size = (uint32_t)__builtin_amdgcn_readfirstlane((int)L.size);
         L.flags = (uint32_t)__builtin_amdgcn_readfirstlane((int)L.flags);
+        L.rbeg = (uint32_t)__builtin_amdgcn_readfirstlane((int)L.rbeg);
         if (!item_ok(L, B) || L.size > kTinyT) {
             if (lane == 0) flag_error(B.cnt, ERR_BOUNDS);
             continue;      // (wave-uniform)
@@ -1155,7 +1278,8 @@ __global__ __launch_bounds__(kWG) void k_leaf_tiny(const Item* items, const uint
             k = src ? B.key1[L.begin + lane] : B.key0[L.begin + lane];
             id = (L.flags & F_IDENT) ? L.begin + lane : src ? B.idx1[L.begin + lane] : B.idx0[L.begin + lane];
         }
-        wave_finish_leaf<NK>(B, L.begin + lane, m, k, id, depth, true, 0u, s_k[w], s_i[w], s_r[w]);
+        wave_finish_leaf<NK>(B, L.begin + lane, m, k, id, seg_depth(B, L.rbeg), key_fmt(L.flags), true, 0u, s_k[w],
+                             s_i[w], s_r[w]);
     }
 }
 
@@ -1198,7 +1322,7 @@ struct TailStack {
 constexpr int kBlkE0 = 4, kBlkE1 = 4, kBlkE2 = 4, kBlkE3 = 4;
 
 // Finish a block's short runs of equal keys (each at most 64 strings, at
-// sorted positions beg + (s_runs[r] >> 16)) at depth + 8: the runs are
+// sorted positions beg + (s_runs[r] >> 16)) at depth, the block's next one: the runs are
 // packed into batches of at most 64 strings, and a wave finishes all runs of
 // a batch in one pass (duplicates come in many short runs).  The batch
 // table lives in s_k after the waves' leaf arrays.
@@ -1253,7 +1377,7 @@ __device__ __forceinline__ void block_finish_runs(const Bufs& B, key64* s_k, con
             kk = B.key0[pos];
             id = B.idx0[pos];
         }
-        wave_finish_leaf<NK>(B, pos, total, kk, id, depth + 8, false, slot0, wk, wi, wr);
+        wave_finish_leaf<NK>(B, pos, total, kk, id, depth, key_fmt(0), false, slot0, wk, wi, wr);
     }
 }
 
@@ -1593,6 +1717,7 @@ __device__ __forceinline__ void block_one(const Item L, const Bufs& B, const Sin
     const key64* K = src ? B.key1 : B.key0;
     const uint32_t* I = src ? B.idx1 : B.idx0;
     const bool ident = L.flags & F_IDENT;
+    const KeyFmt F = key_fmt(L.flags);
     if (tid == 0) s_nruns = 0;
     // the block's input indices are loaded beside its keys and kept in
     // registers through the sort, then staged in s_cnt (free after either
@@ -1637,14 +1762,14 @@ __device__ __forceinline__ void block_one(const Item L, const Bufs& B, const Sin
             if (i > 0) pk = s_k[i - 1];
             eqp = i > 0 && pk == kk;
             eqn = i + 1 < m && s_k[i + 1] == kk;
-            finish_position(B, beg + i, ids[e], kk, i > 0, pk, !eqp && !eqn, depth);
+            finish_position(B, beg + i, ids[e], kk, i > 0, pk, !eqp && !eqn, depth, F);
             if (top && (i == 0 || i == m - 1)) B.bkey[beg + i] = kk;
         }
-        // a run of equal keys without a NUL continues at depth + 8 (its keys
+        // a run of equal keys without a NUL continues at the next depth (its keys
         // there are in place, finish_position fetched them): a run of at most
         // kTinyT strings is finished below by this workgroup, a longer one is
         // a segment of the next round
-        const bool nr = act && !eqp && eqn && (kk & 0xFFull) != 0;
+        const bool nr = act && !eqp && eqn && !key_ends(kk, F);
         if (__ballot(nr) == 0) continue;     // (uniform) nothing to append in this wave
         uint32_t rl = 0;
         if (nr) {     // the run's last position: binary search in the sorted keys
@@ -1666,20 +1791,21 @@ __device__ __forceinline__ void block_one(const Item L, const Bufs& B, const Sin
                 if (t < kTailStack) {
                     ts->pos[t] = beg + i;
                     ts->len[t] = rl;
-                    ts->depth[t] = depth + 8;
+                    ts->depth[t] = depth + F.cpk;
                 } else {
                     flag_error(B.cnt, ERR_BOUNDS);     // (pending runs are disjoint: cannot happen)
                 }
             }
         } else {
             Item ni = { beg + i, rl, beg + i, 0u };
+            if (nr && !keep) B.sdepth_out[beg + i] = depth + F.cpk;
             wave_append_segment(nr && !keep, ni, nxt);
         }
     }
     __syncthreads();     // the runs' keys and indices written above are visible to the whole group
     const uint32_t nruns = min(s_nruns, kMaxRuns);
     for (uint32_t r0 = 0; r0 < nruns; r0 += kBlockRuns) {     // (uniform) batches of at most kBlockRuns runs
-        block_finish_runs<NK>(B, s_k, s_runs + r0, min(kBlockRuns, nruns - r0), beg, depth, T / 64);
+        block_finish_runs<NK>(B, s_k, s_runs + r0, min(kBlockRuns, nruns - r0), beg, depth + F.cpk, T / 64);
         if (TAIL) __syncthreads();     // the next batch reuses the batch table
     }
 }
@@ -1696,7 +1822,7 @@ __device__ __forceinline__ void block_one(const Item L, const Bufs& B, const Sin
 template <uint32_t MAXM, int E, bool LOOP, int NK, bool TAIL>
 __global__ __launch_bounds__(MAXM / E) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_block(const Item* items, uint32_t first, uint32_t last,
                                                      const uint32_t* p_first, const uint32_t* cnt_items, uint32_t cap,
-                                                     Bufs B, Sink nxt, uint32_t depth)
+                                                     Bufs B, Sink nxt)
 {
     __shared__ BlockLds<MAXM, E, TAIL> S;
     if constexpr (TAIL) {
@@ -1709,7 +1835,7 @@ __global__ __launch_bounds__(MAXM / E) __attribute__((amdgpu_waves_per_eu(8, 8))
         // a malformed item: the count is stored before a barrier each time)
         __syncthreads();
         Item cur = items[idx];
-        uint32_t d = depth;
+        uint32_t d = seg_depth(B, cur.rbeg);
         for (bool top = true;; top = false) {     // one call site, so that block_one stays inline
             block_one<MAXM, E, NK, true>(cur, B, nxt, d, S, &ts, top);
             // (the pushes precede a barrier in block_one's finish pass)
@@ -1724,19 +1850,21 @@ __global__ __launch_bounds__(MAXM / E) __attribute__((amdgpu_waves_per_eu(8, 8))
     } else if constexpr (!LOOP) {
         const uint32_t idx = first + blockIdx.x;
         if (idx >= min(last, cap)) return;
-        block_one<MAXM, E, NK, false>(items[idx], B, nxt, depth, S, nullptr, true);
+        const Item L = items[idx];
+        block_one<MAXM, E, NK, false>(L, B, nxt, seg_depth(B, L.rbeg), S, nullptr, true);
     } else {
         const uint32_t lo = *p_first, hi = min(*cnt_items, cap);
         for (uint32_t idx = lo + blockIdx.x; idx < hi; idx += gridDim.x) {
             __syncthreads();     // the previous block's LDS is no longer read
-            block_one<MAXM, E, NK, false>(items[idx], B, nxt, depth, S, nullptr, true);
+            const Item L = items[idx];
+            block_one<MAXM, E, NK, false>(L, B, nxt, seg_depth(B, L.rbeg), S, nullptr, true);
         }
     }
 }
 
 // One workgroup per chunk of an equal-key leaf (all keys equal).
 __global__ __launch_bounds__(kWG) void k_leaf_run(const Item* items, const uint32_t* cnt_items, uint32_t cap,
-                                                  Bufs B, Sink nxt, uint32_t depth)
+                                                  Bufs B, Sink nxt)
 {
     if (B.pending && *B.pending) {      // the round's levels are not finished
         if (B.pending_err && tid_x() == 0) flag_error(B.cnt, ERR_LEVELS);
@@ -1759,22 +1887,25 @@ __global__ __launch_bounds__(kWG) void k_leaf_run(const Item* items, const uint3
         const uint32_t ce = min(rend, cb + kRunChunk);
         const key64 key = K[cb];    // this chunk's own copy of the run key
         __syncthreads();
-        const bool term = (key & 0xFFull) == 0;
+        const KeyFmt F = key_fmt(L.flags);
+        const uint32_t depth = seg_depth(B, L.rbeg);
+        const bool term = key_ends(key, F);
         const bool single = L.size == 1;
         for (uint32_t p = cb + tid_x(); p < ce; p += kWG) {
             const uint32_t id = (L.flags & F_IDENT) ? p : I[p];
             if (single || term) {
                 B.perm[p] = id;
-                if (p > L.begin && B.lcp) B.lcp[p] = depth + key_depth(key);
+                if (p > L.begin && B.lcp) B.lcp[p] = depth + key_depth(key, F);
             } else {
                 if (src || (L.flags & F_IDENT)) B.idx0[p] = id;
-                if (id < B.n) B.key0[p] = load_key(B.arena, B.alen, str_off(B, id) + depth + 8);
+                if (id < B.n) B.key0[p] = load_key(B.arena, B.alen, str_off(B, id) + depth + F.cpk);
                 else flag_error(B.cnt, ERR_BOUNDS);
             }
         }
         if (tid_x() < 64) {
             const bool nr = tid_x() == 0 && c == 0 && !term && !single;
             Item ni = { L.begin, L.size, L.begin, 0u };
+            if (nr) B.sdepth_out[L.begin] = depth + F.cpk;
             wave_append_segment(nr, ni, nxt);
             if (tid_x() == 0) {
                 if (c == 0) B.bkey[L.begin] = key;
@@ -1793,7 +1924,7 @@ struct LeafLists {        // the leaf lists of a round, concatenated in this ord
     uint32_t cap[kBlkClasses + 2];       // their capacities (an overflow has been flagged)
 };
 
-__global__ __launch_bounds__(kWG) void k_leafbound(LeafLists LL, Bufs B, uint32_t depth)
+__global__ __launch_bounds__(kWG) void k_leafbound(LeafLists LL, Bufs B)
 {
     constexpr int NL = kBlkClasses + 2;
     if (B.pending && *B.pending) {      // the round's levels are not finished
@@ -1814,7 +1945,7 @@ __global__ __launch_bounds__(kWG) void k_leafbound(LeafLists LL, Bufs B, uint32_
         if (L.begin >= B.n) { flag_error(B.cnt, ERR_BOUNDS); continue; }
         const key64 a = B.bkey[L.begin - 1], c = B.bkey[L.begin];
         if (a == c) { flag_error(B.cnt, ERR_LCP); continue; }
-        B.lcp[L.begin] = depth + lcp_key(a, c);
+        B.lcp[L.begin] = seg_depth(B, L.rbeg) + lcp_key(a, c, key_fmt(L.flags));
     }
 }
 
@@ -2209,6 +2340,7 @@ struct WorkBuffers {
     uint32_t* idx[2] = { nullptr, nullptr };
     key64* bkey = nullptr;
     uint32_t* bktrank = nullptr;
+    uint32_t* sdepth[2] = { nullptr, nullptr };
     // large segments: first level of a round [round parity], later levels [level parity]
     Item* l_round[2] = { nullptr, nullptr };
     Item* l_lvl[2] = { nullptr, nullptr };
@@ -2226,6 +2358,7 @@ struct WorkBuffers {
     uint64_t tiles_cap = 0;
     key64* trees = nullptr;          // kTreeSlots splitter slots per large segment
     uint64_t trees_cap = 0;
+    uint8_t* lut = nullptr;          // kLutBytes per large segment (trees_cap of them)
     uint32_t* hist = nullptr;
     uint64_t hist_cap = 0;
     uint32_t* part = nullptr;
@@ -2253,7 +2386,7 @@ Plan plan_view(const unsigned char* base, uint64_t cap)
 {
     Plan P;
     P.hdr = reinterpret_cast<const LevelHdr*>(base);
-    P.desc = reinterpret_cast<const LargeDesc*>(base + sizeof(LevelHdr));
+    P.desc = reinterpret_cast<LargeDesc*>(const_cast<unsigned char*>(base) + sizeof(LevelHdr));
     P.tiles = reinterpret_cast<const TileRef*>(base + plan_tiles_off(cap));
     return P;
 }
@@ -2338,13 +2471,15 @@ void free_buffers(ps5_ctx* c)
     auto f = [](void* p) { if (p) (void)hipFree(p); };
     for (int i = 0; i < 2; ++i) {
         f(c->w.key[i]); f(c->w.idx[i]); f(c->w.l_round[i]); f(c->w.l_lvl[i]);
-        f(c->w.l_tiny[i]); f(c->w.l_block[i]); f(c->w.l_run[i]);
+        f(c->w.l_tiny[i]); f(c->w.l_block[i]); f(c->w.l_run[i]); f(c->w.sdepth[i]);
         c->w.key[i] = nullptr; c->w.idx[i] = nullptr; c->w.l_round[i] = nullptr; c->w.l_lvl[i] = nullptr;
         c->w.l_tiny[i] = nullptr; c->w.l_block[i] = nullptr; c->w.l_run[i] = nullptr;
+        c->w.sdepth[i] = nullptr;
     }
-    f(c->w.bkey); f(c->w.bktrank); f(c->w.hist); f(c->w.part); f(c->w.trees); f(c->w.d_plan);
+    f(c->w.bkey); f(c->w.bktrank); f(c->w.hist); f(c->w.part); f(c->w.trees); f(c->w.lut); f(c->w.d_plan);
     c->w.bkey = nullptr; c->w.bktrank = nullptr; c->w.hist = nullptr; c->w.part = nullptr; c->w.trees = nullptr;
     c->w.d_plan = nullptr;
+    c->w.lut = nullptr;
     if (c->w.h_large) (void)hipHostFree(c->w.h_large);
     if (c->w.h_plan) (void)hipHostFree(c->w.h_plan);
     c->w.h_large = nullptr; c->w.h_plan = nullptr; c->w.h_plan_dev = nullptr;
@@ -2366,10 +2501,13 @@ int grow_level(ps5_ctx* c, uint32_t nlarge, uint64_t hl)
                        (unsigned long long)c->w.hist_cap);
     if (nlarge > c->w.trees_cap) {
         if (c->w.trees) (void)hipFree(c->w.trees);
+        if (c->w.lut) (void)hipFree(c->w.lut);
         c->w.trees = nullptr;
+        c->w.lut = nullptr;
         c->w.trees_cap = 0;
         const uint64_t want = std::max<uint64_t>(nlarge + nlarge / 2, 64);
         HIPCHK(hipMalloc(&c->w.trees, want * kTreeSlots * sizeof(key64)));
+        HIPCHK(hipMalloc(&c->w.lut, want * kLutBytes));
         c->w.trees_cap = want;
         c->w_gen++;
     }
@@ -2405,6 +2543,7 @@ int ensure_capacity(ps5_ctx* c, uint64_t n)
     }
     HIPCHK(hipMalloc(&c->w.bkey, cap * sizeof(key64)));
     HIPCHK(hipMalloc(&c->w.bktrank, cap * sizeof(uint32_t)));
+    for (int i = 0; i < 2; ++i) HIPCHK(hipMalloc(&c->w.sdepth[i], cap * sizeof(uint32_t)));
     c->w.cap_large = cap_large_of(cap);
     c->w.cap_block = cap_block_of(cap);
     c->w.cap_tiny = cap_tiny_of(cap);
@@ -2446,7 +2585,7 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 // times at most m/8192 + 1 tiles of kWaves chunks, so cap + cap/4 entries
 // cover a level; a level needs at most cap_large trees.
 struct ScratchLayout {
-    uint64_t key[2], idx[2], bkey, bktrank, l_round[2], l_lvl[2], l_tiny[2], l_block[2], l_run[2];
+    uint64_t key[2], idx[2], bkey, bktrank, sdepth[2], lut, l_round[2], l_lvl[2], l_tiny[2], l_block[2], l_run[2];
     uint64_t desc, trees, hist, part, total;
     uint64_t trees_cap, hist_cap, part_cap;
 };
@@ -2463,6 +2602,7 @@ constexpr ScratchLayout scratch_layout(uint64_t cap)
     }
     L.bkey = take(cap * sizeof(key64));
     L.bktrank = take(cap * sizeof(uint32_t));
+    for (int i = 0; i < 2; ++i) L.sdepth[i] = take(cap * sizeof(uint32_t));
     for (int i = 0; i < 2; ++i) {
         L.l_round[i] = take(cl * sizeof(Item));
         L.l_lvl[i] = take(cl * sizeof(Item));
@@ -2473,6 +2613,7 @@ constexpr ScratchLayout scratch_layout(uint64_t cap)
     L.desc = take(plan_bytes_of(cap));
     L.trees_cap = cl;
     L.trees = take(L.trees_cap * kTreeSlots * sizeof(key64));
+    L.lut = take(L.trees_cap * kLutBytes);
     L.hist_cap = cap + cap / 4 + 64;
     L.hist = take(L.hist_cap * sizeof(uint32_t));
     L.part_cap = L.hist_cap / kScanBlock + 2;
@@ -2529,6 +2670,7 @@ WorkBuffers scratch_buffers(unsigned char* base, Item* h_large, unsigned char* h
         w.l_tiny[i] = reinterpret_cast<Item*>(base + L.l_tiny[i]);
         w.l_block[i] = reinterpret_cast<Item*>(base + L.l_block[i]);
         w.l_run[i] = reinterpret_cast<Item*>(base + L.l_run[i]);
+        w.sdepth[i] = reinterpret_cast<uint32_t*>(base + L.sdepth[i]);
     }
     w.bkey = reinterpret_cast<key64*>(base + L.bkey);
     w.bktrank = reinterpret_cast<uint32_t*>(base + L.bktrank);
@@ -2543,6 +2685,7 @@ WorkBuffers scratch_buffers(unsigned char* base, Item* h_large, unsigned char* h
     w.tiles_cap = tiles_cap_of(cap);
     w.trees = reinterpret_cast<key64*>(base + L.trees);
     w.trees_cap = L.trees_cap;
+    w.lut = base + L.lut;
     w.hist = reinterpret_cast<uint32_t*>(base + L.hist);
     w.hist_cap = L.hist_cap;
     w.part = reinterpret_cast<uint32_t*>(base + L.part);
@@ -2637,6 +2780,10 @@ int wait_stage(ps5_ctx* c, uint32_t seq)
     }
 }
 
+// (not a status of the ABI) the sort's packed keys met a character outside
+// their alphabet: run_sort starts over with plain keys
+constexpr int kUnpack = -1;
+
 int readback(ps5_ctx* c, const Item* list, int ci)
 {
     // one staged copy holds the counters and the head of the list
@@ -2648,6 +2795,7 @@ int readback(ps5_ctx* c, const Item* list, int ci)
     if (rc) return rc;
     c->st_syncs++;
     memcpy(c->h_cnt, c->h_stage, C_NCNT * sizeof(uint32_t));
+    if (c->h_cnt[C_ERR] & ERR_ALPHA) return kUnpack;
     if (c->h_cnt[C_ERR] & ERR_CAP) return set_err(PS5_ERR_CAPACITY, "work list capacity exceeded");
     if (c->h_cnt[C_ERR] & ERR_LCP) return set_err(PS5_ERR_INTERNAL, "equal keys across a leaf boundary");
     if (c->h_cnt[C_ERR] & ERR_BOUNDS) return set_err(PS5_ERR_INTERNAL, "device bounds check failed");
@@ -2686,6 +2834,12 @@ int large_treebits(uint32_t m, uint32_t target, int maxbits)
     return std::max(1, std::min(maxbits, k));
 }
 
+void launch_tree(ps5_ctx* c, const Bufs& B, Plan P, uint32_t grid, uint64_t seed, bool from_arena)
+{
+    const auto f = !from_arena ? k_tree<kNoRoot> : B.lut ? k_tree<kRootPack> : k_tree<kRootPlain>;
+    hipLaunchKernelGGL(f, dim3(grid), dim3(kBigWG), 0, c->stream, P, B, seed, c->w.trees);
+}
+
 // k_count instance for bucket ids of NB = kmax + 1 bits (at least 8)
 void launch_count(ps5_ctx* c, const Bufs& B, Plan P, dim3 g, int kmax, bool from_arena, bool loop)
 {
@@ -2694,12 +2848,10 @@ void launch_count(ps5_ctx* c, const Bufs& B, Plan P, dim3 g, int kmax, bool from
     const uint32_t lds = count_lds_bytes(kmax);
 #define PS5_COUNT_LAUNCH(NB)                                                                                          \
     do {                                                                                                              \
-        if (loop)                                                                                                     \
-            hipLaunchKernelGGL((k_count<NB, true>), g, b, lds, st, P, B, c->w.trees, c->w.hist, (int)from_arena,      \
-                               kmax);                                                                                 \
-        else                                                                                                          \
-            hipLaunchKernelGGL((k_count<NB, false>), g, b, lds, st, P, B, c->w.trees, c->w.hist, (int)from_arena,     \
-                               kmax);                                                                                 \
+        const auto f = !from_arena ? (loop ? k_count<NB, true, kNoRoot> : k_count<NB, false, kNoRoot>)                \
+                       : B.lut ? (loop ? k_count<NB, true, kRootPack> : k_count<NB, false, kRootPack>)                \
+                               : (loop ? k_count<NB, true, kRootPlain> : k_count<NB, false, kRootPlain>);             \
+        hipLaunchKernelGGL(f, g, b, lds, st, P, B, c->w.trees, c->w.hist, kmax);                                      \
     } while (0)
     if (kmax <= 7) PS5_COUNT_LAUNCH(8);
     else if (kmax == 8) PS5_COUNT_LAUNCH(9);
@@ -2769,7 +2921,7 @@ int large_step(ps5_ctx* c, const Bufs& B, uint32_t nlarge, const Sink& sink, uin
     const uint32_t hl32 = (uint32_t)hl;
     {
         Launch L(c, K_TREE, (uint64_t)nlarge * kMaxSamples * 8);
-        hipLaunchKernelGGL(k_tree, dim3(nlarge), dim3(kBigWG), 0, st, P, B, seed, c->w.trees, (int)from_arena);
+        launch_tree(c, B, P, nlarge, seed, from_arena);
     }
     {
         // key 8 R + bktrank 4 W; extracting at the root: offs 4 R + 8 characters R + key 8 W + bktrank 4 W
@@ -2868,6 +3020,13 @@ int setup_roots(ps5_ctx* c, uint32_t n, const uint64_t* set_first, uint32_t nset
 
 constexpr uint32_t kMaxGraphRounds = 64;      // rounds one captured graph may hold
 constexpr uint32_t kForkLeafGroups = 8192;    // leaf workgroups worth a side stream
+// Strings of the largest root from which on roots may pack their keys.  The
+// kernels that can pack take about 11 us more (digits, which do not pack,
+// 0.5 M strings: 221 -> 233 us), and smaller roots of a small alphabet have
+// little to gain (40 K strings of ACGT: 161 us plain, 171 packed); 4 M
+// suffixes of ACGT text take 1.36 ms against 1.58, 20 M windows 1.94 against
+// 2.88, a batch of 192 sets (a third of them ACGT) 3.01 against 3.24.
+constexpr uint64_t kPackMin = 1u << 20;
 constexpr uint64_t kChainMin = 1u << 22;       // strings of a level whose successor is chained on the device
 // Automatic planning plans a single sort of fewer strings on the device.
 // From about 4 M strings on the device plan's bounded grids cost more than
@@ -2901,7 +3060,7 @@ uint32_t block_grid_full(const ps5_ctx* c, int cls)
 // first + count) (or, with dev_first, from the device counter C_BDONE + cls
 // to the list's count), `grid` workgroups.
 void launch_block_class(ps5_ctx* c, const Bufs& B, int rp, int cls, uint32_t first, uint32_t count, bool dev_first,
-                        uint32_t grid, const Sink& nsink, uint32_t depth, bool tail = false, int flags = 0)
+                        uint32_t grid, const Sink& nsink, bool tail = false, int flags = 0)
 {
     const uint32_t last = first + count;
     hipStream_t st = c->stream;
@@ -2915,10 +3074,10 @@ void launch_block_class(ps5_ctx* c, const Bufs& B, int rp, int cls, uint32_t fir
     do {                                                                                                           \
         if (c->leaf_keys == 8)                                                                                     \
             hipExtLaunchKernelGGL((k_block<M, E, LOOP, 8, TAIL>), dim3(grid), dim3(M / E), 0, st, nullptr, nullptr, \
-                                  flags, list, first, last, pf, cnt, cap, B, nsink, depth);                          \
+                                  flags, list, first, last, pf, cnt, cap, B, nsink);                                 \
         else                                                                                                       \
             hipExtLaunchKernelGGL((k_block<M, E, LOOP, 0, TAIL>), dim3(grid), dim3(M / E), 0, st, nullptr, nullptr, \
-                                  flags, list, first, last, pf, cnt, cap, B, nsink, depth);                          \
+                                  flags, list, first, last, pf, cnt, cap, B, nsink);                                 \
     } while (0)
     if (dev_first) {
         if (cls == 0) PS5_BLOCK_LAUNCH(256, kBlkE0, true, false);
@@ -2941,18 +3100,18 @@ void launch_block_class(ps5_ctx* c, const Bufs& B, int rp, int cls, uint32_t fir
 
 // Tiny leaves and equal-key chunks of round parity rp on stream s (grids of
 // g_tiny and g_run workgroups; 0 skips a list).
-void launch_leaves(ps5_ctx* c, const Bufs& B, int rp, const Sink& nsink, uint32_t depth, uint32_t g_tiny,
-                   uint32_t g_run, uint64_t n_tiny, uint64_t n_run, hipStream_t s, int flags = 0)
+void launch_leaves(ps5_ctx* c, const Bufs& B, int rp, const Sink& nsink, uint32_t g_tiny, uint32_t g_run,
+                   uint64_t n_tiny, uint64_t n_run, hipStream_t s, int flags = 0)
 {
     if (g_tiny) {
         {
             Launch L(c, K_LEAF_TINY, 0);
             if (c->leaf_keys == 8)
                 hipExtLaunchKernelGGL(k_leaf_tiny<8>, dim3(g_tiny), dim3(kWG), 0, s, nullptr, nullptr, flags,
-                                      c->w.l_tiny[rp], c->d_cnt + C_TINY + rp, c->w.cap_tiny, B, depth);
+                                      c->w.l_tiny[rp], c->d_cnt + C_TINY + rp, c->w.cap_tiny, B);
             else
                 hipExtLaunchKernelGGL(k_leaf_tiny<0>, dim3(g_tiny), dim3(kWG), 0, s, nullptr, nullptr, flags,
-                                      c->w.l_tiny[rp], c->d_cnt + C_TINY + rp, c->w.cap_tiny, B, depth);
+                                      c->w.l_tiny[rp], c->d_cnt + C_TINY + rp, c->w.cap_tiny, B);
         }
         sum_sizes(c, c->w.l_tiny[rp], 0, c->d_cnt + C_TINY + rp, (uint32_t)n_tiny, S_TINY);
     }
@@ -2960,14 +3119,14 @@ void launch_leaves(ps5_ctx* c, const Bufs& B, int rp, const Sink& nsink, uint32_
         {
             Launch L(c, K_LEAF_RUN, 0);
             hipExtLaunchKernelGGL(k_leaf_run, dim3(g_run), dim3(kWG), 0, s, nullptr, nullptr, flags, c->w.l_run[rp],
-                                  c->d_cnt + C_RUN + rp, c->w.cap_run, B, nsink, depth);
+                                  c->d_cnt + C_RUN + rp, c->w.cap_run, B, nsink);
         }
         sum_sizes(c, c->w.l_run[rp], 0, c->d_cnt + C_RUN + rp, (uint32_t)n_run, S_RUN);
     }
 }
 
 // LCPs between neighbouring leaves of round parity rp (grid workgroups).
-void launch_leafbound(ps5_ctx* c, const Bufs& B, int rp, uint32_t depth, uint32_t grid, uint64_t nleaves)
+void launch_leafbound(ps5_ctx* c, const Bufs& B, int rp, uint32_t grid, uint64_t nleaves)
 {
     Launch L(c, K_LEAFBOUND, nleaves * 36);
     LeafLists LL;
@@ -2982,7 +3141,7 @@ void launch_leafbound(ps5_ctx* c, const Bufs& B, int rp, uint32_t depth, uint32_
     LL.list[kBlkClasses + 1] = c->w.l_run[rp];
     LL.cnt[kBlkClasses + 1] = C_RUN + rp;
     LL.cap[kBlkClasses + 1] = c->w.cap_run;
-    hipLaunchKernelGGL(k_leafbound, dim3(grid), dim3(kWG), 0, c->stream, LL, B, depth);
+    hipLaunchKernelGGL(k_leafbound, dim3(grid), dim3(kWG), 0, c->stream, LL, B);
 }
 
 // One level planned on the device: k_plan turns the large list `list`
@@ -3019,8 +3178,7 @@ void dev_level(ps5_ctx* c, const Bufs& B, const Item* list, int ci, uint32_t bou
     const uint32_t gl = std::max<uint32_t>(1, bound_large);
     {
         Launch L(c, K_TREE, 0);
-        hipLaunchKernelGGL(k_tree, dim3(std::min(gl, kDevTreeWgs)), dim3(kBigWG), 0, st, P, B, seed, c->w.trees,
-                           (int)from_arena);
+        launch_tree(c, B, P, std::min(gl, kDevTreeWgs), seed, from_arena);
     }
     const uint64_t tiles_bound = n / ((uint64_t)kWaves * kChunkMin) + gl;
     {
@@ -3101,7 +3259,6 @@ int host_levels(ps5_ctx* c, const Bufs& B, uint32_t round, int cur_ci, uint32_t*
 {
     *after_blocks = false;     // set when the stream's last packets are the last level's block kernels
     hipStream_t st = c->stream;
-    const uint32_t depth = round * 8;
     const int rp = round & 1, np = rp ^ 1;
     const Sink nsink = make_sink(c, c->w.l_round[np], C_LROUND + np, np);
     int rc;
@@ -3139,7 +3296,7 @@ int host_levels(ps5_ctx* c, const Bufs& B, uint32_t round, int cur_ci, uint32_t*
         if (nlarge == 0 && !c->profile && div_up(nt, kWaves) + nr >= kForkLeafGroups) {
             HIPCHK(hipEventRecord(c->ev_fork, st));
             HIPCHK(hipStreamWaitEvent(c->side, c->ev_fork, 0));
-            launch_leaves(c, B, rp, nsink, depth, leaf_tiny_grid(nt), leaf_run_grid(nr), nt, nr, c->side);
+            launch_leaves(c, B, rp, nsink, leaf_tiny_grid(nt), leaf_run_grid(nr), nt, nr, c->side);
             HIPCHK(hipEventRecord(c->ev_join, c->side));
             *leaves_forked = true;
         }
@@ -3155,7 +3312,7 @@ int host_levels(ps5_ctx* c, const Bufs& B, uint32_t round, int cur_ci, uint32_t*
         int bflags = 0;     // the first class waits for the level; the others may run beside it
         for (int cls = 0; cls < kBlkClasses; ++cls) {
             if (!nblk[cls]) continue;
-            launch_block_class(c, B, rp, cls, blk_done[cls], nblk[cls], false, nblk[cls], nsink, depth, tail, bflags);
+            launch_block_class(c, B, rp, cls, blk_done[cls], nblk[cls], false, nblk[cls], nsink, tail, bflags);
             if (!c->profile) bflags = hipExtAnyOrderLaunch;
             *after_blocks = nlarge == 0;
             sum_sizes(c, c->w.l_block[rp] + (uint64_t)cls * c->w.cap_block, blk_done[cls],
@@ -3208,7 +3365,6 @@ int host_levels(ps5_ctx* c, const Bufs& B, uint32_t round, int cur_ci, uint32_t*
 int host_round_end(ps5_ctx* c, const Bufs& B, uint32_t round, bool leaves_forked, bool after_blocks)
 {
     hipStream_t st = c->stream;
-    const uint32_t depth = round * 8;
     const int rp = round & 1, np = rp ^ 1;
     const Sink nsink = make_sink(c, c->w.l_round[np], C_LROUND + np, np);
     const uint32_t nt = c->h_cnt[C_TINY + rp], nr = c->h_cnt[C_RUN + rp];
@@ -3216,17 +3372,17 @@ int host_round_end(ps5_ctx* c, const Bufs& B, uint32_t round, bool leaves_forked
     for (int cls = 0; cls < kBlkClasses; ++cls) nb += c->h_cnt[C_BLOCK + 2 * cls + rp];
     c->st_leaves += nt + nb + nr;
     if (c->trace) {
-        fprintf(stderr, "[ps5] round %u depth %u: tiny %u, blocks %u/%u/%u/%u, equal chunks %u, levels %llu\n",
-                round, depth, nt, c->h_cnt[C_BLOCK + rp], c->h_cnt[C_BLOCK + 2 + rp], c->h_cnt[C_BLOCK + 4 + rp],
+        fprintf(stderr, "[ps5] round %u: tiny %u, blocks %u/%u/%u/%u, equal chunks %u, levels %llu\n",
+                round, nt, c->h_cnt[C_BLOCK + rp], c->h_cnt[C_BLOCK + 2 + rp], c->h_cnt[C_BLOCK + 4 + rp],
                 c->h_cnt[C_BLOCK + 6 + rp], nr, (unsigned long long)c->st_levels);
     }
     if (leaves_forked) HIPCHK(hipStreamWaitEvent(st, c->ev_join, 0));
     // right after the last level's block kernels (the first of which waited
     // for everything before it) the leaves may start beside them; the leaf
     // boundaries below wait for all of them
-    else launch_leaves(c, B, rp, nsink, depth, leaf_tiny_grid(nt), leaf_run_grid(nr), nt, nr, st,
+    else launch_leaves(c, B, rp, nsink, leaf_tiny_grid(nt), leaf_run_grid(nr), nt, nr, st,
                        after_blocks && !c->profile ? hipExtAnyOrderLaunch : 0);
-    if (nt + nb + nr && B.lcp) launch_leafbound(c, B, rp, depth, div_up((uint64_t)nt + nb + nr, kWG), nt + nb + nr);
+    if (nt + nb + nr && B.lcp) launch_leafbound(c, B, rp, div_up((uint64_t)nt + nb + nr, kWG), nt + nb + nr);
     HIPCHK(hipGetLastError());
     return readback(c, c->w.l_round[np], C_LROUND + np);
 }
@@ -3242,6 +3398,14 @@ struct SortRun {
     uint64_t root_sum;        // strings in large roots
 };
 
+// The depth arrays a round reads (none in round 0: every root starts at
+// depth 0) and writes.
+void set_depths(ps5_ctx* c, Bufs& B, uint32_t round)
+{
+    B.sdepth_in = round ? c->w.sdepth[round & 1] : nullptr;
+    B.sdepth_out = c->w.sdepth[(round & 1) ^ 1];
+}
+
 // Round `round` of a sort, planned on the host or (dev) on the device; sets
 // *done when no work is left for another round.
 int sort_round(ps5_ctx* c, SortRun& R, uint32_t round, bool dev, bool* done)
@@ -3256,8 +3420,8 @@ int sort_round(ps5_ctx* c, SortRun& R, uint32_t round, bool dev, bool* done)
     const uint64_t root_max = R.root_max, root_sum = R.root_sum;
     uint32_t* lcp = B.lcp;
     *done = false;
-    const uint32_t depth = round * 8;
     const int rp = round & 1, np = rp ^ 1;
+    set_depths(c, B, round);
     c->st_rounds++;
     uint32_t round_mask = 0;     // the lists of round r+1 are empty again (consumed in round r-1; set up empty in round 0)
     if (round > 0) {
@@ -3328,7 +3492,7 @@ int sort_round(ps5_ctx* c, SortRun& R, uint32_t round, bool dev, bool* done)
                     const uint64_t full = block_grid_full(c, cls);
                     const uint64_t known = level == 0 ? c->h_cnt[C_BLOCK + 2 * cls + rp] : 0;
                     const uint32_t g = (uint32_t)std::min<uint64_t>(full, known + S / minm + 1);
-                    launch_block_class(c, B, rp, cls, 0, 0, true, g, nsink, depth, false, bflags);
+                    launch_block_class(c, B, rp, cls, 0, 0, true, g, nsink, false, bflags);
                     if (!c->profile) bflags = hipExtAnyOrderLaunch;
                 }
                 HIPCHK(hipGetLastError());
@@ -3342,11 +3506,11 @@ int sort_round(ps5_ctx* c, SortRun& R, uint32_t round, bool dev, bool* done)
             const uint32_t gt = (uint32_t)std::min<uint64_t>(kDevTinyWgs, div_up(nt0 + S, kWaves));
             const uint32_t gr = (uint32_t)std::min<uint64_t>(kDevRunWgs, nr0 + S / kTinyT + 1);
             B.pending = c->d_cnt + in_ci;
-            launch_leaves(c, B, rp, nsink, depth, gt, gr, nt0 + S, nr0 + S, st);
+            launch_leaves(c, B, rp, nsink, gt, gr, nt0 + S, nr0 + S, st);
             if (lcp) {
                 uint64_t known = nt0 + nr0;
                 for (int cls = 0; cls < kBlkClasses; ++cls) known += c->h_cnt[C_BLOCK + 2 * cls + rp];
-                launch_leafbound(c, B, rp, depth,
+                launch_leafbound(c, B, rp,
                                  (uint32_t)std::min<uint64_t>(kDevBoundWgs, div_up(known + S, kWG)), known + S);
             }
             B.pending = nullptr;
@@ -3370,7 +3534,7 @@ int sort_round(ps5_ctx* c, SortRun& R, uint32_t round, bool dev, bool* done)
     uint64_t pending = (uint64_t)c->h_cnt[C_LROUND + np] + c->h_cnt[C_TINY + np] + c->h_cnt[C_RUN + np];
     for (int cls = 0; cls < kBlkClasses; ++cls) pending += c->h_cnt[C_BLOCK + 2 * cls + np];
     if (pending == 0) { *done = true; return PS5_OK; }
-    if (depth > alen + 8) return set_err(PS5_ERR_INTERNAL, "depth exceeds the arena: no progress");
+    if ((uint64_t)round * 8 > alen + 8) return set_err(PS5_ERR_INTERNAL, "depth exceeds the arena: no progress");
     return PS5_OK;
 }
 
@@ -3383,8 +3547,8 @@ void graph_round(ps5_ctx* c, SortRun& R, uint32_t round, uint32_t L, uint32_t nl
     hipStream_t st = c->stream;
     Bufs B = R.B;
     const uint64_t n = R.n;
-    const uint32_t depth = round * 8;
     const int rp = round & 1, np = rp ^ 1;
+    set_depths(c, B, round);
     if (round > 0) {
         uint32_t mask = (1u << (C_LROUND + np)) | (1u << (C_TINY + np)) | (1u << (C_RUN + np));
         for (int cls = 0; cls < kBlkClasses; ++cls) mask |= (1u << (C_BLOCK + 2 * cls + np)) | (1u << (C_BDONE + cls));
@@ -3405,16 +3569,16 @@ void graph_round(ps5_ctx* c, SortRun& R, uint32_t round, uint32_t L, uint32_t nl
         dev_level(c, B, in_list, in_ci, rootlvl ? nl_root : any_large, S, sink, seed, R.fused_root && rootlvl,
                   rootlvl, rootlvl ? (int)R.root_kmax : dev_level_kmax(c, R.root_max, level), level > 0 ? rp : -1);
         for (int cls = 0; cls < kBlkClasses; ++cls) {
-            launch_block_class(c, B, rp, cls, 0, 0, true, block_grid_full(c, cls), nsink, depth);
+            launch_block_class(c, B, rp, cls, 0, 0, true, block_grid_full(c, cls), nsink);
         }
         in_ci = out_ci;
         in_list = c->w.l_lvl[level & 1];
     }
     B.pending = c->d_cnt + in_ci;
     B.pending_err = 1;
-    launch_leaves(c, B, rp, nsink, depth, (uint32_t)std::min<uint64_t>(kDevTinyWgs, div_up(n, kWaves)),
+    launch_leaves(c, B, rp, nsink, (uint32_t)std::min<uint64_t>(kDevTinyWgs, div_up(n, kWaves)),
                   (uint32_t)std::min<uint64_t>(kDevRunWgs, c->w.cap_run), n, n, st);
-    if (B.lcp) launch_leafbound(c, B, rp, depth, (uint32_t)std::min<uint64_t>(kDevBoundWgs, div_up(n, kWG)), n);
+    if (B.lcp) launch_leafbound(c, B, rp, (uint32_t)std::min<uint64_t>(kDevBoundWgs, div_up(n, kWG)), n);
 }
 
 // Round 0 keys the first classification pass does not extract: every
@@ -3441,8 +3605,8 @@ int init_root_keys(ps5_ctx* c, const Bufs& B, uint32_t n, const uint64_t* set_fi
     return PS5_OK;
 }
 
-int run_sort(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_t* offs, const uint64_t* offs64,
-             uint32_t n, uint32_t* perm, uint32_t* lcp, const uint64_t* set_first, uint32_t nsets)
+int run_sort_keys(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_t* offs, const uint64_t* offs64,
+                  uint32_t n, uint32_t* perm, uint32_t* lcp, const uint64_t* set_first, uint32_t nsets, bool pack)
 {
     int rc = ensure_capacity(c, n);
     if (rc) return rc;
@@ -3467,6 +3631,8 @@ int run_sort(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_t* of
     B.pending = nullptr;
     B.pending_err = 0;
     B.leaf_keys = c->leaf_keys;
+    set_depths(c, B, 0);
+    B.lut = nullptr;     // (set below, once the trees' buffers have their size)
 
     // the roots (one, or a batch's sets) and their sizes
     uint32_t root_kmax = 1;                     // largest treebits of a large root
@@ -3516,6 +3682,14 @@ int run_sort(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_t* of
         c->h_cnt[n <= kTinyT ? C_TINY : C_BLOCK + 2 * block_class(n)] = 1;
     }
 
+    if (fused_root && pack && root_max >= kPackMin) {     // a root's keys may be packed: its code table beside its tree
+        if (!set_first) {
+            if ((rc = grow_level(c, 1, 0))) return rc;
+        } else if ((rc = grow_level(c, c->w.cap_large, 0))) {
+            return rc;
+        }
+        B.lut = c->w.lut;
+    }
     SortRun R{ B, n, alen, fused_root, root_kmax, root_max, root_sum };
     uint32_t start = 0;
     if (c->graph_rounds && !c->profile) {
@@ -3602,6 +3776,20 @@ int run_sort(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_t* of
     return PS5_OK;
 }
 
+// (a captured graph holds plain keys only: its replay cannot start over)
+int run_sort(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_t* offs, const uint64_t* offs64,
+             uint32_t n, uint32_t* perm, uint32_t* lcp, const uint64_t* set_first, uint32_t nsets)
+{
+    const bool graph = c->graph_rounds && !c->profile;
+    int rc = run_sort_keys(c, arena, alen, offs, offs64, n, perm, lcp, set_first, nsets, !graph);
+    if (rc != kUnpack) return rc;
+    HIPCHK(hipStreamSynchronize(c->side));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    if (c->profile) collect_events(c);
+    rc = run_sort_keys(c, arena, alen, offs, offs64, n, perm, lcp, set_first, nsets, false);
+    return rc == kUnpack ? set_err(PS5_ERR_INTERNAL, "plain keys flagged as packed") : rc;
+}
+
 }  // namespace
 
 // ===========================================================================
@@ -3621,10 +3809,13 @@ int ps5_ctx_create(ps5_ctx** out, int device)
                                ScatLds<false>::kBytes));
     HIPCHK(hipFuncSetAttribute((const void*)k_scatter<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                ScatLds<true>::kBytes));
-    for (const void* f : { (const void*)k_count<8, false>, (const void*)k_count<9, false>,
-                           (const void*)k_count<10, false>, (const void*)k_count<11, false>,
-                           (const void*)k_count<8, true>, (const void*)k_count<9, true>,
-                           (const void*)k_count<10, true>, (const void*)k_count<11, true> })
+#define PS5_COUNT_INSTANCES(NB)                                                              \
+    (const void*)k_count<NB, false, kNoRoot>, (const void*)k_count<NB, false, kRootPlain>,   \
+    (const void*)k_count<NB, false, kRootPack>, (const void*)k_count<NB, true, kNoRoot>,     \
+    (const void*)k_count<NB, true, kRootPlain>, (const void*)k_count<NB, true, kRootPack>
+    for (const void* f : { PS5_COUNT_INSTANCES(8), PS5_COUNT_INSTANCES(9), PS5_COUNT_INSTANCES(10),
+                           PS5_COUNT_INSTANCES(11) })
+#undef PS5_COUNT_INSTANCES
         HIPCHK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, count_lds_bytes(kMaxTreebits)));
     ps5_ctx* c = new ps5_ctx;
     c->device = device;

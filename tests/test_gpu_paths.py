@@ -30,3 +30,71 @@ def test_new_context_ignores_recycled_sequence_words(ps5, oracle, syncs):
         check(second, oracle, *large)
     finally:
         second.close()
+
+
+def packed_case(sigma, n, seed, hi=60, rare=None):
+    """(arena, offs) of n strings over sigma characters drawn from the whole
+    byte range, many sharing 8 characters and more; `rare` puts a character
+    outside that alphabet at that place of one string"""
+    rng = np.random.default_rng(seed)
+    alpha = np.sort(rng.choice(np.arange(1, 255), sigma, replace=False)).astype(np.uint8)
+    lens = rng.integers(0, hi, n)
+    chars = alpha[rng.integers(0, sigma, (n, hi))]
+    stems = alpha[rng.integers(0, sigma, (40, 24))][rng.integers(0, 40, n)]
+    keep = np.arange(24)[None, :] < rng.integers(0, 25, n)[:, None]
+    chars[:, :24] = np.where(keep, stems, chars[:, :24])
+    if rare is not None:
+        i = int(rng.integers(0, n))
+        lens[i] = hi - 1
+        chars[i, rare] = 255
+    ends = np.cumsum(lens + 1)
+    offs = (ends - lens - 1).astype(np.uint32)
+    arena = np.zeros(int(ends[-1]) + 16, np.uint8)
+    inside = np.arange(hi)[None, :] < lens[:, None]
+    arena[(offs[:, None].astype(np.int64) + np.arange(hi)[None, :])[inside]] = chars[inside]
+    return arena, offs
+
+
+def concatenated(sets):
+    """one arena, uint64 offsets and set boundaries of several (arena, offs)"""
+    base = np.cumsum([0] + [len(a) for a, _ in sets])
+    arena = np.concatenate([a for a, _ in sets])
+    offs = np.concatenate([o.astype(np.uint64) + np.uint64(b) for (_, o), b in zip(sets, base)])
+    return arena, offs, np.cumsum([0] + [len(o) for _, o in sets]).astype(np.uint64)
+
+
+@pytest.mark.parametrize("sigma", [1, 2, 4, 7, 8, 15, 16, 31, 32])
+@pytest.mark.parametrize("n", [2049, 30011, 1050003])
+def test_packed_roots(ctx, oracle, sigma, n):
+    """every code width (3, 4, 5 bits and none) at the edges of its alphabet"""
+    check(ctx, oracle, *packed_case(sigma, n, 100 * sigma + n))
+
+
+@pytest.mark.parametrize("at", [0, 7, 20, 21, 40])
+def test_packed_root_meets_an_unknown_character(ctx, oracle, at):
+    """one string holds a character the samples do not show: in the packed
+    key (the sort starts over) or behind it (it stands)"""
+    check(ctx, oracle, *packed_case(4, 1060000, at, rare=at))
+    check(ctx, oracle, *packed_case(4, 1060000, 7 + at, rare=at), with_lcp=False)
+
+
+@pytest.mark.parametrize("planning", [0, 1])
+def test_packed_batch_of_mixed_alphabets(ps5, oracle, planning):
+    """sets of one batch choose their own key formats; one of them meets an
+    unknown character, and small sets stay unpacked"""
+    sets = [packed_case(4, 9000, 1), packed_case(12, 5000, 2), packed_case(40, 7000, 3), packed_case(2, 700, 4), pack([b""]),
+            packed_case(20, 6000, 5), packed_case(4, 1060000, 6)]
+    for rare in (None, 5):
+        if rare is not None:
+            sets[-1] = packed_case(4, 1060000, 6, rare=rare)
+        arena, offs, first = concatenated(sets)
+        c = ps5.Context(0)
+        try:
+            c.set_planning(planning)
+            perm, lcp = c.sort_batch(arena, offs, first)
+        finally:
+            c.close()
+        for k in range(len(sets)):
+            b, e = int(first[k]), int(first[k + 1])
+            r, msg = oracle.verify(arena, offs[b:e].astype(np.uint32), perm[b:e], lcp[b:e])
+            assert r == 0, (k, msg)
