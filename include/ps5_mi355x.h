@@ -119,7 +119,7 @@ int ps5_sort_device(ps5_ctx* ctx, const uint8_t* d_arena, uint64_t arena_bytes,
  * it is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Arguments
  * and results are those of ps5_sort_device; the work buffers come from a
- * static device array of 96 MiB that every GPU the library runs on holds
+ * static device array of 128 MiB that every GPU the library runs on holds
  * (one copy per GPU and process) until the process ends, so n is limited to
  * ps5_noalloc_max_strings() (2^20); a larger n is rejected with
  * PS5_ERR_ARG.  The call makes no hipMalloc/hipFree or other allocating call
@@ -249,14 +249,15 @@ int ps5_ctx_get_tuning(ps5_ctx* ctx, uint32_t* leaf_target, uint32_t* max_treebi
 /* Tile shapes and key width of a context's sorts (they never change the
  * output).  No counterpart in the reference (its tiles are per-thread
  * buckets and its key cache is one uint64, bingmann-sample_sort.hpp:49):
- *   chunk_max      keys per wave chunk of a multi-workgroup level, in
- *                  [2048, 9216] (default 9216): the unit of stable ranks
- *                  and of the scatter's LDS reorder;
+ *   chunk_max      keys per chunk of a multi-workgroup level, the unit one
+ *                  workgroup ranks and reorders in LDS, in [2048, 9216]
+ *                  (default 9216; a chunk holds at most 4096 keys, so larger
+ *                  limits act as 4096);
  *   chunk_max_root the same in a level of roots, in [2048, 12032] (default
- *                  12032; the root scatter stages 2-byte positions);
- *   min_tiles      tiles a level is spread over at least, its chunks
- *                  shrinking (not below 2048 keys) when it is small, in
- *                  [1, 65536] (default 512);
+ *                  12032, likewise);
+ *   min_tiles      chunks a level is spread over at least, shrinking (not
+ *                  below 2048 keys) when it is small, in [1, 65536]
+ *                  (default 512);
  *   leaf_keys      keys (8 characters each) a leaf pass fetches per string
  *                  at a time, in [1, 8] (default 8). */
 int ps5_ctx_set_shape(ps5_ctx* ctx, uint32_t chunk_max, uint32_t chunk_max_root, uint32_t min_tiles,

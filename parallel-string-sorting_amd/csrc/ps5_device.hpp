@@ -290,10 +290,56 @@ __device__ __forceinline__ uint64_t str_off(const Bufs& B, uint32_t i)
     return B.offs64 ? B.offs64[i] : (uint64_t)B.offs[i];
 }
 
+// Where a bucket's strings lie: run c holds the positions from V[c] on, at
+// S[c] and after in K and I.
+struct Runs {
+    const key64* K;
+    const uint32_t* I;
+    const uint32_t* V;
+    const uint32_t* S;
+    uint32_t nch;
+};
+__device__ __forceinline__ Runs runs_of(const Bufs& B, const Item& it)
+{
+    const uint64_t b = it.flags & F_BUFB;
+    const uint64_t t = it.row + b * B.cap_h;
+    return Runs{ B.key + b * B.cap, B.idx + b * B.cap, B.vpos + t, B.src + t, it.nch };
+}
+// the run holding position pos: the last of n whose first position is not
+// above it (an empty run shares its position with the run after it)
+__device__ __forceinline__ uint32_t find_run(const uint32_t* V, uint32_t n, uint32_t pos)
+{
+    uint32_t lo = 0, hi = n;
+    while (lo + 1 < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (V[mid] <= pos) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+// a place computed from run tables, checked against the buffers' size
+__device__ __forceinline__ uint32_t checked_place(const Bufs& B, uint32_t q)
+{
+    if (q >= B.n) { flag_error(B.cnt, ERR_BOUNDS); q = 0; }
+    return q;
+}
+__device__ __forceinline__ uint32_t run_place(const Bufs& B, const Runs& R, uint32_t pos)
+{
+    const uint32_t c = find_run(R.V, R.nch, pos);
+    return checked_place(B, R.S[c] + (pos - R.V[c]));
+}
+// the key at depth d of input string id
+__device__ __forceinline__ key64 string_key(const Bufs& B, uint32_t id, uint32_t d)
+{
+    if (id >= B.n) { flag_error(B.cnt, ERR_BOUNDS); id = 0; }
+    return load_key(B.arena, B.alen, str_off(B, id) + d);
+}
+
 // an item must describe a non-empty range inside [0, n)
 __device__ __forceinline__ bool item_ok(const Item& it, const Bufs& B)
 {
-    return it.size != 0 && it.begin < B.n && it.size <= B.n - it.begin;
+    return it.size != 0 && it.begin < B.n && it.size <= B.n - it.begin &&
+           ((it.flags & (F_IDENT | F_NEXT)) || it.nch != 0);
 }
 
 __device__ __forceinline__ void put_item(Item* list, uint32_t cap, uint32_t slot, Item it, uint32_t* cnt)
@@ -409,13 +455,13 @@ __device__ __forceinline__ int inorder_of(int t, int k)
 // Buckets of G keys: b = 2 * lower_bound + [splitter == key]
 // (ClassifyTreeSimple::find_bkt, bingmann-sample_sortBTC.hpp:45-72).  The
 // descent i = 2i + (key > tree[i]) over the level-order tree ends at the
-// number of splitters below the key; the equality test reads that splitter
-// from the sorted array (one load instead of tracking a candidate per level).
+// number x of splitters below the key; the equality test reads splitter x,
+// whose node follows from the number of trailing zeros of x + 1 (one load
+// instead of tracking a candidate per level, and no second array).
 // The G descents advance level by level together, so their LDS reads are in
 // flight at the same time.
 template <int G>
-__device__ __forceinline__ void classify_keys(const key64 (&key)[G], const key64* s_tree, const key64* s_sorted,
-                                              int k, uint32_t (&b)[G])
+__device__ __forceinline__ void classify_keys(const key64 (&key)[G], const key64* s_tree, int k, uint32_t (&b)[G])
 {
     // the descent tracks byte offsets into s_tree (8 * node): each level is
     // one LDS read, one compare and one shift-add
@@ -428,11 +474,14 @@ __device__ __forceinline__ void classify_keys(const key64 (&key)[G], const key64
         for (int j = 0; j < G; ++j)
             a[j] = 2 * a[j] + (key[j] > *reinterpret_cast<const key64*>(tb + a[j]) ? 8u : 0u);
     }
-    const uint32_t nspl = (1u << k) - 1;
+    // a / 8 = 2^k + x; splitter x is node (2^k + x + 1) >> (z + 1), z the
+    // trailing zeros of x + 1 (node 0 when every splitter is below the key)
 #pragma unroll
     for (int j = 0; j < G; ++j) {
-        const uint32_t x = (a[j] >> 3) - (1u << k);
-        b[j] = 2 * x + ((x < nspl && s_sorted[x] == key[j]) ? 1u : 0u);
+        const uint32_t n = (a[j] >> 3) + 1;
+        const uint32_t node = n >> (__builtin_ctz(n) + 1);
+        const uint32_t x = n - 1 - (1u << k);
+        b[j] = 2 * x + ((node != 0 && s_tree[node] == key[j]) ? 1u : 0u);
     }
 }
 

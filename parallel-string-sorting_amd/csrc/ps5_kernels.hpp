@@ -1,26 +1,35 @@
 // ps5_kernels.hpp -- shared definitions of the gfx950 pS5 kernels.
 //
-// Device data layout (one sort, n strings, positions 0..n-1):
+// Device data layout (one sort, n strings, positions 0..n-1 of the sorted order):
 //   arena      characters as given by the caller (never written)
 //   offs[n]    uint32 start offset of input string i
-//   key[2][n]  uint64 ping-pong: 8 characters at the current depth,
-//              big-endian, zero from the first NUL on
-//   idx[2][n]  uint32 ping-pong: input index of the string at a position
-//   bktrank[n] uint32 scratch: (bucket << 21) | rank inside its wave chunk
+//   key[2][n], idx[2][n]  keys (uint64) and input indices as a level of the
+//              sample sort leaves them: every chunk of a segment reordered by
+//              bucket, in place of the chunk.  Even levels of a round write
+//              buffer 0, odd levels buffer 1
+//   vpos[2], src[2]  per buffer: for bucket b and chunk c of a segment, the
+//              first sorted position and the place in key/idx of the bucket's
+//              strings in that chunk (its run), bucket-major
 //   bkey[n]    uint64 scratch: depth key of the first/last position of a leaf
 //   sdepth[2][n] uint32 by round parity: characters the strings of the round
 //              segment starting at a position are known to share
-//   perm[n], lcp[n]  results (caller memory)
+//   perm[n], lcp[n]  results (caller memory); between rounds perm holds the
+//              input indices of the strings that continue
 //
 // A sort proceeds in rounds; a round compares one key (8 characters, or up to
 // 21 in round 0, see KeyFmt) of every string at the depth of its segment.
 // Inside a round, segments (contiguous position ranges whose strings share
-// the characters before that depth) are split by multi-workgroup splitter-tree steps
-// until every piece is a leaf: a block (at most kBlkT strings, sorted
-// completely in LDS by one workgroup), a tiny leaf (at most 64 strings, one
-// wave) or an equal-key bucket.  Leaves finish their strings at this depth
-// (order, LCPs, permutation) and turn every run of equal keys without a NUL
-// into a segment of round r+1.
+// the characters before that depth) are split by multi-workgroup
+// splitter-tree steps until every piece is a leaf: a block (at most kBlkT
+// strings, sorted completely in LDS by one workgroup), a tiny leaf (at most
+// 64 strings, one wave) or an equal-key bucket.  Leaves finish their strings
+// at this depth (order, LCPs, permutation) and turn every run of equal keys
+// without a NUL into a segment of the next round.
+//
+// A level moves every string once: its chunks are reordered in LDS and
+// written back whole, and whoever reads a bucket gathers its runs, one per
+// chunk.  Counting first, so that buckets come out contiguous, would read
+// every key once more and write and read its bucket and rank (12 bytes).
 #pragma once
 #include <cstdint>
 
@@ -38,17 +47,24 @@ constexpr int kMaxSpl = (1 << kMaxTreebits) - 1;    // 1023 splitters
 constexpr int kMaxBkt = 2 * kMaxSpl + 1;            // 2047 buckets
 constexpr int kMaxSamples = 4096;            // sample keys of one splitter tree
 constexpr uint32_t kTreeSlots = 2048;        // per segment: level-order tree [0,1024), sorted splitters [1024,2048)
-// A large segment is cut into T tiles of kWaves equal wave chunks; a wave
-// chunk (the unit of stable ranks and of the scatter's LDS reorder) holds at
-// most a per-level limit of keys, and T is the fewest tiles that allows, so
-// a level's tiles are as few and as full as possible.  The limit is
-// kChunkMax (kChunkMaxIdent in a level of roots, whose scatter stages
-// 2-byte positions) unless the level is too small to give kMinTiles tiles that way;
-// then it shrinks (not below kChunkMin) so small sorts still spread over
-// the GPU.
-constexpr int kChunkMax = 9216;              // keys ranked by one wave (multi-workgroup step)
-constexpr int kChunkMaxIdent = 12032;        // the same in a level of root segments (indices = positions)
+// A large segment is cut into the fewest equal chunks of at most a per-level
+// limit of keys: kPartMax, unless the level is too small to give min_tiles
+// chunks that way; then the limit shrinks (not below kChunkMin) so small
+// sorts still spread over the GPU.  A chunk is the unit of k_part: one
+// workgroup of kPartWaves waves ranks its keys stably and reorders them.
+// 4096 keys (52 KB of LDS with a 9-level tree) leave room for three workgroups
+// per CU, so that one loads while others rank: 64 M random strings take 605 us
+// at the root level and a batch of 50 M strings with 10-level trees 650 us (two
+// workgroups per CU), with 6144 keys 620 and 1000 us (one workgroup with 10
+// levels).
+constexpr int kPartWaves = 8;
+constexpr int kPartThreads = kPartWaves * 64;
+constexpr int kPartGroups = 8;               // 64-key groups per wave
+constexpr int kPartMax = kPartThreads * kPartGroups;
 constexpr int kChunkMin = 2048;
+constexpr uint32_t kHistGroup = 64;          // chunks whose bucket counts are summed together
+// limits and defaults of ps5_ctx_set_shape
+constexpr uint32_t kShapeChunkMax = 9216, kShapeChunkMaxRoot = 12032;
 constexpr uint32_t kMinTiles = 512;
 constexpr uint32_t kTinyT = 64;              // leaves sorted by one wave
 constexpr uint32_t kBlkT = 2048;             // leaves sorted on chip by one workgroup
@@ -68,11 +84,17 @@ struct Item {            // a segment or a leaf
     uint32_t begin;      // first position
     uint32_t size;       // number of positions
     uint32_t rbeg;       // first position of the round segment it belongs to
-    uint32_t flags;      // F_BUFB | F_SORTED | chunk index << 8
+    uint32_t flags;      // F_* | key format << kFmtShift | chunk index << kFlagShift
+    uint32_t row, nch;   // a bucket: its first entry in vpos/src and its runs (one per chunk of its segment)
 };
-constexpr uint32_t F_BUFB = 1u;              // data lives in key[1]/idx[1]
+// Where a segment's strings are found: F_IDENT (a root: the string at position
+// p is input string p) and F_NEXT (a segment of an earlier round: perm[p]) say
+// that its keys are still to be read from the arena; otherwise it is a bucket,
+// whose strings lie in the runs of its row in buffer F_BUFB.
+constexpr uint32_t F_BUFB = 1u;              // key[1]/idx[1]/vpos[1]/src[1]
 constexpr uint32_t F_SORTED = 2u;            // all keys equal (equal bucket)
-constexpr uint32_t F_IDENT = 4u;             // a root: idx[p] = p, not stored
+constexpr uint32_t F_IDENT = 4u;
+constexpr uint32_t F_NEXT = 32u;
 constexpr uint32_t kFmtShift = 3;            // (flags >> kFmtShift) & 3: format of the segment's keys (KeyFmt)
 constexpr uint32_t kFmtMask = 3u << kFmtShift;
 constexpr uint32_t kFlagShift = 8;           // flags >> kFlagShift: chunk index of an equal-key chunk
@@ -87,7 +109,9 @@ enum : int {
     C_ERR = 16,    // error flags
     C_BDONE = 17,  // [4] blocks of the current round already sorted, per size class (device-driven levels)
     C_RUNCONT = 21,  // [2] equal-key leaves whose strings continue into the next round (round parity)
-    C_NCNT = 23
+    C_TDONE = 23,  // tiny leaves and equal-key chunks of the current round finished before its end (device-driven
+    C_RDONE = 24,  // levels)
+    C_NCNT = 25
 };
 constexpr uint32_t ERR_CAP = 1u, ERR_LCP = 2u, ERR_BOUNDS = 4u;
 constexpr uint32_t ERR_LEVELS = 8u;          // a captured round had more levels than it was built with
@@ -113,34 +137,37 @@ __host__ __device__ constexpr KeyFmt key_fmt(uint32_t flags)
 
 struct LargeDesc {       // one segment of the multi-workgroup sample-sort step
     Item seg;
-    uint32_t T;          // tiles of kWaves * chunk keys (the last one may be short)
-    uint32_t chunk;      // keys per wave chunk, <= kChunkMax (kChunkMaxIdent for a root)
-    uint32_t pad;
-    uint32_t hist_base;  // first histogram entry of this segment
+    uint32_t nch;        // chunks
+    uint32_t chunk;      // keys per chunk (the last one may be short), <= kPartMax
+    uint32_t hist_base;  // first entry of this segment's bucket counts (chunk-major, 2 << k per chunk) and of
+                         // its vpos/src rows (bucket-major, nch per bucket)
+    uint32_t gbase;      // first entry of its group sums: a row of 2 << k first positions, then a row per group
     uint32_t k;          // treebits
     uint32_t oversample; // sample keys per splitter
 };
+__host__ __device__ constexpr uint32_t hist_groups(uint32_t nch) { return (nch + kHistGroup - 1) / kHistGroup; }
 
-struct TileRef {         // one workgroup of the multi-workgroup step
+struct TileRef {         // one chunk, or one group of kHistGroup chunks
     uint32_t seg;        // index into the LargeDesc array
-    uint32_t t;          // tile inside the segment
+    uint32_t t;          // chunk or group inside the segment
 };
 
 struct LevelHdr {        // totals of one level's multi-workgroup step
     uint32_t nlarge;     // segments (LargeDesc entries)
-    uint32_t ntiles;     // tiles (TileRef entries), kWaves chunks each
-    uint32_t hl;         // histogram entries
+    uint32_t ntiles;     // chunks (TileRef entries)
+    uint32_t ngroups;    // groups of chunks (TileRef entries of the second table)
     uint32_t kmax;       // largest treebits of the level
     uint32_t pad[4];
 };
 
 // A level's plan in device memory: the header, then cap_large descriptors,
-// then the tile table (fixed offsets, so a plan written on the device needs
-// no pointer arithmetic on the host).
+// then the tables of chunks and of groups (fixed offsets, so a plan written
+// on the device needs no pointer arithmetic on the host).
 struct Plan {
     const LevelHdr* hdr;
     LargeDesc* desc;     // (k_tree records a root's key format in it)
     const TileRef* tiles;
+    const TileRef* groups;
 };
 
 struct Sink {            // where new items are appended
@@ -159,12 +186,16 @@ struct Bufs {
     uint64_t alen;
     const uint32_t* offs;      // string start offsets (uint32), or
     const uint64_t* offs64;    // uint64 offsets when non-null (batches over 4 GiB)
-    key64* key0; key64* key1;
-    uint32_t* idx0; uint32_t* idx1;
+    key64* key;          // two buffers of cap entries each, one after the other
+    uint32_t* idx;
+    uint32_t* vpos;      // two tables of cap_h entries each
+    uint32_t* src;
+    uint64_t cap, cap_h;
     uint32_t* perm;
     uint32_t* lcp;       // may be null
     key64* bkey;
-    uint32_t* bktrank;
+    uint32_t* hist;      // bucket counts of the level being split
+    uint32_t* gsum;      // their sums over groups of chunks
     const uint32_t* pending;   // non-null and non-zero: large segments remain, the round's leaves wait
     uint32_t pending_err;      // ... and that is an error (ERR_LEVELS: a captured graph cannot continue the round)
     const uint32_t* sdepth_in; // depths of this round's segments (null in round 0: depth 0)

@@ -37,30 +37,12 @@ using namespace ps5;
 // kernels
 // ===========================================================================
 
-// Round 0 keys: key0[i] = 8 characters of string i at depth 0.  The index
-// at every root position is the position itself (root items carry F_IDENT),
-// so idx0 is not written.
+// First 8 characters of every string, in input order (the LCP merge's keys).
 __global__ __launch_bounds__(kWG) void k_init(Bufs B, uint32_t n)
 {
     const uint32_t i = blockIdx.x * kWG + tid_x();
     if (i >= n) return;
-    B.key0[i] = load_key(B.arena, B.alen, str_off(B, i));
-}
-
-// Round 0 keys of the positions of listed items (the sets of a batch that
-// start as tiny leaves or blocks, when the first count pass extracts the keys
-// of the large ones), one workgroup per item at a time.
-__global__ __launch_bounds__(kWG) void k_init_items(const Item* items, uint32_t nitems, Bufs B)
-{
-    for (uint32_t ii = blockIdx.x; ii < nitems; ii += gridDim.x) {
-        const Item it = items[ii];
-        if (!item_ok(it, B)) {
-            if (tid_x() == 0) flag_error(B.cnt, ERR_BOUNDS);
-            continue;
-        }
-        for (uint32_t p = it.begin + tid_x(); p < it.begin + it.size; p += kWG)
-            B.key0[p] = load_key(B.arena, B.alen, str_off(B, p));
-    }
+    B.key[i] = load_key(B.arena, B.alen, str_off(B, i));
 }
 
 // Reset counters and place the root item.
@@ -69,9 +51,35 @@ __global__ void k_setup(uint32_t* cnt, Item* list, int c_index, uint32_t n)
     if (tid_x() < C_NCNT) cnt[tid_x()] = 0;
     __syncthreads();
     if (tid_x() == 0) {
-        Item it = { 0u, n, 0u, F_IDENT };
-        list[0] = it;
+        list[0] = Item{ 0u, n, 0u, F_IDENT, 0u, 0u };
         cnt[c_index] = 1;
+    }
+}
+
+// The roots of a batch, staged by kind in mapped host memory: the lists and
+// the counters in one launch.
+constexpr int kRootKinds = kBlkClasses + 2;      // tiny, blocks by size class, large
+struct RootLists {
+    const Item* src;                 // all roots, kind by kind
+    Item* dst[kRootKinds];
+    uint32_t count[kRootKinds];
+    int counter[kRootKinds];
+};
+__global__ __launch_bounds__(kWG) void k_roots(RootLists R, uint32_t* cnt)
+{
+    if (blockIdx.x == 0) {
+        if (tid_x() < C_NCNT) cnt[tid_x()] = 0;
+        __syncthreads();
+        if (tid_x() == 0) {
+#pragma unroll
+            for (int k = 0; k < kRootKinds; ++k) cnt[R.counter[k]] = R.count[k];
+        }
+    }
+    uint32_t first = 0;
+#pragma unroll
+    for (int k = 0; k < kRootKinds; ++k) {
+        for (uint32_t i = blockIdx.x * kWG + tid_x(); i < R.count[k]; i += gridDim.x * kWG) R.dst[k][i] = R.src[first + i];
+        first += R.count[k];
     }
 }
 
@@ -104,37 +112,39 @@ __global__ __launch_bounds__(kWG) void k_stage(const uint32_t* cnt, const Item* 
 }
 
 // copy 8-byte words of a level plan from mapped host memory to the device:
-// the header with the descriptors, then the tile table
-__device__ __forceinline__ void fetch_plan(const uint64_t* src, uint64_t* dst, uint64_t words, const uint64_t* src2,
-                                           uint64_t* dst2, uint64_t words2)
+// the header with the descriptors, the table of chunks, the table of groups
+struct FetchArgs {
+    const uint64_t* src[3];
+    uint64_t* dst[3];
+    uint64_t words[3];
+};
+__device__ __forceinline__ void fetch_plan(const FetchArgs& F)
 {
     const uint64_t stride = (uint64_t)gridDim.x * kWG;
-    for (uint64_t i = (uint64_t)blockIdx.x * kWG + tid_x(); i < words; i += stride) dst[i] = src[i];
-    for (uint64_t i = (uint64_t)blockIdx.x * kWG + tid_x(); i < words2; i += stride) dst2[i] = src2[i];
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        for (uint64_t i = (uint64_t)blockIdx.x * kWG + tid_x(); i < F.words[k]; i += stride) F.dst[k][i] = F.src[k][i];
 }
 
-__global__ __launch_bounds__(kWG) void k_fetch(const uint64_t* src, uint64_t* dst, uint64_t words,
-                                               const uint64_t* src2, uint64_t* dst2, uint64_t words2)
+__global__ __launch_bounds__(kWG) void k_fetch(FetchArgs F)
 {
-    fetch_plan(src, dst, words, src2, dst2, words2);
+    fetch_plan(F);
 }
 
 // The same for the root level of a single root planned on the host, the
 // sort's first kernel: its first workgroup also does k_setup's work
 // (counters, the root item), one launch fewer before the root level.
-__global__ __launch_bounds__(kWG) void k_root_fetch(const uint64_t* src, uint64_t* dst, uint64_t words,
-                                                    const uint64_t* src2, uint64_t* dst2, uint64_t words2,
-                                                    uint32_t* cnt, Item* list, uint32_t n)
+__global__ __launch_bounds__(kWG) void k_root_fetch(FetchArgs F, uint32_t* cnt, Item* list, uint32_t n)
 {
     if (blockIdx.x == 0) {
         if (tid_x() < C_NCNT) cnt[tid_x()] = 0;
         __syncthreads();
         if (tid_x() == 0) {
-            list[0] = Item{ 0u, n, 0u, F_IDENT };
+            list[0] = Item{ 0u, n, 0u, F_IDENT, 0u, 0u };
             cnt[C_LROUND] = 1;
         }
     }
-    fetch_plan(src, dst, words, src2, dst2, words2);
+    fetch_plan(F);
 }
 
 // zero the counters whose bit is set in `mask`
@@ -142,6 +152,15 @@ __global__ void k_reset(uint32_t* cnt, uint32_t mask)
 {
     const int t = tid_x();
     if (t < C_NCNT && ((mask >> t) & 1u)) cnt[t] = 0;
+}
+
+// the leaves listed so far are finished (device-driven levels, round parity rp)
+__global__ void k_leaves_done(uint32_t* cnt, int rp)
+{
+    if (tid_x() == 0) {
+        cnt[C_TDONE] = cnt[C_TINY + rp];
+        cnt[C_RDONE] = cnt[C_RUN + rp];
+    }
 }
 
 // ---- multi-workgroup sample-sort step (segments > kBlkT) -------------------
@@ -163,27 +182,28 @@ struct PlanArgs {
     const Item* list;        // the level's large segments
     int ci;                  // their counter
     uint32_t cap_large;      // capacity of that list
-    unsigned char* plan;     // header, descriptors, tile table (tiles at tiles_off)
-    uint64_t tiles_off, tiles_cap, hist_cap, trees_cap;
+    unsigned char* plan;     // header, descriptors, tables (at tiles_off and groups_off)
+    uint64_t tiles_off, tiles_cap, groups_off, groups_cap, hist_cap, gsum_cap, trees_cap;
     uint32_t leaf_target, max_treebits, max_oversample;
-    uint32_t chunk_max, chunk_max_root, min_tiles;    // tile shapes (ps5_ctx_set_shape)
-    uint32_t kmax;           // bound of the count launch (treebits are clamped to it)
+    uint32_t chunk_max, chunk_max_root, min_tiles;    // chunk shapes (ps5_ctx_set_shape)
+    uint32_t kmax;           // bound of the level's launches (treebits are clamped to it)
     int done_rp;             // >= 0: mark the blocks of round parity done_rp listed so far as sorted
 };
 
 // Plan one level on the device (one workgroup of kBigWG threads): the same
-// descriptors, tile table and totals that the host's large_step computes
+// descriptors, tables and totals that the host's large_step computes
 // from a read-back list.  A level that does not fit the buffers is flagged
 // (ERR_CAP) and planned empty.
 __global__ __launch_bounds__(kBigWG) void k_plan(PlanArgs A, uint32_t* cnt)
 {
     __shared__ uint32_t s_tmp[kBigWaves];
-    __shared__ uint32_t s_tb[kBigWG];        // tile offsets of a block of segments, for its tile table
+    __shared__ uint32_t s_tb[kBigWG], s_gb[kBigWG];   // chunk and group offsets of a block of segments, for the tables
     __shared__ unsigned long long s_tot;
     __shared__ uint32_t s_ident, s_kmax;
     LevelHdr* hdr = reinterpret_cast<LevelHdr*>(A.plan);
     LargeDesc* desc = reinterpret_cast<LargeDesc*>(A.plan + sizeof(LevelHdr));
     TileRef* tiles = reinterpret_cast<TileRef*>(A.plan + A.tiles_off);
+    TileRef* groups = reinterpret_cast<TileRef*>(A.plan + A.groups_off);
     const uint32_t tid = tid_x();
     if (A.done_rp >= 0 && tid < kBlkClasses) cnt[C_BDONE + tid] = cnt[C_BLOCK + 2 * tid + A.done_rp];
     uint32_t nl = cnt[A.ci];
@@ -207,59 +227,64 @@ __global__ __launch_bounds__(kBigWG) void k_plan(PlanArgs A, uint32_t* cnt)
     if (!ident) atomicAnd(&s_ident, 0u);
     __syncthreads();
     const uint64_t cmax = s_ident ? A.chunk_max_root : A.chunk_max;
-    const uint64_t climit = min(cmax, max((uint64_t)kChunkMin, (s_tot + kWaves * A.min_tiles - 1) / (kWaves * A.min_tiles)));
-    // descriptors: tile and histogram bases are exclusive scans over the
-    // segments (blocks of kBigWG with carries); pad holds the tile base
-    uint32_t tcarry = 0;
-    uint64_t hcarry = 0;
+    const uint64_t climit = min(cmax, max((uint64_t)kChunkMin, (s_tot + A.min_tiles - 1) / A.min_tiles));
+    // descriptors: table, histogram and group bases are exclusive scans over
+    // the segments (blocks of kBigWG with carries)
+    uint32_t tcarry = 0, gcarry = 0;
+    uint64_t hcarry = 0, scarry = 0;
     for (uint32_t b0 = 0; b0 < nl; b0 += kBigWG) {
         const uint32_t i = b0 + tid;
-        uint32_t T = 0, hc = 0;
+        uint32_t T = 0, G = 0, hc = 0, sc = 0;
         LargeDesc D{};
         if (i < nl) {
             D.seg = A.list[i];
-            T = (uint32_t)((D.seg.size + climit * kWaves - 1) / (climit * kWaves));
-            D.T = T;
-            D.chunk = (uint32_t)((D.seg.size + (uint64_t)T * kWaves - 1) / ((uint64_t)T * kWaves));
+            T = (uint32_t)((D.seg.size + climit - 1) / climit);
+            G = hist_groups(T);
+            D.nch = T;
+            D.chunk = (D.seg.size + T - 1) / T;
             D.k = min(dev_treebits(D.seg.size, A.leaf_target, A.max_treebits), A.kmax);
             const uint32_t nspl = (1u << D.k) - 1;
             D.oversample = max(2u, min(A.max_oversample, (kMaxSamples / nspl) & ~1u));
-            hc = ((2u << D.k) - 1) * T * kWaves;
+            hc = (2u << D.k) * T;
+            sc = (2u << D.k) * (G + 1);
             atomicMax(&s_kmax, D.k);
         }
-        uint32_t ttot, htot;
+        uint32_t ttot, gtot, htot, stot;
         const uint32_t tex = block_excl_scan<kBigWaves>(T, &ttot, s_tmp);
+        const uint32_t gex = block_excl_scan<kBigWaves>(G, &gtot, s_tmp);
         const uint32_t hex = block_excl_scan<kBigWaves>(hc, &htot, s_tmp);
+        const uint32_t sex = block_excl_scan<kBigWaves>(sc, &stot, s_tmp);
         if (i < nl) {
-            D.pad = tcarry + tex;
             D.hist_base = (uint32_t)(hcarry + hex);
+            D.gbase = (uint32_t)(scarry + sex);
             desc[i] = D;
         }
-        // this block's entries of the tile table, written by the whole
-        // workgroup (within its capacity; an overflow is flagged below):
-        // tile t of the block belongs to the last segment whose offset is
-        // <= t (every segment has at least one tile)
+        // this block's entries of the two tables, written by the whole
+        // workgroup (within their capacity; an overflow is flagged below):
+        // entry t of the block belongs to the last segment whose offset is
+        // <= t (every segment has at least one chunk and one group)
         s_tb[tid] = tex;
+        s_gb[tid] = gex;
         __syncthreads();
         const uint32_t nseg = min(nl - b0, (uint32_t)kBigWG);
-        for (uint32_t t = tid; t < ttot && tcarry + t < A.tiles_cap; t += kBigWG) {
-            uint32_t lo = 0, hi = nseg;
-            while (hi - lo > 1) {
-                const uint32_t mid = (lo + hi) >> 1;
-                if (s_tb[mid] <= t) lo = mid;
-                else hi = mid;
+        auto fill = [&](TileRef* out, const uint32_t* first, uint32_t total, uint32_t carry, uint64_t cap) {
+            for (uint32_t t = tid; t < total && carry + t < cap; t += kBigWG) {
+                const uint32_t lo = find_run(first, nseg, t);
+                out[carry + t] = TileRef{ b0 + lo, t - first[lo] };
             }
-            tiles[tcarry + t] = TileRef{ b0 + lo, t - s_tb[lo] };
-        }
-        __syncthreads();     // s_tb is written again by the next block
+        };
+        fill(tiles, s_tb, ttot, tcarry, A.tiles_cap);
+        fill(groups, s_gb, gtot, gcarry, A.groups_cap);
+        __syncthreads();     // the offsets are written again by the next block
         tcarry += ttot;
+        gcarry += gtot;
         hcarry += htot;
+        scarry += stot;
     }
-    const bool fits = tcarry <= A.tiles_cap && hcarry <= A.hist_cap && hcarry <= 0xFFFFFFFFull && nl <= A.trees_cap;
+    const bool fits = tcarry <= A.tiles_cap && gcarry <= A.groups_cap && hcarry <= A.hist_cap && scarry <= A.gsum_cap &&
+                      hcarry <= 0xFFFFFFFFull && nl <= A.trees_cap;
     if (!fits && tid == 0) flag_error(cnt, ERR_CAP);
-    const uint32_t ntiles = fits ? tcarry : 0u;
-    if (tid == 0)
-        *hdr = LevelHdr{ fits ? nl : 0u, ntiles, fits ? (uint32_t)hcarry : 0u, s_kmax, { 0u, 0u, 0u, 0u } };
+    if (tid == 0) *hdr = LevelHdr{ fits ? nl : 0u, fits ? tcarry : 0u, fits ? gcarry : 0u, s_kmax, { 0u, 0u, 0u, 0u } };
 }
 
 // Splitter trees of the large segments of a level, one workgroup each.
@@ -268,9 +293,7 @@ __global__ __launch_bounds__(kBigWG) void k_plan(PlanArgs A, uint32_t* cnt)
 // oversample/2 + oversample*i (the reference's choice for oversample factor 2,
 // bingmann-sample_sort_tree_builder.hpp:44-58) and the tree is stored in
 // level order: trees[seg*2048 + t], t = 1..nspl, followed by the splitters in
-// sorted order at trees[seg*2048 + 1024 + i], i < nspl.  ROOT: the roots
-// of a sort, whose keys are not extracted yet; the samples are read from the
-// arena directly.
+// sorted order at trees[seg*2048 + 1024 + i], i < nspl.
 //
 // A root's samples also choose the format of its keys (KeyFmt).  Eight
 // characters of a small alphabet leave many strings equal: 20 M windows of
@@ -283,9 +306,11 @@ __global__ __launch_bounds__(kBigWG) void k_plan(PlanArgs A, uint32_t* cnt)
 // keys hold 21, 16 or 12 packed characters instead.  A character the sample
 // missed is found by the extraction (ERR_ALPHA) and the sort starts over
 // unpacked.
-// what a kernel of a level knows of its segments: no roots, roots with plain
-// keys, or roots that may pack theirs
-constexpr int kNoRoot = 0, kRootPlain = 1, kRootPack = 2;
+
+// what the kernels of a level know of its segments' strings: buckets of the
+// level before, roots with plain keys, roots that may pack theirs, or
+// segments of an earlier round
+constexpr int kFromRuns = 0, kRootPlain = 1, kRootPack = 2, kFromPerm = 3;
 
 struct TreeLds {
     key64 samp[kMaxSamples + 1];      // + 1: a merge step reads the slot after the one it takes
@@ -294,7 +319,6 @@ struct TreeLds {
     uint8_t lut[kLutBytes];           // code table
 };
 constexpr float kPackRun = 1.0f;
-
 constexpr uint32_t kAlphaSamples = 256;
 
 // the alphabet of one string per thread, as a bitmap in S.alpha (cleared by the caller)
@@ -320,7 +344,7 @@ __device__ __forceinline__ void sample_alphabet(const Item& seg, const Bufs& B, 
     }
 }
 
-template <int ROOT>
+template <int SRC>
 __device__ __forceinline__ void tree_of_segment(LargeDesc* Dp, uint32_t si, const Bufs& B, uint64_t seed, key64* tree,
                                                 TreeLds& S)
 {
@@ -331,7 +355,6 @@ __device__ __forceinline__ void tree_of_segment(LargeDesc* Dp, uint32_t si, cons
         if (tid_x() == 0) flag_error(B.cnt, ERR_BOUNDS);
         return;
     }
-    const key64* K = (seg.flags & F_BUFB) ? B.key1 : B.key0;
     const int k = (int)D.k, nspl = (1 << k) - 1, a = (int)D.oversample;
     const uint32_t ss = (uint32_t)(a * nspl);
     uint32_t P = 64;
@@ -349,7 +372,7 @@ __device__ __forceinline__ void tree_of_segment(LargeDesc* Dp, uint32_t si, cons
     static_assert(kMaxSamples % kBigWG == 0 && kPer == 4, "four samples per thread");
     const uint32_t o = tid_x() * kPer;
     const bool act = o < P;
-    constexpr bool may_pack = ROOT == kRootPack;
+    constexpr bool may_pack = SRC == kRootPack;
     if (may_pack) {     // (cleared before the merge rounds' barriers)
         if (tid_x() < 8) S.alpha[tid_x()] = 0;
         if (tid_x() == 8) S.dups = 0;
@@ -359,10 +382,39 @@ __device__ __forceinline__ void tree_of_segment(LargeDesc* Dp, uint32_t si, cons
         return seg.begin + (uint32_t)(((h >> 32) * (uint64_t)seg.size) >> 32);
     };
     key64 v[kPer];
+    if (SRC == kFromRuns) {
+        // the samples' runs are searched in a copy of the bucket's row of
+        // first positions (in LDS, before the samples go there), or of every
+        // stride-th entry of it and then in the row itself
+        const Runs R = runs_of(B, seg);
+        constexpr uint32_t kRowMax = 2 * kMaxSamples;
+        uint32_t* s_v = reinterpret_cast<uint32_t*>(s_samp);
+        const uint32_t stride = (R.nch + kRowMax - 1) / kRowMax, ns = (R.nch + stride - 1) / stride;
+        for (uint32_t c = tid_x(); c < ns; c += kBigWG) s_v[c] = R.V[c * stride];
+        __syncthreads();
+        uint32_t q[kPer];
 #pragma unroll
-    for (int e = 0; e < kPer; ++e) {
-        v[e] = ~0ull;
-        if (o + e < ss) v[e] = ROOT ? load_key(B.arena, B.alen, str_off(B, sample(o + e))) : K[sample(o + e)];
+        for (int e = 0; e < kPer; ++e) {
+            const uint32_t pos = sample(min(o + e, ss - 1));
+            uint32_t c = find_run(s_v, ns, pos) * stride;
+            if (stride > 1) c += find_run(R.V + c, min(stride, R.nch - c), pos);     // (uniform branch)
+            q[e] = R.S[c] + (pos - R.V[c]);
+        }
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) {
+            const key64 x = R.K[checked_place(B, q[e])];
+            v[e] = o + e < ss ? x : ~0ull;
+        }
+        __syncthreads();     // the row's copy is no longer read
+    } else {
+        const uint32_t depth = SRC == kFromPerm ? seg_depth(B, seg.rbeg) : 0u;
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) {
+            v[e] = ~0ull;
+            if (o + e >= ss) continue;
+            const uint32_t pos = sample(o + e);
+            v[e] = string_key(B, SRC == kFromPerm ? B.perm[pos] : pos, depth);
+        }
     }
     uint32_t fmt = 0;
     for (;;) {
@@ -461,35 +513,15 @@ __device__ __forceinline__ void tree_of_segment(LargeDesc* Dp, uint32_t si, cons
     for (int i = tid_x(); i < nspl; i += kBigWG) tree[1024 + i] = sorted[a / 2 + a * i];
 }
 
-template <int ROOT>
+template <int SRC>
 __global__ __launch_bounds__(kBigWG) void k_tree(Plan P, Bufs B, uint64_t seed, key64* trees)
 {
     __shared__ TreeLds S;
     const uint32_t nlarge = P.hdr->nlarge;
     for (uint32_t si = blockIdx.x; si < nlarge; si += gridDim.x) {
         __syncthreads();     // the previous segment's samples are consumed
-        tree_of_segment<ROOT>(P.desc + si, si, B, seed, trees + (uint64_t)si * kTreeSlots, S);
+        tree_of_segment<SRC>(P.desc + si, si, B, seed, trees + (uint64_t)si * kTreeSlots, S);
     }
-}
-
-// Classify one tile of kWaves wave chunks.  Each wave ranks its own chunk
-// of D.chunk keys stably (ballot matching, ranks follow input order) and the
-// chunk counts go to hist[hist_base + (b * T + t) * kWaves + w]: bucket-major,
-// then tile, then wave -- the order of the reference's prefix sum
-// (.hpp:1437-1460) with wave chunks as the parts -- so an exclusive scan of
-// hist gives every chunk's base offset per bucket.  bktrank gets bucket and
-// rank inside the chunk.  ROOT (the roots of a sort, positions =
-// input indices) the keys are extracted from the arena here and stored: this
-// replaces the separate extraction pass and saves reading the keys back.
-// The tree and the sorted splitters sit in static LDS (their addresses are
-// constants, so a descent step needs no address arithmetic); the per-wave
-// 16-bit counts[kWaves][2^(kmax+1)] in dynamic LDS, sized by the largest
-// tree of the level (kmax treebits); a packed root's code table takes their
-// place while its keys are extracted.
-__host__ __device__ constexpr uint32_t count_lds_bytes(int kmax)
-{
-    const uint32_t counts = kWaves * (2u << kmax) * 2u;
-    return counts > kLutBytes ? counts : kLutBytes;
 }
 
 // Load a read-only value that every lane of the wave reads at the same
@@ -508,289 +540,9 @@ __device__ __forceinline__ T load_uniform(const T* p)
     return v;
 }
 
-// NB: bits of a bucket id in this launch (kmax + 1, at least 8).  Lanes of
-// one bucket are matched through a per-wave LDS table of lane masks on the
-// id's low kPeerBits bits and by ballots on the rest (a few vector
-// instructions per bit); ids of 11 bits use ballots only, since their
-// launch's LDS leaves no room for the tables at full occupancy.
-template <int NB>
-constexpr int kPeerBits = NB <= 10 ? (NB < 8 ? NB : 8) : 0;
-
-template <int NB, int ROOT>
-__device__ __forceinline__ void count_tile(uint32_t ti, const Plan& P, const Bufs& B, const key64* trees,
-                                           uint32_t* hist, int kmax, key64* s_tree, key64* s_sorted,
-                                           uint16_t* s_hist_base, uint64_t* s_peer)
-{
-    constexpr uint32_t kNoBkt = (1u << NB) - 1;   // id of inactive lanes, above every bucket of the launch
-    const uint32_t nb2 = 2u << kmax;               // bucket slots per wave
-    ti = __builtin_amdgcn_readfirstlane(ti);
-    const TileRef tr = load_uniform(P.tiles + ti);     // (read-only here, the same for the workgroup)
-    const LargeDesc D = load_uniform(P.desc + tr.seg);
-    const Item seg = D.seg;
-    const int k = (int)D.k, nbkt = (2 << k) - 1;
-    if (k > kmax || k + 1 > NB) {   // the launch must size LDS and ids for every tree of the level
-        if (tid_x() == 0) flag_error(B.cnt, ERR_BOUNDS);
-        return;
-    }
-    const key64* tree = trees + (uint64_t)tr.seg * kTreeSlots;
-    const int nspl = (1 << k) - 1;
-    for (int i = tid_x(); i <= nspl; i += kWG) s_tree[i] = tree[i];
-    for (int i = tid_x(); i < nspl; i += kWG) s_sorted[i] = tree[1024 + i];
-    const key64* K = (seg.flags & F_BUFB) ? B.key1 : B.key0;
-    const uint32_t t = tr.t;
-    const uint32_t w = wave_id(), lane = lane_id();
-    uint16_t* s_hist = s_hist_base + w * nb2;      // this wave's counts
-    uint64_t* peer_tab = s_peer + (w << kPeerBits<NB>);
-    const uint64_t lanebit = 1ull << lane;
-    const uint32_t cb = (t * kWaves + w) * D.chunk;
-    const uint32_t cmax = (seg.flags & F_IDENT) ? kChunkMaxIdent : kChunkMax;
-    const uint32_t ce = (item_ok(seg, B) && t < D.T && D.chunk <= cmax) ? min(seg.size, cb + D.chunk) : 0u;
-    const uint32_t fmt = ROOT == kRootPack ? (seg.flags & kFmtMask) >> kFmtShift : 0u;
-    const bool plain = ROOT && fmt == 0;     // (uniform)
-    if (fmt) {
-        // a packed root's keys are extracted first, in a loop of their own, and
-        // read back from the cache below: extracting them inside the main loop
-        // takes 116 registers instead of 72 (4 instead of 7 waves per SIMD)
-        uint8_t* s_lut = reinterpret_cast<uint8_t*>(s_hist_base);
-        static_assert(kLutBytes == kWG, "a table byte per thread");
-        s_lut[tid_x()] = B.lut[(uint64_t)tr.seg * kLutBytes + tid_x()];
-        __syncthreads();
-        bool bad = false;
-#pragma unroll 2
-        for (uint32_t p = cb + lane; p < ce; p += 64)
-            B.key0[seg.begin + p] =
-                pack_key_fmt(load_chars24(B.arena, B.alen, str_off(B, seg.begin + p)), fmt, s_lut, &bad);
-        if (bad) flag_error(B.cnt, ERR_ALPHA);
-        __syncthreads();     // the table is no longer read
-    }
-    for (uint32_t i = tid_x(); i < kWaves * nb2; i += kWG) s_hist_base[i] = 0;
-    __syncthreads();
-    // kGroups 64-key groups per iteration: all loads are in flight before the
-    // tree descents, then the groups are ranked in order (stable)
-    constexpr int kGroups = 8;
-    // extracting at the root, the string offsets of the next iteration are
-    // loaded one iteration ahead (the first link of offset -> characters)
-    uint64_t off_next[kGroups];
-    if (plain) {
-#pragma unroll
-        for (int j = 0; j < kGroups; ++j) {
-            const uint32_t p = cb + 64 * j + lane;
-            off_next[j] = p < ce ? str_off(B, seg.begin + p) : 0ull;
-        }
-    }
-    for (uint32_t g = cb; g < ce; g += 64 * kGroups) {
-        key64 kv[kGroups];
-        if (plain) {
-            uint64_t off[kGroups];
-#pragma unroll
-            for (int j = 0; j < kGroups; ++j) off[j] = off_next[j];
-#pragma unroll
-            for (int j = 0; j < kGroups; ++j) {
-                const uint32_t p = g + 64 * kGroups + 64 * j + lane;
-                off_next[j] = p < ce ? str_off(B, seg.begin + p) : 0ull;
-            }
-#pragma unroll
-            for (int j = 0; j < kGroups; ++j) {
-                const uint32_t p = g + 64 * j + lane;
-                kv[j] = p < ce ? load_key(B.arena, B.alen, off[j]) : 0ull;
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < kGroups; ++j) {
-                const uint32_t p = g + 64 * j + lane;
-                kv[j] = p < ce ? K[seg.begin + p] : 0ull;
-            }
-        }
-        uint32_t bv[kGroups];
-        classify_keys<kGroups>(kv, s_tree, s_sorted, k, bv);
-#pragma unroll
-        for (int j = 0; j < kGroups; ++j) {
-            const uint32_t p = g + 64 * j + lane;
-            if (p >= ce) bv[j] = kNoBkt;
-        }
-#pragma unroll
-        for (int j = 0; j < kGroups; ++j) {
-            const uint32_t p = g + 64 * j + lane;
-            uint64_t peers;
-            if constexpr (kPeerBits<NB> > 0) peers = match_bucket_lds<NB, kPeerBits<NB>>(bv[j], peer_tab, lanebit);
-            else peers = match_bucket<NB>(bv[j]);
-            const uint32_t r = (uint32_t)__popcll(peers & lanemask_lt());
-            if (p < ce) {
-                const uint32_t old = s_hist[bv[j]];
-                if (r == 0) s_hist[bv[j]] = (uint16_t)(old + (uint32_t)__popcll(peers));
-                B.bktrank[seg.begin + p] = (bv[j] << kRankBits) | (old + r);
-            }
-        }
-        if (plain) {     // the extracted keys, for the scatter
-#pragma unroll
-            for (int j = 0; j < kGroups; ++j) {
-                const uint32_t p = g + 64 * j + lane;
-                if (p < ce) B.key0[seg.begin + p] = kv[j];
-            }
-        }
-    }
-    __syncthreads();
-    uint32_t* h = hist + D.hist_base;
-    for (int i = tid_x(); i < nbkt * kWaves; i += kWG) {
-        const uint32_t b = (uint32_t)i / kWaves, ww = (uint32_t)i % kWaves;
-        h[((uint32_t)b * D.T + t) * kWaves + ww] = s_hist_base[ww * nb2 + b];
-    }
-}
-
-// XCD-contiguous tiles: workgroup g runs on XCD g % kXcds (the grid is a
-// multiple of kXcds), and XCD x takes the tiles [N x / kXcds, N (x+1) /
-// kXcds): one per workgroup, or with LOOP (levels planned on the device)
-// each workgroup loops over its XCD's share.
-template <int NB, bool LOOP, int ROOT>
-__global__ __launch_bounds__(kWG) void k_count(Plan P, Bufs B, const key64* trees, uint32_t* hist, int kmax)
-{
-    static_assert(NB >= 2 && NB <= kMaxTreebits + 1, "bucket ids of up to 2047 buckets");
-    static_assert(kChunkMax <= 65535 && kChunkMaxIdent <= 65535, "per-wave bucket counts must fit 16 bits");
-    extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ key64 s_tree[1 << (NB - 1)];        // trees of up to NB - 1 levels
-    __shared__ key64 s_sorted[1 << (NB - 1)];
-    __shared__ uint64_t s_peer[kWaves << kPeerBits<NB>];     // lane-mask tables, kept zero between uses
-    uint16_t* s_hist_base = reinterpret_cast<uint16_t*>(smem);
-    if constexpr (kPeerBits<NB> > 0)
-        for (int i = tid_x(); i < (kWaves << kPeerBits<NB>); i += kWG) s_peer[i] = 0;   // (a barrier follows in count_tile)
-    const uint32_t N = P.hdr->ntiles, per = gridDim.x / kXcds, xcd = blockIdx.x % kXcds;
-    const uint32_t thi = (uint32_t)((uint64_t)N * (xcd + 1) / kXcds);
-    uint32_t ti = (uint32_t)((uint64_t)N * xcd / kXcds) + blockIdx.x / kXcds;
-    if (!LOOP) {
-        if (ti < thi) count_tile<NB, ROOT>(ti, P, B, trees, hist, kmax, s_tree, s_sorted, s_hist_base, s_peer);
-        return;
-    }
-    for (; ti < thi; ti += per) {
-        __syncthreads();     // the previous tile's counts are written out
-        count_tile<NB, ROOT>(ti, P, B, trees, hist, kmax, s_tree, s_sorted, s_hist_base, s_peer);
-    }
-}
-
-// exclusive scan of hist[0..len): block sums
-constexpr int kScanPer = 16;
-constexpr int kScanBlock = kWG * kScanPer;   // 4096 entries per block
-
-// (the length is the level's hl; workgroups loop over the blocks of kScanBlock entries)
-__global__ __launch_bounds__(kWG) void k_scan_reduce(const uint32_t* in, const LevelHdr* hdr, uint32_t* part)
-{
-    __shared__ uint32_t s_tmp[16];
-    const uint32_t len = hdr->hl, nb = (len + kScanBlock - 1) / kScanBlock;
-    for (uint32_t blk = blockIdx.x; blk < nb; blk += gridDim.x) {
-        const uint32_t base = blk * kScanBlock;
-        uint32_t sum = 0;
-#pragma unroll
-        for (int j = 0; j < kScanPer; ++j) {
-            const uint32_t i = base + j * kWG + tid_x();
-            if (i < len) sum += in[i];
-        }
-        uint32_t tot;
-        block_excl_scan<kWaves>(sum, &tot, s_tmp);
-        if (tid_x() == 0) part[blk] = tot;
-    }
-}
-
-// exclusive scan of the block sums (one workgroup, any count)
-__global__ __launch_bounds__(kWG) void k_scan_top(uint32_t* part, const LevelHdr* hdr)
-{
-    __shared__ uint32_t s_tmp[16];
-    const uint32_t nparts = (hdr->hl + kScanBlock - 1) / kScanBlock;
-    uint32_t carry = 0;
-    for (uint32_t base = 0; base < nparts; base += kWG) {
-        const uint32_t i = base + tid_x();
-        const uint32_t v = i < nparts ? part[i] : 0u;
-        uint32_t tot;
-        const uint32_t ex = block_excl_scan<kWaves>(v, &tot, s_tmp);
-        if (i < nparts) part[i] = carry + ex;
-        carry += tot;
-    }
-}
-
-// exclusive scan inside each block, offset by its block prefix (in place)
-// (data is 16-byte aligned: a thread's kScanPer consecutive entries move as
-// 16-byte vectors, except in a block cut short by len)
-__global__ __launch_bounds__(kWG) void k_scan_down(uint32_t* data, const LevelHdr* hdr, const uint32_t* part)
-{
-    static_assert(kScanPer % 4 == 0, "whole 16-byte vectors per thread");
-    __shared__ uint32_t s_tmp[16];
-    const uint32_t len = hdr->hl, nb = (len + kScanBlock - 1) / kScanBlock;
-    for (uint32_t blk = blockIdx.x; blk < nb; blk += gridDim.x) {
-        const uint32_t base = blk * kScanBlock + tid_x() * kScanPer;
-        const bool full = base + kScanPer <= len;
-        uint32_t v[kScanPer];
-        if (full) {
-            const uint4* p = reinterpret_cast<const uint4*>(data + base);
-#pragma unroll
-            for (int q = 0; q < kScanPer / 4; ++q) {
-                const uint4 x = p[q];
-                v[4 * q] = x.x;
-                v[4 * q + 1] = x.y;
-                v[4 * q + 2] = x.z;
-                v[4 * q + 3] = x.w;
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < kScanPer; ++j) v[j] = base + j < len ? data[base + j] : 0u;
-        }
-        uint32_t sum = 0;
-#pragma unroll
-        for (int j = 0; j < kScanPer; ++j) sum += v[j];
-        uint32_t tot;
-        uint32_t run = block_excl_scan<kWaves>(sum, &tot, s_tmp) + part[blk];
-        uint32_t o[kScanPer];
-#pragma unroll
-        for (int j = 0; j < kScanPer; ++j) {
-            o[j] = run;
-            run += v[j];
-        }
-        if (full) {
-            uint4* p = reinterpret_cast<uint4*>(data + base);
-#pragma unroll
-            for (int q = 0; q < kScanPer / 4; ++q) p[q] = make_uint4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]);
-        } else {
-#pragma unroll
-            for (int j = 0; j < kScanPer; ++j)
-                if (base + j < len) data[base + j] = o[j];
-        }
-    }
-}
-
-// LDS layout of k_scatter (dynamic shared memory).  In a level of root
-// segments (IDENT: indices = positions) a chunk stages 2-byte positions
-// instead of 4-byte indices, which leaves room for longer chunks: longer
-// runs per bucket, fewer partial cache lines written.
-template <bool IDENT>
-struct ScatLds {
-    static constexpr uint32_t kMax = IDENT ? kChunkMaxIdent : kChunkMax;
-    static constexpr int kPer = (kMax + kBigWG - 1) / kBigWG;   // keys per thread
-    static constexpr uint32_t kKeyOff = 0;
-    static constexpr uint32_t kIdxOff = kKeyOff + kMax * 8;
-    static constexpr uint32_t kBktOff = kIdxOff + kMax * (IDENT ? 2 : 4);
-    static constexpr uint32_t kStartOff = (kBktOff + kMax * 2 + 15) / 16 * 16;
-    static constexpr uint32_t kBaseOff = kStartOff + 2048 * 4;
-    static constexpr uint32_t kTmpOff = kBaseOff + 2048 * 4;
-    static constexpr uint32_t kBytes = kTmpOff + 64 * 4;
-};
-static_assert(ScatLds<false>::kBytes <= 160 * 1024 && ScatLds<true>::kBytes <= 160 * 1024,
-              "a chunk image fits a CU's LDS");
-
-// Move wave chunks (at most kChunkMax keys each, kChunkMaxIdent in a level
-// of roots) to their buckets (distribute, .hpp:1464-1490, but stable).  A
-// chunk is first reordered by bucket in
-// LDS, then written out position by position, so consecutive lanes store
-// consecutive addresses inside each bucket: full cache lines instead of the
-// scattered 8-byte stores of a direct scatter.
-//
-// The chunk's LDS image takes most of a CU's LDS, so one workgroup runs per
-// CU; to keep memory busy, each workgroup loops over chunks and loads the
-// next chunk (keys, indices, ranks and histogram entries) into registers
-// before it reorders and writes the current one.  Chunks are split into
-// kXcds contiguous ranges, one per XCD (workgroup g runs on XCD g % kXcds),
-// so the chunks in flight on an XCD are neighbours that share histogram
-// lines and bucket output lines in its L2.
-
 // tid_x() through an opaque move: addresses derived from it are
-// recomputed per chunk instead of being hoisted out of the chunk loop,
-// where they would hold registers the two chunk buffers need
+// recomputed where they are used instead of being hoisted out of loops,
+// where they would hold registers
 __device__ __forceinline__ uint32_t scat_tid()
 {
     uint32_t t;
@@ -798,235 +550,452 @@ __device__ __forceinline__ uint32_t scat_tid()
     return t;
 }
 
-template <int PER>
-struct ScatChunk {       // one chunk's description and its prefetched inputs
-    LargeDesc D;
-    uint32_t t, w, cb, m;
-    uint32_t br[PER], iv[PER];
-    key64 kv[PER];
-    uint32_t h0, h0n, h1, h1n, hseg;   // histogram entries of buckets tid, tid + kBigWG; segment base
+// The places of a bucket's positions [v0, v0 + m) for a workgroup of NW
+// waves: position v0 + p lies at p + delta[r] for the run r holding it, and r
+// is the number of run starts at or before p in a bitmap, less one.  Runs
+// average tens of strings, so a bit per position costs less to build and to
+// read than a search per position.
+template <int MAXP>
+struct RunMap {
+    uint32_t delta[MAXP];
+    uint32_t bits[MAXP / 32];
+    uint32_t pre[MAXP / 32];
+    uint32_t tmp[16];
+};
+template <int NW, int MAXP>
+__device__ __forceinline__ void map_runs(const Runs& R, uint32_t vend, uint32_t v0, uint32_t m, RunMap<MAXP>& M)
+{
+    constexpr uint32_t T = NW * 64;
+    constexpr uint32_t W = MAXP / 32;
+    static_assert(W <= T, "a thread per bitmap word");
+    const uint32_t tid = scat_tid(), w = wave_id(), lane = lane_id();
+    if (tid < W) M.bits[tid] = 0;
+    // the run holding v0: T samples of the row, then their interval
+    const uint32_t step = (R.nch + T - 1) / T;
+    const uint32_t si = tid * step;
+    const uint32_t le = (uint32_t)__popcll(__ballot(si < R.nch && R.V[si] <= v0));
+    if (lane == 0) M.tmp[w] = le;
+    __syncthreads();
+    uint32_t c0 = 0;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) c0 += M.tmp[i];
+    c0 = (c0 ? c0 - 1 : 0u) * step;
+    if (step > 1) {     // (uniform) every wave looks at the interval
+        if (step <= 64) {
+            const uint32_t c = c0 + lane;
+            const uint32_t in = (uint32_t)__popcll(__ballot(lane < step && c < R.nch && R.V[c] <= v0));
+            c0 += in ? in - 1 : 0u;
+        } else {
+            c0 += find_run(R.V + c0, min(step, R.nch - c0), v0);
+        }
+    }
+    uint32_t base = 0;       // runs mapped so far
+    for (uint32_t cb = c0;; cb += T) {
+        __syncthreads();     // tmp is read (first pass: and the bitmap is cleared)
+        const uint32_t c = cb + tid;
+        uint32_t v = 0, nx = 0, s = 0;
+        if (c < R.nch) {
+            v = R.V[c];
+            nx = c + 1 < R.nch ? R.V[c + 1] : vend;
+            s = R.S[c];
+        }
+        const bool use = nx > v && nx > v0 && v < v0 + m;
+        const uint64_t bal = __ballot(use);
+        if (lane == 0) M.tmp[w] = (uint32_t)__popcll(bal);
+        __syncthreads();
+        uint32_t before = 0, all = 0;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            const uint32_t t = M.tmp[i];
+            before += i < (int)w ? t : 0u;
+            all += t;
+        }
+        if (use) {
+            const uint32_t r = base + before + (uint32_t)__popcll(bal & lanemask_lt());
+            const uint32_t p = v > v0 ? v - v0 : 0u;
+            if (r < MAXP) M.delta[r] = s + v0 - v;
+            atomicOr(&M.bits[p >> 5], 1u << (p & 31));
+        }
+        base += all;
+        if (cb + T >= R.nch || R.V[cb + T] >= v0 + m) break;     // (uniform)
+    }
+    __syncthreads();
+    // exclusive prefix of the words' bit counts
+    const uint32_t pc = tid < W ? (uint32_t)__popc(M.bits[tid]) : 0u;
+    uint32_t x = pc;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t y = (uint32_t)__shfl_up((int)x, d, 64);
+        if (lane >= (uint32_t)d) x += y;
+    }
+    if (lane == 63) M.tmp[w] = x;
+    __syncthreads();
+    uint32_t wp = 0;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) wp += i < (int)w ? M.tmp[i] : 0u;
+    if (tid < W) M.pre[tid] = wp + x - pc;
+    __syncthreads();
+}
+template <int MAXP>
+__device__ __forceinline__ uint32_t mapped_place(const Bufs& B, const RunMap<MAXP>& M, uint32_t p)
+{
+    const uint32_t below = M.bits[p >> 5] & (0xFFFFFFFFu >> (31 - (p & 31)));
+    const uint32_t r = M.pre[p >> 5] + (uint32_t)__popc(below);
+    return checked_place(B, p + M.delta[r ? min(r - 1, (uint32_t)MAXP - 1) : 0u]);
+}
+
+// Partition one chunk of a segment (classify, .hpp:1413-1435, and distribute,
+// .hpp:1464-1490, in one pass): each wave classifies its part of the chunk
+// with the splitter tree in LDS and ranks it stably (ballot matching and
+// per-wave bucket counts, ranks follow input order), a scan of the counts
+// places every (bucket, wave), the keys and then the indices are staged in
+// LDS in that order and written back in place of the chunk, whole lines at a
+// time.  The chunk's bucket counts and starts go to its row of hist.
+//
+// 2 GiB of random strings, root level (reading the arena, 511 splitters):
+// 0.60 ms, 5.3 TB/s of the 3.2 GB it reads and writes, the rate of a plain
+// copy; counting first and scattering afterwards took 0.71 + 0.50 ms.
+//
+// LDS: the key stage (the lane-mask tables of match_bucket_lds, or the run
+// map of a bucket's chunk, before that), the per-wave counts and the tree;
+// three workgroups per CU up to 9 treebits, two with 10.
+template <int NB>
+struct PartLds {
+    static constexpr uint32_t kSlots = 1u << NB;             // bucket slots per wave
+    static constexpr uint32_t kKeyOff = 0;
+    static constexpr uint32_t kCntOff = kPartMax * 8;
+    static constexpr uint32_t kTreeOff = kCntOff + kPartWaves * kSlots * 2;
+    static constexpr uint32_t kTmpOff = kTreeOff + kSlots / 2 * 8;
+    static constexpr uint32_t kBytes = kTmpOff + 64;
+    static constexpr int kPeerBits = NB < 8 ? NB : 8;
+    static constexpr uint32_t kMapOff = 0;
+    static_assert(((uint32_t)kPartWaves << kPeerBits << 3) <= kCntOff, "the lane-mask tables fit the key stage");
+    static_assert(kMapOff + sizeof(RunMap<kPartMax>) <= kCntOff, "the run map fits the key stage");
 };
 
-// Issue the loads of chunk c.  Every load is unconditional (indices are
-// clamped into the arrays and invalid lanes discard their values when the
-// chunk is processed): the same number of loads every time lets the
-// compiler wait for exactly the older loads when the chunk is used, while
-// the next chunk's loads stay in flight.
-template <bool IDENT>
-__device__ __forceinline__ void scat_fetch(const LargeDesc* __restrict__ desc, const TileRef* __restrict__ tiles,
-                                           const Bufs& B, const uint32_t* __restrict__ hscan, uint32_t c,
-                                           ScatChunk<ScatLds<IDENT>::kPer>& S)
-{
-    const uint32_t tid = scat_tid();
-    // the chunk's tile and descriptor are read-only in this kernel and the
-    // same for the whole workgroup: scalar loads, counted apart from the
-    // vector loads and stores of the chunks
-    c = __builtin_amdgcn_readfirstlane(c);
-    const TileRef tr = load_uniform(tiles + c / kWaves);
-    S.w = c % kWaves;
-    S.t = tr.t;
-    S.D = load_uniform(desc + tr.seg);
-    const Item seg = S.D.seg;
-    S.cb = (S.t * kWaves + S.w) * S.D.chunk;
-    const bool ok = item_ok(seg, B) && S.t < S.D.T && S.D.chunk <= ScatLds<IDENT>::kMax && S.cb < seg.size;
-    S.m = ok ? min(seg.size - S.cb, S.D.chunk) : 0u;
-    const key64* K = (seg.flags & F_BUFB) ? B.key1 : B.key0;
-    // a root's indices are implicit: its third load repeats the rank load
-    const uint32_t* I = (seg.flags & F_IDENT) ? B.bktrank : (seg.flags & F_BUFB) ? B.idx1 : B.idx0;
-    const uint32_t qmax = B.n - 1;
-#pragma unroll
-    for (int e = 0; e < ScatLds<IDENT>::kPer; ++e) {
-        const uint32_t q = min(seg.begin + S.cb + e * kBigWG + tid, qmax);
-        S.br[e] = B.bktrank[q];
-        S.kv[e] = K[q];
-        if (!IDENT) S.iv[e] = I[q];     // (a level of roots stages positions)
-    }
-    // histogram entries; entry e's count is scan[e + 1] - scan[e], and the
-    // entry after the segment's last one is segbase + size (fixed up on use)
-    const uint32_t* h = hscan + S.D.hist_base;
-    const uint32_t T = max(S.D.T, 1u), nbkt = (2u << S.D.k) - 1;
-    const uint32_t last = ((nbkt - 1) * T + (T - 1)) * kWaves + (kWaves - 1);
-    const uint32_t t = min(S.t, T - 1);
-    const uint32_t e0 = (min(tid, nbkt - 1) * T + t) * kWaves + S.w;
-    const uint32_t e1 = (min(tid + kBigWG, nbkt - 1) * T + t) * kWaves + S.w;
-    S.hseg = h[0];
-    S.h0 = h[e0];
-    S.h0n = h[min(e0 + 1, last)];
-    S.h1 = h[e1];
-    S.h1n = h[min(e1 + 1, last)];
-}
-
-// Stage one prefetched chunk in LDS, reordered by bucket (after the
-// previous chunk's image has been written out).  Returns false (uniformly)
-// for an empty or inconsistent chunk.
-template <bool IDENT>
-__device__ __forceinline__ bool scat_stage(const ScatChunk<ScatLds<IDENT>::kPer>& S, const Bufs& B,
+template <int NB, int SRC>
+__device__ __forceinline__ void part_chunk(uint32_t ti, const Plan& P, const Bufs& B, const key64* trees, bool one,
                                            unsigned char* smem)
 {
-    using L = ScatLds<IDENT>;
-    const uint32_t tid = scat_tid();
+    using L = PartLds<NB>;
+    constexpr int kE = kPartGroups;
+    constexpr uint32_t T = kPartThreads;
     key64* s_key = reinterpret_cast<key64*>(smem + L::kKeyOff);
-    uint32_t* s_idx = reinterpret_cast<uint32_t*>(smem + L::kIdxOff);
-    uint16_t* s_pos = reinterpret_cast<uint16_t*>(smem + L::kIdxOff);
-    uint16_t* s_bkt = reinterpret_cast<uint16_t*>(smem + L::kBktOff);
-    uint32_t* s_start = reinterpret_cast<uint32_t*>(smem + L::kStartOff);
-    uint32_t* s_base = reinterpret_cast<uint32_t*>(smem + L::kBaseOff);
+    uint64_t* s_peer = reinterpret_cast<uint64_t*>(smem + L::kKeyOff);
+    uint16_t* s_cnt = reinterpret_cast<uint16_t*>(smem + L::kCntOff);
+    key64* s_tree = reinterpret_cast<key64*>(smem + L::kTreeOff);
     uint32_t* s_tmp = reinterpret_cast<uint32_t*>(smem + L::kTmpOff);
-    __syncthreads();     // the previous chunk's LDS image has been written out
-    const uint32_t m = S.m;
-    if (m == 0) return false;
-    const Item seg = S.D.seg;
-    const uint32_t nbkt = (2u << S.D.k) - 1;
-    const uint32_t segend = S.hseg + seg.size;
-    const uint32_t last = ((nbkt - 1) * S.D.T + (S.D.T - 1)) * kWaves + (kWaves - 1);
-    const uint32_t b0 = tid, b1 = tid + kBigWG;
-    uint32_t c0 = 0, c1 = 0;
-    if (b0 < nbkt) {
-        const uint32_t e = (b0 * S.D.T + S.t) * kWaves + S.w;
-        c0 = (e == last ? segend : S.h0n) - S.h0;
-        s_base[b0] = S.h0 - S.hseg;
+    ti = __builtin_amdgcn_readfirstlane(ti);
+    // (read-only here, the same for the workgroup)
+    const TileRef tr = one ? TileRef{ 0u, ti } : load_uniform(P.tiles + ti);
+    const LargeDesc D = load_uniform(P.desc + tr.seg);
+    const Item seg = D.seg;
+    const int k = (int)D.k;
+    const uint32_t cb = tr.t * D.chunk;
+    if (!item_ok(seg, B) || k + 1 > NB || tr.t >= D.nch || D.chunk > (uint32_t)kPartMax || cb >= seg.size) {   // (uniform)
+        if (tid_x() == 0) flag_error(B.cnt, ERR_BOUNDS);
+        return;
     }
-    if (b1 < nbkt) {
-        const uint32_t e = (b1 * S.D.T + S.t) * kWaves + S.w;
-        c1 = (e == last ? segend : S.h1n) - S.h1;
-        s_base[b1] = S.h1 - S.hseg;
-    }
-    // local bucket starts: buckets 0..1023 first, then 1024..2046
-    uint32_t tot0, tot1;
-    const uint32_t ex0 = block_excl_scan<kBigWaves>(c0, &tot0, s_tmp);
-    const uint32_t ex1 = block_excl_scan<kBigWaves>(c1, &tot1, s_tmp);
-    if (b0 < nbkt) s_start[b0] = ex0;
-    if (b1 < nbkt) s_start[b1] = tot0 + ex1;
-    __syncthreads();
-    if (tot0 + tot1 != m) {   // the histogram must account for every key of the chunk
-        if (tid == 0) flag_error(B.cnt, ERR_BOUNDS);
-        return false;
-    }
+    const uint32_t tid = scat_tid(), w = wave_id(), lane = lane_id();
+    const uint32_t m = min(seg.size - cb, D.chunk);
+    const uint32_t per = ((m + kPartWaves - 1) / kPartWaves + 63) & ~63u;     // positions per wave
+    const uint32_t wb = w * per;
+    const uint32_t nspl = (1u << k) - 1, nbs = 2u << k;
+    const key64* tree = trees + (uint64_t)tr.seg * kTreeSlots;
+    const uint32_t fmt = SRC == kRootPack ? (seg.flags & kFmtMask) >> kFmtShift : 0u;
+    key64 kv[kE];
+    uint32_t iv[kE];        // (indices; a root's are its positions)
+    // clamped positions: every load is unconditional, so all of them are in flight together
+#define PS5_PART_POS(e) min(wb + (e) * 64 + lane, m - 1)
+    if (SRC == kFromRuns) {
+        const Runs R = runs_of(B, seg);
+        RunMap<kPartMax>& M = *reinterpret_cast<RunMap<kPartMax>*>(smem + L::kMapOff);
+        map_runs<kPartWaves, kPartMax>(R, seg.begin + seg.size, seg.begin + cb, m, M);
 #pragma unroll
-    for (int e = 0; e < L::kPer; ++e) {
-        const uint32_t p = e * kBigWG + tid;
-        if (p >= m) continue;
-        const uint32_t b = S.br[e] >> kRankBits;
-        const uint32_t l = b < nbkt ? s_start[b] + (S.br[e] & kRankMask) : 0xFFFFFFFFu;
-        if (l >= m) { flag_error(B.cnt, ERR_BOUNDS); continue; }
-        s_key[l] = S.kv[e];
-        if (IDENT) s_pos[l] = (uint16_t)p;
-        else s_idx[l] = (seg.flags & F_IDENT) ? seg.begin + S.cb + p : S.iv[e];
-        s_bkt[l] = (uint16_t)b;
+        for (int e = 0; e < kE; ++e) {
+            const uint32_t q = mapped_place(B, M, PS5_PART_POS(e));
+            kv[e] = R.K[q];
+            iv[e] = R.I[q];
+        }
+    } else if (SRC == kFromPerm) {
+        const uint32_t depth = seg_depth(B, seg.rbeg);
+#pragma unroll
+        for (int e = 0; e < kE; ++e) iv[e] = B.perm[seg.begin + cb + PS5_PART_POS(e)];
+#pragma unroll
+        for (int e = 0; e < kE; ++e) kv[e] = string_key(B, iv[e], depth);
+    } else if (fmt == 0) {     // (uniform)
+        uint64_t off[kE];
+        if (B.offs64) {     // (uniform)
+#pragma unroll
+            for (int e = 0; e < kE; ++e) off[e] = B.offs64[seg.begin + cb + PS5_PART_POS(e)];
+        } else {
+#pragma unroll
+            for (int e = 0; e < kE; ++e) off[e] = B.offs[seg.begin + cb + PS5_PART_POS(e)];
+        }
+#pragma unroll
+        for (int e = 0; e < kE; ++e) kv[e] = load_key(B.arena, B.alen, off[e]);
+    }
+    for (uint32_t i = tid; i <= nspl; i += T) s_tree[i] = tree[i];
+    for (uint32_t i = tid; i < kPartWaves * L::kSlots / 2; i += T) reinterpret_cast<uint32_t*>(s_cnt)[i] = 0;
+    if (SRC == kRootPack && fmt) {
+        // packed keys are extracted in a rolled loop through the wave's part
+        // of the key stage: unrolled with the others they would take twice
+        // the registers.  The code table sits where the counts go afterwards
+        uint8_t* s_lut = reinterpret_cast<uint8_t*>(s_cnt);
+        __syncthreads();
+        if (tid < kLutBytes) s_lut[tid] = B.lut[(uint64_t)tr.seg * kLutBytes + tid];
+        __syncthreads();
+        bool bad = false;
+#pragma unroll 2
+        for (uint32_t p = lane; p < per; p += 64) {
+            const uint32_t q = min(wb + p, m - 1);
+            s_key[wb + p] = pack_key_fmt(load_chars24(B.arena, B.alen, str_off(B, seg.begin + cb + q)), fmt, s_lut, &bad);
+        }
+        if (bad) flag_error(B.cnt, ERR_ALPHA);
+#pragma unroll
+        for (int e = 0; e < kE; ++e) kv[e] = (uint32_t)e * 64 < per ? s_key[wb + e * 64 + lane] : 0ull;
+        __syncthreads();     // the table and the keys are read
+        if (tid < kLutBytes / 4) reinterpret_cast<uint32_t*>(s_cnt)[tid] = 0;
+    }
+    if (SRC == kFromRuns) __syncthreads();     // the run map is read
+    for (uint32_t i = tid; i < ((uint32_t)kPartWaves << L::kPeerBits); i += T) s_peer[i] = 0;
+    __syncthreads();
+    uint16_t* cnt_w = s_cnt + w * L::kSlots;
+    uint64_t* peer = s_peer + (w << L::kPeerBits);
+    const uint64_t lanebit = 1ull << lane;
+    uint32_t br[kE];        // bucket << 16 | rank inside the wave's part, later the staged slot
+    constexpr int kG = 4;   // groups whose descents advance together
+    static_assert(kE % kG == 0, "whole batches");
+#pragma unroll
+    for (int e0 = 0; e0 < kE; e0 += kG) {
+        if ((uint32_t)e0 * 64 >= per) {     // (uniform) nothing here in a short chunk
+#pragma unroll
+            for (int j = 0; j < kG; ++j) br[e0 + j] = 0;
+            continue;
+        }
+        key64 kk[kG];
+        uint32_t bv[kG];
+#pragma unroll
+        for (int j = 0; j < kG; ++j) kk[j] = kv[e0 + j];
+        classify_keys<kG>(kk, s_tree, k, bv);
+#pragma unroll
+        for (int j = 0; j < kG; ++j) {
+            const uint32_t p = (e0 + j) * 64 + lane;
+            const bool act = p < per && wb + p < m;
+            if (!act) bv[j] = L::kSlots - 1;     // (above every bucket)
+            const uint64_t peers = match_bucket_lds<NB, L::kPeerBits>(bv[j], peer, lanebit);
+            const uint32_t r = (uint32_t)__popcll(peers & lanemask_lt());
+            const uint32_t old = cnt_w[bv[j]];
+            if (act && r == 0) cnt_w[bv[j]] = (uint16_t)(old + (uint32_t)__popcll(peers));
+            br[e0 + j] = (bv[j] << 16) | (old + r);
+        }
     }
     __syncthreads();
-    return true;
+    // places: a thread takes kPB neighbouring buckets, two 16-bit counts to a
+    // word; the counts become the wave's first slot per bucket
+    constexpr int kPB = (int)L::kSlots / (int)T > 2 ? (int)L::kSlots / (int)T : 2;
+    static_assert(kPartMax < 65536, "slots fit 16 bits");
+    uint32_t* s_pair = reinterpret_cast<uint32_t*>(s_cnt);
+    const uint32_t pair0 = tid * (kPB / 2);
+    uint32_t cnt[kPB], sum = 0;
+#pragma unroll
+    for (int q = 0; q < kPB / 2; ++q) {
+        uint32_t run = 0;
+        if (pair0 + q < nbs / 2) {
+            uint32_t* col = s_pair + pair0 + q;
+#pragma unroll
+            for (int ww = 0; ww < kPartWaves; ++ww) {
+                const uint32_t v = col[ww * (L::kSlots / 2)];
+                col[ww * (L::kSlots / 2)] = run;
+                run += v;
+            }
+        }
+        cnt[2 * q] = run & 0xFFFFu;
+        cnt[2 * q + 1] = run >> 16;
+        sum += cnt[2 * q] + cnt[2 * q + 1];
+    }
+    uint32_t tot;
+    uint32_t st = block_excl_scan<kPartWaves>(sum, &tot, s_tmp);
+    uint32_t* hrow = B.hist + D.hist_base + (uint64_t)tr.t * nbs;
+#pragma unroll
+    for (int q = 0; q < kPB / 2; ++q) {
+        const uint32_t b0 = st, b1 = st + cnt[2 * q];
+        st = b1 + cnt[2 * q + 1];
+        if (pair0 + q >= nbs / 2) continue;
+        uint32_t* col = s_pair + pair0 + q;
+        const uint32_t add = b0 | (b1 << 16);
+#pragma unroll
+        for (int ww = 0; ww < kPartWaves; ++ww) col[ww * (L::kSlots / 2)] += add;
+        *reinterpret_cast<uint2*>(hrow + 2 * (pair0 + q)) =
+            make_uint2(cnt[2 * q] | (b0 << 16), cnt[2 * q + 1] | (b1 << 16));
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kE; ++e) {
+        const uint32_t p = e * 64 + lane;
+        const bool act = p < per && wb + p < m;
+        uint32_t slot = act ? cnt_w[br[e] >> 16] + (br[e] & 0xFFFFu) : 0xFFFFFFFFu;
+        if (act && slot >= m) { flag_error(B.cnt, ERR_BOUNDS); slot = 0xFFFFFFFFu; }
+        br[e] = slot;
+        if (slot < m) s_key[slot] = kv[e];
+    }
+    __syncthreads();
+    // the buffer the segment's strings are not in
+    const uint64_t at = (SRC == kFromRuns && !(seg.flags & F_BUFB) ? B.cap : 0ull) + seg.begin + cb;
+    key64* KD = B.key + at;
+    uint32_t* ID = B.idx + at;
+#pragma unroll
+    for (int e = 0; e < kE; ++e) {
+        const uint32_t j = e * T + tid;
+        if (j < m) KD[j] = s_key[j];
+    }
+    __syncthreads();
+    uint32_t* s_idx = reinterpret_cast<uint32_t*>(smem + L::kKeyOff);
+#pragma unroll
+    for (int e = 0; e < kE; ++e)
+        if (br[e] < m)
+            s_idx[br[e]] = SRC == kRootPlain || SRC == kRootPack ? seg.begin + cb + wb + e * 64 + lane : iv[e];
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kE; ++e) {
+        const uint32_t j = e * T + tid;
+        if (j < m) ID[j] = s_idx[j];
+    }
+#undef PS5_PART_POS
 }
 
-// Write a staged chunk of m keys of segment seg (chunk base cb) out, position
-// by position.
-template <bool IDENT>
-__device__ __forceinline__ void scat_write(const Item& seg, uint32_t m, uint32_t cb, const Bufs& B,
-                                           unsigned char* smem)
-{
-    using L = ScatLds<IDENT>;
-    const uint32_t tid = scat_tid();
-    const key64* s_key = reinterpret_cast<const key64*>(smem + L::kKeyOff);
-    const uint32_t* s_idx = reinterpret_cast<const uint32_t*>(smem + L::kIdxOff);
-    const uint16_t* s_pos = reinterpret_cast<const uint16_t*>(smem + L::kIdxOff);
-    const uint16_t* s_bkt = reinterpret_cast<const uint16_t*>(smem + L::kBktOff);
-    const uint32_t* s_start = reinterpret_cast<const uint32_t*>(smem + L::kStartOff);
-    const uint32_t* s_base = reinterpret_cast<const uint32_t*>(smem + L::kBaseOff);
-    key64* KD = (seg.flags & F_BUFB) ? B.key0 : B.key1;
-    uint32_t* ID = (seg.flags & F_BUFB) ? B.idx0 : B.idx1;
-#pragma unroll
-    for (int e = 0; e < L::kPer; ++e) {
-        const uint32_t j = e * kBigWG + tid;
-        if (j >= m) continue;
-        const uint32_t b = s_bkt[j];
-        const uint32_t rel = s_base[b] + (j - s_start[b]);
-        if (rel >= seg.size) { flag_error(B.cnt, ERR_BOUNDS); continue; }
-        KD[seg.begin + rel] = s_key[j];
-        ID[seg.begin + rel] = IDENT ? seg.begin + cb + s_pos[j] : s_idx[j];
-    }
-}
-
-template <bool IDENT>
-__global__ __launch_bounds__(kBigWG) void k_scatter(Plan P, Bufs B, const uint32_t* __restrict__ hscan)
+// XCD-contiguous chunks: workgroup g runs on XCD g % kXcds (the grid is a
+// multiple of kXcds), and XCD x takes the chunks [N x / kXcds, N (x+1) /
+// kXcds), so neighbouring chunks, whose runs of a bucket share cache lines
+// with those of its neighbours, meet in one L2; each workgroup loops over its
+// share (one chunk, in a level planned on the host).  ntiles: the level's
+// chunks if the host knows them, else 0; one: a level of one segment, whose
+// chunks need no table.
+template <int NB, int SRC>
+__global__ __launch_bounds__(kPartThreads, 4) void k_part(Plan P, Bufs B, const key64* trees, uint32_t ntiles, int one)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    const LargeDesc* __restrict__ desc = P.desc;
-    const TileRef* __restrict__ tiles = P.tiles;
-    const uint32_t nchunks = P.hdr->ntiles * kWaves;
-    const uint32_t per = gridDim.x / kXcds;      // workgroups per XCD (the grid is a multiple of kXcds)
-    const uint32_t xcd = blockIdx.x % kXcds, slot = blockIdx.x / kXcds;
-    const uint32_t chi = (uint32_t)((uint64_t)nchunks * (xcd + 1) / kXcds);
-    uint32_t c = (uint32_t)((uint64_t)nchunks * xcd / kXcds) + slot;
-    if (slot >= per || c >= chi) return;
-    // one register set: once a chunk is staged in LDS its registers take the
-    // next chunk's loads, which overlap the write-out (past the end of its
-    // range a workgroup fetches its last chunk again, unused, so that every
-    // iteration issues the same loads)
-    ScatChunk<ScatLds<IDENT>::kPer> R;
-    scat_fetch<IDENT>(desc, tiles, B, hscan, c, R);
-    for (;;) {
-        const Item seg = R.D.seg;
-        const uint32_t m = R.m, cb = R.cb;
-        const bool staged = scat_stage<IDENT>(R, B, smem);
-        scat_fetch<IDENT>(desc, tiles, B, hscan, min(c + per, chi - 1), R);
-        if (staged) scat_write<IDENT>(seg, m, cb, B, smem);
-        c += per;
-        if (c >= chi) break;
+    const uint32_t N = ntiles ? ntiles : P.hdr->ntiles, per = gridDim.x / kXcds, xcd = blockIdx.x % kXcds;
+    const uint32_t thi = (uint32_t)((uint64_t)N * (xcd + 1) / kXcds);
+    uint32_t ti = (uint32_t)((uint64_t)N * xcd / kXcds) + blockIdx.x / kXcds;
+    for (; ti < thi; ti += per) {
+        __syncthreads();     // the previous chunk's stage is written out
+        part_chunk<NB, SRC>(ti, P, B, trees, one, smem);
     }
 }
 
-// Emit the children buckets of a multi-workgroup step.  start(b) =
-// bstart[b*stride] - base relative to seg.begin; the last bucket ends at
-// seg.size.  Tiny buckets become tiny leaves, other equal buckets (odd b)
-// equal-key leaves in chunks, other less-than buckets blocks or large
-// segments of the next level (distribute_finished, .hpp:1492-1584).
+// Bucket counts summed over groups of kHistGroup chunks (segments of more
+// than one group): row 1 + g of the segment's gsum.
+__global__ __launch_bounds__(kWG) void k_hist_sum(Plan P, Bufs B)
+{
+    const uint32_t ng = P.hdr->ngroups;
+    for (uint32_t gi = blockIdx.x; gi < ng; gi += gridDim.x) {
+        const TileRef gr = load_uniform(P.groups + gi);
+        const LargeDesc D = load_uniform(P.desc + gr.seg);
+        const uint32_t G = hist_groups(D.nch), nbs = 2u << D.k;
+        if (G == 1) continue;     // (k_children sums its rows)
+        const uint32_t c0 = gr.t * kHistGroup, c1 = min(D.nch, c0 + kHistGroup);
+        const uint32_t* h = B.hist + D.hist_base;
+        for (uint32_t b = blockIdx.y * kWG + tid_x(); b < nbs; b += gridDim.y * kWG) {
+            uint32_t s = 0;
+#pragma unroll 8
+            for (uint32_t c = c0; c < c1; ++c) s += h[(uint64_t)c * nbs + b] & 0xFFFFu;
+                B.gsum[D.gbase + (1 + gr.t) * nbs + b] = s;
+        }
+    }
+}
+
+// The rows of the run tables: for bucket b and chunk c of a segment,
+// vpos = the bucket's first position + its strings in the chunks before c,
+// src = the chunk's place + the bucket's start inside it.  A workgroup takes
+// 64 chunks x 64 buckets, turned in LDS from chunk-major to bucket-major.
+__global__ __launch_bounds__(kWG) void k_hist_runs(Plan P, Bufs B, int buf)
+{
+    __shared__ uint32_t s_h[64][65];
+    static_assert(kHistGroup == 64, "a lane per chunk of a group");
+    const uint32_t ng = P.hdr->ngroups;
+    uint32_t* V = B.vpos + (buf ? B.cap_h : 0ull);
+    uint32_t* S = B.src + (buf ? B.cap_h : 0ull);
+    const uint32_t w = wave_id(), lane = lane_id();
+    for (uint32_t gi = blockIdx.x; gi < ng; gi += gridDim.x) {
+        const TileRef gr = load_uniform(P.groups + gi);
+        const LargeDesc D = load_uniform(P.desc + gr.seg);
+        const uint32_t nbs = 2u << D.k, b0 = blockIdx.y * 64;
+        if (b0 >= nbs) continue;     // (uniform)
+        const uint32_t c0 = gr.t * kHistGroup, nc = min(D.nch - c0, kHistGroup);
+        const uint32_t* h = B.hist + D.hist_base;
+        __syncthreads();     // the previous tile is read
+#pragma unroll 4
+        for (uint32_t r = w; r < 64; r += kWaves)
+            s_h[r][lane] = r < nc && b0 + lane < nbs ? h[(uint64_t)(c0 + r) * nbs + b0 + lane] : 0u;
+        __syncthreads();
+        const uint32_t chunk_at = D.seg.begin + (c0 + lane) * D.chunk;
+        // lane: the first position of bucket b0 + lane in this group of chunks
+        const uint32_t* g = B.gsum + D.gbase + min(b0 + lane, nbs - 1);
+        const uint32_t firsts = g[0] + g[(1 + gr.t) * nbs];
+        for (uint32_t r = w; r < 64; r += kWaves) {
+            const uint32_t b = b0 + r;
+            if (b + 1 >= nbs) break;     // (uniform) the last slot is no bucket
+            const uint32_t x = s_h[lane][r], n = x & 0xFFFFu;
+            uint32_t inc = n;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const uint32_t y = (uint32_t)__shfl_up((int)inc, d, 64);
+                if (lane >= (uint32_t)d) inc += y;
+            }
+            const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)firsts, (int)r);
+            if (lane < nc) {
+                const uint32_t at = D.hist_base + b * D.nch + c0 + lane;
+                V[at] = first + inc - n;
+                S[at] = chunk_at + (x >> 16);
+            }
+        }
+    }
+}
+
+// Emit the children buckets of a multi-workgroup step.  Tiny buckets become
+// tiny leaves, other equal buckets (odd b) equal-key leaves in chunks, other
+// less-than buckets blocks or large segments of the next level
+// (distribute_finished, .hpp:1492-1584).  A thread takes the kPer buckets
+// from tid * kPer on, of sz[] strings, the first of them starting at
+// position start; dst: the buffer they lie in.
 //
 // spl: the segment's sorted splitters; equal bucket b holds the key spl[b >> 1],
 // and one whose key holds no NUL continues into the next round (counted).
-constexpr int kChildScan = 32;     // scan scratch of emit_children (at least kWaves * 7 entries)
+constexpr int kChildPer = (kMaxBkt + kBigWG) / kBigWG;     // 2 buckets per thread
+constexpr int kChildLists = 3 + kBlkClasses;
 
-__device__ void emit_children(const Item& seg, int nbkt, const uint32_t* bstart, uint32_t stride, uint32_t base,
-                              const key64* spl, const Sink& s, uint32_t* s_tmp)
+__device__ __forceinline__ void emit_children(const LargeDesc& D, uint32_t start, const uint32_t (&sz)[kChildPer], uint32_t dst,
+                                              const key64* spl, const Sink& s, uint32_t* s_tmp)
 {
-    constexpr int kPer = (kMaxBkt + kWG - 1) / kWG;   // 8
-    const uint32_t dstbuf = ((seg.flags & F_BUFB) ^ F_BUFB) | (seg.flags & kFmtMask);
+    const Item seg = D.seg;
+    const uint32_t base_flags = dst | (seg.flags & kFmtMask);
     const KeyFmt F = key_fmt(seg.flags);
     uint32_t c_t = 0, c_l = 0, c_r = 0, c_b[kBlkClasses] = {}, c_cont = 0;
-    uint32_t st[kPer], sz[kPer];
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        const int b = tid_x() * kPer + j;
-        st[j] = 0;
-        sz[j] = 0;
-        if (b < nbkt) {
-            st[j] = bstart[(uint32_t)b * stride] - base;
-            const uint32_t en = (b + 1 < nbkt) ? bstart[(uint32_t)(b + 1) * stride] - base : seg.size;
-            sz[j] = en - st[j];
-            const uint32_t m = sz[j];
-            if (m == 0) continue;
-            if (m <= kTinyT) c_t++;
-            else if (b & 1) {
-                c_r += (m + kRunChunk - 1) / kRunChunk;
-                if (!key_ends(spl[b >> 1], F)) c_cont++;
-            }
-            else if (m <= kBlkT) c_b[block_class(m)]++;
-            else c_l++;
+    for (int j = 0; j < kChildPer; ++j) {
+        const uint32_t b = tid_x() * kChildPer + j, m = sz[j];
+        if (m == 0) continue;
+        if (m <= kTinyT) c_t++;
+        else if (b & 1) {
+            c_r += (m + kRunChunk - 1) / kRunChunk;
+            if (!key_ends(spl[b >> 1], F)) c_cont++;
         }
+        else if (m <= kBlkT) c_b[block_class(m)]++;
+        else c_l++;
     }
     // the list offsets of this thread's children: one scan of all seven
     // counts (tiny, large, equal-key chunks, the block classes), then one
     // atomic per list for the segment's place in it
-    constexpr int kLists = 3 + kBlkClasses;
-    static_assert(kWaves * kLists <= kChildScan, "scan scratch");
-    uint32_t cv[kLists], ov[kLists], tv[kLists];
+    uint32_t cv[kChildLists], ov[kChildLists], tv[kChildLists];
     cv[0] = c_t;
     cv[1] = c_l;
     cv[2] = c_r;
 #pragma unroll
     for (int c = 0; c < kBlkClasses; ++c) cv[3 + c] = c_b[c];
-    block_excl_scan_k<kWaves, kLists>(cv, ov, tv, s_tmp);
+    block_excl_scan_k<kBigWaves, kChildLists>(cv, ov, tv, s_tmp);
     if (c_cont) atomicAdd(&s.cnt[s.c_runcont], c_cont);
-    uint32_t* s_base = s_tmp + kChildScan;
+    uint32_t* s_base = s_tmp + kBigWaves * kChildLists;
     if (tid_x() == 0) {
         s_base[0] = tv[0] ? atomicAdd(&s.cnt[s.c_tiny], tv[0]) : 0;
         s_base[1] = tv[1] ? atomicAdd(&s.cnt[s.c_large], tv[1]) : 0;
@@ -1040,22 +1009,18 @@ __device__ void emit_children(const Item& seg, int nbkt, const uint32_t* bstart,
 #pragma unroll
     for (int c = 0; c < kBlkClasses; ++c) o_b[c] = ov[3 + c] + s_base[3 + c];
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        const int b = tid_x() * kPer + j;
-        const uint32_t m = sz[j];
-        if (b >= nbkt || m == 0) continue;
-        Item it;
-        it.begin = seg.begin + st[j];
-        it.size = m;
-        it.rbeg = seg.rbeg;
-        it.flags = dstbuf;
+    for (int j = 0; j < kChildPer; ++j) {
+        const uint32_t b = tid_x() * kChildPer + j, m = sz[j];
+        if (m == 0) continue;
+        const Item it = { start, m, seg.rbeg, base_flags, D.hist_base + b * D.nch, D.nch };
+        start += m;
         if (m <= kTinyT) {
             put_item(s.tiny, s.cap_tiny, o_t++, it, s.cnt);
         } else if (b & 1) {
             const uint32_t nch = (m + kRunChunk - 1) / kRunChunk;
             for (uint32_t c = 0; c < nch; ++c) {
                 Item r = it;
-                r.flags = dstbuf | F_SORTED | (c << kFlagShift);
+                r.flags = base_flags | F_SORTED | (c << kFlagShift);
                 put_item(s.run, s.cap_run, o_r++, r, s.cnt);
             }
         } else if (m <= kBlkT) {
@@ -1067,16 +1032,71 @@ __device__ void emit_children(const Item& seg, int nbkt, const uint32_t* bstart,
     }
 }
 
-__global__ __launch_bounds__(kWG) void k_children(Plan P, const uint32_t* hscan, const key64* trees, Sink s)
+// Bucket sizes of the segments of a level, one workgroup each: their starts
+// (gsum), and the children.  A segment of one group of chunks sums its bucket
+// counts here, of more it scans the groups' sums, a thread per bucket.  dst:
+// the buffer the level wrote.
+__global__ __launch_bounds__(kBigWG) void k_children(Plan P, Bufs B, const key64* trees, Sink s, uint32_t dst)
 {
-    __shared__ uint32_t s_tmp[kChildScan + 8];     // the counts' scan, then the lists' bases
+    __shared__ uint32_t s_sz[kMaxBkt + 1];
+    __shared__ uint32_t s_tmp[kBigWaves * kChildLists + 8];     // the scans' scratch, then the lists' bases
     const uint32_t nlarge = P.hdr->nlarge;
     for (uint32_t si = blockIdx.x; si < nlarge; si += gridDim.x) {
-        const LargeDesc D = P.desc[si];
-        const uint32_t* h = hscan + D.hist_base;
-        emit_children(D.seg, (2 << D.k) - 1, h, D.T * kWaves, h[0], trees + (uint64_t)si * kTreeSlots + 1024, s,
-                      s_tmp);
-        __syncthreads();     // s_tmp is reused by the next segment
+        const LargeDesc D = load_uniform(P.desc + si);
+        const uint32_t G = hist_groups(D.nch), nbs = 2u << D.k;
+        uint32_t* g = B.gsum + D.gbase;
+        uint32_t sz[kChildPer];
+        if (G == 1) {     // (uniform)
+            const uint32_t* h = B.hist + D.hist_base;
+            for (uint32_t b = tid_x(); b < nbs; b += kBigWG) {
+                uint32_t n = 0;
+#pragma unroll 8
+                for (uint32_t c = 0; c < D.nch; ++c) n += h[c * nbs + b] & 0xFFFFu;
+                s_sz[b] = n;
+            }
+        } else {
+            for (uint32_t b = tid_x(); b < nbs; b += kBigWG) {
+                uint32_t* col = g + nbs + b;
+                uint32_t n = 0;
+                for (uint32_t i0 = 0; i0 < G; i0 += 8) {     // eight loads in flight
+                    uint32_t x[8];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) x[j] = i0 + j < G ? col[(i0 + j) * nbs] : 0u;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        if (i0 + j < G) col[(i0 + j) * nbs] = n;
+                        n += x[j];
+                    }
+                }
+                s_sz[b] = n;
+            }
+        }
+        __syncthreads();
+        uint32_t sum = 0;
+#pragma unroll
+        for (int j = 0; j < kChildPer; ++j) {
+            const uint32_t b = tid_x() * kChildPer + j;
+            sz[j] = b < nbs ? s_sz[b] : 0u;
+            sum += sz[j];
+        }
+        uint32_t tot;
+        const uint32_t start = D.seg.begin + block_excl_scan<kBigWaves>(sum, &tot, s_tmp);
+        if (tot != D.seg.size) {     // (uniform) the counts must account for every string of the segment
+            if (tid_x() == 0) flag_error(B.cnt, ERR_BOUNDS);
+        } else {
+            uint32_t at = start;
+#pragma unroll
+            for (int j = 0; j < kChildPer; ++j) {
+                const uint32_t b = tid_x() * kChildPer + j;
+                if (b < nbs) {
+                    g[b] = at;
+                    if (G == 1) g[nbs + b] = 0;
+                }
+                at += sz[j];
+            }
+            emit_children(D, start, sz, dst, trees + (uint64_t)si * kTreeSlots + 1024, s, s_tmp);
+        }
+        __syncthreads();     // the LDS is reused by the next segment
     }
 }
 
@@ -1085,21 +1105,14 @@ __global__ __launch_bounds__(kWG) void k_children(Plan P, const uint32_t* hscan,
 // Finish one sorted position at depth d: LCP with the predecessor when the
 // keys differ; inside a run of equal keys the LCP is known when the key holds
 // a NUL (fill_lcp with lcpKeyDepth, .hpp:1546-1547), otherwise the run moves
-// on to the next depth and the string's next key is gathered for round r+1.
+// on to the next depth, where its keys are read through the permutation.
 __device__ __forceinline__ void finish_position(const Bufs& B, uint32_t pos, uint32_t id, key64 k, bool has_prev,
-                                                key64 pk, bool run_single, uint32_t depth, KeyFmt F)
+                                                key64 pk, uint32_t depth, KeyFmt F)
 {
-    const bool eqp = has_prev && pk == k;
-    if (has_prev && !eqp && B.lcp) B.lcp[pos] = depth + lcp_key(pk, k, F);
-    const bool term = key_ends(k, F);
-    if (run_single || term) {
-        B.perm[pos] = id;
-        if (eqp && B.lcp) B.lcp[pos] = depth + key_depth(k, F);
-    } else {
-        B.idx0[pos] = id;
-        if (id < B.n) B.key0[pos] = load_key(B.arena, B.alen, str_off(B, id) + depth + F.cpk);
-        else flag_error(B.cnt, ERR_BOUNDS);
-    }
+    B.perm[pos] = id;
+    if (!has_prev || !B.lcp) return;
+    if (pk != k) B.lcp[pos] = depth + lcp_key(pk, k, F);
+    else if (key_ends(k, F)) B.lcp[pos] = depth + key_depth(k, F);
 }
 
 // LDS exchange between the lanes of one wave: its LDS operations execute in
@@ -1245,10 +1258,52 @@ __device__ void wave_finish_leaf(const Bufs& B, uint32_t pos, uint32_t m, key64 
     }
 }
 
-// One wave per tiny leaf (at most 64 strings), finished completely.
+// Key and input index of the string at lane's position L.begin + lane of a
+// leaf of at most 64 strings (lane < L.size).  A bucket of at most 64 runs has
+// them in the lanes; longer rows are searched.
+__device__ __forceinline__ void load_tiny(const Bufs& B, const Item& L, uint32_t depth, key64* k, uint32_t* id)
+{
+    const uint32_t lane = lane_id(), pos = L.begin + lane;
+    const bool act = lane < L.size;
+    if (L.flags & (F_IDENT | F_NEXT)) {     // (uniform)
+        if (act) {
+            *id = (L.flags & F_IDENT) ? pos : B.perm[pos];
+            *k = string_key(B, *id, depth);
+        }
+        return;
+    }
+    const Runs R = runs_of(B, L);
+    uint32_t q = 0;
+    if (R.nch <= 64) {     // (uniform)
+        uint32_t v = 0, sp = 0;
+        if (lane < R.nch) {
+            v = R.V[lane];
+            sp = R.S[lane];
+        }
+        // (an empty run starts where the next one does, or at the leaf's end)
+        const uint32_t down = (uint32_t)__shfl_down((int)v, 1, 64);     // (by all lanes)
+        const uint32_t nx = lane + 1 < R.nch ? down : L.begin + L.size;
+        for (uint64_t m = __ballot(lane < R.nch && nx > v); m; m &= m - 1) {     // (uniform)
+            const int c = __builtin_ctzll(m);
+            const uint32_t rv = (uint32_t)__builtin_amdgcn_readlane((int)v, c);
+            const uint32_t rs = (uint32_t)__builtin_amdgcn_readlane((int)sp, c);
+            if (pos >= rv) q = rs + (pos - rv);
+        }
+        if (act) q = checked_place(B, q);
+    } else if (act) {
+        q = run_place(B, R, pos);
+    }
+    if (act) {
+        *k = R.K[q];
+        *id = R.I[q];
+    }
+}
+
+// One wave per tiny leaf (at most 64 strings), finished completely: the
+// entries from *p_first (first, if null) on of a list.
 template <int NK>
-__global__ __launch_bounds__(kWG) void k_leaf_tiny(const Item* items, const uint32_t* cnt_items, uint32_t cap,
-                                                   Bufs B)
+__global__ __launch_bounds__(kWG) void k_leaf_tiny(const Item* items, const uint32_t* p_first, uint32_t first,
+                                                   const uint32_t* cnt_items, uint32_t cap, Bufs B)
 {
     __shared__ key64 s_k[kWaves][64];
     __shared__ uint32_t s_i[kWaves][64];
@@ -1259,27 +1314,20 @@ __global__ __launch_bounds__(kWG) void k_leaf_tiny(const Item* items, const uint
         return;
     }
     const uint32_t nitems = min(*cnt_items, cap);     // (an overflow has been flagged)
+    if (p_first) first = *p_first;
     // each wave takes leaves it, it + stride, ... (no workgroup barriers below)
-    for (uint32_t it = blockIdx.x * kWaves + w; it < nitems; it += gridDim.x * kWaves) {
-        Item L = items[it];
-        L.begin = (uint32_t)__builtin_amdgcn_readfirstlane((int)L.begin);
-        L.size = (uint32_t)__builtin_amdgcn_readfirstlane((int)L.size);
-        L.flags = (uint32_t)__builtin_amdgcn_readfirstlane((int)L.flags);
-        L.rbeg = (uint32_t)__builtin_amdgcn_readfirstlane((int)L.rbeg);
+    for (uint32_t it = first + blockIdx.x * kWaves + w; it < nitems; it += gridDim.x * kWaves) {
+        const Item L = load_uniform(items + __builtin_amdgcn_readfirstlane((int)it));
         if (!item_ok(L, B) || L.size > kTinyT) {
             if (lane == 0) flag_error(B.cnt, ERR_BOUNDS);
             continue;      // (wave-uniform)
         }
-        const uint32_t m = L.size;
-        const int src = L.flags & F_BUFB;
         key64 k = ~0ull;
         uint32_t id = 0;
-        if (lane < m) {
-            k = src ? B.key1[L.begin + lane] : B.key0[L.begin + lane];
-            id = (L.flags & F_IDENT) ? L.begin + lane : src ? B.idx1[L.begin + lane] : B.idx0[L.begin + lane];
-        }
-        wave_finish_leaf<NK>(B, L.begin + lane, m, k, id, seg_depth(B, L.rbeg), key_fmt(L.flags), true, 0u, s_k[w],
-                             s_i[w], s_r[w]);
+        const uint32_t depth = seg_depth(B, L.rbeg);
+        load_tiny(B, L, depth, &k, &id);
+        wave_finish_leaf<NK>(B, L.begin + lane, L.size, k, id, depth, key_fmt(L.flags), true, 0u, s_k[w], s_i[w],
+                             s_r[w]);
     }
 }
 
@@ -1322,7 +1370,8 @@ struct TailStack {
 constexpr int kBlkE0 = 4, kBlkE1 = 4, kBlkE2 = 4, kBlkE3 = 4;
 
 // Finish a block's short runs of equal keys (each at most 64 strings, at
-// sorted positions beg + (s_runs[r] >> 16)) at depth, the block's next one: the runs are
+// sorted positions beg + (s_runs[r] >> 16)) at depth, the block's next one
+// (their strings are in perm): the runs are
 // packed into batches of at most 64 strings, and a wave finishes all runs of
 // a batch in one pass (duplicates come in many short runs).  The batch
 // table lives in s_k after the waves' leaf arrays.
@@ -1374,8 +1423,8 @@ __device__ __forceinline__ void block_finish_runs(const Bufs& B, key64* s_k, con
         uint32_t id = 0, pos = 0;
         if (mine) {
             pos = beg + rs + (lane - slot0);
-            kk = B.key0[pos];
-            id = B.idx0[pos];
+            id = B.perm[pos];
+            kk = string_key(B, id, depth);
         }
         wave_finish_leaf<NK>(B, pos, total, kk, id, depth, key_fmt(0), false, slot0, wk, wi, wr);
     }
@@ -1521,7 +1570,7 @@ __device__ __forceinline__ key64 shfl_xor64(key64 v, int d)
     return ((key64)hi << 32) | lo;
 }
 
-// Radix-partitioned rank sort of a block's m keys (position i = key K[beg+i]):
+// Radix-partitioned rank sort of a block's m keys (w: thread t's keys of the positions t, t + T, ..):
 // values v are grouped in LDS by d = v >> (16 + sh), the top log2(MAXM)
 // bits of the offset (slots from LDS atomics, in no particular order), and
 // each value's sorted slot is its group's start plus the group members below
@@ -1531,8 +1580,8 @@ __device__ __forceinline__ key64 shfl_xor64(key64 v, int d)
 // success s_k holds the sorted keys and s_p their positions.  s_cnt: MAXM +
 // 2 counters (group counts, the total, a spare for lanes past m).
 template <uint32_t MAXM, int E>
-__device__ __forceinline__ bool block_radix_sort(const key64* __restrict__ K, uint32_t beg, uint32_t m,
-                                                 key64* s_k, uint16_t* s_p, uint32_t* s_cnt, uint32_t* s_tmp)
+__device__ __forceinline__ bool block_radix_sort(key64 (&w)[E], uint32_t m, key64* s_k, uint16_t* s_p,
+                                                 uint32_t* s_cnt, uint32_t* s_tmp)
 {
     constexpr uint32_t T = MAXM / E;
     constexpr int NW = (int)(T / 64);
@@ -1542,11 +1591,8 @@ __device__ __forceinline__ bool block_radix_sort(const key64* __restrict__ K, ui
     // block instead of being hoisted out of a tail workgroup's loop)
     const uint32_t tid = scat_tid();
     const uint32_t Pm = (m + E - 1) / E * E;
-    // w: this thread's keys (positions e*T + tid), later their packed values
-    // every load is unconditional (clamped index), so all E are in flight at once
-    key64 w[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) w[e] = K[beg + min((uint32_t)e * T + tid, m - 1)];
+    // w: this thread's keys (positions e*T + tid, clamped to the block), later
+    // their packed values
     key64 kmin = ~0ull, kmax = 0;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -1713,41 +1759,68 @@ __device__ __forceinline__ void block_one(const Item L, const Bufs& B, const Sin
     }
     const uint32_t m = L.size, beg = L.begin;
     uint32_t tid = scat_tid();     // (opaque: see block_radix_sort)
-    const int src = L.flags & F_BUFB;
-    const key64* K = src ? B.key1 : B.key0;
-    const uint32_t* I = src ? B.idx1 : B.idx0;
-    const bool ident = L.flags & F_IDENT;
     const KeyFmt F = key_fmt(L.flags);
     if (tid == 0) s_nruns = 0;
-    // the block's input indices are loaded beside its keys and kept in
-    // registers through the sort, then staged in s_cnt (free after either
-    // sort), so that sorted positions read them from LDS instead of waiting
-    // for a second global gather
+    // keys and input indices; every load is unconditional (clamped position),
+    // so all of a thread's are in flight at once.  The indices stay in
+    // registers through the sort, then are staged in s_cnt (free after either
+    // sort), so that sorted positions read them from LDS
     constexpr int kPerThread = MAXM / T;
+    key64 w[kPerThread];
     uint32_t idv[kPerThread];
-    if (!ident) {
-#pragma unroll
-        for (int e = 0; e < kPerThread; ++e) idv[e] = I[beg + min(tid + (uint32_t)e * T, m - 1)];
-    }
-    if (!block_radix_sort<MAXM, E>(K, beg, m, s_k, s_p, s_cnt, s_tmp))
-        block_merge_sort<MAXM, E>(m, s_k, s_p);
-    tid = scat_tid();     // (a fresh copy: positions from it are not held through the sort)
-    if (!ident) {     // (uniform)
+    if (L.flags & (F_IDENT | F_NEXT)) {     // (uniform)
 #pragma unroll
         for (int e = 0; e < kPerThread; ++e) {
-            const uint32_t i = tid + (uint32_t)e * T;
-            if (i < m) s_cnt[i] = idv[e];
+            const uint32_t pos = beg + min(tid + (uint32_t)e * T, m - 1);
+            idv[e] = (L.flags & F_IDENT) ? pos : B.perm[pos];
         }
-        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < kPerThread; ++e) w[e] = string_key(B, idv[e], depth);
+    } else {
+        // a bucket: the runs' starts and places are copied to s_k and searched
+        // there (a row longer than that is searched where it is)
+        const Runs R = runs_of(B, L);
+        uint32_t* s_v = reinterpret_cast<uint32_t*>(s_k);
+        uint32_t q[kPerThread];
+        if (R.nch <= MAXM) {     // (uniform)
+            for (uint32_t c = tid; c < R.nch; c += T) {
+                s_v[c] = R.V[c];
+                s_v[R.nch + c] = R.S[c];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < kPerThread; ++e) {
+                const uint32_t pos = beg + min(tid + (uint32_t)e * T, m - 1);
+                const uint32_t c = find_run(s_v, R.nch, pos);
+                q[e] = checked_place(B, s_v[R.nch + c] + (pos - s_v[c]));
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < kPerThread; ++e) q[e] = run_place(B, R, beg + min(tid + (uint32_t)e * T, m - 1));
+        }
+#pragma unroll
+        for (int e = 0; e < kPerThread; ++e) {
+            w[e] = R.K[q[e]];
+            idv[e] = R.I[q[e]];
+        }
     }
+    // (the sort writes s_k only after a barrier)
+    if (!block_radix_sort<MAXM, E>(w, m, s_k, s_p, s_cnt, s_tmp)) block_merge_sort<MAXM, E>(m, s_k, s_p);
+    tid = scat_tid();     // (a fresh copy: positions from it are not held through the sort)
+#pragma unroll
+    for (int e = 0; e < kPerThread; ++e) {
+        const uint32_t i = tid + (uint32_t)e * T;
+        if (i < m) s_cnt[i] = idv[e];
+    }
+    __syncthreads();
     // the input index of every sorted position, read before finish_position
-    // may overwrite its slot in idx0 (continuing runs store theirs)
+    // overwrites its slot in perm (a segment of an earlier round reads it there)
     uint32_t ids[kPerThread];
 #pragma unroll
     for (int e = 0; e < kPerThread; ++e) {
         const uint32_t i = tid + (uint32_t)e * T;
         ids[e] = 0;
-        if (i < m) ids[e] = ident ? beg + s_p[i] : s_cnt[s_p[i]];
+        if (i < m) ids[e] = s_cnt[s_p[i]];
     }
     __syncthreads();
 #pragma unroll
@@ -1762,11 +1835,11 @@ __device__ __forceinline__ void block_one(const Item L, const Bufs& B, const Sin
             if (i > 0) pk = s_k[i - 1];
             eqp = i > 0 && pk == kk;
             eqn = i + 1 < m && s_k[i + 1] == kk;
-            finish_position(B, beg + i, ids[e], kk, i > 0, pk, !eqp && !eqn, depth, F);
+            finish_position(B, beg + i, ids[e], kk, i > 0, pk, depth, F);
             if (top && (i == 0 || i == m - 1)) B.bkey[beg + i] = kk;
         }
-        // a run of equal keys without a NUL continues at the next depth (its keys
-        // there are in place, finish_position fetched them): a run of at most
+        // a run of equal keys without a NUL continues at the next depth (its
+        // strings are in perm): a run of at most
         // kTinyT strings is finished below by this workgroup, a longer one is
         // a segment of the next round
         const bool nr = act && !eqp && eqn && !key_ends(kk, F);
@@ -1797,12 +1870,12 @@ __device__ __forceinline__ void block_one(const Item L, const Bufs& B, const Sin
                 }
             }
         } else {
-            Item ni = { beg + i, rl, beg + i, 0u };
+            Item ni = { beg + i, rl, beg + i, F_NEXT, 0u, 0u };
             if (nr && !keep) B.sdepth_out[beg + i] = depth + F.cpk;
             wave_append_segment(nr && !keep, ni, nxt);
         }
     }
-    __syncthreads();     // the runs' keys and indices written above are visible to the whole group
+    __syncthreads();     // the runs' indices written above are visible to the whole group
     const uint32_t nruns = min(s_nruns, kMaxRuns);
     for (uint32_t r0 = 0; r0 < nruns; r0 += kBlockRuns) {     // (uniform) batches of at most kBlockRuns runs
         block_finish_runs<NK>(B, s_k, s_runs + r0, min(kBlockRuns, nruns - r0), beg, depth + F.cpk, T / 64);
@@ -1842,7 +1915,7 @@ __global__ __launch_bounds__(MAXM / E) __attribute__((amdgpu_waves_per_eu(8, 8))
             const uint32_t n = min(ts.n, kTailStack);
             if (n == 0) break;     // (uniform)
             __syncthreads();     // the last pass's LDS is no longer read, every thread has read ts.n
-            cur = Item{ ts.pos[n - 1], ts.len[n - 1], ts.pos[n - 1], 0u };
+            cur = Item{ ts.pos[n - 1], ts.len[n - 1], ts.pos[n - 1], F_NEXT, 0u, 0u };
             d = ts.depth[n - 1];
             if (tid_x() == 0) ts.n = n - 1;     // (pushes into the freed entry come after block_one's barriers)
             __syncthreads();     // every thread has read the top entry; the count is stored
@@ -1862,54 +1935,69 @@ __global__ __launch_bounds__(MAXM / E) __attribute__((amdgpu_waves_per_eu(8, 8))
     }
 }
 
-// One workgroup per chunk of an equal-key leaf (all keys equal).
-__global__ __launch_bounds__(kWG) void k_leaf_run(const Item* items, const uint32_t* cnt_items, uint32_t cap,
-                                                  Bufs B, Sink nxt)
+constexpr uint32_t kRunRow = 512;       // runs of a row that k_leaf_run searches
+
+// One workgroup per chunk of an equal-key leaf (all keys equal): the entries
+// from *p_first (first, if null) on of a list.
+__global__ __launch_bounds__(kWG) void k_leaf_run(const Item* items, const uint32_t* p_first, uint32_t first,
+                                                  const uint32_t* cnt_items, uint32_t cap, Bufs B, Sink nxt)
 {
+    __shared__ RunMap<kRunChunk> M;
     if (B.pending && *B.pending) {      // the round's levels are not finished
         if (B.pending_err && tid_x() == 0) flag_error(B.cnt, ERR_LEVELS);
         return;
     }
     const uint32_t nitems = min(*cnt_items, cap);     // (an overflow has been flagged)
-    for (uint32_t ii = blockIdx.x; ii < nitems; ii += gridDim.x) {
-        __syncthreads();     // the previous chunk's key read is complete
-        const Item L = items[ii];
+    if (p_first) first = *p_first;
+    for (uint32_t ii = first + blockIdx.x; ii < nitems; ii += gridDim.x) {
+        __syncthreads();     // the previous chunk's map is no longer read
+        const Item L = load_uniform(items + ii);
         const uint32_t c = L.flags >> kFlagShift;
-        if (!item_ok(L, B) || (uint64_t)c * kRunChunk >= L.size) {
+        if (!item_ok(L, B) || (uint64_t)c * kRunChunk >= L.size || (L.flags & (F_IDENT | F_NEXT))) {
             if (tid_x() == 0) flag_error(B.cnt, ERR_BOUNDS);
             continue;
         }
-        const int src = L.flags & F_BUFB;
-        const key64* K = src ? B.key1 : B.key0;
-        const uint32_t* I = src ? B.idx1 : B.idx0;
+        const Runs R = runs_of(B, L);
         const uint32_t rend = L.begin + L.size;
         const uint32_t cb = L.begin + c * kRunChunk;
-        const uint32_t ce = min(rend, cb + kRunChunk);
-        const key64 key = K[cb];    // this chunk's own copy of the run key
-        __syncthreads();
+        const uint32_t m = min(rend - cb, kRunChunk);
+        // a short row (a bucket of a small segment) is copied and searched, a
+        // long one mapped
+        uint32_t* s_v = M.delta;
+        const bool small = R.nch <= kRunRow;     // (uniform)
+        if (small) {
+            for (uint32_t i = tid_x(); i < R.nch; i += kWG) {
+                s_v[i] = R.V[i];
+                s_v[kRunRow + i] = R.S[i];
+            }
+            __syncthreads();
+        } else {
+            map_runs<kWaves, (int)kRunChunk>(R, rend, cb, m, M);
+        }
+        auto place = [&](uint32_t p) {
+            if (!small) return mapped_place(B, M, p);
+            const uint32_t r = find_run(s_v, R.nch, cb + p);
+            return checked_place(B, s_v[kRunRow + r] + (cb + p - s_v[r]));
+        };
+        const key64 key = R.K[place(0u)];
         const KeyFmt F = key_fmt(L.flags);
         const uint32_t depth = seg_depth(B, L.rbeg);
-        const bool term = key_ends(key, F);
-        const bool single = L.size == 1;
-        for (uint32_t p = cb + tid_x(); p < ce; p += kWG) {
-            const uint32_t id = (L.flags & F_IDENT) ? p : I[p];
-            if (single || term) {
-                B.perm[p] = id;
-                if (p > L.begin && B.lcp) B.lcp[p] = depth + key_depth(key, F);
-            } else {
-                if (src || (L.flags & F_IDENT)) B.idx0[p] = id;
-                if (id < B.n) B.key0[p] = load_key(B.arena, B.alen, str_off(B, id) + depth + F.cpk);
-                else flag_error(B.cnt, ERR_BOUNDS);
-            }
+        // identical strings are done, others continue at the next depth
+        const bool term = key_ends(key, F), single = L.size == 1;
+        const uint32_t l = depth + key_depth(key, F);
+#pragma unroll 4
+        for (uint32_t p = tid_x(); p < m; p += kWG) {
+            B.perm[cb + p] = R.I[place(p)];
+            if (term && B.lcp && cb + p > L.begin) B.lcp[cb + p] = l;
         }
         if (tid_x() < 64) {
             const bool nr = tid_x() == 0 && c == 0 && !term && !single;
-            Item ni = { L.begin, L.size, L.begin, 0u };
+            Item ni = { L.begin, L.size, L.begin, F_NEXT, 0u, 0u };
             if (nr) B.sdepth_out[L.begin] = depth + F.cpk;
             wave_append_segment(nr, ni, nxt);
             if (tid_x() == 0) {
                 if (c == 0) B.bkey[L.begin] = key;
-                if (ce == rend) B.bkey[rend - 1] = key;
+                if (cb + m == rend) B.bkey[rend - 1] = key;
             }
         }
     }
@@ -2320,11 +2408,11 @@ int set_err(int code, const char* fmt, ...)
     } while (0)
 
 enum KernelId {
-    K_INIT, K_TREE, K_COUNT, K_SCAN, K_SCATTER, K_CHILDREN, K_BLOCK,
+    K_INIT, K_TREE, K_PART, K_HIST, K_CHILDREN, K_BLOCK,
     K_LEAF_TINY, K_LEAF_RUN, K_LEAFBOUND, K_MISC, K_NUM
 };
 const char* kKernelNames[K_NUM] = {
-    "k_init", "k_tree", "k_count", "k_scan", "k_scatter", "k_children", "k_block",
+    "k_init", "k_tree", "k_part", "k_hist", "k_children", "k_block",
     "k_leaf_tiny", "k_leaf_run", "k_leafbound", "k_misc"
 };
 
@@ -2336,10 +2424,9 @@ enum { S_BLOCK, S_TINY, S_RUN, S_NUM };
 struct WorkBuffers {
     bool fixed = false;              // carved from the static scratch: never grown or freed
     uint64_t cap = 0;
-    key64* key[2] = { nullptr, nullptr };
-    uint32_t* idx[2] = { nullptr, nullptr };
+    key64* key = nullptr;            // two buffers of cap entries, one after the other
+    uint32_t* idx = nullptr;
     key64* bkey = nullptr;
-    uint32_t* bktrank = nullptr;
     uint32_t* sdepth[2] = { nullptr, nullptr };
     // large segments: first level of a round [round parity], later levels [level parity]
     Item* l_round[2] = { nullptr, nullptr };
@@ -2348,46 +2435,69 @@ struct WorkBuffers {
     Item* l_tiny[2] = { nullptr, nullptr };
     Item* l_block[2] = { nullptr, nullptr };
     Item* l_run[2] = { nullptr, nullptr };
-    uint32_t cap_large = 0, cap_block = 0, cap_tiny = 0, cap_run = 0;
+    uint32_t cap_large = 0, cap_block = 0, cap_tiny[2] = { 0, 0 }, cap_run = 0;
     Item* h_large = nullptr;         // pinned copy of a large list
     // plan of a level: its nlarge descriptors followed by its tile table, in
     // one buffer so that one copy uploads both
     unsigned char* d_plan = nullptr;
     unsigned char* h_plan = nullptr;     // pinned, mapped: the host's plans are pulled by k_fetch
     unsigned char* h_plan_dev = nullptr; // its device address
-    uint64_t tiles_cap = 0;
+    uint64_t tiles_cap = 0, groups_cap = 0;
     key64* trees = nullptr;          // kTreeSlots splitter slots per large segment
     uint64_t trees_cap = 0;
     uint8_t* lut = nullptr;          // kLutBytes per large segment (trees_cap of them)
+    // bucket counts of a level (hist_cap entries), their group sums, and the
+    // run tables (hist_cap entries for each of the two buffers)
     uint32_t* hist = nullptr;
+    uint32_t* vpos = nullptr;
+    uint32_t* src = nullptr;
     uint64_t hist_cap = 0;
-    uint32_t* part = nullptr;
-    uint64_t part_cap = 0;
+    uint32_t* gsum = nullptr;
+    uint64_t gsum_cap = 0;
 };
 
 // List capacities of a sort of up to cap strings (each list bounds what the
 // device can append to it; an overflow is flagged, never written).
 constexpr uint32_t cap_large_of(uint64_t cap) { return (uint32_t)(cap / kBlkT + 16); }
 constexpr uint32_t cap_block_of(uint64_t cap) { return (uint32_t)(cap / kTinyT + 16); }
-constexpr uint32_t cap_tiny_of(uint64_t cap) { return (uint32_t)(cap + 16); }
+// Tiny leaves: a batch may consist of as many sets; later rounds' (odd first)
+// come from runs of two strings or more, or are buckets of segments with at
+// most a sixteenth as many buckets as strings.
+constexpr uint32_t cap_tiny_of(uint64_t cap, int rp) { return (uint32_t)(rp ? cap / 4 * 3 + 16 : cap + 16); }
 // an equal-key run of m > kTinyT strings yields ceil(m / kRunChunk) <= m / 64 chunks
 constexpr uint32_t cap_run_of(uint64_t cap) { return (uint32_t)(cap / 64 + 16); }
-// every large segment has at most size/(kWaves * kChunkMin) + 1 tiles
-constexpr uint64_t tiles_cap_of(uint64_t cap) { return cap / ((uint64_t)kWaves * kChunkMin) + cap_large_of(cap) + 1; }
-// a plan: the level header, cap_large descriptors, the tile table
+// every large segment has at most size / kChunkMin + 1 chunks
+constexpr uint64_t tiles_cap_of(uint64_t cap) { return cap / kChunkMin + cap_large_of(cap) + 1; }
+constexpr uint64_t groups_cap_of(uint64_t cap) { return tiles_cap_of(cap) / kHistGroup + cap_large_of(cap) + 1; }
+// Entries of a level's bucket counts and of its run tables: segments of S
+// strings in all, in chunks of `limit` keys, have at most 2048 S / limit +
+// S / 16 (2 << treebits is at most 2048 and at most a sixteenth of a segment,
+// the leaf target being 64 or more); a level of min_tiles chunks or fewer has
+// chunks of kChunkMin or more keys.
+constexpr uint64_t hist_cap_of(uint64_t cap, uint64_t chunk_max, uint64_t min_tiles)
+{
+    const uint64_t limit = chunk_max < (uint64_t)kPartMax ? chunk_max : (uint64_t)kPartMax;
+    const uint64_t few = cap < kChunkMin * min_tiles ? cap : kChunkMin * min_tiles, many = cap * 2048 / limit;
+    return (few > many ? few : many) + cap / 16 + 4096;
+}
+// per bucket its first position and one sum per group of chunks
+constexpr uint64_t gsum_cap_of(uint64_t cap, uint64_t hist_cap) { return hist_cap / kHistGroup + cap / 8 + 8192; }
+// a plan: the level header, cap_large descriptors, the tables of chunks and groups
 constexpr uint64_t plan_tiles_off(uint64_t cap)
 {
     return sizeof(LevelHdr) + (uint64_t)cap_large_of(cap) * sizeof(LargeDesc);
 }
-constexpr uint64_t plan_bytes_of(uint64_t cap) { return plan_tiles_off(cap) + tiles_cap_of(cap) * sizeof(TileRef); }
+constexpr uint64_t plan_groups_off(uint64_t cap) { return plan_tiles_off(cap) + tiles_cap_of(cap) * sizeof(TileRef); }
+constexpr uint64_t plan_bytes_of(uint64_t cap) { return plan_groups_off(cap) + groups_cap_of(cap) * sizeof(TileRef); }
 static_assert(sizeof(LevelHdr) % 8 == 0 && sizeof(LargeDesc) % 8 == 0 && sizeof(TileRef) % 8 == 0,
               "a plan is copied in 8-byte words");
-Plan plan_view(const unsigned char* base, uint64_t cap)
+Plan plan_view(unsigned char* base, uint64_t cap)
 {
     Plan P;
     P.hdr = reinterpret_cast<const LevelHdr*>(base);
-    P.desc = reinterpret_cast<LargeDesc*>(const_cast<unsigned char*>(base) + sizeof(LevelHdr));
+    P.desc = reinterpret_cast<LargeDesc*>(base + sizeof(LevelHdr));
     P.tiles = reinterpret_cast<const TileRef*>(base + plan_tiles_off(cap));
+    P.groups = reinterpret_cast<const TileRef*>(base + plan_groups_off(cap));
     return P;
 }
 
@@ -2414,12 +2524,12 @@ struct ps5_ctx {
     unsigned char* h_stage_dev = nullptr;    // its device address
     uint32_t stage_seq = 0;                  // sequence number of the last staged copy
     uint32_t pending_root = 0;               // strings of a single root whose set-up the next plan fetch does
-    uint32_t* h_upcnt = nullptr;     // pinned: counters uploaded with batch roots
-    Item* h_roots = nullptr;         // pinned: root items of a batch
+    Item* h_roots = nullptr;         // pinned, mapped: root items of a batch, kind by kind
+    Item* h_roots_dev = nullptr;     // its device address
     uint64_t roots_cap = 0;
     uint64_t* d_merge = nullptr;     // plan of a merge round
     uint64_t merge_cap = 0;
-    uint32_t scatter_wgs = 256;         // k_scatter workgroups: one per CU, a multiple of kXcds
+    uint32_t cus = 256;                 // CUs, rounded down to a multiple of kXcds
     uint64_t* d_sets = nullptr;      // set boundaries of a batch
     uint64_t sets_cap = 0;
     unsigned long long* d_sums = nullptr;   // profiling: elements per kernel class
@@ -2429,8 +2539,8 @@ struct ps5_ctx {
     uint32_t max_treebits = kMaxTreebits;   // splitter-tree depth limit of one level
     uint32_t max_oversample = 32;    // sample keys per splitter (limited by kMaxSamples)
     // tile shapes of the multi-workgroup levels and the leaf passes' key width
-    uint32_t chunk_max = kChunkMax;          // keys per wave chunk, ordinary levels
-    uint32_t chunk_max_root = kChunkMaxIdent;    // the same in a level of roots
+    uint32_t chunk_max = kShapeChunkMax;     // keys per chunk, ordinary levels (at most kPartMax take effect)
+    uint32_t chunk_max_root = kShapeChunkMaxRoot;    // the same in a level of roots
     uint32_t min_tiles = kMinTiles;          // a small level's chunks shrink to give this many tiles
     uint32_t leaf_keys = 8;                  // keys a leaf pass fetches per string at a time
     uint64_t seed = 0x5EED5EEDull;
@@ -2462,6 +2572,15 @@ struct ps5_ctx {
 
 namespace {
 
+void free_tables(ps5_ctx* c)
+{
+    for (uint32_t** q : { &c->w.hist, &c->w.gsum, &c->w.vpos, &c->w.src }) {
+        if (*q) (void)hipFree(*q);
+        *q = nullptr;
+    }
+    c->w.hist_cap = c->w.gsum_cap = 0;
+}
+
 void free_buffers(ps5_ctx* c)
 {
     if (c->w.fixed) {     // views into the static scratch: nothing to free
@@ -2470,58 +2589,52 @@ void free_buffers(ps5_ctx* c)
     }
     auto f = [](void* p) { if (p) (void)hipFree(p); };
     for (int i = 0; i < 2; ++i) {
-        f(c->w.key[i]); f(c->w.idx[i]); f(c->w.l_round[i]); f(c->w.l_lvl[i]);
+        f(c->w.l_round[i]); f(c->w.l_lvl[i]);
         f(c->w.l_tiny[i]); f(c->w.l_block[i]); f(c->w.l_run[i]); f(c->w.sdepth[i]);
-        c->w.key[i] = nullptr; c->w.idx[i] = nullptr; c->w.l_round[i] = nullptr; c->w.l_lvl[i] = nullptr;
+        c->w.l_round[i] = nullptr; c->w.l_lvl[i] = nullptr;
         c->w.l_tiny[i] = nullptr; c->w.l_block[i] = nullptr; c->w.l_run[i] = nullptr;
         c->w.sdepth[i] = nullptr;
     }
-    f(c->w.bkey); f(c->w.bktrank); f(c->w.hist); f(c->w.part); f(c->w.trees); f(c->w.lut); f(c->w.d_plan);
-    c->w.bkey = nullptr; c->w.bktrank = nullptr; c->w.hist = nullptr; c->w.part = nullptr; c->w.trees = nullptr;
-    c->w.d_plan = nullptr;
-    c->w.lut = nullptr;
+    f(c->w.key); f(c->w.idx); f(c->w.bkey); f(c->w.trees); f(c->w.lut); f(c->w.d_plan);
+    c->w.key = nullptr; c->w.idx = nullptr; c->w.bkey = nullptr; c->w.trees = nullptr; c->w.lut = nullptr; c->w.d_plan = nullptr;
+    free_tables(c);
     if (c->w.h_large) (void)hipHostFree(c->w.h_large);
     if (c->w.h_plan) (void)hipHostFree(c->w.h_plan);
     c->w.h_large = nullptr; c->w.h_plan = nullptr; c->w.h_plan_dev = nullptr;
     c->w.cap = 0;
-    c->w.hist_cap = 0;
-    c->w.part_cap = 0;
-    c->w.tiles_cap = 0;
+    c->w.tiles_cap = c->w.groups_cap = 0;
     c->w.trees_cap = 0;
 }
 
-// Splitter trees for `nlarge` segments and `hl` histogram counters of one
-// level.  Called between levels, when the stream has drained (the level's
-// counts were just read back), so old buffers are idle.
-int grow_level(ps5_ctx* c, uint32_t nlarge, uint64_t hl)
+// The splitter trees, bucket counts and run tables of any level of a sort of
+// the context's capacity and shape.  Called before a sort, when its stream is
+// idle; they keep their size until the capacity or the shape asks for more
+// (a level's tables are still read by the leaves of the one before).
+int ensure_tables(ps5_ctx* c)
 {
-    if (c->w.fixed && (nlarge > c->w.trees_cap || hl > c->w.hist_cap))
-        return set_err(PS5_ERR_CAPACITY, "a level needs %u trees and %llu histogram entries; the scratch holds "
-                       "%llu and %llu", nlarge, (unsigned long long)hl, (unsigned long long)c->w.trees_cap,
-                       (unsigned long long)c->w.hist_cap);
-    if (nlarge > c->w.trees_cap) {
+    const uint64_t hist = hist_cap_of(c->w.cap, std::min(c->chunk_max, c->chunk_max_root), c->min_tiles);
+    const uint64_t gsum = gsum_cap_of(c->w.cap, hist);
+    if (c->w.cap_large <= c->w.trees_cap && hist <= c->w.hist_cap && gsum <= c->w.gsum_cap) return PS5_OK;
+    if (c->w.fixed) return set_err(PS5_ERR_CAPACITY, "the scratch holds no tables of this shape");
+    if (c->w.cap_large > c->w.trees_cap) {
         if (c->w.trees) (void)hipFree(c->w.trees);
         if (c->w.lut) (void)hipFree(c->w.lut);
         c->w.trees = nullptr;
         c->w.lut = nullptr;
         c->w.trees_cap = 0;
-        const uint64_t want = std::max<uint64_t>(nlarge + nlarge / 2, 64);
-        HIPCHK(hipMalloc(&c->w.trees, want * kTreeSlots * sizeof(key64)));
-        HIPCHK(hipMalloc(&c->w.lut, want * kLutBytes));
-        c->w.trees_cap = want;
+        HIPCHK(hipMalloc(&c->w.trees, (uint64_t)c->w.cap_large * kTreeSlots * sizeof(key64)));
+        HIPCHK(hipMalloc(&c->w.lut, (uint64_t)c->w.cap_large * kLutBytes));
+        c->w.trees_cap = c->w.cap_large;
         c->w_gen++;
     }
-    if (hl > c->w.hist_cap) {
-        if (c->w.hist) (void)hipFree(c->w.hist);
-        if (c->w.part) (void)hipFree(c->w.part);
-        c->w.hist = nullptr;
-        c->w.part = nullptr;
-        c->w.hist_cap = c->w.part_cap = 0;
-        const uint64_t want = std::min<uint64_t>(std::max<uint64_t>(hl + hl / 2, 1u << 20), 0xFFFFFFFFull);
-        HIPCHK(hipMalloc(&c->w.hist, want * sizeof(uint32_t)));
-        c->w.part_cap = want / kScanBlock + 2;
-        HIPCHK(hipMalloc(&c->w.part, c->w.part_cap * sizeof(uint32_t)));
-        c->w.hist_cap = want;
+    if (hist > c->w.hist_cap || gsum > c->w.gsum_cap) {
+        free_tables(c);
+        HIPCHK(hipMalloc(&c->w.hist, hist * sizeof(uint32_t)));
+        HIPCHK(hipMalloc(&c->w.gsum, gsum * sizeof(uint32_t)));
+        HIPCHK(hipMalloc(&c->w.vpos, 2 * hist * sizeof(uint32_t)));
+        HIPCHK(hipMalloc(&c->w.src, 2 * hist * sizeof(uint32_t)));
+        c->w.hist_cap = hist;
+        c->w.gsum_cap = gsum;
         c->w_gen++;
     }
     return PS5_OK;
@@ -2537,26 +2650,23 @@ int ensure_capacity(ps5_ctx* c, uint64_t n)
     uint64_t cap = std::max<uint64_t>(std::max<uint64_t>(n, 1024), c->w.cap + c->w.cap / 2);
     cap = std::min<uint64_t>(cap, std::max<uint64_t>(n, 0xFFFFFF00ull));
     free_buffers(c);
-    for (int i = 0; i < 2; ++i) {
-        HIPCHK(hipMalloc(&c->w.key[i], cap * sizeof(key64)));
-        HIPCHK(hipMalloc(&c->w.idx[i], cap * sizeof(uint32_t)));
-    }
+    HIPCHK(hipMalloc(&c->w.key, 2 * cap * sizeof(key64)));
+    HIPCHK(hipMalloc(&c->w.idx, 2 * cap * sizeof(uint32_t)));
     HIPCHK(hipMalloc(&c->w.bkey, cap * sizeof(key64)));
-    HIPCHK(hipMalloc(&c->w.bktrank, cap * sizeof(uint32_t)));
     for (int i = 0; i < 2; ++i) HIPCHK(hipMalloc(&c->w.sdepth[i], cap * sizeof(uint32_t)));
     c->w.cap_large = cap_large_of(cap);
     c->w.cap_block = cap_block_of(cap);
-    c->w.cap_tiny = cap_tiny_of(cap);
+    for (int i = 0; i < 2; ++i) c->w.cap_tiny[i] = cap_tiny_of(cap, i);
     c->w.cap_run = cap_run_of(cap);
     for (int i = 0; i < 2; ++i) {
         HIPCHK(hipMalloc(&c->w.l_round[i], (uint64_t)c->w.cap_large * sizeof(Item)));
         HIPCHK(hipMalloc(&c->w.l_lvl[i], (uint64_t)c->w.cap_large * sizeof(Item)));
-        HIPCHK(hipMalloc(&c->w.l_tiny[i], (uint64_t)c->w.cap_tiny * sizeof(Item)));
+        HIPCHK(hipMalloc(&c->w.l_tiny[i], (uint64_t)c->w.cap_tiny[i] * sizeof(Item)));
         HIPCHK(hipMalloc(&c->w.l_block[i], (uint64_t)kBlkClasses * c->w.cap_block * sizeof(Item)));
         HIPCHK(hipMalloc(&c->w.l_run[i], (uint64_t)c->w.cap_run * sizeof(Item)));
     }
-    // the splitter trees and histograms of a level grow on demand (grow_level)
     c->w.tiles_cap = tiles_cap_of(cap);
+    c->w.groups_cap = groups_cap_of(cap);
     const uint64_t plan_bytes = plan_bytes_of(cap);
     HIPCHK(hipMalloc(&c->w.d_plan, plan_bytes));
     HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&c->w.h_large), (uint64_t)c->w.cap_large * sizeof(Item)));
@@ -2575,19 +2685,16 @@ int ensure_capacity(ps5_ctx* c, uint64_t n)
 // loaded until the process ends.  Host code never uses the array's name as a
 // device address; the address is resolved once per device with
 // hipGetSymbolAddress (scratch_address) and kept in the context.
-constexpr uint64_t kScratchBytes = 96ull << 20;
+constexpr uint64_t kScratchBytes = 128ull << 20;
 constexpr uint64_t kNoAllocMaxStrings = 1ull << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 // Byte offsets of the work buffers of a sort of up to `cap` strings inside
-// the scratch.  Histogram bound per large segment of m strings: at most
-// min(2047, m/16) buckets (2^treebits < 2m/leaf_target, leaf_target >= 64)
-// times at most m/8192 + 1 tiles of kWaves chunks, so cap + cap/4 entries
-// cover a level; a level needs at most cap_large trees.
+// the scratch, its tables sized for any shape (chunks of kChunkMin keys).
 struct ScratchLayout {
-    uint64_t key[2], idx[2], bkey, bktrank, sdepth[2], lut, l_round[2], l_lvl[2], l_tiny[2], l_block[2], l_run[2];
-    uint64_t desc, trees, hist, part, total;
-    uint64_t trees_cap, hist_cap, part_cap;
+    uint64_t key, idx, bkey, sdepth[2], lut, l_round[2], l_lvl[2], l_tiny[2], l_block[2], l_run[2];
+    uint64_t desc, trees, hist, gsum, vpos, src, total;
+    uint64_t trees_cap, hist_cap, gsum_cap;
 };
 constexpr uint64_t align256(uint64_t x) { return (x + 255) / 256 * 256; }
 constexpr ScratchLayout scratch_layout(uint64_t cap)
@@ -2595,18 +2702,15 @@ constexpr ScratchLayout scratch_layout(uint64_t cap)
     ScratchLayout L{};
     uint64_t o = 0;
     auto take = [&o](uint64_t bytes) { const uint64_t at = o; o = align256(o + bytes); return at; };
-    const uint64_t cl = cap_large_of(cap), cb = cap_block_of(cap), ct = cap_tiny_of(cap), cr = cap_run_of(cap);
-    for (int i = 0; i < 2; ++i) {
-        L.key[i] = take(cap * sizeof(key64));
-        L.idx[i] = take(cap * sizeof(uint32_t));
-    }
+    const uint64_t cl = cap_large_of(cap), cb = cap_block_of(cap), cr = cap_run_of(cap);
+    L.key = take(2 * cap * sizeof(key64));
+    L.idx = take(2 * cap * sizeof(uint32_t));
     L.bkey = take(cap * sizeof(key64));
-    L.bktrank = take(cap * sizeof(uint32_t));
     for (int i = 0; i < 2; ++i) L.sdepth[i] = take(cap * sizeof(uint32_t));
     for (int i = 0; i < 2; ++i) {
         L.l_round[i] = take(cl * sizeof(Item));
         L.l_lvl[i] = take(cl * sizeof(Item));
-        L.l_tiny[i] = take(ct * sizeof(Item));
+        L.l_tiny[i] = take(cap_tiny_of(cap, i) * sizeof(Item));
         L.l_block[i] = take(kBlkClasses * cb * sizeof(Item));
         L.l_run[i] = take(cr * sizeof(Item));
     }
@@ -2614,10 +2718,12 @@ constexpr ScratchLayout scratch_layout(uint64_t cap)
     L.trees_cap = cl;
     L.trees = take(L.trees_cap * kTreeSlots * sizeof(key64));
     L.lut = take(L.trees_cap * kLutBytes);
-    L.hist_cap = cap + cap / 4 + 64;
+    L.hist_cap = hist_cap_of(cap, kChunkMin, kMinTiles);
     L.hist = take(L.hist_cap * sizeof(uint32_t));
-    L.part_cap = L.hist_cap / kScanBlock + 2;
-    L.part = take(L.part_cap * sizeof(uint32_t));
+    L.vpos = take(2 * L.hist_cap * sizeof(uint32_t));
+    L.src = take(2 * L.hist_cap * sizeof(uint32_t));
+    L.gsum_cap = gsum_cap_of(cap, L.hist_cap);
+    L.gsum = take(L.gsum_cap * sizeof(uint32_t));
     L.total = o;
     return L;
 }
@@ -2663,33 +2769,35 @@ WorkBuffers scratch_buffers(unsigned char* base, Item* h_large, unsigned char* h
     w.fixed = true;
     w.cap = cap;
     for (int i = 0; i < 2; ++i) {
-        w.key[i] = reinterpret_cast<key64*>(base + L.key[i]);
-        w.idx[i] = reinterpret_cast<uint32_t*>(base + L.idx[i]);
         w.l_round[i] = reinterpret_cast<Item*>(base + L.l_round[i]);
         w.l_lvl[i] = reinterpret_cast<Item*>(base + L.l_lvl[i]);
         w.l_tiny[i] = reinterpret_cast<Item*>(base + L.l_tiny[i]);
         w.l_block[i] = reinterpret_cast<Item*>(base + L.l_block[i]);
         w.l_run[i] = reinterpret_cast<Item*>(base + L.l_run[i]);
         w.sdepth[i] = reinterpret_cast<uint32_t*>(base + L.sdepth[i]);
+        w.cap_tiny[i] = cap_tiny_of(cap, i);
     }
+    w.key = reinterpret_cast<key64*>(base + L.key);
+    w.idx = reinterpret_cast<uint32_t*>(base + L.idx);
+    w.vpos = reinterpret_cast<uint32_t*>(base + L.vpos);
+    w.src = reinterpret_cast<uint32_t*>(base + L.src);
     w.bkey = reinterpret_cast<key64*>(base + L.bkey);
-    w.bktrank = reinterpret_cast<uint32_t*>(base + L.bktrank);
     w.cap_large = cap_large_of(cap);
     w.cap_block = cap_block_of(cap);
-    w.cap_tiny = cap_tiny_of(cap);
     w.cap_run = cap_run_of(cap);
     w.h_large = h_large;
     w.d_plan = base + L.desc;
     w.h_plan = h_plan;
     w.h_plan_dev = h_plan_dev;
     w.tiles_cap = tiles_cap_of(cap);
+    w.groups_cap = groups_cap_of(cap);
     w.trees = reinterpret_cast<key64*>(base + L.trees);
     w.trees_cap = L.trees_cap;
     w.lut = base + L.lut;
     w.hist = reinterpret_cast<uint32_t*>(base + L.hist);
     w.hist_cap = L.hist_cap;
-    w.part = reinterpret_cast<uint32_t*>(base + L.part);
-    w.part_cap = L.part_cap;
+    w.gsum = reinterpret_cast<uint32_t*>(base + L.gsum);
+    w.gsum_cap = L.gsum_cap;
     return w;
 }
 
@@ -2752,7 +2860,7 @@ Sink make_sink(ps5_ctx* c, Item* large, int c_large, int rp)
     s.c_runcont = C_RUNCONT + rp;
     s.cap_large = c->w.cap_large;
     s.cap_block = c->w.cap_block;
-    s.cap_tiny = c->w.cap_tiny;
+    s.cap_tiny = c->w.cap_tiny[rp];
     s.cap_run = c->w.cap_run;
     return s;
 }
@@ -2834,130 +2942,142 @@ int large_treebits(uint32_t m, uint32_t target, int maxbits)
     return std::max(1, std::min(maxbits, k));
 }
 
-void launch_tree(ps5_ctx* c, const Bufs& B, Plan P, uint32_t grid, uint64_t seed, bool from_arena)
+void launch_tree(ps5_ctx* c, const Bufs& B, Plan P, uint32_t grid, uint64_t seed, int src)
 {
-    const auto f = !from_arena ? k_tree<kNoRoot> : B.lut ? k_tree<kRootPack> : k_tree<kRootPlain>;
+    const auto f = src == kFromRuns ? k_tree<kFromRuns> : src == kRootPlain ? k_tree<kRootPlain>
+                 : src == kRootPack ? k_tree<kRootPack> : k_tree<kFromPerm>;
     hipLaunchKernelGGL(f, dim3(grid), dim3(kBigWG), 0, c->stream, P, B, seed, c->w.trees);
 }
 
-// k_count instance for bucket ids of NB = kmax + 1 bits (at least 8)
-void launch_count(ps5_ctx* c, const Bufs& B, Plan P, dim3 g, int kmax, bool from_arena, bool loop)
+// the k_part instance for trees of up to kmax treebits, with its LDS
+using PartKernel = void (*)(Plan, Bufs, const key64*, uint32_t, int);
+template <int NB>
+PartKernel part_kernel_nb(int src)
 {
-    hipStream_t st = c->stream;
-    const dim3 b(kWG);
-    const uint32_t lds = count_lds_bytes(kmax);
-#define PS5_COUNT_LAUNCH(NB)                                                                                          \
-    do {                                                                                                              \
-        const auto f = !from_arena ? (loop ? k_count<NB, true, kNoRoot> : k_count<NB, false, kNoRoot>)                \
-                       : B.lut ? (loop ? k_count<NB, true, kRootPack> : k_count<NB, false, kRootPack>)                \
-                               : (loop ? k_count<NB, true, kRootPlain> : k_count<NB, false, kRootPlain>);             \
-        hipLaunchKernelGGL(f, g, b, lds, st, P, B, c->w.trees, c->w.hist, kmax);                                      \
-    } while (0)
-    if (kmax <= 7) PS5_COUNT_LAUNCH(8);
-    else if (kmax == 8) PS5_COUNT_LAUNCH(9);
-    else if (kmax == 9) PS5_COUNT_LAUNCH(10);
-    else PS5_COUNT_LAUNCH(11);
-#undef PS5_COUNT_LAUNCH
+    return src == kFromRuns ? k_part<NB, kFromRuns> : src == kRootPlain ? k_part<NB, kRootPlain>
+         : src == kRootPack ? k_part<NB, kRootPack> : k_part<NB, kFromPerm>;
+}
+PartKernel part_kernel(int kmax, int src, uint32_t* lds)
+{
+    if (kmax <= 7) { *lds = PartLds<8>::kBytes; return part_kernel_nb<8>(src); }
+    if (kmax == 8) { *lds = PartLds<9>::kBytes; return part_kernel_nb<9>(src); }
+    if (kmax == 9) { *lds = PartLds<10>::kBytes; return part_kernel_nb<10>(src); }
+    *lds = PartLds<11>::kBytes;
+    return part_kernel_nb<11>(src);
+}
+void launch_part(ps5_ctx* c, const Bufs& B, Plan P, uint32_t grid, int kmax, int src, uint32_t ntiles, bool one)
+{
+    uint32_t lds = 0;
+    const PartKernel f = part_kernel(kmax, src, &lds);
+    hipLaunchKernelGGL(f, dim3(grid), dim3(kPartThreads), lds, c->stream, P, B, c->w.trees, ntiles, (int)one);
+}
+// bytes per string of a partition: its input, and key 8 + idx 4 written
+uint64_t part_bytes(int src)
+{
+    return src == kFromRuns ? 8 + 4 + 12                 // key, idx
+         : src == kFromPerm ? 4 + 4 + 8 + 12             // perm, offset, characters
+                            : 4 + 8 + 12;                // offset, characters
+}
+
+// What follows a level's partition: bucket sizes, children, run tables.
+void launch_hist(ps5_ctx* c, const Bufs& B, Plan P, const Sink& sink, uint32_t dst, int kmax, uint32_t g_sum,
+                 uint32_t g_children, uint32_t g_runs, uint64_t hl)
+{
+    const uint32_t nbs = 2u << kmax;
+    if (g_sum) {     // (segments of more than one group of chunks)
+        Launch L(c, K_HIST, hl * 4);
+        hipLaunchKernelGGL(k_hist_sum, dim3(g_sum, div_up(nbs, kWG)), dim3(kWG), 0, c->stream, P, B);
+    }
+    {
+        Launch L(c, K_CHILDREN, g_sum ? hl * 8 / kHistGroup : hl * 4);
+        hipLaunchKernelGGL(k_children, dim3(g_children), dim3(kBigWG), 0, c->stream, P, B, c->w.trees, sink, dst);
+    }
+    {
+        Launch L(c, K_HIST, hl * 12);
+        hipLaunchKernelGGL(k_hist_runs, dim3(g_runs, div_up(nbs, 64)), dim3(kWG), 0, c->stream, P, B, (int)dst);
+    }
 }
 
 // One multi-workgroup sample-sort step over all large segments of a level,
 // planned on the host from the level's large list (read back into h_large).
-int large_step(ps5_ctx* c, const Bufs& B, uint32_t nlarge, const Sink& sink, uint64_t seed, bool from_arena)
+// src: where the segments' strings are; dst: the buffer the level writes.
+int large_step(ps5_ctx* c, const Bufs& B, uint32_t nlarge, const Sink& sink, uint64_t seed, int src, uint32_t dst)
 {
     hipStream_t st = c->stream;
-    uint64_t ntiles = 0, hl = 0, elems = 0, elems_ident = 0;
+    uint64_t ntiles = 0, ngroups = 0, hl = 0, gs = 0, elems = 0;
     int kmax = 1;
     if (nlarge > c->w.cap_large) return set_err(PS5_ERR_CAPACITY, "large list overflow");
     LevelHdr* h_hdr = reinterpret_cast<LevelHdr*>(c->w.h_plan);
     LargeDesc* h_descs = reinterpret_cast<LargeDesc*>(c->w.h_plan + sizeof(LevelHdr));
     TileRef* h_tiles = reinterpret_cast<TileRef*>(c->w.h_plan + plan_tiles_off(c->w.cap));
-    uint64_t total = 0;
-    bool all_ident = true;     // a level of roots: the scatter stages positions, chunks may be longer
-    for (uint32_t i = 0; i < nlarge; ++i) {
-        total += c->w.h_large[i].size;
-        all_ident = all_ident && (c->w.h_large[i].flags & F_IDENT);
-    }
-    const uint64_t cmax = all_ident ? c->chunk_max_root : c->chunk_max;
-    const uint64_t climit = std::min<uint64_t>(cmax, std::max<uint64_t>(kChunkMin, div_up(total, kWaves * c->min_tiles)));
+    TileRef* h_groups = reinterpret_cast<TileRef*>(c->w.h_plan + plan_groups_off(c->w.cap));
+    for (uint32_t i = 0; i < nlarge; ++i) elems += c->w.h_large[i].size;
+    const bool roots = src == kRootPlain || src == kRootPack;
+    const uint64_t cmax = std::min<uint64_t>(roots ? c->chunk_max_root : c->chunk_max, kPartMax);
+    const uint64_t climit = std::min<uint64_t>(cmax, std::max<uint64_t>(kChunkMin, div_up(elems, c->min_tiles)));
     for (uint32_t i = 0; i < nlarge; ++i) {
         const Item seg = c->w.h_large[i];
-        const uint32_t T = div_up(seg.size, climit * kWaves);
+        const uint32_t T = div_up(seg.size, climit), G = hist_groups(T);
         LargeDesc& D = h_descs[i];
         D.seg = seg;
-        D.T = T;
-        D.chunk = div_up(seg.size, (uint64_t)T * kWaves);   // <= climit: equal chunks, the last one short
-        D.pad = 0;
+        D.nch = T;
+        D.chunk = div_up(seg.size, T);   // <= climit: equal chunks, the last one short
         D.hist_base = (uint32_t)hl;
+        D.gbase = (uint32_t)gs;
         D.k = (uint32_t)large_treebits(seg.size, c->leaf_target, (int)c->max_treebits);
         const uint32_t nspl = (1u << D.k) - 1;
         kmax = std::max(kmax, (int)D.k);
         D.oversample = std::max<uint32_t>(2, std::min<uint32_t>(c->max_oversample, (kMaxSamples / nspl) & ~1u));
-        if (ntiles + T > c->w.tiles_cap) return set_err(PS5_ERR_CAPACITY, "tile table capacity");
+        if (ntiles + T > c->w.tiles_cap || ngroups + G > c->w.groups_cap)
+            return set_err(PS5_ERR_CAPACITY, "chunk table capacity");
         for (uint32_t t = 0; t < T; ++t) h_tiles[ntiles + t] = TileRef{ i, t };
+        for (uint32_t g = 0; g < G; ++g) h_groups[ngroups + g] = TileRef{ i, g };
         ntiles += T;
-        hl += (uint64_t)((2u << D.k) - 1) * T * kWaves;
-        elems += seg.size;
-        if (seg.flags & F_IDENT) elems_ident += seg.size;
-        if (hl > 0xFFFFFFFFull) return set_err(PS5_ERR_CAPACITY, "histogram capacity");
+        ngroups += G;
+        hl += (uint64_t)(2u << D.k) * T;
+        gs += (uint64_t)(2u << D.k) * (G + 1);
+        if (hl > c->w.hist_cap || hl > 0xFFFFFFFFull || gs > c->w.gsum_cap)
+            return set_err(PS5_ERR_CAPACITY, "histogram capacity");
     }
-    *h_hdr = LevelHdr{ nlarge, (uint32_t)ntiles, (uint32_t)hl, (uint32_t)kmax, { 0u, 0u, 0u, 0u } };
-    if (int rc = grow_level(c, nlarge, hl)) return rc;
+    *h_hdr = LevelHdr{ nlarge, (uint32_t)ntiles, (uint32_t)ngroups, (uint32_t)kmax, { 0u, 0u, 0u, 0u } };
     {   // the plan: pulled from mapped host memory by a kernel (no copy engine)
-        const uint64_t words = (sizeof(LevelHdr) + nlarge * sizeof(LargeDesc)) / 8, words2 = ntiles * sizeof(TileRef) / 8;
-        const uint64_t toff = plan_tiles_off(c->w.cap);
-        const dim3 g((uint32_t)std::min<uint64_t>(div_up(std::max(words, words2), kWG), 1024));
-        const uint64_t* s1 = reinterpret_cast<const uint64_t*>(c->w.h_plan_dev);
-        const uint64_t* s2 = reinterpret_cast<const uint64_t*>(c->w.h_plan_dev + toff);
-        uint64_t* d1 = reinterpret_cast<uint64_t*>(c->w.d_plan);
-        uint64_t* d2 = reinterpret_cast<uint64_t*>(c->w.d_plan + toff);
+        FetchArgs F;
+        const uint64_t off[3] = { 0, plan_tiles_off(c->w.cap), plan_groups_off(c->w.cap) };
+        F.words[0] = (sizeof(LevelHdr) + nlarge * sizeof(LargeDesc)) / 8;
+        F.words[1] = ntiles * sizeof(TileRef) / 8;
+        F.words[2] = ngroups * sizeof(TileRef) / 8;
+        for (int k = 0; k < 3; ++k) {
+            F.src[k] = reinterpret_cast<const uint64_t*>(c->w.h_plan_dev + off[k]);
+            F.dst[k] = reinterpret_cast<uint64_t*>(c->w.d_plan + off[k]);
+        }
+        const dim3 g((uint32_t)std::min<uint64_t>(div_up(std::max(F.words[0], F.words[1]), kWG), 1024));
         if (c->pending_root)
-            hipLaunchKernelGGL(k_root_fetch, g, dim3(kWG), 0, st, s1, d1, words, s2, d2, words2, c->d_cnt,
-                               c->w.l_round[0], c->pending_root);
+            hipLaunchKernelGGL(k_root_fetch, g, dim3(kWG), 0, st, F, c->d_cnt, c->w.l_round[0], c->pending_root);
         else
-            hipLaunchKernelGGL(k_fetch, g, dim3(kWG), 0, st, s1, d1, words, s2, d2, words2);
+            hipLaunchKernelGGL(k_fetch, g, dim3(kWG), 0, st, F);
         c->pending_root = 0;
     }
     const Plan P = plan_view(c->w.d_plan, c->w.cap);
-    const uint32_t hl32 = (uint32_t)hl;
     {
         Launch L(c, K_TREE, (uint64_t)nlarge * kMaxSamples * 8);
-        launch_tree(c, B, P, nlarge, seed, from_arena);
+        launch_tree(c, B, P, nlarge, seed, src);
     }
     {
-        // key 8 R + bktrank 4 W; extracting at the root: offs 4 R + 8 characters R + key 8 W + bktrank 4 W
-        Launch L(c, K_COUNT, (from_arena ? elems * 24 : elems * 12) + hl * 4);
-        launch_count(c, B, P, dim3(div_up(ntiles, kXcds) * kXcds), kmax, from_arena, false);
+        Launch L(c, K_PART, elems * part_bytes(src) + hl * 4);
+        launch_part(c, B, P, div_up(ntiles, kXcds) * kXcds, kmax, src, (uint32_t)ntiles, nlarge == 1);
     }
-    {
-        const uint32_t nb = div_up(hl32, kScanBlock);
-        Launch L(c, K_SCAN, hl * 12);
-        hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(kWG), 0, st, c->w.hist, P.hdr, c->w.part);
-        hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kWG), 0, st, c->w.part, P.hdr);
-        hipLaunchKernelGGL(k_scan_down, dim3(nb), dim3(kWG), 0, st, c->w.hist, P.hdr, c->w.part);
-    }
-    {
-        // bktrank 4 + key 8 + idx 4 R (no idx at a root), key 8 + idx 4 W
-        Launch L(c, K_SCATTER, elems * 28 - elems_ident * 4 + hl * 8);
-        const uint32_t nchunks = (uint32_t)ntiles * kWaves;
-        const uint32_t wgs = std::min(c->scatter_wgs, div_up(nchunks, kXcds) * kXcds);
-        if (all_ident)
-            hipLaunchKernelGGL(k_scatter<true>, dim3(wgs), dim3(kBigWG), ScatLds<true>::kBytes, st, P, B, c->w.hist);
-        else
-            hipLaunchKernelGGL(k_scatter<false>, dim3(wgs), dim3(kBigWG), ScatLds<false>::kBytes, st, P, B, c->w.hist);
-    }
-    {
-        Launch L(c, K_CHILDREN, hl * 4 / kWaves);
-        hipLaunchKernelGGL(k_children, dim3(nlarge), dim3(kWG), 0, st, P, c->w.hist, c->w.trees, sink);
-    }
+    launch_hist(c, B, P, sink, dst, kmax, ngroups > nlarge ? (uint32_t)ngroups : 0u, nlarge, (uint32_t)ngroups, hl);
     c->st_segments += nlarge;
     return PS5_OK;
 }
 
 // Roots of a sort: one segment [0, n), or one per set of a batch (sets never
 // mix: every set is its own round segment, so no LCP crosses a set border).
+// h_cnt and h_large get what the first round finds in its lists.
 int setup_roots(ps5_ctx* c, uint32_t n, const uint64_t* set_first, uint32_t nsets)
 {
     hipStream_t st = c->stream;
+    for (int i = 0; i < C_NCNT; ++i) c->h_cnt[i] = 0;
     if (!set_first) {
         Item* list; int ci;
         if (n <= kTinyT) { list = c->w.l_tiny[0]; ci = C_TINY; }
@@ -2967,54 +3087,57 @@ int setup_roots(ps5_ctx* c, uint32_t n, const uint64_t* set_first, uint32_t nset
             ci = C_BLOCK + 2 * cls;
         }
         else { list = c->w.l_round[0]; ci = C_LROUND; }
+        c->h_cnt[ci] = 1;
+        if (ci == C_LROUND) c->w.h_large[0] = Item{ 0u, n, 0u, F_IDENT, 0u, 0u };
         Launch L(c, K_MISC, 0);
         hipLaunchKernelGGL(k_setup, dim3(1), dim3(64), 0, st, c->d_cnt, list, ci, n);
+        HIPCHK(hipGetLastError());
         return PS5_OK;
     }
-    // root items staged in pinned memory and copied on the context's stream
-    // (a blocking copy on the null stream would wait for every other
-    // context's work on the device)
+    // root items staged in mapped host memory and pulled by a kernel (the
+    // last sort that read them is complete)
     if ((uint64_t)nsets > c->roots_cap) {
         const uint64_t want = std::max<uint64_t>(nsets, 2 * c->roots_cap);
         if (c->h_roots) (void)hipHostFree(c->h_roots);
         c->h_roots = nullptr;
         c->roots_cap = 0;
-        HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&c->h_roots), want * sizeof(Item)));
+        HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&c->h_roots), want * sizeof(Item),
+                             hipHostMallocMapped | hipHostMallocCoherent));
+        HIPCHK(hipHostGetDevicePointer(reinterpret_cast<void**>(&c->h_roots_dev), c->h_roots, 0));
         c->roots_cap = want;
     }
     // kinds: 0 tiny, 1..kBlkClasses blocks by size class, last large
-    constexpr int NK = kBlkClasses + 2;
-    uint32_t cnt[NK] = {};
-    uint32_t tot = 0;
-    for (int kind = 0; kind < NK; ++kind) {
-        for (uint32_t s = 0; s < nsets; ++s) {
-            const uint64_t b = set_first[s], e = set_first[s + 1];
-            if (e < b || e > n) return set_err(PS5_ERR_ARG, "set boundaries must be non-decreasing and <= n");
-            if (e == b) continue;
-            const Item it = { (uint32_t)b, (uint32_t)(e - b), (uint32_t)b, F_IDENT };
-            const int k = it.size <= kTinyT ? 0 : it.size <= kBlkT ? 1 + block_class(it.size) : NK - 1;
-            if (k != kind) continue;
-            c->h_roots[tot++] = it;
-            cnt[kind]++;
-        }
+    auto kind_of = [](uint32_t m) { return m <= kTinyT ? 0 : m <= kBlkT ? 1 + block_class(m) : kRootKinds - 1; };
+    RootLists R{};
+    for (uint32_t s = 0; s < nsets; ++s) {
+        const uint64_t b = set_first[s], e = set_first[s + 1];
+        if (e < b || e > n) return set_err(PS5_ERR_ARG, "set boundaries must be non-decreasing and <= n");
+        if (e > b) R.count[kind_of((uint32_t)(e - b))]++;
     }
-    if (cnt[NK - 1] > c->w.cap_large || cnt[0] > c->w.cap_tiny) return set_err(PS5_ERR_CAPACITY, "too many sets");
-    for (int k = 1; k <= kBlkClasses; ++k)
-        if (cnt[k] > c->w.cap_block) return set_err(PS5_ERR_CAPACITY, "too many sets");
-    HIPCHK(hipStreamSynchronize(st));     // h_upcnt may still feed an earlier copy
-    for (int i = 0; i < C_NCNT; ++i) c->h_upcnt[i] = 0;
-    c->h_upcnt[C_TINY] = cnt[0];
-    for (int k = 1; k <= kBlkClasses; ++k) c->h_upcnt[C_BLOCK + 2 * (k - 1)] = cnt[k];
-    c->h_upcnt[C_LROUND] = cnt[NK - 1];
-    const Item* h = c->h_roots;
-    for (int kind = 0; kind < NK; ++kind) {
-        Item* dst = kind == 0 ? c->w.l_tiny[0]
-                  : kind == NK - 1 ? c->w.l_round[0]
-                  : c->w.l_block[0] + (uint64_t)(kind - 1) * c->w.cap_block;
-        if (cnt[kind]) HIPCHK(hipMemcpyAsync(dst, h, cnt[kind] * sizeof(Item), hipMemcpyHostToDevice, st));
-        h += cnt[kind];
+    if (R.count[kRootKinds - 1] > c->w.cap_large || R.count[0] > c->w.cap_tiny[0])
+        return set_err(PS5_ERR_CAPACITY, "too many sets");
+    uint32_t at[kRootKinds], total = 0;
+    for (int k = 0; k < kRootKinds; ++k) {
+        at[k] = total;
+        total += R.count[k];
+        const bool large = k == kRootKinds - 1;
+        if (k > 0 && !large && R.count[k] > c->w.cap_block) return set_err(PS5_ERR_CAPACITY, "too many sets");
+        R.dst[k] = k == 0 ? c->w.l_tiny[0] : large ? c->w.l_round[0] : c->w.l_block[0] + (uint64_t)(k - 1) * c->w.cap_block;
+        R.counter[k] = k == 0 ? C_TINY : large ? C_LROUND : C_BLOCK + 2 * (k - 1);
+        c->h_cnt[R.counter[k]] = R.count[k];
     }
-    HIPCHK(hipMemcpyAsync(c->d_cnt, c->h_upcnt, C_NCNT * sizeof(uint32_t), hipMemcpyHostToDevice, st));
+    const uint32_t large0 = at[kRootKinds - 1];
+    for (uint32_t s = 0; s < nsets; ++s) {
+        const uint64_t b = set_first[s], e = set_first[s + 1];
+        if (e > b) c->h_roots[at[kind_of((uint32_t)(e - b))]++] =
+            Item{ (uint32_t)b, (uint32_t)(e - b), (uint32_t)b, F_IDENT, 0u, 0u };
+    }
+    memcpy(c->w.h_large, c->h_roots + large0, R.count[kRootKinds - 1] * sizeof(Item));
+    R.src = c->h_roots_dev;
+    Launch L(c, K_MISC, 0);
+    hipLaunchKernelGGL(k_roots, dim3(std::min<uint32_t>(div_up(std::max(total, 1u), kWG), 1024)), dim3(kWG), 0, st, R,
+                       c->d_cnt);
+    HIPCHK(hipGetLastError());
     return PS5_OK;
 }
 
@@ -3038,7 +3161,7 @@ constexpr uint64_t kAutoDevMax = 1u << 22;
 
 // Largest grids of the device-planned levels: their kernels loop over the
 // work the device lists, so these bound the workgroups of a launch.
-constexpr uint32_t kDevTreeWgs = 512, kDevCountWgs = 2048, kDevScanWgs = 1024, kDevChildWgs = 1024,
+constexpr uint32_t kDevTreeWgs = 512, kDevHistWgs = 1024, kDevChildWgs = 512,
                    kDevTinyWgs = 8192, kDevRunWgs = 2048, kDevBoundWgs = 1024;
 static_assert(kBlkE0 == kBlkE1 && kBlkE1 == kBlkE2 && kBlkE2 == kBlkE3, "one thread count per 256 keys");
 
@@ -3053,7 +3176,7 @@ uint32_t leaf_run_grid(uint64_t nr) { return (uint32_t)std::min<uint64_t>(kDevRu
 uint32_t block_grid_full(const ps5_ctx* c, int cls)
 {
     const uint32_t waves = (256u << cls) / (uint32_t)kBlkE0 / 64;
-    return (uint32_t)((uint64_t)c->scatter_wgs * 128 / waves);
+    return (uint32_t)((uint64_t)c->cus * 128 / waves);
 }
 
 // Blocks of size class cls and round parity rp: the list entries [first,
@@ -3098,31 +3221,44 @@ void launch_block_class(ps5_ctx* c, const Bufs& B, int rp, int cls, uint32_t fir
 #undef PS5_BLOCK_LAUNCH
 }
 
-// Tiny leaves and equal-key chunks of round parity rp on stream s (grids of
-// g_tiny and g_run workgroups; 0 skips a list).
-void launch_leaves(ps5_ctx* c, const Bufs& B, int rp, const Sink& nsink, uint32_t g_tiny, uint32_t g_run,
-                   uint64_t n_tiny, uint64_t n_run, hipStream_t s, int flags = 0)
+// Tiny leaves and equal-key chunks of round parity rp on stream s, from the
+// entries done.tiny and done.run on (from the counters C_TDONE and C_RDONE on
+// with dev_first), in grids of g_tiny and g_run workgroups (0 skips a list).
+struct LeavesDone { uint32_t tiny = 0, run = 0; };
+void launch_leaves(ps5_ctx* c, const Bufs& B, int rp, const Sink& nsink, LeavesDone done, bool dev_first,
+                   uint32_t g_tiny, uint32_t g_run, uint64_t n_tiny, uint64_t n_run, hipStream_t s, int flags = 0)
 {
     if (g_tiny) {
+        const uint32_t* first = dev_first ? c->d_cnt + C_TDONE : nullptr;
         {
             Launch L(c, K_LEAF_TINY, 0);
-            if (c->leaf_keys == 8)
-                hipExtLaunchKernelGGL(k_leaf_tiny<8>, dim3(g_tiny), dim3(kWG), 0, s, nullptr, nullptr, flags,
-                                      c->w.l_tiny[rp], c->d_cnt + C_TINY + rp, c->w.cap_tiny, B);
-            else
-                hipExtLaunchKernelGGL(k_leaf_tiny<0>, dim3(g_tiny), dim3(kWG), 0, s, nullptr, nullptr, flags,
-                                      c->w.l_tiny[rp], c->d_cnt + C_TINY + rp, c->w.cap_tiny, B);
+            const auto f = c->leaf_keys == 8 ? k_leaf_tiny<8> : k_leaf_tiny<0>;
+            hipExtLaunchKernelGGL(f, dim3(g_tiny), dim3(kWG), 0, s, nullptr, nullptr, flags, c->w.l_tiny[rp], first,
+                                  done.tiny, c->d_cnt + C_TINY + rp, c->w.cap_tiny[rp], B);
         }
-        sum_sizes(c, c->w.l_tiny[rp], 0, c->d_cnt + C_TINY + rp, (uint32_t)n_tiny, S_TINY);
+        sum_sizes(c, c->w.l_tiny[rp], done.tiny, c->d_cnt + C_TINY + rp, (uint32_t)n_tiny, S_TINY);
     }
     if (g_run) {
+        const uint32_t* first = dev_first ? c->d_cnt + C_RDONE : nullptr;
         {
             Launch L(c, K_LEAF_RUN, 0);
-            hipExtLaunchKernelGGL(k_leaf_run, dim3(g_run), dim3(kWG), 0, s, nullptr, nullptr, flags, c->w.l_run[rp],
-                                  c->d_cnt + C_RUN + rp, c->w.cap_run, B, nsink);
+            hipExtLaunchKernelGGL(k_leaf_run, dim3(g_run), dim3(kWG), 0, s, nullptr, nullptr, flags, c->w.l_run[rp], first,
+                                  done.run, c->d_cnt + C_RUN + rp, c->w.cap_run, B, nsink);
         }
-        sum_sizes(c, c->w.l_run[rp], 0, c->d_cnt + C_RUN + rp, (uint32_t)n_run, S_RUN);
+        sum_sizes(c, c->w.l_run[rp], done.run, c->d_cnt + C_RUN + rp, (uint32_t)n_run, S_RUN);
     }
+}
+
+// The leaves known to the host (h_cnt) that are not finished yet, on the
+// context's stream: before a level overwrites the buffer and the run tables
+// of the level before the last, where some of them lie.
+void finish_known_leaves(ps5_ctx* c, const Bufs& B, int rp, const Sink& nsink, LeavesDone* done)
+{
+    const uint32_t nt = c->h_cnt[C_TINY + rp], nr = c->h_cnt[C_RUN + rp];
+    launch_leaves(c, B, rp, nsink, *done, false, leaf_tiny_grid(nt - done->tiny), leaf_run_grid(nr - done->run),
+                  nt - done->tiny, nr - done->run, c->stream);
+    done->tiny = nt;
+    done->run = nr;
 }
 
 // LCPs between neighbouring leaves of round parity rp (grid workgroups).
@@ -3132,7 +3268,7 @@ void launch_leafbound(ps5_ctx* c, const Bufs& B, int rp, uint32_t grid, uint64_t
     LeafLists LL;
     LL.list[0] = c->w.l_tiny[rp];
     LL.cnt[0] = C_TINY + rp;
-    LL.cap[0] = c->w.cap_tiny;
+    LL.cap[0] = c->w.cap_tiny[rp];
     for (int cls = 0; cls < kBlkClasses; ++cls) {
         LL.list[1 + cls] = c->w.l_block[rp] + (uint64_t)cls * c->w.cap_block;
         LL.cnt[1 + cls] = C_BLOCK + 2 * cls + rp;
@@ -3144,15 +3280,23 @@ void launch_leafbound(ps5_ctx* c, const Bufs& B, int rp, uint32_t grid, uint64_t
     hipLaunchKernelGGL(k_leafbound, dim3(grid), dim3(kWG), 0, c->stream, LL, B);
 }
 
+// The leaves listed so far, in a round planned on the device (at most n of
+// them): before a level from the third on (finish_known_leaves).
+void dev_finish_leaves(ps5_ctx* c, const Bufs& B, int rp, const Sink& nsink, uint64_t n)
+{
+    launch_leaves(c, B, rp, nsink, LeavesDone{}, true, (uint32_t)std::min<uint64_t>(kDevTinyWgs, div_up(n, kWaves)),
+                  (uint32_t)std::min<uint64_t>(kDevRunWgs, n / kTinyT + 1), n, n, c->stream);
+    hipLaunchKernelGGL(k_leaves_done, dim3(1), dim3(64), 0, c->stream, c->d_cnt, rp);
+}
+
 // One level planned on the device: k_plan turns the large list `list`
 // (counter ci) into the level's plan, and the step's kernels read their work
 // from it, in grids bounded by what the host knows (at most bound_large
 // segments holding S strings), so nothing comes back to the host.
 void dev_level(ps5_ctx* c, const Bufs& B, const Item* list, int ci, uint32_t bound_large, uint64_t S,
-               const Sink& sink, uint64_t seed, bool from_arena, bool ident, int kmax, int done_rp)
+               const Sink& sink, uint64_t seed, int src, uint32_t dst, int kmax, int done_rp)
 {
     hipStream_t st = c->stream;
-    const uint64_t n = S;     // strings the level's segments hold at most
     PlanArgs A;
     A.list = list;
     A.ci = ci;
@@ -3160,13 +3304,16 @@ void dev_level(ps5_ctx* c, const Bufs& B, const Item* list, int ci, uint32_t bou
     A.plan = c->w.d_plan;
     A.tiles_off = plan_tiles_off(c->w.cap);
     A.tiles_cap = c->w.tiles_cap;
+    A.groups_off = plan_groups_off(c->w.cap);
+    A.groups_cap = c->w.groups_cap;
     A.hist_cap = c->w.hist_cap;
+    A.gsum_cap = c->w.gsum_cap;
     A.trees_cap = c->w.trees_cap;
     A.leaf_target = c->leaf_target;
     A.max_treebits = c->max_treebits;
     A.max_oversample = c->max_oversample;
-    A.chunk_max = c->chunk_max;
-    A.chunk_max_root = c->chunk_max_root;
+    A.chunk_max = std::min<uint32_t>(c->chunk_max, kPartMax);
+    A.chunk_max_root = std::min<uint32_t>(c->chunk_max_root, kPartMax);
     A.min_tiles = c->min_tiles;
     A.kmax = (uint32_t)kmax;
     A.done_rp = done_rp;
@@ -3178,34 +3325,17 @@ void dev_level(ps5_ctx* c, const Bufs& B, const Item* list, int ci, uint32_t bou
     const uint32_t gl = std::max<uint32_t>(1, bound_large);
     {
         Launch L(c, K_TREE, 0);
-        launch_tree(c, B, P, std::min(gl, kDevTreeWgs), seed, from_arena);
+        launch_tree(c, B, P, std::min(gl, kDevTreeWgs), seed, src);
     }
-    const uint64_t tiles_bound = n / ((uint64_t)kWaves * kChunkMin) + gl;
+    const uint64_t tiles_bound = S / kChunkMin + gl;
     {
-        Launch L(c, K_COUNT, 0);
-        launch_count(c, B, P, dim3((uint32_t)std::min<uint64_t>(kDevCountWgs, div_up(tiles_bound, kXcds) * kXcds)),
-                     kmax, from_arena, true);
+        // three workgroups per CU are resident
+        Launch L(c, K_PART, 0);
+        launch_part(c, B, P, (uint32_t)std::min<uint64_t>(3 * c->cus, div_up(tiles_bound, kXcds) * kXcds), kmax, src, 0u,
+                    false);
     }
-    {
-        const uint32_t nb = (uint32_t)std::min<uint64_t>(kDevScanWgs, div_up(c->w.hist_cap, kScanBlock));
-        Launch L(c, K_SCAN, 0);
-        hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(kWG), 0, st, c->w.hist, P.hdr, c->w.part);
-        hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kWG), 0, st, c->w.part, P.hdr);
-        hipLaunchKernelGGL(k_scan_down, dim3(nb), dim3(kWG), 0, st, c->w.hist, P.hdr, c->w.part);
-    }
-    {
-        Launch L(c, K_SCATTER, 0);
-        const uint32_t wgs = (uint32_t)std::min<uint64_t>(c->scatter_wgs, div_up(tiles_bound * kWaves, kXcds) * kXcds);
-        if (ident)
-            hipLaunchKernelGGL(k_scatter<true>, dim3(wgs), dim3(kBigWG), ScatLds<true>::kBytes, st, P, B, c->w.hist);
-        else
-            hipLaunchKernelGGL(k_scatter<false>, dim3(wgs), dim3(kBigWG), ScatLds<false>::kBytes, st, P, B, c->w.hist);
-    }
-    {
-        Launch L(c, K_CHILDREN, 0);
-        hipLaunchKernelGGL(k_children, dim3(std::min(gl, kDevChildWgs)), dim3(kWG), 0, st, P, c->w.hist, c->w.trees,
-                           sink);
-    }
+    const uint32_t groups_bound = (uint32_t)std::min<uint64_t>(kDevHistWgs, tiles_bound / kHistGroup + gl);
+    launch_hist(c, B, P, sink, dst, kmax, groups_bound, std::min(gl, kDevChildWgs), groups_bound, 0);
 }
 
 // Bound on the buckets of a level over segments of at most m strings (its
@@ -3251,18 +3381,19 @@ int dev_level_kmax(const ps5_ctx* c, uint64_t m, uint32_t level)
 }
 
 // The host-planned levels of a round from the large list of counter cur_ci
-// (in h_cnt / h_large): each level's large list is read back and planned on
-// the host, and the blocks listed before a level are sorted in it
-// (blk_done: blocks already sorted per size class).
-int host_levels(ps5_ctx* c, const Bufs& B, uint32_t round, int cur_ci, uint32_t* blk_done, bool fused_root,
-                bool* leaves_forked, uint32_t reset_mask, bool* after_blocks)
+// (in h_cnt / h_large), the round's level `level` and on: each level's large
+// list is read back and planned on the host, and the blocks listed before a
+// level are sorted in it (blk_done: blocks already sorted per size class;
+// done: leaves already finished).  Level l of a round writes buffer l & 1.
+int host_levels(ps5_ctx* c, const Bufs& B, uint32_t round, uint32_t level, int cur_ci, uint32_t* blk_done,
+                LeavesDone* done, bool* leaves_forked, uint32_t reset_mask, bool* after_blocks)
 {
     *after_blocks = false;     // set when the stream's last packets are the last level's block kernels
     hipStream_t st = c->stream;
     const int rp = round & 1, np = rp ^ 1;
     const Sink nsink = make_sink(c, c->w.l_round[np], C_LROUND + np, np);
     int rc;
-    for (uint32_t level = 0;; ++level) {
+    for (;; ++level) {
         if (level > 4096) return set_err(PS5_ERR_INTERNAL, "sample-sort levels do not terminate");
         const uint32_t nlarge = c->h_cnt[cur_ci];
         uint32_t nblk[kBlkClasses], nblk_all = 0;
@@ -3292,32 +3423,41 @@ int host_levels(ps5_ctx* c, const Bufs& B, uint32_t round, int cur_ci, uint32_t*
         // listed, and when they are many they run on the side stream
         // beside the blocks (not when profiling, whose events time the
         // main stream; for few leaves the fork costs more than it hides)
-        const uint32_t nt = c->h_cnt[C_TINY + rp], nr = c->h_cnt[C_RUN + rp];
+        const uint32_t nt = c->h_cnt[C_TINY + rp] - done->tiny, nr = c->h_cnt[C_RUN + rp] - done->run;
         if (nlarge == 0 && !c->profile && div_up(nt, kWaves) + nr >= kForkLeafGroups) {
             HIPCHK(hipEventRecord(c->ev_fork, st));
             HIPCHK(hipStreamWaitEvent(c->side, c->ev_fork, 0));
-            launch_leaves(c, B, rp, nsink, leaf_tiny_grid(nt), leaf_run_grid(nr), nt, nr, c->side);
+            launch_leaves(c, B, rp, nsink, *done, false, leaf_tiny_grid(nt), leaf_run_grid(nr), nt, nr, c->side);
             HIPCHK(hipEventRecord(c->ev_join, c->side));
             *leaves_forked = true;
         }
         const Sink sink = make_sink(c, nx_large, nx_ci, rp);
         const uint64_t seed = c->seed ^ ((uint64_t)round << 40) ^ ((uint64_t)level << 32);
-        if (nlarge && (rc = large_step(c, B, nlarge, sink, seed, fused_root && round == 0 && level == 0)))
-            return rc;
         // a level without large segments, in a round whose equal-key
         // leaves all end here (their keys hold a NUL), holds the round's
         // last work: its blocks finish every string themselves (tail mode)
         // and no further round is needed
         const bool tail = c->tail_blocks && nlarge == 0 && c->h_cnt[C_RUNCONT + rp] == 0;
-        int bflags = 0;     // the first class waits for the level; the others may run beside it
-        for (int cls = 0; cls < kBlkClasses; ++cls) {
-            if (!nblk[cls]) continue;
-            launch_block_class(c, B, rp, cls, blk_done[cls], nblk[cls], false, nblk[cls], nsink, tail, bflags);
-            if (!c->profile) bflags = hipExtAnyOrderLaunch;
-            *after_blocks = nlarge == 0;
-            sum_sizes(c, c->w.l_block[rp] + (uint64_t)cls * c->w.cap_block, blk_done[cls],
-                      c->d_cnt + C_BLOCK + 2 * cls + rp, blk_done[cls] + nblk[cls], S_BLOCK);
-            blk_done[cls] += nblk[cls];
+        auto sort_blocks = [&] {
+            int bflags = 0;     // the first class waits for the level; the others may run beside it
+            for (int cls = 0; cls < kBlkClasses; ++cls) {
+                if (!nblk[cls]) continue;
+                launch_block_class(c, B, rp, cls, blk_done[cls], nblk[cls], false, nblk[cls], nsink, tail, bflags);
+                if (!c->profile) bflags = hipExtAnyOrderLaunch;
+                *after_blocks = nlarge == 0;
+                sum_sizes(c, c->w.l_block[rp] + (uint64_t)cls * c->w.cap_block, blk_done[cls],
+                          c->d_cnt + C_BLOCK + 2 * cls + rp, blk_done[cls] + nblk[cls], S_BLOCK);
+                blk_done[cls] += nblk[cls];
+            }
+        };
+        // from level 2 on, the step overwrites the buffer and the run tables
+        // of the level before the last: what was listed from them goes first
+        if (level >= 2 || nlarge == 0) sort_blocks();
+        if (nlarge) {
+            if (level >= 2) finish_known_leaves(c, B, rp, nsink, done);
+            const int src = level > 0 ? kFromRuns : round > 0 ? kFromPerm : B.lut ? kRootPack : kRootPlain;
+            if ((rc = large_step(c, B, nlarge, sink, seed, src, level & 1))) return rc;
+            if (level < 2) sort_blocks();
         }
         HIPCHK(hipGetLastError());
         // blocks only append to the next round's lists: after a level
@@ -3347,8 +3487,9 @@ int host_levels(ps5_ctx* c, const Bufs& B, uint32_t round, int cur_ci, uint32_t*
             const uint64_t seed2 = c->seed ^ ((uint64_t)round << 40) ^ ((uint64_t)level << 32);
             const int kmax = large_treebits((uint32_t)std::min<uint64_t>(mmax, 0xFFFFFFFFull), c->leaf_target,
                                             (int)c->max_treebits);
+            if (level >= 2) finish_known_leaves(c, B, rp, nsink, done);
             dev_level(c, B, nx_large, nx_ci, (uint32_t)std::min<uint64_t>(c->w.cap_large, S / (kBlkT + 1) + 1), S,
-                      make_sink(c, nn_large, nn_ci, rp), seed2, false, false, kmax, -1);
+                      make_sink(c, nn_large, nn_ci, rp), seed2, kFromRuns, level & 1, kmax, -1);
             HIPCHK(hipGetLastError());
             if ((rc = readback(c, nn_large, nn_ci))) return rc;
             cur_ci = nn_ci;
@@ -3362,7 +3503,7 @@ int host_levels(ps5_ctx* c, const Bufs& B, uint32_t round, int cur_ci, uint32_t*
 
 // Leaves and leaf boundaries of a round planned on the host (h_cnt holds
 // the round's final counts), then the read-back of the next round's lists.
-int host_round_end(ps5_ctx* c, const Bufs& B, uint32_t round, bool leaves_forked, bool after_blocks)
+int host_round_end(ps5_ctx* c, const Bufs& B, uint32_t round, LeavesDone done, bool leaves_forked, bool after_blocks)
 {
     hipStream_t st = c->stream;
     const int rp = round & 1, np = rp ^ 1;
@@ -3380,8 +3521,8 @@ int host_round_end(ps5_ctx* c, const Bufs& B, uint32_t round, bool leaves_forked
     // right after the last level's block kernels (the first of which waited
     // for everything before it) the leaves may start beside them; the leaf
     // boundaries below wait for all of them
-    else launch_leaves(c, B, rp, nsink, leaf_tiny_grid(nt), leaf_run_grid(nr), nt, nr, st,
-                       after_blocks && !c->profile ? hipExtAnyOrderLaunch : 0);
+    else launch_leaves(c, B, rp, nsink, done, false, leaf_tiny_grid(nt - done.tiny), leaf_run_grid(nr - done.run),
+                       nt - done.tiny, nr - done.run, st, after_blocks && !c->profile ? hipExtAnyOrderLaunch : 0);
     if (nt + nb + nr && B.lcp) launch_leafbound(c, B, rp, div_up((uint64_t)nt + nb + nr, kWG), nt + nb + nr);
     HIPCHK(hipGetLastError());
     return readback(c, c->w.l_round[np], C_LROUND + np);
@@ -3392,7 +3533,6 @@ struct SortRun {
     Bufs B;
     uint32_t n;
     uint64_t alen;
-    bool fused_root;          // one root whose keys the first count pass extracts
     uint32_t root_kmax;       // largest treebits of a large root
     uint64_t root_max;        // largest root: no segment of any round is larger
     uint64_t root_sum;        // strings in large roots
@@ -3415,7 +3555,6 @@ int sort_round(ps5_ctx* c, SortRun& R, uint32_t round, bool dev, bool* done)
     Bufs& B = R.B;
     const uint32_t n = R.n;
     const uint64_t alen = R.alen;
-    const bool fused_root = R.fused_root;
     const uint32_t root_kmax = R.root_kmax;
     const uint64_t root_max = R.root_max, root_sum = R.root_sum;
     uint32_t* lcp = B.lcp;
@@ -3428,7 +3567,7 @@ int sort_round(ps5_ctx* c, SortRun& R, uint32_t round, bool dev, bool* done)
         round_mask = (1u << (C_LROUND + np)) | (1u << (C_TINY + np)) | (1u << (C_RUN + np));
         for (int cls = 0; cls < kBlkClasses; ++cls)
             round_mask |= (1u << (C_BLOCK + 2 * cls + np)) | (1u << (C_BDONE + cls));
-        round_mask |= 1u << (C_RUNCONT + np);
+        round_mask |= (1u << (C_RUNCONT + np)) | (1u << C_TDONE) | (1u << C_RDONE);
     }
     if (round_mask && dev) {     // (host-planned levels clear them with their first level's counters)
         Launch L(c, K_MISC, 0);
@@ -3436,12 +3575,13 @@ int sort_round(ps5_ctx* c, SortRun& R, uint32_t round, bool dev, bool* done)
     }
     const Sink nsink = make_sink(c, c->w.l_round[np], C_LROUND + np, np);
     uint32_t blk_done[kBlkClasses] = {};
+    LeavesDone done_leaves;
     bool leaves_forked = false, after_blocks = false;
     if (!dev) {
-        if ((rc = host_levels(c, B, round, C_LROUND + rp, blk_done, fused_root, &leaves_forked, round_mask,
+        if ((rc = host_levels(c, B, round, 0, C_LROUND + rp, blk_done, &done_leaves, &leaves_forked, round_mask,
                               &after_blocks)))
             return rc;
-        if ((rc = host_round_end(c, B, round, leaves_forked, after_blocks))) return rc;
+        if ((rc = host_round_end(c, B, round, done_leaves, leaves_forked, after_blocks))) return rc;
     } else {
         // every level of the round without a host synchronisation.  The
         // host knows the round's lists (read back with the previous
@@ -3463,9 +3603,10 @@ int sort_round(ps5_ctx* c, SortRun& R, uint32_t round, bool dev, bool* done)
         }
         const uint32_t L = nl0 ? dev_levels_for(c, mmax) : 0;
         if (L == 0) {
-            if ((rc = host_levels(c, B, round, C_LROUND + rp, blk_done, false, &leaves_forked, 0u, &after_blocks)))
+            if ((rc = host_levels(c, B, round, 0, C_LROUND + rp, blk_done, &done_leaves, &leaves_forked, 0u,
+                                  &after_blocks)))
                 return rc;
-            if ((rc = host_round_end(c, B, round, leaves_forked, after_blocks))) return rc;
+            if ((rc = host_round_end(c, B, round, done_leaves, leaves_forked, after_blocks))) return rc;
         } else {
             int in_ci = C_LROUND + rp;
             const Item* in_list = c->w.l_round[rp];
@@ -3480,9 +3621,10 @@ int sort_round(ps5_ctx* c, SortRun& R, uint32_t round, bool dev, bool* done)
                 const Sink sink = make_sink(c, c->w.l_lvl[level & 1], out_ci, rp);
                 const uint64_t seed = c->seed ^ ((uint64_t)round << 40) ^ ((uint64_t)level << 32);
                 const bool rootlvl = round == 0 && level == 0;
-                dev_level(c, B, in_list, in_ci, level == 0 ? nl0 : deeper_large, S, sink, seed,
-                          fused_root && rootlvl, rootlvl, rootlvl ? (int)root_kmax : dev_level_kmax(c, mmax, level),
-                          level > 0 ? rp : -1);
+                const int src = level > 0 ? kFromRuns : round > 0 ? kFromPerm : B.lut ? kRootPack : kRootPlain;
+                if (level >= 2) dev_finish_leaves(c, B, rp, nsink, S);
+                dev_level(c, B, in_list, in_ci, level == 0 ? nl0 : deeper_large, S, sink, seed, src, level & 1,
+                          rootlvl ? (int)root_kmax : dev_level_kmax(c, mmax, level), level > 0 ? rp : -1);
                 int bflags = 0;     // the first class waits for the level; the others run beside it
                 for (int cls = 0; cls < kBlkClasses; ++cls) {
                     // four workgroups for every wave slot of the GPU (32
@@ -3506,7 +3648,7 @@ int sort_round(ps5_ctx* c, SortRun& R, uint32_t round, bool dev, bool* done)
             const uint32_t gt = (uint32_t)std::min<uint64_t>(kDevTinyWgs, div_up(nt0 + S, kWaves));
             const uint32_t gr = (uint32_t)std::min<uint64_t>(kDevRunWgs, nr0 + S / kTinyT + 1);
             B.pending = c->d_cnt + in_ci;
-            launch_leaves(c, B, rp, nsink, gt, gr, nt0 + S, nr0 + S, st);
+            launch_leaves(c, B, rp, nsink, done_leaves, true, gt, gr, nt0 + S, nr0 + S, st);
             if (lcp) {
                 uint64_t known = nt0 + nr0;
                 for (int cls = 0; cls < kBlkClasses; ++cls) known += c->h_cnt[C_BLOCK + 2 * cls + rp];
@@ -3521,9 +3663,10 @@ int sort_round(ps5_ctx* c, SortRun& R, uint32_t round, bool dev, bool* done)
                 // back and finish the round on the host
                 for (int cls = 0; cls < kBlkClasses; ++cls) blk_done[cls] = c->h_cnt[C_BLOCK + 2 * cls + rp];
                 if ((rc = readback(c, in_list, in_ci))) return rc;
-                if ((rc = host_levels(c, B, round, in_ci, blk_done, false, &leaves_forked, 0u, &after_blocks)))
+                done_leaves = LeavesDone{ c->h_cnt[C_TDONE], c->h_cnt[C_RDONE] };
+                if ((rc = host_levels(c, B, round, L, in_ci, blk_done, &done_leaves, &leaves_forked, 0u, &after_blocks)))
                     return rc;
-                if ((rc = host_round_end(c, B, round, leaves_forked, after_blocks))) return rc;
+                if ((rc = host_round_end(c, B, round, done_leaves, leaves_forked, after_blocks))) return rc;
             } else {
                 uint32_t nb = 0;
                 for (int cls = 0; cls < kBlkClasses; ++cls) nb += c->h_cnt[C_BLOCK + 2 * cls + rp];
@@ -3552,7 +3695,7 @@ void graph_round(ps5_ctx* c, SortRun& R, uint32_t round, uint32_t L, uint32_t nl
     if (round > 0) {
         uint32_t mask = (1u << (C_LROUND + np)) | (1u << (C_TINY + np)) | (1u << (C_RUN + np));
         for (int cls = 0; cls < kBlkClasses; ++cls) mask |= (1u << (C_BLOCK + 2 * cls + np)) | (1u << (C_BDONE + cls));
-        mask |= 1u << (C_RUNCONT + np);
+        mask |= (1u << (C_RUNCONT + np)) | (1u << C_TDONE) | (1u << C_RDONE);
         hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, st, c->d_cnt, mask);
     }
     const Sink nsink = make_sink(c, c->w.l_round[np], C_LROUND + np, np);
@@ -3566,8 +3709,10 @@ void graph_round(ps5_ctx* c, SortRun& R, uint32_t round, uint32_t L, uint32_t nl
         const Sink sink = make_sink(c, c->w.l_lvl[level & 1], out_ci, rp);
         const uint64_t seed = c->seed ^ ((uint64_t)round << 40) ^ ((uint64_t)level << 32);
         const bool rootlvl = round == 0 && level == 0;
-        dev_level(c, B, in_list, in_ci, rootlvl ? nl_root : any_large, S, sink, seed, R.fused_root && rootlvl,
-                  rootlvl, rootlvl ? (int)R.root_kmax : dev_level_kmax(c, R.root_max, level), level > 0 ? rp : -1);
+        const int src = level > 0 ? kFromRuns : round > 0 ? kFromPerm : kRootPlain;
+        if (level >= 2) dev_finish_leaves(c, B, rp, nsink, n);
+        dev_level(c, B, in_list, in_ci, rootlvl ? nl_root : any_large, S, sink, seed, src, level & 1,
+                  rootlvl ? (int)R.root_kmax : dev_level_kmax(c, R.root_max, level), level > 0 ? rp : -1);
         for (int cls = 0; cls < kBlkClasses; ++cls) {
             launch_block_class(c, B, rp, cls, 0, 0, true, block_grid_full(c, cls), nsink);
         }
@@ -3576,39 +3721,16 @@ void graph_round(ps5_ctx* c, SortRun& R, uint32_t round, uint32_t L, uint32_t nl
     }
     B.pending = c->d_cnt + in_ci;
     B.pending_err = 1;
-    launch_leaves(c, B, rp, nsink, (uint32_t)std::min<uint64_t>(kDevTinyWgs, div_up(n, kWaves)),
+    launch_leaves(c, B, rp, nsink, LeavesDone{}, true, (uint32_t)std::min<uint64_t>(kDevTinyWgs, div_up(n, kWaves)),
                   (uint32_t)std::min<uint64_t>(kDevRunWgs, c->w.cap_run), n, n, st);
     if (B.lcp) launch_leafbound(c, B, rp, (uint32_t)std::min<uint64_t>(kDevBoundWgs, div_up(n, kWG)), n);
-}
-
-// Round 0 keys the first classification pass does not extract: every
-// position's (no fused root), or those of a batch's sets that start as tiny
-// leaves or blocks (their lists and counts as setup_roots left them).
-int init_root_keys(ps5_ctx* c, const Bufs& B, uint32_t n, const uint64_t* set_first, bool fused_root)
-{
-    hipStream_t st = c->stream;
-    if (!fused_root) {
-        Launch L(c, K_INIT, (uint64_t)n * 20);   // offs 4 R + 8 characters R + key 8 W
-        hipLaunchKernelGGL(k_init, dim3(div_up(n, kWG)), dim3(kWG), 0, st, B, n);
-    } else if (set_first) {
-        Launch L(c, K_INIT, 0);
-        const uint32_t nt = c->h_upcnt[C_TINY];
-        if (nt) hipLaunchKernelGGL(k_init_items, dim3(std::min<uint32_t>(nt, 4096)), dim3(kWG), 0, st,
-                                   c->w.l_tiny[0], nt, B);
-        for (int cls = 0; cls < kBlkClasses; ++cls) {
-            const uint32_t nb = c->h_upcnt[C_BLOCK + 2 * cls];
-            if (nb) hipLaunchKernelGGL(k_init_items, dim3(std::min<uint32_t>(nb, 4096)), dim3(kWG), 0, st,
-                                       c->w.l_block[0] + (uint64_t)cls * c->w.cap_block, nb, B);
-        }
-    }
-    HIPCHK(hipGetLastError());
-    return PS5_OK;
 }
 
 int run_sort_keys(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_t* offs, const uint64_t* offs64,
                   uint32_t n, uint32_t* perm, uint32_t* lcp, const uint64_t* set_first, uint32_t nsets, bool pack)
 {
     int rc = ensure_capacity(c, n);
+    if (!rc) rc = ensure_tables(c);
     if (rc) return rc;
     for (int i = 0; i < K_NUM; ++i) { c->k_ms[i] = 0; c->k_launch[i] = 0; c->k_bytes[i] = 0; }
     c->st_rounds = c->st_levels = c->st_segments = c->st_leaves = c->st_syncs = 0;
@@ -3622,17 +3744,22 @@ int run_sort_keys(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_
     B.alen = alen;
     B.offs = offs;
     B.offs64 = offs64;
-    B.key0 = c->w.key[0]; B.key1 = c->w.key[1];
-    B.idx0 = c->w.idx[0]; B.idx1 = c->w.idx[1];
+    B.key = c->w.key;
+    B.idx = c->w.idx;
+    B.vpos = c->w.vpos;
+    B.src = c->w.src;
+    B.cap = c->w.cap;
+    B.cap_h = c->w.hist_cap;
     B.perm = perm;
     B.lcp = lcp;
     B.bkey = c->w.bkey;
-    B.bktrank = c->w.bktrank;
+    B.hist = c->w.hist;
+    B.gsum = c->w.gsum;
     B.pending = nullptr;
     B.pending_err = 0;
     B.leaf_keys = c->leaf_keys;
     set_depths(c, B, 0);
-    B.lut = nullptr;     // (set below, once the trees' buffers have their size)
+    B.lut = nullptr;
 
     // the roots (one, or a batch's sets) and their sizes
     uint32_t root_kmax = 1;                     // largest treebits of a large root
@@ -3652,45 +3779,22 @@ int run_sort_keys(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_
                                                                                (int)c->max_treebits));
         }
     }
-    // Roots larger than a block have their keys extracted by the first
-    // classification pass itself (its level holds only roots, whose indices
-    // are their positions); k_init covers the rest.  One such root alone is
-    // known to the host without asking.
     const bool single_root = !set_first && n > kBlkT;
-    const bool fused_root = single_root || (set_first && root_sum > 0);
     bool dev = c->planning == 1 ||
                (c->planning == 2 && !c->profile && !set_first && n < kAutoDevMax);   // (profiled sorts: host, whose
                                                                                      // launches know their bytes)
     // a single root planned on the host: the root level's plan fetch, the
     // sort's first kernel, also sets the counters and the root item up
     c->pending_root = single_root && !dev && !(c->graph_rounds && !c->profile) ? n : 0u;
-    if (!c->pending_root && (rc = setup_roots(c, n, set_first, nsets))) return rc;
-    if ((rc = init_root_keys(c, B, n, set_first, fused_root))) return rc;
-    // device-planned levels: the plan buffers take their largest size now
-    // (the levels' sizes are not known on the host)
-    if ((dev || c->chain_levels) && (rc = grow_level(c, c->w.cap_large, c->w.cap + c->w.cap / 4 + 64))) return rc;
-    if (single_root) {
+    if (c->pending_root) {
         for (int i = 0; i < C_NCNT; ++i) c->h_cnt[i] = 0;
         c->h_cnt[C_LROUND] = 1;
-        c->w.h_large[0] = Item{ 0u, n, 0u, F_IDENT };
-    } else if (!dev) {
-        if ((rc = readback(c, c->w.l_round[0], C_LROUND))) return rc;
-    } else if (set_first) {     // the counts setup_roots uploaded
-        memcpy(c->h_cnt, c->h_upcnt, C_NCNT * sizeof(uint32_t));
-    } else {                    // one root, a tiny leaf or a block
-        for (int i = 0; i < C_NCNT; ++i) c->h_cnt[i] = 0;
-        c->h_cnt[n <= kTinyT ? C_TINY : C_BLOCK + 2 * block_class(n)] = 1;
+        c->w.h_large[0] = Item{ 0u, n, 0u, F_IDENT, 0u, 0u };
+    } else if ((rc = setup_roots(c, n, set_first, nsets))) {
+        return rc;
     }
-
-    if (fused_root && pack && root_max >= kPackMin) {     // a root's keys may be packed: its code table beside its tree
-        if (!set_first) {
-            if ((rc = grow_level(c, 1, 0))) return rc;
-        } else if ((rc = grow_level(c, c->w.cap_large, 0))) {
-            return rc;
-        }
-        B.lut = c->w.lut;
-    }
-    SortRun R{ B, n, alen, fused_root, root_kmax, root_max, root_sum };
+    if (pack && root_max >= kPackMin) B.lut = c->w.lut;     // large roots may pack their keys
+    SortRun R{ B, n, alen, root_kmax, root_max, root_sum };
     uint32_t start = 0;
     if (c->graph_rounds && !c->profile) {
         // the first graph_rounds rounds as one captured graph, replayed while
@@ -3700,13 +3804,12 @@ int run_sort_keys(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_
         if (!set_first) nl_root = n > kBlkT ? 1 : 0;
         std::vector<uint64_t> key = { (uint64_t)(uintptr_t)arena, alen, (uint64_t)(uintptr_t)offs,
                                       (uint64_t)(uintptr_t)offs64, n, (uint64_t)(uintptr_t)perm,
-                                      (uint64_t)(uintptr_t)lcp, nsets, (uint64_t)(uintptr_t)c->w.key[0], c->w.cap,
+                                      (uint64_t)(uintptr_t)lcp, nsets, (uint64_t)(uintptr_t)c->w.key, c->w.cap,
                                       (uint64_t)(uintptr_t)c->w.trees, c->w.trees_cap, c->leaf_target,
                                       c->max_treebits, c->max_oversample, c->graph_rounds, c->seed,
                                       c->w_gen, c->w.fixed ? 1u : 0u, c->graph_levels, c->chunk_max,
                                       c->chunk_max_root, c->min_tiles, c->leaf_keys };
         for (uint32_t s = 0; set_first && s <= nsets; ++s) key.push_back(set_first[s]);
-        if ((rc = grow_level(c, c->w.cap_large, c->w.cap + c->w.cap / 4 + 64))) return rc;
         if (!c->graph_exec || key != c->graph_key) {
             if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
             if (c->graph) (void)hipGraphDestroy(c->graph);
@@ -3737,14 +3840,6 @@ int run_sort_keys(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_
             // a round needed more levels than the graph holds: sort again,
             // every level planned on the host
             if ((rc = setup_roots(c, n, set_first, nsets))) return rc;
-            if ((rc = init_root_keys(c, B, n, set_first, fused_root))) return rc;
-            if (single_root) {
-                for (int i = 0; i < C_NCNT; ++i) c->h_cnt[i] = 0;
-                c->h_cnt[C_LROUND] = 1;
-                c->w.h_large[0] = Item{ 0u, n, 0u, F_IDENT };
-            } else if ((rc = readback(c, c->w.l_round[0], C_LROUND))) {
-                return rc;
-            }
             dev = false;
         } else {
             if (c->h_cnt[C_ERR] & ERR_CAP) return set_err(PS5_ERR_CAPACITY, "work list capacity exceeded");
@@ -3805,18 +3900,12 @@ int ps5_ctx_create(ps5_ctx** out, int device)
     if (!out) return set_err(PS5_ERR_ARG, "out is NULL");
     *out = nullptr;
     HIPCHK(hipSetDevice(device));
-    HIPCHK(hipFuncSetAttribute((const void*)k_scatter<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               ScatLds<false>::kBytes));
-    HIPCHK(hipFuncSetAttribute((const void*)k_scatter<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               ScatLds<true>::kBytes));
-#define PS5_COUNT_INSTANCES(NB)                                                              \
-    (const void*)k_count<NB, false, kNoRoot>, (const void*)k_count<NB, false, kRootPlain>,   \
-    (const void*)k_count<NB, false, kRootPack>, (const void*)k_count<NB, true, kNoRoot>,     \
-    (const void*)k_count<NB, true, kRootPlain>, (const void*)k_count<NB, true, kRootPack>
-    for (const void* f : { PS5_COUNT_INSTANCES(8), PS5_COUNT_INSTANCES(9), PS5_COUNT_INSTANCES(10),
-                           PS5_COUNT_INSTANCES(11) })
-#undef PS5_COUNT_INSTANCES
-        HIPCHK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, count_lds_bytes(kMaxTreebits)));
+    for (int kmax = 7; kmax <= kMaxTreebits; ++kmax)
+        for (int src : { kFromRuns, kRootPlain, kRootPack, kFromPerm }) {
+            uint32_t lds = 0;
+            const PartKernel f = part_kernel(kmax, src, &lds);
+            HIPCHK(hipFuncSetAttribute((const void*)f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        }
     ps5_ctx* c = new ps5_ctx;
     c->device = device;
     c->trace = getenv("PS5_TRACE") != nullptr;
@@ -3827,14 +3916,13 @@ int ps5_ctx_create(ps5_ctx** out, int device)
     if (const char* cl = getenv("PS5_CHAIN_LEVELS")) c->chain_levels = atoi(cl) != 0;
     int ncu = 0;
     hipError_t e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device);
-    c->scatter_wgs = std::max<uint32_t>(kXcds, (uint32_t)std::max(ncu, 0) / kXcds * kXcds);
+    c->cus = std::max<uint32_t>(kXcds, (uint32_t)std::max(ncu, 0) / kXcds * kXcds);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming);
     if (e == hipSuccess) e = hipMalloc(&c->d_cnt, C_NCNT * sizeof(uint32_t));
     if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&c->h_cnt), C_NCNT * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&c->h_upcnt), C_NCNT * sizeof(uint32_t));
     if (e == hipSuccess)
         e = hipHostMalloc(reinterpret_cast<void**>(&c->h_stage), kStageHead + kPeek * sizeof(Item),
                           hipHostMallocMapped | hipHostMallocCoherent);
@@ -3875,7 +3963,6 @@ void ps5_ctx_destroy(ps5_ctx* c)
     if (c->d_sets) (void)hipFree(c->d_sets);
     if (c->d_merge) (void)hipFree(c->d_merge);
     if (c->h_cnt) (void)hipHostFree(c->h_cnt);
-    if (c->h_upcnt) (void)hipHostFree(c->h_upcnt);
     if (c->h_stage) (void)hipHostFree(c->h_stage);
     if (c->h_roots) (void)hipHostFree(c->h_roots);
     if (c->h_sums) (void)hipHostFree(c->h_sums);
@@ -3993,21 +4080,22 @@ int ps5_merge_device(ps5_ctx* c, const uint8_t* d_arena, uint64_t arena_bytes, c
     B.arena = d_arena;
     B.alen = arena_bytes;
     B.offs = d_offs;
-    // ping-pong buffers: indices in idx[0]/idx[1], first 8 characters in
-    // key[0]/key[1], LCPs in the two halves of bkey
-    uint32_t* ti[2] = { c->w.idx[0], c->w.idx[1] };
-    key64* tk[2] = { c->w.key[0], c->w.key[1] };
+    // ping-pong buffers: indices in the two halves of idx, first 8 characters
+    // in those of key, LCPs in those of bkey
+    uint32_t* ti[2] = { c->w.idx, c->w.idx + c->w.cap };
+    key64* tk[2] = { c->w.key, c->w.key + c->w.cap };
     uint32_t* tl[2] = { reinterpret_cast<uint32_t*>(c->w.bkey), reinterpret_cast<uint32_t*>(c->w.bkey) + c->w.cap };
     std::vector<uint64_t> bounds(run_first, run_first + nruns + 1);
     const uint32_t* si = d_idx;
     const uint32_t* sl = d_lcp;
     // the first round reads every string's first 8 characters from ik, keys
     // extracted in input order by one streaming pass (the previous round's
-    // output carries them afterwards); key[1] is free until the second merge round writes it
-    key64* ik = c->w.key[1];
+    // output carries them afterwards); the second half of key is free until the
+    // second merge round writes it
+    key64* ik = tk[1];
     {
         Bufs BI = B;
-        BI.key0 = ik;
+        BI.key = ik;
         hipLaunchKernelGGL(k_init, dim3(div_up(n, kWG)), dim3(kWG), 0, st, BI, (uint32_t)n);
         HIPCHK(hipGetLastError());
     }
@@ -4154,10 +4242,10 @@ int ps5_ctx_set_tuning(ps5_ctx* c, uint32_t leaf_target, uint32_t max_treebits, 
 int ps5_ctx_set_shape(ps5_ctx* c, uint32_t chunk_max, uint32_t chunk_max_root, uint32_t min_tiles, uint32_t leaf_keys)
 {
     if (!c) return set_err(PS5_ERR_ARG, "ctx is NULL");
-    if (chunk_max < (uint32_t)kChunkMin || chunk_max > (uint32_t)kChunkMax)
-        return set_err(PS5_ERR_ARG, "chunk_max must be in [%d, %d]", kChunkMin, kChunkMax);
-    if (chunk_max_root < (uint32_t)kChunkMin || chunk_max_root > (uint32_t)kChunkMaxIdent)
-        return set_err(PS5_ERR_ARG, "chunk_max_root must be in [%d, %d]", kChunkMin, kChunkMaxIdent);
+    if (chunk_max < (uint32_t)kChunkMin || chunk_max > kShapeChunkMax)
+        return set_err(PS5_ERR_ARG, "chunk_max must be in [%d, %u]", kChunkMin, kShapeChunkMax);
+    if (chunk_max_root < (uint32_t)kChunkMin || chunk_max_root > kShapeChunkMaxRoot)
+        return set_err(PS5_ERR_ARG, "chunk_max_root must be in [%d, %u]", kChunkMin, kShapeChunkMaxRoot);
     if (min_tiles < 1 || min_tiles > 65536) return set_err(PS5_ERR_ARG, "min_tiles must be in [1, 65536]");
     if (leaf_keys < 1 || leaf_keys > 8) return set_err(PS5_ERR_ARG, "leaf_keys must be in [1, 8]");
     c->chunk_max = chunk_max;

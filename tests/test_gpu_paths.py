@@ -98,3 +98,38 @@ def test_packed_batch_of_mixed_alphabets(ps5, oracle, planning):
             b, e = int(first[k]), int(first[k + 1])
             r, msg = oracle.verify(arena, offs[b:e].astype(np.uint32), perm[b:e], lcp[b:e])
             assert r == 0, (k, msg)
+
+
+@pytest.mark.parametrize("n", [2049, 4095, 4096, 4097, 6145, 65537, 262143, 262145, 600011])
+@pytest.mark.parametrize("kind", ["spread", "sorted", "heavy"])
+def test_partition_edges(ctx, oracle, n, kind):
+    """chunk and group remainders; buckets that lie in few chunks (sorted
+    input) and in all of them (heavy duplicates)"""
+    rng = np.random.default_rng(n)
+    hi = 24
+    lens = rng.integers(0, hi, n) if kind != "heavy" else rng.integers(0, 3, n)
+    chars = rng.integers(33, 127, (n, hi)).astype(np.uint8)
+    if kind == "sorted":
+        chars[:, :4] = np.sort(rng.integers(33, 127, (n, 4)).astype(np.uint8).view(">u4").ravel()).view(np.uint8).reshape(n, 4)
+    ends = np.cumsum(lens + 1)
+    offs = (ends - lens - 1).astype(np.uint32)
+    arena = np.zeros(int(ends[-1]) + 16, np.uint8)
+    inside = np.arange(hi)[None, :] < lens[:, None]
+    arena[(offs[:, None].astype(np.int64) + np.arange(hi)[None, :])[inside]] = chars[inside]
+    check(ctx, oracle, arena, offs)
+    check(ctx, oracle, arena, offs, with_lcp=False)
+
+
+@pytest.mark.parametrize("planning", [0, 1])
+@pytest.mark.parametrize("tuning", [(64, 2, 4), (64, 3, 2), (256, 10, 32)])
+def test_many_levels_and_rounds(ps5, oracle, planning, tuning):
+    """rounds of three levels and more reuse the buffers and run tables their
+    earlier leaves lie in, and later rounds start from the permutation"""
+    c = ps5.Context(0)
+    try:
+        c.set_planning(planning)
+        c.set_tuning(*tuning)
+        for sigma, n, seed in ((3, 300007, 1), (60, 150001, 2), (2, 70001, 3)):
+            check(c, oracle, *packed_case(sigma, n, seed, hi=40))
+    finally:
+        c.close()
