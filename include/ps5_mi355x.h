@@ -251,8 +251,8 @@ int ps5_ctx_get_tuning(ps5_ctx* ctx, uint32_t* leaf_target, uint32_t* max_treebi
  * buckets and its key cache is one uint64, bingmann-sample_sort.hpp:49):
  *   chunk_max      keys per chunk of a multi-workgroup level, the unit one
  *                  workgroup ranks and reorders in LDS, in [2048, 9216]
- *                  (default 9216; a chunk holds at most 4096 keys, so larger
- *                  limits act as 4096);
+ *                  (default 9216; a chunk holds at most 8192 keys, so larger
+ *                  limits act as 8192);
  *   chunk_max_root the same in a level of roots, in [2048, 12032] (default
  *                  12032, likewise);
  *   min_tiles      chunks a level is spread over at least, shrinking (not

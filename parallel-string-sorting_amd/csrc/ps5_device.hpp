@@ -290,11 +290,13 @@ __device__ __forceinline__ uint64_t str_off(const Bufs& B, uint32_t i)
     return B.offs64 ? B.offs64[i] : (uint64_t)B.offs[i];
 }
 
+struct Rec { uint32_t lo, hi, id; };
+__device__ __forceinline__ key64 rec_key(const Rec& r) { return ((key64)r.hi << 32) | r.lo; }
+
 // Where a bucket's strings lie: run c holds the positions from V[c] on, at
-// S[c] and after in K and I.
+// S[c] and after in R.
 struct Runs {
-    const key64* K;
-    const uint32_t* I;
+    const Rec* R;
     const uint32_t* V;
     const uint32_t* S;
     uint32_t nch;
@@ -303,7 +305,7 @@ __device__ __forceinline__ Runs runs_of(const Bufs& B, const Item& it)
 {
     const uint64_t b = it.flags & F_BUFB;
     const uint64_t t = it.row + b * B.cap_h;
-    return Runs{ B.key + b * B.cap, B.idx + b * B.cap, B.vpos + t, B.src + t, it.nch };
+    return Runs{ reinterpret_cast<const Rec*>(B.rec) + b * B.cap, B.vpos + t, B.src + t, it.nch };
 }
 // the run holding position pos: the last of n whose first position is not
 // above it (an empty run shares its position with the run after it)

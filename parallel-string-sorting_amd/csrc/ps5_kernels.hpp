@@ -3,12 +3,15 @@
 // Device data layout (one sort, n strings, positions 0..n-1 of the sorted order):
 //   arena      characters as given by the caller (never written)
 //   offs[n]    uint32 start offset of input string i
-//   key[2][n], idx[2][n]  keys (uint64) and input indices as a level of the
+//   rec[2][n]  records of 12 bytes (key and input index) as a level of the
 //              sample sort leaves them: every chunk of a segment reordered by
 //              bucket, in place of the chunk.  Even levels of a round write
-//              buffer 0, odd levels buffer 1
+//              buffer 0, odd levels buffer 1.  Key and index lie together
+//              because a bucket is gathered in short runs: 8 strings of a
+//              511-bucket level's chunk of 4096 touched 340 bytes of cache
+//              lines in two arrays
 //   vpos[2], src[2]  per buffer: for bucket b and chunk c of a segment, the
-//              first sorted position and the place in key/idx of the bucket's
+//              first sorted position and the place in rec of the bucket's
 //              strings in that chunk (its run), bucket-major
 //   bkey[n]    uint64 scratch: depth key of the first/last position of a leaf
 //   sdepth[2][n] uint32 by round parity: characters the strings of the round
@@ -52,15 +55,17 @@ constexpr uint32_t kTreeSlots = 2048;        // per segment: level-order tree [0
 // chunks that way; then the limit shrinks (not below kChunkMin) so small
 // sorts still spread over the GPU.  A chunk is the unit of k_part: one
 // workgroup of kPartWaves waves ranks its keys stably and reorders them.
-// 4096 keys (52 KB of LDS with a 9-level tree) leave room for three workgroups
-// per CU, so that one loads while others rank: 64 M random strings take 605 us
-// at the root level and a batch of 50 M strings with 10-level trees 650 us (two
-// workgroups per CU), with 6144 keys 620 and 1000 us (one workgroup with 10
-// levels).
+// Longer chunks make longer runs, which the next reader gathers with fewer
+// partial cache lines; the records are staged in parts, so that the LDS of
+// two workgroups or more fits a CU and one loads while another ranks.  2 GiB
+// of random strings sort in 2.24 ms with chunks of 8192 keys, 2.29 with 6144
+// and 2.37 with 4096 (the root level alone is faster with 4096, 0.61 ms
+// against 0.66, where three workgroups fit).
 constexpr int kPartWaves = 8;
 constexpr int kPartThreads = kPartWaves * 64;
-constexpr int kPartGroups = 8;               // 64-key groups per wave
+constexpr int kPartGroups = 16;              // 64-key groups per wave
 constexpr int kPartMax = kPartThreads * kPartGroups;
+constexpr uint32_t kPartStage = 2752;        // records staged in LDS at a time (a multiple of 4)
 constexpr int kChunkMin = 2048;
 constexpr uint32_t kHistGroup = 64;          // chunks whose bucket counts are summed together
 // limits and defaults of ps5_ctx_set_shape
@@ -91,7 +96,7 @@ struct Item {            // a segment or a leaf
 // p is input string p) and F_NEXT (a segment of an earlier round: perm[p]) say
 // that its keys are still to be read from the arena; otherwise it is a bucket,
 // whose strings lie in the runs of its row in buffer F_BUFB.
-constexpr uint32_t F_BUFB = 1u;              // key[1]/idx[1]/vpos[1]/src[1]
+constexpr uint32_t F_BUFB = 1u;              // rec[1]/vpos[1]/src[1]
 constexpr uint32_t F_SORTED = 2u;            // all keys equal (equal bucket)
 constexpr uint32_t F_IDENT = 4u;
 constexpr uint32_t F_NEXT = 32u;
@@ -134,6 +139,8 @@ __host__ __device__ constexpr KeyFmt key_fmt(uint32_t flags)
     return f == 0 ? KeyFmt{ 32, 8, 0, 0xFFu } : f == 1 ? KeyFmt{ 86, 21, 1, 7u << 1 }
          : f == 2 ? KeyFmt{ 64, 16, 0, 15u } : KeyFmt{ 52, 12, 4, 31u << 4 };
 }
+
+constexpr uint32_t kRecWords = 3;            // key low, key high, index
 
 struct LargeDesc {       // one segment of the multi-workgroup sample-sort step
     Item seg;
@@ -186,8 +193,7 @@ struct Bufs {
     uint64_t alen;
     const uint32_t* offs;      // string start offsets (uint32), or
     const uint64_t* offs64;    // uint64 offsets when non-null (batches over 4 GiB)
-    key64* key;          // two buffers of cap entries each, one after the other
-    uint32_t* idx;
+    uint32_t* rec;       // two buffers of cap records (kRecWords words) each, one after the other
     uint32_t* vpos;      // two tables of cap_h entries each
     uint32_t* src;
     uint64_t cap, cap_h;

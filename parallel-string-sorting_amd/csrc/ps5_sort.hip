@@ -38,11 +38,11 @@ using namespace ps5;
 // ===========================================================================
 
 // First 8 characters of every string, in input order (the LCP merge's keys).
-__global__ __launch_bounds__(kWG) void k_init(Bufs B, uint32_t n)
+__global__ __launch_bounds__(kWG) void k_init(Bufs B, key64* key, uint32_t n)
 {
     const uint32_t i = blockIdx.x * kWG + tid_x();
     if (i >= n) return;
-    B.key[i] = load_key(B.arena, B.alen, str_off(B, i));
+    key[i] = load_key(B.arena, B.alen, str_off(B, i));
 }
 
 // Reset counters and place the root item.
@@ -402,7 +402,7 @@ __device__ __forceinline__ void tree_of_segment(LargeDesc* Dp, uint32_t si, cons
         }
 #pragma unroll
         for (int e = 0; e < kPer; ++e) {
-            const key64 x = R.K[checked_place(B, q[e])];
+            const key64 x = rec_key(R.R[checked_place(B, q[e])]);
             v[e] = o + e < ss ? x : ~0ull;
         }
         __syncthreads();     // the row's copy is no longer read
@@ -648,29 +648,28 @@ __device__ __forceinline__ uint32_t mapped_place(const Bufs& B, const RunMap<MAX
 // .hpp:1464-1490, in one pass): each wave classifies its part of the chunk
 // with the splitter tree in LDS and ranks it stably (ballot matching and
 // per-wave bucket counts, ranks follow input order), a scan of the counts
-// places every (bucket, wave), the keys and then the indices are staged in
-// LDS in that order and written back in place of the chunk, whole lines at a
-// time.  The chunk's bucket counts and starts go to its row of hist.
+// places every (bucket, wave), and the records are staged in LDS in that
+// order and written back in place of the chunk, 16 bytes a lane.  The chunk's
+// bucket counts and starts go to its row of hist.
 //
 // 2 GiB of random strings, root level (reading the arena, 511 splitters):
-// 0.60 ms, 5.3 TB/s of the 3.2 GB it reads and writes, the rate of a plain
+// 0.66 ms, 4.9 TB/s of the 3.2 GB it reads and writes, against 5.5 of a plain
 // copy; counting first and scattering afterwards took 0.71 + 0.50 ms.
 //
-// LDS: the key stage (the lane-mask tables of match_bucket_lds, or the run
-// map of a bucket's chunk, before that), the per-wave counts and the tree;
-// three workgroups per CU up to 9 treebits, two with 10.
+// LDS: the stage (the lane-mask tables of match_bucket_lds, or the run map of
+// a bucket's chunk, before that), the per-wave counts and the tree.
 template <int NB>
 struct PartLds {
     static constexpr uint32_t kSlots = 1u << NB;             // bucket slots per wave
-    static constexpr uint32_t kKeyOff = 0;
-    static constexpr uint32_t kCntOff = kPartMax * 8;
+    static constexpr uint32_t kStageOff = 0;                 // (+ 3 words: the image is aligned like its destination)
+    static constexpr uint32_t kCntOff = (kPartStage * kRecWords + 4) * 4;
     static constexpr uint32_t kTreeOff = kCntOff + kPartWaves * kSlots * 2;
     static constexpr uint32_t kTmpOff = kTreeOff + kSlots / 2 * 8;
     static constexpr uint32_t kBytes = kTmpOff + 64;
     static constexpr int kPeerBits = NB < 8 ? NB : 8;
-    static constexpr uint32_t kMapOff = 0;
-    static_assert(((uint32_t)kPartWaves << kPeerBits << 3) <= kCntOff, "the lane-mask tables fit the key stage");
-    static_assert(kMapOff + sizeof(RunMap<kPartMax>) <= kCntOff, "the run map fits the key stage");
+    static_assert(((uint32_t)kPartWaves << kPeerBits << 3) <= kCntOff, "the lane-mask tables fit the stage");
+    static_assert(sizeof(RunMap<kPartMax>) <= kTmpOff, "the run map fits the stage and the counts");
+    static_assert(kCntOff % 16 == 0 && kPartStage % 4 == 0, "16-byte copies");
 };
 
 template <int NB, int SRC>
@@ -680,8 +679,8 @@ __device__ __forceinline__ void part_chunk(uint32_t ti, const Plan& P, const Buf
     using L = PartLds<NB>;
     constexpr int kE = kPartGroups;
     constexpr uint32_t T = kPartThreads;
-    key64* s_key = reinterpret_cast<key64*>(smem + L::kKeyOff);
-    uint64_t* s_peer = reinterpret_cast<uint64_t*>(smem + L::kKeyOff);
+    uint32_t* s_rec = reinterpret_cast<uint32_t*>(smem + L::kStageOff);
+    uint64_t* s_peer = reinterpret_cast<uint64_t*>(smem + L::kStageOff);
     uint16_t* s_cnt = reinterpret_cast<uint16_t*>(smem + L::kCntOff);
     key64* s_tree = reinterpret_cast<key64*>(smem + L::kTreeOff);
     uint32_t* s_tmp = reinterpret_cast<uint32_t*>(smem + L::kTmpOff);
@@ -709,14 +708,15 @@ __device__ __forceinline__ void part_chunk(uint32_t ti, const Plan& P, const Buf
 #define PS5_PART_POS(e) min(wb + (e) * 64 + lane, m - 1)
     if (SRC == kFromRuns) {
         const Runs R = runs_of(B, seg);
-        RunMap<kPartMax>& M = *reinterpret_cast<RunMap<kPartMax>*>(smem + L::kMapOff);
+        RunMap<kPartMax>& M = *reinterpret_cast<RunMap<kPartMax>*>(smem);
         map_runs<kPartWaves, kPartMax>(R, seg.begin + seg.size, seg.begin + cb, m, M);
 #pragma unroll
         for (int e = 0; e < kE; ++e) {
-            const uint32_t q = mapped_place(B, M, PS5_PART_POS(e));
-            kv[e] = R.K[q];
-            iv[e] = R.I[q];
+            const Rec r = R.R[mapped_place(B, M, PS5_PART_POS(e))];
+            kv[e] = rec_key(r);
+            iv[e] = r.id;
         }
+        __syncthreads();     // the run map is read
     } else if (SRC == kFromPerm) {
         const uint32_t depth = seg_depth(B, seg.rbeg);
 #pragma unroll
@@ -738,26 +738,38 @@ __device__ __forceinline__ void part_chunk(uint32_t ti, const Plan& P, const Buf
     for (uint32_t i = tid; i <= nspl; i += T) s_tree[i] = tree[i];
     for (uint32_t i = tid; i < kPartWaves * L::kSlots / 2; i += T) reinterpret_cast<uint32_t*>(s_cnt)[i] = 0;
     if (SRC == kRootPack && fmt) {
-        // packed keys are extracted in a rolled loop through the wave's part
-        // of the key stage: unrolled with the others they would take twice
-        // the registers.  The code table sits where the counts go afterwards
+        // packed keys are extracted in a rolled loop, four groups at a time
+        // through the wave's part of the stage: unrolled with the others they
+        // would take twice the registers.  The code table sits where the
+        // counts go afterwards
         uint8_t* s_lut = reinterpret_cast<uint8_t*>(s_cnt);
+        constexpr int kH = 4;
+        static_assert(kPartWaves * kH * 64 * 8 <= L::kCntOff && kE % kH == 0, "the groups' keys fit the stage");
+        key64* s_w = reinterpret_cast<key64*>(smem + L::kStageOff) + w * kH * 64;
         __syncthreads();
         if (tid < kLutBytes) s_lut[tid] = B.lut[(uint64_t)tr.seg * kLutBytes + tid];
         __syncthreads();
         bool bad = false;
+#pragma unroll
+        for (int e0 = 0; e0 < kE; e0 += kH) {
+            if ((uint32_t)e0 * 64 >= per) {     // (uniform)
+#pragma unroll
+                for (int j = 0; j < kH; ++j) kv[e0 + j] = 0;
+                continue;
+            }
 #pragma unroll 2
-        for (uint32_t p = lane; p < per; p += 64) {
-            const uint32_t q = min(wb + p, m - 1);
-            s_key[wb + p] = pack_key_fmt(load_chars24(B.arena, B.alen, str_off(B, seg.begin + cb + q)), fmt, s_lut, &bad);
+            for (int j = 0; j < kH; ++j) {
+                const uint32_t q = min(wb + (e0 + j) * 64 + lane, m - 1);
+                s_w[j * 64 + lane] =
+                    pack_key_fmt(load_chars24(B.arena, B.alen, str_off(B, seg.begin + cb + q)), fmt, s_lut, &bad);
+            }
+#pragma unroll
+            for (int j = 0; j < kH; ++j) kv[e0 + j] = s_w[j * 64 + lane];
         }
         if (bad) flag_error(B.cnt, ERR_ALPHA);
-#pragma unroll
-        for (int e = 0; e < kE; ++e) kv[e] = (uint32_t)e * 64 < per ? s_key[wb + e * 64 + lane] : 0ull;
-        __syncthreads();     // the table and the keys are read
+        __syncthreads();     // the table is read
         if (tid < kLutBytes / 4) reinterpret_cast<uint32_t*>(s_cnt)[tid] = 0;
     }
-    if (SRC == kFromRuns) __syncthreads();     // the run map is read
     for (uint32_t i = tid; i < ((uint32_t)kPartWaves << L::kPeerBits); i += T) s_peer[i] = 0;
     __syncthreads();
     uint16_t* cnt_w = s_cnt + w * L::kSlots;
@@ -837,29 +849,39 @@ __device__ __forceinline__ void part_chunk(uint32_t ti, const Plan& P, const Buf
         uint32_t slot = act ? cnt_w[br[e] >> 16] + (br[e] & 0xFFFFu) : 0xFFFFFFFFu;
         if (act && slot >= m) { flag_error(B.cnt, ERR_BOUNDS); slot = 0xFFFFFFFFu; }
         br[e] = slot;
-        if (slot < m) s_key[slot] = kv[e];
     }
-    __syncthreads();
-    // the buffer the segment's strings are not in
+    // the records in their new order, kPartStage at a time; the image in LDS
+    // is shifted so that it is aligned to 16 bytes where its destination is.
+    // The destination is the buffer the segment's strings are not in
     const uint64_t at = (SRC == kFromRuns && !(seg.flags & F_BUFB) ? B.cap : 0ull) + seg.begin + cb;
-    key64* KD = B.key + at;
-    uint32_t* ID = B.idx + at;
+    uint32_t* out = B.rec + at * kRecWords;
+    const uint32_t shift = (uint32_t)((uintptr_t)out >> 2) & 3u;
+    for (uint32_t s0 = 0; s0 < m; s0 += kPartStage) {     // (uniform)
+        const uint32_t ns = min(m - s0, kPartStage);
+        if (s0) __syncthreads();     // the last part is copied (first: the lane-mask tables are read, a barrier ago)
 #pragma unroll
-    for (int e = 0; e < kE; ++e) {
-        const uint32_t j = e * T + tid;
-        if (j < m) KD[j] = s_key[j];
-    }
-    __syncthreads();
-    uint32_t* s_idx = reinterpret_cast<uint32_t*>(smem + L::kKeyOff);
+        for (int e = 0; e < kE; ++e) {
+            const uint32_t r = br[e] - s0;
+            if (r < ns) {
+                uint32_t* x = s_rec + shift + r * kRecWords;
+                x[0] = (uint32_t)kv[e];
+                x[1] = (uint32_t)(kv[e] >> 32);
+                x[2] = SRC == kRootPlain || SRC == kRootPack ? seg.begin + cb + wb + e * 64 + lane : iv[e];
+            }
+        }
+        __syncthreads();
+        const uint32_t words = ns * kRecWords;
+        uint32_t* o = out + (uint64_t)s0 * kRecWords - shift;      // (a 16-byte boundary)
+        const uint4* img = reinterpret_cast<const uint4*>(s_rec);
+        for (uint32_t v = tid; 4 * v < shift + words; v += T) {
+            if (4 * v >= shift && 4 * v + 4 <= shift + words) {
+                reinterpret_cast<uint4*>(o)[v] = img[v];
+            } else {     // the ends
 #pragma unroll
-    for (int e = 0; e < kE; ++e)
-        if (br[e] < m)
-            s_idx[br[e]] = SRC == kRootPlain || SRC == kRootPack ? seg.begin + cb + wb + e * 64 + lane : iv[e];
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < kE; ++e) {
-        const uint32_t j = e * T + tid;
-        if (j < m) ID[j] = s_idx[j];
+                for (uint32_t j = 4 * v; j < 4 * v + 4; ++j)
+                    if (j >= shift && j < shift + words) o[j] = s_rec[j];
+            }
+        }
     }
 #undef PS5_PART_POS
 }
@@ -1294,8 +1316,9 @@ __device__ __forceinline__ void load_tiny(const Bufs& B, const Item& L, uint32_t
         q = run_place(B, R, pos);
     }
     if (act) {
-        *k = R.K[q];
-        *id = R.I[q];
+        const Rec r = R.R[q];
+        *k = rec_key(r);
+        *id = r.id;
     }
 }
 
@@ -1800,8 +1823,9 @@ __device__ __forceinline__ void block_one(const Item L, const Bufs& B, const Sin
         }
 #pragma unroll
         for (int e = 0; e < kPerThread; ++e) {
-            w[e] = R.K[q[e]];
-            idv[e] = R.I[q[e]];
+            const Rec r = R.R[q[e]];
+            w[e] = rec_key(r);
+            idv[e] = r.id;
         }
     }
     // (the sort writes s_k only after a barrier)
@@ -1979,7 +2003,7 @@ __global__ __launch_bounds__(kWG) void k_leaf_run(const Item* items, const uint3
             const uint32_t r = find_run(s_v, R.nch, cb + p);
             return checked_place(B, s_v[kRunRow + r] + (cb + p - s_v[r]));
         };
-        const key64 key = R.K[place(0u)];
+        const key64 key = rec_key(R.R[place(0u)]);
         const KeyFmt F = key_fmt(L.flags);
         const uint32_t depth = seg_depth(B, L.rbeg);
         // identical strings are done, others continue at the next depth
@@ -1987,7 +2011,7 @@ __global__ __launch_bounds__(kWG) void k_leaf_run(const Item* items, const uint3
         const uint32_t l = depth + key_depth(key, F);
 #pragma unroll 4
         for (uint32_t p = tid_x(); p < m; p += kWG) {
-            B.perm[cb + p] = R.I[place(p)];
+            B.perm[cb + p] = R.R[place(p)].id;
             if (term && B.lcp && cb + p > L.begin) B.lcp[cb + p] = l;
         }
         if (tid_x() < 64) {
@@ -2424,8 +2448,7 @@ enum { S_BLOCK, S_TINY, S_RUN, S_NUM };
 struct WorkBuffers {
     bool fixed = false;              // carved from the static scratch: never grown or freed
     uint64_t cap = 0;
-    key64* key = nullptr;            // two buffers of cap entries, one after the other
-    uint32_t* idx = nullptr;
+    uint32_t* rec = nullptr;         // two buffers of cap records, one after the other
     key64* bkey = nullptr;
     uint32_t* sdepth[2] = { nullptr, nullptr };
     // large segments: first level of a round [round parity], later levels [level parity]
@@ -2595,8 +2618,8 @@ void free_buffers(ps5_ctx* c)
         c->w.l_tiny[i] = nullptr; c->w.l_block[i] = nullptr; c->w.l_run[i] = nullptr;
         c->w.sdepth[i] = nullptr;
     }
-    f(c->w.key); f(c->w.idx); f(c->w.bkey); f(c->w.trees); f(c->w.lut); f(c->w.d_plan);
-    c->w.key = nullptr; c->w.idx = nullptr; c->w.bkey = nullptr; c->w.trees = nullptr; c->w.lut = nullptr; c->w.d_plan = nullptr;
+    f(c->w.rec); f(c->w.bkey); f(c->w.trees); f(c->w.lut); f(c->w.d_plan);
+    c->w.rec = nullptr; c->w.bkey = nullptr; c->w.trees = nullptr; c->w.lut = nullptr; c->w.d_plan = nullptr;
     free_tables(c);
     if (c->w.h_large) (void)hipHostFree(c->w.h_large);
     if (c->w.h_plan) (void)hipHostFree(c->w.h_plan);
@@ -2650,8 +2673,7 @@ int ensure_capacity(ps5_ctx* c, uint64_t n)
     uint64_t cap = std::max<uint64_t>(std::max<uint64_t>(n, 1024), c->w.cap + c->w.cap / 2);
     cap = std::min<uint64_t>(cap, std::max<uint64_t>(n, 0xFFFFFF00ull));
     free_buffers(c);
-    HIPCHK(hipMalloc(&c->w.key, 2 * cap * sizeof(key64)));
-    HIPCHK(hipMalloc(&c->w.idx, 2 * cap * sizeof(uint32_t)));
+    HIPCHK(hipMalloc(&c->w.rec, 2 * cap * kRecWords * sizeof(uint32_t)));
     HIPCHK(hipMalloc(&c->w.bkey, cap * sizeof(key64)));
     for (int i = 0; i < 2; ++i) HIPCHK(hipMalloc(&c->w.sdepth[i], cap * sizeof(uint32_t)));
     c->w.cap_large = cap_large_of(cap);
@@ -2692,7 +2714,7 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 // Byte offsets of the work buffers of a sort of up to `cap` strings inside
 // the scratch, its tables sized for any shape (chunks of kChunkMin keys).
 struct ScratchLayout {
-    uint64_t key, idx, bkey, sdepth[2], lut, l_round[2], l_lvl[2], l_tiny[2], l_block[2], l_run[2];
+    uint64_t rec, bkey, sdepth[2], lut, l_round[2], l_lvl[2], l_tiny[2], l_block[2], l_run[2];
     uint64_t desc, trees, hist, gsum, vpos, src, total;
     uint64_t trees_cap, hist_cap, gsum_cap;
 };
@@ -2703,8 +2725,7 @@ constexpr ScratchLayout scratch_layout(uint64_t cap)
     uint64_t o = 0;
     auto take = [&o](uint64_t bytes) { const uint64_t at = o; o = align256(o + bytes); return at; };
     const uint64_t cl = cap_large_of(cap), cb = cap_block_of(cap), cr = cap_run_of(cap);
-    L.key = take(2 * cap * sizeof(key64));
-    L.idx = take(2 * cap * sizeof(uint32_t));
+    L.rec = take(2 * cap * kRecWords * sizeof(uint32_t));
     L.bkey = take(cap * sizeof(key64));
     for (int i = 0; i < 2; ++i) L.sdepth[i] = take(cap * sizeof(uint32_t));
     for (int i = 0; i < 2; ++i) {
@@ -2777,8 +2798,7 @@ WorkBuffers scratch_buffers(unsigned char* base, Item* h_large, unsigned char* h
         w.sdepth[i] = reinterpret_cast<uint32_t*>(base + L.sdepth[i]);
         w.cap_tiny[i] = cap_tiny_of(cap, i);
     }
-    w.key = reinterpret_cast<key64*>(base + L.key);
-    w.idx = reinterpret_cast<uint32_t*>(base + L.idx);
+    w.rec = reinterpret_cast<uint32_t*>(base + L.rec);
     w.vpos = reinterpret_cast<uint32_t*>(base + L.vpos);
     w.src = reinterpret_cast<uint32_t*>(base + L.src);
     w.bkey = reinterpret_cast<key64*>(base + L.bkey);
@@ -3329,9 +3349,9 @@ void dev_level(ps5_ctx* c, const Bufs& B, const Item* list, int ci, uint32_t bou
     }
     const uint64_t tiles_bound = S / kChunkMin + gl;
     {
-        // three workgroups per CU are resident
+        // two workgroups per CU are resident
         Launch L(c, K_PART, 0);
-        launch_part(c, B, P, (uint32_t)std::min<uint64_t>(3 * c->cus, div_up(tiles_bound, kXcds) * kXcds), kmax, src, 0u,
+        launch_part(c, B, P, (uint32_t)std::min<uint64_t>(2 * c->cus, div_up(tiles_bound, kXcds) * kXcds), kmax, src, 0u,
                     false);
     }
     const uint32_t groups_bound = (uint32_t)std::min<uint64_t>(kDevHistWgs, tiles_bound / kHistGroup + gl);
@@ -3744,8 +3764,7 @@ int run_sort_keys(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_
     B.alen = alen;
     B.offs = offs;
     B.offs64 = offs64;
-    B.key = c->w.key;
-    B.idx = c->w.idx;
+    B.rec = c->w.rec;
     B.vpos = c->w.vpos;
     B.src = c->w.src;
     B.cap = c->w.cap;
@@ -3804,7 +3823,7 @@ int run_sort_keys(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_
         if (!set_first) nl_root = n > kBlkT ? 1 : 0;
         std::vector<uint64_t> key = { (uint64_t)(uintptr_t)arena, alen, (uint64_t)(uintptr_t)offs,
                                       (uint64_t)(uintptr_t)offs64, n, (uint64_t)(uintptr_t)perm,
-                                      (uint64_t)(uintptr_t)lcp, nsets, (uint64_t)(uintptr_t)c->w.key, c->w.cap,
+                                      (uint64_t)(uintptr_t)lcp, nsets, (uint64_t)(uintptr_t)c->w.rec, c->w.cap,
                                       (uint64_t)(uintptr_t)c->w.trees, c->w.trees_cap, c->leaf_target,
                                       c->max_treebits, c->max_oversample, c->graph_rounds, c->seed,
                                       c->w_gen, c->w.fixed ? 1u : 0u, c->graph_levels, c->chunk_max,
@@ -4080,25 +4099,23 @@ int ps5_merge_device(ps5_ctx* c, const uint8_t* d_arena, uint64_t arena_bytes, c
     B.arena = d_arena;
     B.alen = arena_bytes;
     B.offs = d_offs;
-    // ping-pong buffers: indices in the two halves of idx, first 8 characters
-    // in those of key, LCPs in those of bkey
-    uint32_t* ti[2] = { c->w.idx, c->w.idx + c->w.cap };
-    key64* tk[2] = { c->w.key, c->w.key + c->w.cap };
+    // ping-pong buffers in the records' memory: two of first 8 characters, two
+    // of indices; LCPs in the two halves of bkey
+    key64* keys = reinterpret_cast<key64*>(c->w.rec);
+    uint32_t* idxs = reinterpret_cast<uint32_t*>(keys + 2 * c->w.cap);
+    uint32_t* ti[2] = { idxs, idxs + c->w.cap };
+    key64* tk[2] = { keys, keys + c->w.cap };
     uint32_t* tl[2] = { reinterpret_cast<uint32_t*>(c->w.bkey), reinterpret_cast<uint32_t*>(c->w.bkey) + c->w.cap };
     std::vector<uint64_t> bounds(run_first, run_first + nruns + 1);
     const uint32_t* si = d_idx;
     const uint32_t* sl = d_lcp;
     // the first round reads every string's first 8 characters from ik, keys
     // extracted in input order by one streaming pass (the previous round's
-    // output carries them afterwards); the second half of key is free until the
-    // second merge round writes it
+    // output carries them afterwards); tk[1] is free until the second merge
+    // round writes it
     key64* ik = tk[1];
-    {
-        Bufs BI = B;
-        BI.key = ik;
-        hipLaunchKernelGGL(k_init, dim3(div_up(n, kWG)), dim3(kWG), 0, st, BI, (uint32_t)n);
-        HIPCHK(hipGetLastError());
-    }
+    hipLaunchKernelGGL(k_init, dim3(div_up(n, kWG)), dim3(kWG), 0, st, B, ik, (uint32_t)n);
+    HIPCHK(hipGetLastError());
     const key64* sk = nullptr;
     int cur = 0;
     while (bounds.size() > 2) {
