@@ -988,7 +988,7 @@ constexpr int kChildPer = (kMaxBkt + kBigWG) / kBigWG;     // 2 buckets per thre
 constexpr int kChildLists = 3 + kBlkClasses;
 
 __device__ __forceinline__ void emit_children(const LargeDesc& D, uint32_t start, const uint32_t (&sz)[kChildPer], uint32_t dst,
-                                              const key64* spl, const Sink& s, uint32_t* s_tmp)
+                                              const key64* spl, const Sink& s, uint32_t* sdepth_out, uint32_t* s_tmp)
 {
     const Item seg = D.seg;
     const uint32_t base_flags = dst | (seg.flags & kFmtMask);
@@ -1040,6 +1040,7 @@ __device__ __forceinline__ void emit_children(const LargeDesc& D, uint32_t start
             put_item(s.tiny, s.cap_tiny, o_t++, it, s.cnt);
         } else if (b & 1) {
             const uint32_t nch = (m + kRunChunk - 1) / kRunChunk;
+            sdepth_out[it.begin] = 0xFFFFFFFFu;     // (k_leaf_run's chunks lower it)
             for (uint32_t c = 0; c < nch; ++c) {
                 Item r = it;
                 r.flags = base_flags | F_SORTED | (c << kFlagShift);
@@ -1116,7 +1117,8 @@ __global__ __launch_bounds__(kBigWG) void k_children(Plan P, Bufs B, const key64
                 }
                 at += sz[j];
             }
-            emit_children(D, start, sz, dst, trees + (uint64_t)si * kTreeSlots + 1024, s, s_tmp);
+            emit_children(D, start, sz, dst, trees + (uint64_t)si * kTreeSlots + 1024, s,
+                          B.sdepth_out, s_tmp);
         }
         __syncthreads();     // the LDS is reused by the next segment
     }
@@ -1641,6 +1643,18 @@ __device__ __forceinline__ bool block_radix_sort(key64 (&w)[E], uint32_t m, key6
     }
     // (s_tmp is written again only after the counting barrier below)
     const key64 range = kmax - kmin;
+    if (range == 0) {     // (uniform) all keys equal (a run sorted at its next depth): already in order
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const uint32_t i = (uint32_t)e * T + tid;
+            if (i < m) {
+                s_k[i] = kmin;
+                s_p[i] = (uint16_t)i;
+            }
+        }
+        __syncthreads();
+        return true;
+    }
     if ((range >> 48) != 0) {     // (uniform) offsets too wide to pack: merge sort
 #pragma unroll
         for (int e = 0; e < E; ++e) {
@@ -1961,8 +1975,34 @@ __global__ __launch_bounds__(MAXM / E) __attribute__((amdgpu_waves_per_eu(8, 8))
 
 constexpr uint32_t kRunRow = 512;       // runs of a row that k_leaf_run searches
 
+// Characters that string a (from offset off on) shares with the string whose
+// next characters are ref[]: at most 64, and none past a NUL of it.
+constexpr int kExtKeys = 8;
+__device__ __forceinline__ uint32_t common_chars(const Bufs& B, const key64 (&ref)[kExtKeys], uint64_t off)
+{
+    key64 a[kExtKeys];
+    load_keys<kExtKeys>(B.arena, B.alen, off, a);
+    uint32_t n = 8 * kExtKeys;
+#pragma unroll
+    for (int i = kExtKeys - 1; i >= 0; --i) {     // (the first difference or end counts)
+        if (a[i] != ref[i]) n = 8 * i + lcp_key(a[i], ref[i]);
+        else if ((ref[i] & 0xFFull) == 0) n = 8 * i + key_depth(ref[i]);
+    }
+    return n;
+}
+
 // One workgroup per chunk of an equal-key leaf (all keys equal): the entries
 // from *p_first (first, if null) on of a list.
+//
+// A run that continues is a segment of the next round, at the depth its
+// strings are known to share.  Strings with a common prefix (URLs of one host)
+// share more than one key: without looking ahead, every 8 characters of the
+// prefix cost a round of tree, partition and host round trips that split
+// nothing.  64 strings of the chunk say how far looking ahead can go; if
+// anywhere, every string of the chunk is compared with the run's first one
+// over 64 characters, and the run continues after what they all share.
+// 4.4 M URL-like strings (prefixes of 8 to 40 characters, 256 MB): 3.07 -> 1.50
+// ms, 2 instead of 5 rounds with large segments.
 __global__ __launch_bounds__(kWG) void k_leaf_run(const Item* items, const uint32_t* p_first, uint32_t first,
                                                   const uint32_t* cnt_items, uint32_t cap, Bufs B, Sink nxt)
 {
@@ -2014,10 +2054,33 @@ __global__ __launch_bounds__(kWG) void k_leaf_run(const Item* items, const uint3
             B.perm[cb + p] = R.R[place(p)].id;
             if (term && B.lcp && cb + p > L.begin) B.lcp[cb + p] = l;
         }
+        if (!term) {     // (uniform)
+            const uint32_t next = depth + F.cpk;
+            const uint32_t id0 = R.R[run_place(B, R, L.begin)].id;
+            key64 ref[kExtKeys];
+            load_keys<kExtKeys>(B.arena, B.alen, str_off(B, min(id0, B.n - 1)) + next, ref);
+            // all waves take the same sample
+            const uint32_t lane = lane_id();
+            const uint32_t sp = (uint32_t)(((uint64_t)lane * m) >> 6);
+            const uint32_t sid = R.R[place(sp)].id;
+            uint32_t ext = common_chars(B, ref, str_off(B, min(sid, B.n - 1)) + next);
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) ext = min(ext, (uint32_t)__shfl_xor((int)ext, d, 64));
+            if (ext) {     // (uniform)
+                uint32_t e = ext;
+                for (uint32_t p = tid_x(); p < m; p += kWG) {
+                    const uint32_t id = R.R[place(p)].id;
+                    e = min(e, common_chars(B, ref, str_off(B, min(id, B.n - 1)) + next));
+                }
+#pragma unroll
+                for (int d = 32; d >= 1; d >>= 1) e = min(e, (uint32_t)__shfl_xor((int)e, d, 64));
+                ext = e;     // (of this wave's strings)
+            }
+            if (lane == 0) atomicMin(&B.sdepth_out[L.begin], next + ext);
+        }
         if (tid_x() < 64) {
             const bool nr = tid_x() == 0 && c == 0 && !term && !single;
             Item ni = { L.begin, L.size, L.begin, F_NEXT, 0u, 0u };
-            if (nr) B.sdepth_out[L.begin] = depth + F.cpk;
             wave_append_segment(nr, ni, nxt);
             if (tid_x() == 0) {
                 if (c == 0) B.bkey[L.begin] = key;

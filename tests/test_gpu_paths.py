@@ -133,3 +133,32 @@ def test_many_levels_and_rounds(ps5, oracle, planning, tuning):
             check(c, oracle, *packed_case(sigma, n, seed, hi=40))
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("planning", [0, 1])
+@pytest.mark.parametrize("shared", [0, 7, 8, 15, 63, 64, 65, 200])
+def test_runs_with_long_common_prefixes(ps5, oracle, shared, planning):
+    """equal-key runs that share `shared` characters past their key, some
+    strings ending inside them, some identical"""
+    rng = np.random.default_rng(shared)
+    strs = []
+    for g in range(3):
+        stem = bytes([65 + g]) * 8 + rng.integers(97, 123, shared).astype(np.uint8).tobytes()
+        for _ in range(6000):
+            kind = rng.integers(0, 20)
+            tail = rng.integers(97, 123, rng.integers(0, 12)).astype(np.uint8).tobytes()
+            if kind == 0 and shared:
+                strs.append(stem[:8 + rng.integers(0, shared + 1)])
+            elif kind == 1:
+                strs.append(stem)
+            else:
+                strs.append(stem + tail)
+        if g == 2:      # one run that shares all of it
+            strs = [s if not s.startswith(b"C") else stem + s[len(stem):] for s in strs]
+    order = rng.permutation(len(strs))
+    c = ps5.Context(0)
+    try:
+        c.set_planning(planning)
+        check(c, oracle, *pack([strs[i] for i in order]))
+    finally:
+        c.close()
