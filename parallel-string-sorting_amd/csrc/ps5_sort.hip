@@ -1018,13 +1018,13 @@ __device__ __forceinline__ void emit_children(const LargeDesc& D, uint32_t start
     block_excl_scan_k<kBigWaves, kChildLists>(cv, ov, tv, s_tmp);
     if (c_cont) atomicAdd(&s.cnt[s.c_runcont], c_cont);
     uint32_t* s_base = s_tmp + kBigWaves * kChildLists;
-    if (tid_x() == 0) {
-        s_base[0] = tv[0] ? atomicAdd(&s.cnt[s.c_tiny], tv[0]) : 0;
-        s_base[1] = tv[1] ? atomicAdd(&s.cnt[s.c_large], tv[1]) : 0;
-        s_base[2] = tv[2] ? atomicAdd(&s.cnt[s.c_run], tv[2]) : 0;
+    if (tid_x() < kChildLists) {     // (a lane per list, so that the atomics are in flight together)
+        const uint32_t l = tid_x();
+        const int ci = l == 0 ? s.c_tiny : l == 1 ? s.c_large : l == 2 ? s.c_run : s.c_block + 2 * ((int)l - 3);
+        uint32_t n = tv[0];
 #pragma unroll
-        for (int c = 0; c < kBlkClasses; ++c)
-            s_base[3 + c] = tv[3 + c] ? atomicAdd(&s.cnt[s.c_block + 2 * c], tv[3 + c]) : 0;
+        for (int c = 1; c < kChildLists; ++c) n = l == (uint32_t)c ? tv[c] : n;
+        s_base[l] = n ? atomicAdd(&s.cnt[ci], n) : 0u;
     }
     __syncthreads();
     uint32_t o_t = ov[0] + s_base[0], o_l = ov[1] + s_base[1], o_r = ov[2] + s_base[2], o_b[kBlkClasses];
@@ -1249,24 +1249,33 @@ __device__ void wave_finish_leaf(const Bufs& B, uint32_t pos, uint32_t m, key64 
         cur += F.cpk;
         F = key_fmt(0);      // (what is fetched here is plain characters)
         if (nbuf == 0 || __ballot(live && id != bid) != 0) {     // (uniform)
-            if (live) {
-                if (id < B.n) load_keys<kLeafKeys>(B.arena, B.alen, str_off(B, id) + cur, kbuf, nk);
-                else { flag_error(B.cnt, ERR_BOUNDS); for (int i = 0; i < kLeafKeys; ++i) kbuf[i] = 0; }
-                bid = id;
+            const bool ok = live && id < B.n;
+            if (live && !ok) flag_error(B.cnt, ERR_BOUNDS);
+            const uint64_t off = ok ? str_off(B, id) : 0ull;
+            bid = id;
+            // depths where, in every run, all strings agree with the run's
+            // first one and none ends decide nothing: skip them together.
+            // While all fetched keys do, the wave fetches on without sorting
+            // (the suffixes of a 4.2 MB text with long repeats: 1.24 -> 0.89 ms)
+            int skip;
+            for (;;) {
+                if (live) {
+                    if (ok) load_keys<kLeafKeys>(B.arena, B.alen, off + cur, kbuf, nk);
+                    else for (int i = 0; i < kLeafKeys; ++i) kbuf[i] = 0;
+                }
+                skip = nk;
+#pragma unroll
+                for (int i = 0; i < kLeafKeys; ++i) {
+                    if (i >= nk) break;     // (uniform)
+                    const uint32_t lo = __shfl((uint32_t)kbuf[i], (int)run, 64);
+                    const uint32_t hi = __shfl((uint32_t)(kbuf[i] >> 32), (int)run, 64);
+                    const bool same = kbuf[i] == (((uint64_t)hi << 32) | lo) && (kbuf[i] & 0xFFull) != 0;
+                    if (skip == nk && __ballot(live && !same) != 0) skip = i;     // (uniform)
+                }
+                if (skip < nk) break;     // (uniform)
+                cur += 8 * (uint32_t)nk;
             }
             nbuf = nk;
-            // depths where, in every run, all strings agree with the run's
-            // first one and none ends decide nothing: skip them together
-            // (identical strings then cost one pass per 8 * (nk - 1) characters)
-            int skip = nk - 1;
-#pragma unroll
-            for (int i = 0; i < kLeafKeys - 1; ++i) {
-                if (i >= nk - 1) break;     // (uniform)
-                const uint32_t lo = __shfl((uint32_t)kbuf[i], (int)run, 64);
-                const uint32_t hi = __shfl((uint32_t)(kbuf[i] >> 32), (int)run, 64);
-                const bool same = kbuf[i] == (((uint64_t)hi << 32) | lo) && (kbuf[i] & 0xFFull) != 0;
-                if (skip == nk - 1 && __ballot(live && !same) != 0) skip = i;     // (uniform)
-            }
             for (int s = 0; s < skip; ++s) {     // (uniform)
 #pragma unroll
                 for (int i = 0; i + 1 < kLeafKeys; ++i) kbuf[i] = kbuf[i + 1];
@@ -1588,11 +1597,40 @@ __device__ __forceinline__ uint32_t block_scan_sum_max(uint32_t a, uint32_t b, u
     return wpre + x - a;
 }
 
-__device__ __forceinline__ key64 shfl_xor64(key64 v, int d)
+// minimum and maximum over the wave by lane moves inside the vector unit (the
+// lanes' values need no trip through the LDS), then over the workgroup (NW
+// waves; s_tmp: 2 NW words, written again by the caller only after a barrier)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ void dpp_min_max(uint32_t& lo, uint32_t& hi)
 {
-    const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)v, d, 64);
-    const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(v >> 32), d, 64);
-    return ((key64)hi << 32) | lo;
+    lo = min(lo, (uint32_t)__builtin_amdgcn_update_dpp((int)0xFFFFFFFFu, (int)lo, CTRL, ROWS, 0xF, false));
+    hi = max(hi, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)hi, CTRL, ROWS, 0xF, false));
+}
+template <int NW>
+__device__ __forceinline__ void block_min_max(uint32_t& lo, uint32_t& hi, uint32_t* s_tmp)
+{
+    dpp_min_max<0x111, 0xF>(lo, hi);     // row_shr:1, 2, 4, 8: lane 15 of a row has the row's
+    dpp_min_max<0x112, 0xF>(lo, hi);
+    dpp_min_max<0x114, 0xF>(lo, hi);
+    dpp_min_max<0x118, 0xF>(lo, hi);
+    dpp_min_max<0x142, 0xA>(lo, hi);     // row_bcast:15 into rows 1 and 3
+    dpp_min_max<0x143, 0xC>(lo, hi);     // row_bcast:31 into rows 2 and 3: lane 63 has the wave's
+    if (NW == 1) {
+        lo = (uint32_t)__builtin_amdgcn_readlane((int)lo, 63);
+        hi = (uint32_t)__builtin_amdgcn_readlane((int)hi, 63);
+        __syncthreads();
+        return;
+    }
+    if (lane_id() == 63) {
+        s_tmp[wave_id()] = lo;
+        s_tmp[NW + wave_id()] = hi;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+        lo = min(lo, s_tmp[i]);
+        hi = max(hi, s_tmp[NW + i]);
+    }
 }
 
 // Radix-partitioned rank sort of a block's m keys (w: thread t's keys of the positions t, t + T, ..):
@@ -1618,28 +1656,28 @@ __device__ __forceinline__ bool block_radix_sort(key64 (&w)[E], uint32_t m, key6
     const uint32_t Pm = (m + E - 1) / E * E;
     // w: this thread's keys (positions e*T + tid, clamped to the block), later
     // their packed values
-    key64 kmin = ~0ull, kmax = 0;
+    for (uint32_t j = tid; j < MAXM + 2; j += T) s_cnt[j] = 0;
+    // bounds of the keys from their high words, or from their low words where
+    // those agree: any bounds do, and words take a quarter of the instructions
+    uint32_t lo32 = ~0u, hi32 = 0u;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-        kmin = min(kmin, w[e]);     // (clamped copies of the last key change neither)
-        kmax = max(kmax, w[e]);
+        lo32 = min(lo32, (uint32_t)(w[e] >> 32));     // (clamped copies of the last key change neither)
+        hi32 = max(hi32, (uint32_t)(w[e] >> 32));
     }
-    for (uint32_t j = tid; j < MAXM + 2; j += T) s_cnt[j] = 0;
+    block_min_max<NW>(lo32, hi32, s_tmp);
+    key64 kmin = (key64)lo32 << 32, kmax = ((key64)hi32 << 32) | 0xFFFFFFFFull;
+    if (lo32 == hi32) {     // (uniform)
+        lo32 = ~0u;
+        hi32 = 0u;
 #pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-        kmin = min(kmin, shfl_xor64(kmin, d));
-        kmax = max(kmax, shfl_xor64(kmax, d));
-    }
-    key64* s_mm = reinterpret_cast<key64*>(s_tmp);      // [NW] minima, then [NW] maxima
-    if (lane_id() == 0) {
-        s_mm[wave_id()] = kmin;
-        s_mm[NW + wave_id()] = kmax;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < NW; ++i) {
-        kmin = min(kmin, s_mm[i]);
-        kmax = max(kmax, s_mm[NW + i]);
+        for (int e = 0; e < E; ++e) {
+            lo32 = min(lo32, (uint32_t)w[e]);
+            hi32 = max(hi32, (uint32_t)w[e]);
+        }
+        block_min_max<NW>(lo32, hi32, s_tmp + 2 * NW);
+        kmax = kmin | hi32;
+        kmin |= lo32;
     }
     // (s_tmp is written again only after the counting barrier below)
     const key64 range = kmax - kmin;
@@ -1814,12 +1852,38 @@ __device__ __forceinline__ void block_one(const Item L, const Bufs& B, const Sin
 #pragma unroll
         for (int e = 0; e < kPerThread; ++e) w[e] = string_key(B, idv[e], depth);
     } else {
-        // a bucket: the runs' starts and places are copied to s_k and searched
-        // there (a row longer than that is searched where it is)
+        // a bucket of at most 64 runs has them in the lanes of every wave, and
+        // a wave's 64 consecutive positions walk the few runs they meet (the
+        // blocks of 42 M keys are bound by instruction issue: with the bounds
+        // below by words, 750 -> 630 us); longer rows are copied to s_k and
+        // searched there, or searched where they are
         const Runs R = runs_of(B, L);
         uint32_t* s_v = reinterpret_cast<uint32_t*>(s_k);
         uint32_t q[kPerThread];
-        if (R.nch <= MAXM) {     // (uniform)
+        if (R.nch <= 64) {     // (uniform)
+            const uint32_t lane = tid & 63u;
+            uint32_t v = 0xFFFFFFFFu, sp = 0;
+            if (lane < R.nch) {
+                v = R.V[lane];
+                sp = R.S[lane] - v;     // a string's place less its position
+            }
+#pragma unroll
+            for (int e = 0; e < kPerThread; ++e) {
+                const uint32_t pos = beg + min(tid + (uint32_t)e * T, m - 1);
+                const uint32_t p0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)pos);
+                uint64_t rest = __ballot(v <= p0 + 63u);       // runs starting before the wave's positions end
+                uint64_t upto = __ballot(v <= p0);              // the last of them holds its first one
+                int c = 63 - (int)__builtin_clzll(upto | 1ull);
+                uint32_t d = (uint32_t)__builtin_amdgcn_readlane((int)sp, c);
+                for (rest &= ~((2ull << c) - 1ull); rest; rest &= rest - 1) {     // (uniform)
+                    c = __builtin_ctzll(rest);
+                    const uint32_t rv = (uint32_t)__builtin_amdgcn_readlane((int)v, c);
+                    const uint32_t rd = (uint32_t)__builtin_amdgcn_readlane((int)sp, c);
+                    if (pos >= rv) d = rd;
+                }
+                q[e] = checked_place(B, pos + d);
+            }
+        } else if (R.nch <= MAXM) {     // (uniform)
             for (uint32_t c = tid; c < R.nch; c += T) {
                 s_v[c] = R.V[c];
                 s_v[R.nch + c] = R.S[c];
