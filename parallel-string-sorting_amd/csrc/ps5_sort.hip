@@ -1333,8 +1333,24 @@ __device__ __forceinline__ void load_tiny(const Bufs& B, const Item& L, uint32_t
     }
 }
 
-// One wave per tiny leaf (at most 64 strings), finished completely: the
-// entries from *p_first (first, if null) on of a list.
+// One tiny leaf (at most 64 strings), finished completely by one wave.
+// s_k, s_i, s_r: its 64-entry LDS arrays.
+template <int NK>
+__device__ __forceinline__ void tiny_leaf(const Item& L, const Bufs& B, key64* s_k, uint32_t* s_i, uint32_t* s_r)
+{
+    const uint32_t lane = lane_id();
+    if (!item_ok(L, B) || L.size > kTinyT) {     // (uniform)
+        if (lane == 0) flag_error(B.cnt, ERR_BOUNDS);
+        return;
+    }
+    key64 k = ~0ull;
+    uint32_t id = 0;
+    const uint32_t depth = seg_depth(B, L.rbeg);
+    load_tiny(B, L, depth, &k, &id);
+    wave_finish_leaf<NK>(B, L.begin + lane, L.size, k, id, depth, key_fmt(L.flags), true, 0u, s_k, s_i, s_r);
+}
+
+// The tiny leaves from *p_first (first, if null) on of a list, a wave each.
 template <int NK>
 __global__ __launch_bounds__(kWG) void k_leaf_tiny(const Item* items, const uint32_t* p_first, uint32_t first,
                                                    const uint32_t* cnt_items, uint32_t cap, Bufs B)
@@ -1342,7 +1358,7 @@ __global__ __launch_bounds__(kWG) void k_leaf_tiny(const Item* items, const uint
     __shared__ key64 s_k[kWaves][64];
     __shared__ uint32_t s_i[kWaves][64];
     __shared__ uint32_t s_r[kWaves][64];     // first sorted position of the run holding a position
-    const uint32_t w = wave_id(), lane = lane_id();
+    const uint32_t w = wave_id();
     if (B.pending && *B.pending) {      // the round's levels are not finished
         if (B.pending_err && tid_x() == 0) flag_error(B.cnt, ERR_LEVELS);
         return;
@@ -1352,16 +1368,7 @@ __global__ __launch_bounds__(kWG) void k_leaf_tiny(const Item* items, const uint
     // each wave takes leaves it, it + stride, ... (no workgroup barriers below)
     for (uint32_t it = first + blockIdx.x * kWaves + w; it < nitems; it += gridDim.x * kWaves) {
         const Item L = load_uniform(items + __builtin_amdgcn_readfirstlane((int)it));
-        if (!item_ok(L, B) || L.size > kTinyT) {
-            if (lane == 0) flag_error(B.cnt, ERR_BOUNDS);
-            continue;      // (wave-uniform)
-        }
-        key64 k = ~0ull;
-        uint32_t id = 0;
-        const uint32_t depth = seg_depth(B, L.rbeg);
-        load_tiny(B, L, depth, &k, &id);
-        wave_finish_leaf<NK>(B, L.begin + lane, L.size, k, id, depth, key_fmt(L.flags), true, 0u, s_k[w], s_i[w],
-                             s_r[w]);
+        tiny_leaf<NK>(L, B, s_k[w], s_i[w], s_r[w]);
     }
 }
 
@@ -1985,6 +1992,28 @@ __device__ __forceinline__ void block_one(const Item L, const Bufs& B, const Sin
     }
 }
 
+// A block in tail mode, finished completely by its workgroup.
+template <uint32_t MAXM, int E, int NK>
+__device__ __forceinline__ void block_tail(Item cur, const Bufs& B, const Sink& nxt, BlockLds<MAXM, E, true>& S, TailStack& ts)
+{
+    if (tid_x() == 0) ts.n = 0;
+    // (every thread reads ts.n after block_one, which returns at once on
+    // a malformed item: the count is stored before a barrier each time)
+    __syncthreads();
+    uint32_t d = seg_depth(B, cur.rbeg);
+    for (bool top = true;; top = false) {     // one call site, so that block_one stays inline
+        block_one<MAXM, E, NK, true>(cur, B, nxt, d, S, &ts, top);
+        // (the pushes precede a barrier in block_one's finish pass)
+        const uint32_t n = min(ts.n, kTailStack);
+        if (n == 0) break;     // (uniform)
+        __syncthreads();     // the last pass's LDS is no longer read, every thread has read ts.n
+        cur = Item{ ts.pos[n - 1], ts.len[n - 1], ts.pos[n - 1], F_NEXT, 0u, 0u };
+        d = ts.depth[n - 1];
+        if (tid_x() == 0) ts.n = n - 1;     // (pushes into the freed entry come after block_one's barriers)
+        __syncthreads();     // every thread has read the top entry; the count is stored
+    }
+}
+
 // Blocks [first, last) of a list (one per workgroup), or with LOOP (levels
 // planned on the device) from *p_first to the list's count, each workgroup
 // looping over them; a count over the list's capacity has been flagged and
@@ -2005,23 +2034,7 @@ __global__ __launch_bounds__(MAXM / E) __attribute__((amdgpu_waves_per_eu(8, 8))
         __shared__ TailStack ts;
         const uint32_t idx = first + blockIdx.x;
         if (idx >= min(last, cap)) return;
-        if (tid_x() == 0) ts.n = 0;
-        // (every thread reads ts.n after block_one, which returns at once on
-        // a malformed item: the count is stored before a barrier each time)
-        __syncthreads();
-        Item cur = items[idx];
-        uint32_t d = seg_depth(B, cur.rbeg);
-        for (bool top = true;; top = false) {     // one call site, so that block_one stays inline
-            block_one<MAXM, E, NK, true>(cur, B, nxt, d, S, &ts, top);
-            // (the pushes precede a barrier in block_one's finish pass)
-            const uint32_t n = min(ts.n, kTailStack);
-            if (n == 0) break;     // (uniform)
-            __syncthreads();     // the last pass's LDS is no longer read, every thread has read ts.n
-            cur = Item{ ts.pos[n - 1], ts.len[n - 1], ts.pos[n - 1], F_NEXT, 0u, 0u };
-            d = ts.depth[n - 1];
-            if (tid_x() == 0) ts.n = n - 1;     // (pushes into the freed entry come after block_one's barriers)
-            __syncthreads();     // every thread has read the top entry; the count is stored
-        }
+        block_tail<MAXM, E, NK>(items[idx], B, nxt, S, ts);
     } else if constexpr (!LOOP) {
         const uint32_t idx = first + blockIdx.x;
         if (idx >= min(last, cap)) return;
@@ -2055,8 +2068,7 @@ __device__ __forceinline__ uint32_t common_chars(const Bufs& B, const key64 (&re
     return n;
 }
 
-// One workgroup per chunk of an equal-key leaf (all keys equal): the entries
-// from *p_first (first, if null) on of a list.
+// One chunk of an equal-key leaf (all keys equal), by a workgroup of kWG threads.
 //
 // A run that continues is a segment of the next round, at the depth its
 // strings are known to share.  Strings with a common prefix (URLs of one host)
@@ -2067,6 +2079,82 @@ __device__ __forceinline__ uint32_t common_chars(const Bufs& B, const key64 (&re
 // over 64 characters, and the run continues after what they all share.
 // 4.4 M URL-like strings (prefixes of 8 to 40 characters, 256 MB): 3.07 -> 1.50
 // ms, 2 instead of 5 rounds with large segments.
+__device__ __forceinline__ void run_chunk(const Item& L, const Bufs& B, const Sink& nxt, RunMap<kRunChunk>& M)
+{
+    const uint32_t c = L.flags >> kFlagShift;
+    if (!item_ok(L, B) || (uint64_t)c * kRunChunk >= L.size || (L.flags & (F_IDENT | F_NEXT))) {
+        if (tid_x() == 0) flag_error(B.cnt, ERR_BOUNDS);
+        return;
+    }
+    const Runs R = runs_of(B, L);
+    const uint32_t rend = L.begin + L.size;
+    const uint32_t cb = L.begin + c * kRunChunk;
+    const uint32_t m = min(rend - cb, kRunChunk);
+    // a short row (a bucket of a small segment) is copied and searched, a
+    // long one mapped
+    uint32_t* s_v = M.delta;
+    const bool small = R.nch <= kRunRow;     // (uniform)
+    if (small) {
+        for (uint32_t i = tid_x(); i < R.nch; i += kWG) {
+            s_v[i] = R.V[i];
+            s_v[kRunRow + i] = R.S[i];
+        }
+        __syncthreads();
+    } else {
+        map_runs<kWaves, (int)kRunChunk>(R, rend, cb, m, M);
+    }
+    auto place = [&](uint32_t p) {
+        if (!small) return mapped_place(B, M, p);
+        const uint32_t r = find_run(s_v, R.nch, cb + p);
+        return checked_place(B, s_v[kRunRow + r] + (cb + p - s_v[r]));
+    };
+    const key64 key = rec_key(R.R[place(0u)]);
+    const KeyFmt F = key_fmt(L.flags);
+    const uint32_t depth = seg_depth(B, L.rbeg);
+    // identical strings are done, others continue at the next depth
+    const bool term = key_ends(key, F), single = L.size == 1;
+    const uint32_t l = depth + key_depth(key, F);
+#pragma unroll 4
+    for (uint32_t p = tid_x(); p < m; p += kWG) {
+        B.perm[cb + p] = R.R[place(p)].id;
+        if (term && B.lcp && cb + p > L.begin) B.lcp[cb + p] = l;
+    }
+    if (!term) {     // (uniform)
+        const uint32_t next = depth + F.cpk;
+        const uint32_t id0 = R.R[run_place(B, R, L.begin)].id;
+        key64 ref[kExtKeys];
+        load_keys<kExtKeys>(B.arena, B.alen, str_off(B, min(id0, B.n - 1)) + next, ref);
+        // all waves take the same sample
+        const uint32_t lane = lane_id();
+        const uint32_t sp = (uint32_t)(((uint64_t)lane * m) >> 6);
+        const uint32_t sid = R.R[place(sp)].id;
+        uint32_t ext = common_chars(B, ref, str_off(B, min(sid, B.n - 1)) + next);
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) ext = min(ext, (uint32_t)__shfl_xor((int)ext, d, 64));
+        if (ext) {     // (uniform)
+            uint32_t e = ext;
+            for (uint32_t p = tid_x(); p < m; p += kWG) {
+                const uint32_t id = R.R[place(p)].id;
+                e = min(e, common_chars(B, ref, str_off(B, min(id, B.n - 1)) + next));
+            }
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) e = min(e, (uint32_t)__shfl_xor((int)e, d, 64));
+            ext = e;     // (of this wave's strings)
+        }
+        if (lane == 0) atomicMin(&B.sdepth_out[L.begin], next + ext);
+    }
+    if (tid_x() < 64) {
+        const bool nr = tid_x() == 0 && c == 0 && !term && !single;
+        Item ni = { L.begin, L.size, L.begin, F_NEXT, 0u, 0u };
+        wave_append_segment(nr, ni, nxt);
+        if (tid_x() == 0) {
+            if (c == 0) B.bkey[L.begin] = key;
+            if (cb + m == rend) B.bkey[rend - 1] = key;
+        }
+    }
+}
+
+// The chunks of equal-key leaves from *p_first (first, if null) on of a list.
 __global__ __launch_bounds__(kWG) void k_leaf_run(const Item* items, const uint32_t* p_first, uint32_t first,
                                                   const uint32_t* cnt_items, uint32_t cap, Bufs B, Sink nxt)
 {
@@ -2079,79 +2167,65 @@ __global__ __launch_bounds__(kWG) void k_leaf_run(const Item* items, const uint3
     if (p_first) first = *p_first;
     for (uint32_t ii = first + blockIdx.x; ii < nitems; ii += gridDim.x) {
         __syncthreads();     // the previous chunk's map is no longer read
-        const Item L = load_uniform(items + ii);
-        const uint32_t c = L.flags >> kFlagShift;
-        if (!item_ok(L, B) || (uint64_t)c * kRunChunk >= L.size || (L.flags & (F_IDENT | F_NEXT))) {
-            if (tid_x() == 0) flag_error(B.cnt, ERR_BOUNDS);
-            continue;
-        }
-        const Runs R = runs_of(B, L);
-        const uint32_t rend = L.begin + L.size;
-        const uint32_t cb = L.begin + c * kRunChunk;
-        const uint32_t m = min(rend - cb, kRunChunk);
-        // a short row (a bucket of a small segment) is copied and searched, a
-        // long one mapped
-        uint32_t* s_v = M.delta;
-        const bool small = R.nch <= kRunRow;     // (uniform)
-        if (small) {
-            for (uint32_t i = tid_x(); i < R.nch; i += kWG) {
-                s_v[i] = R.V[i];
-                s_v[kRunRow + i] = R.S[i];
-            }
-            __syncthreads();
-        } else {
-            map_runs<kWaves, (int)kRunChunk>(R, rend, cb, m, M);
-        }
-        auto place = [&](uint32_t p) {
-            if (!small) return mapped_place(B, M, p);
-            const uint32_t r = find_run(s_v, R.nch, cb + p);
-            return checked_place(B, s_v[kRunRow + r] + (cb + p - s_v[r]));
-        };
-        const key64 key = rec_key(R.R[place(0u)]);
-        const KeyFmt F = key_fmt(L.flags);
-        const uint32_t depth = seg_depth(B, L.rbeg);
-        // identical strings are done, others continue at the next depth
-        const bool term = key_ends(key, F), single = L.size == 1;
-        const uint32_t l = depth + key_depth(key, F);
-#pragma unroll 4
-        for (uint32_t p = tid_x(); p < m; p += kWG) {
-            B.perm[cb + p] = R.R[place(p)].id;
-            if (term && B.lcp && cb + p > L.begin) B.lcp[cb + p] = l;
-        }
-        if (!term) {     // (uniform)
-            const uint32_t next = depth + F.cpk;
-            const uint32_t id0 = R.R[run_place(B, R, L.begin)].id;
-            key64 ref[kExtKeys];
-            load_keys<kExtKeys>(B.arena, B.alen, str_off(B, min(id0, B.n - 1)) + next, ref);
-            // all waves take the same sample
-            const uint32_t lane = lane_id();
-            const uint32_t sp = (uint32_t)(((uint64_t)lane * m) >> 6);
-            const uint32_t sid = R.R[place(sp)].id;
-            uint32_t ext = common_chars(B, ref, str_off(B, min(sid, B.n - 1)) + next);
-#pragma unroll
-            for (int d = 32; d >= 1; d >>= 1) ext = min(ext, (uint32_t)__shfl_xor((int)ext, d, 64));
-            if (ext) {     // (uniform)
-                uint32_t e = ext;
-                for (uint32_t p = tid_x(); p < m; p += kWG) {
-                    const uint32_t id = R.R[place(p)].id;
-                    e = min(e, common_chars(B, ref, str_off(B, min(id, B.n - 1)) + next));
-                }
-#pragma unroll
-                for (int d = 32; d >= 1; d >>= 1) e = min(e, (uint32_t)__shfl_xor((int)e, d, 64));
-                ext = e;     // (of this wave's strings)
-            }
-            if (lane == 0) atomicMin(&B.sdepth_out[L.begin], next + ext);
-        }
-        if (tid_x() < 64) {
-            const bool nr = tid_x() == 0 && c == 0 && !term && !single;
-            Item ni = { L.begin, L.size, L.begin, F_NEXT, 0u, 0u };
-            wave_append_segment(nr, ni, nxt);
-            if (tid_x() == 0) {
-                if (c == 0) B.bkey[L.begin] = key;
-                if (cb + m == rend) B.bkey[rend - 1] = key;
-            }
-        }
+        run_chunk(load_uniform(items + ii), B, nxt, M);
     }
+}
+
+// Few leaves of all kinds in one launch (host-planned): workgroups of
+// kLeavesWG threads, the largest blocks first; waves that a leaf has no use
+// for end at once (a barrier waits for those that are left).  Kernels of one
+// kind each run after one another, and with few leaves each lasts as long as
+// its slowest workgroup, 20 to 40 us.  40 K strings of ACGT: 147 -> 117 us.
+struct LeafRange {
+    const Item* list;
+    uint32_t first, count;
+};
+struct LeafSet {          // kinds: tiny, blocks by class, equal-key chunks
+    LeafRange r[kBlkClasses + 2];
+};
+constexpr uint32_t kLeavesWG = kBlkT / kBlkE3;
+constexpr uint32_t kLeavesTiny = kLeavesWG / 64;     // tiny leaves of a workgroup
+
+template <uint32_t MAXM, int E, int NK, bool TAIL>
+__device__ __forceinline__ void leaves_block(const Item L, const Bufs& B, const Sink& nxt, BlockLds<MAXM, E, TAIL>& S, TailStack& ts)
+{
+    if constexpr (TAIL) block_tail<MAXM, E, NK>(L, B, nxt, S, ts);
+    else block_one<MAXM, E, NK, false>(L, B, nxt, seg_depth(B, L.rbeg), S, nullptr, true);
+}
+template <int NK, bool TAIL>
+__global__ __launch_bounds__(kLeavesWG) __attribute__((amdgpu_waves_per_eu(5))) void k_leaves(LeafSet Q, Bufs B, Sink nxt)
+{
+    union Lds {
+        BlockLds<kBlkT, kBlkE3, TAIL> b3;
+        BlockLds<1024, kBlkE2, TAIL> b2;
+        BlockLds<512, kBlkE1, TAIL> b1;
+        BlockLds<256, kBlkE0, TAIL> b0;
+        RunMap<kRunChunk> m;
+        struct { key64 k[kLeavesTiny][64]; uint32_t i[kLeavesTiny][64], r[kLeavesTiny][64]; } t;
+    };
+    __shared__ Lds S;
+    __shared__ TailStack ts;
+    uint32_t i = blockIdx.x;
+#define PS5_LEAVES_BLOCK(J, M, E, LDS)                                                  \
+    if (i < Q.r[J].count) {                                                             \
+        if (tid_x() >= (M) / (E)) return;     /* (whole waves) */                       \
+        leaves_block<M, E, NK, TAIL>(Q.r[J].list[Q.r[J].first + i], B, nxt, LDS, ts);   \
+        return;                                                                         \
+    }                                                                                   \
+    i -= Q.r[J].count;
+    PS5_LEAVES_BLOCK(4, kBlkT, kBlkE3, S.b3)
+    PS5_LEAVES_BLOCK(3, 1024, kBlkE2, S.b2)
+    PS5_LEAVES_BLOCK(2, 512, kBlkE1, S.b1)
+    PS5_LEAVES_BLOCK(1, 256, kBlkE0, S.b0)
+#undef PS5_LEAVES_BLOCK
+    if (i < Q.r[5].count) {
+        if (tid_x() < kWG) run_chunk(load_uniform(Q.r[5].list + Q.r[5].first + i), B, nxt, S.m);
+        return;
+    }
+    i -= Q.r[5].count;
+    const uint32_t w = wave_id(), t = i * kLeavesTiny + w;
+    if (t < Q.r[0].count)
+        tiny_leaf<NK>(load_uniform(Q.r[0].list + __builtin_amdgcn_readfirstlane((int)(Q.r[0].first + t))), B, S.t.k[w], S.t.i[w], S.t.r[w]);
 }
 
 // LCP between neighbouring leaves of one round segment:
@@ -3290,6 +3364,13 @@ int setup_roots(ps5_ctx* c, uint32_t n, const uint64_t* set_first, uint32_t nset
 
 constexpr uint32_t kMaxGraphRounds = 64;      // rounds one captured graph may hold
 constexpr uint32_t kForkLeafGroups = 8192;    // leaf workgroups worth a side stream
+// Workgroups per CU of one launch for all kinds of leaves (k_leaves).  Their
+// LDS, that of the largest block each, fills a CU with four, so this is twice
+// what the chip holds at once.  0.5 M digits (1020 workgroups): 201 us with
+// the kinds' own kernels, 159 together; 512 sets, 4.7 K workgroups of two
+// block classes and 0.4 K others: 363 us apart, 329 with the others together,
+// 316 with those on the side stream, 338 with one of the classes as well.
+constexpr uint32_t kFewLeavesPerCu = 8;
 // Strings of the largest root from which on roots may pack their keys.  The
 // kernels that can pack take about 11 us more (digits, which do not pack,
 // 0.5 M strings: 221 -> 233 us), and smaller roots of a small alphabet have
@@ -3394,6 +3475,63 @@ void launch_leaves(ps5_ctx* c, const Bufs& B, int rp, const Sink& nsink, LeavesD
         }
         sum_sizes(c, c->w.l_run[rp], done.run, c->d_cnt + C_RUN + rp, (uint32_t)n_run, S_RUN);
     }
+}
+
+// The kinds of leaves that go into one launch (k_leaves): of the blocks of
+// round parity rp from blk_first on (nblk by class), and the nt tiny leaves
+// and nr equal-key chunks from `done` on, the kinds with the fewest
+// workgroups, as long as they are few together (kFewLeavesPerCu).  Takes their
+// counts; grid 0: none (a single kind is left to its own kernel, and so are
+// all when profiling, which asks for each kind's time).
+struct FewLeaves {
+    LeafSet q;
+    uint32_t grid;
+};
+FewLeaves take_few_leaves(const ps5_ctx* c, int rp, const uint32_t* blk_first, uint32_t* nblk, LeavesDone done, uint32_t* nt,
+                          uint32_t* nr)
+{
+    constexpr int NL = kBlkClasses + 2;
+    uint32_t* count[NL];
+    FewLeaves F;
+    F.grid = 0;
+    count[0] = nt;
+    F.q.r[0] = LeafRange{ c->w.l_tiny[rp], done.tiny, 0u };
+    for (int cls = 0; cls < kBlkClasses; ++cls) {
+        count[1 + cls] = nblk + cls;
+        F.q.r[1 + cls] = LeafRange{ c->w.l_block[rp] + (uint64_t)cls * c->w.cap_block, blk_first[cls], 0u };
+    }
+    count[NL - 1] = nr;
+    F.q.r[NL - 1] = LeafRange{ c->w.l_run[rp], done.run, 0u };
+    uint32_t grid = 0, kinds = 0;
+    uint64_t room = c->profile ? 0 : (uint64_t)c->cus * kFewLeavesPerCu;
+    for (;;) {
+        int best = -1;
+        uint64_t bw = 0;
+        for (int j = 0; j < NL; ++j) {
+            // (a chunk counts twice: its own kernel holds twice as many at once)
+            const uint64_t w = j == 0 ? div_up(*nt, kLeavesTiny) : j == NL - 1 ? 2ull * *nr : *count[j];
+            if (w == 0 || F.q.r[j].count || (best >= 0 && w >= bw)) continue;
+            best = j;
+            bw = w;
+        }
+        if (best < 0 || bw > room) break;
+        F.q.r[best].count = *count[best];
+        room -= bw;
+        grid += best == 0 ? (uint32_t)bw : *count[best];
+        ++kinds;
+    }
+    if (kinds < 2) return F;
+    F.grid = grid;
+    for (int j = 0; j < NL; ++j)
+        if (F.q.r[j].count) *count[j] = 0;
+    return F;
+}
+void launch_few_leaves(ps5_ctx* c, const Bufs& B, const FewLeaves& F, const Sink& nsink, bool tail, hipStream_t s)
+{
+    if (F.grid == 0) return;
+    const auto f = c->leaf_keys == 8 ? (tail ? k_leaves<8, true> : k_leaves<8, false>)
+                                     : (tail ? k_leaves<0, true> : k_leaves<0, false>);
+    hipLaunchKernelGGL(f, dim3(F.grid), dim3(kLeavesWG), 0, s, F.q, B, nsink);
 }
 
 // The leaves known to the host (h_cnt) that are not finished yet, on the
@@ -3566,18 +3704,6 @@ int host_levels(ps5_ctx* c, const Bufs& B, uint32_t round, uint32_t level, int c
         }
         if (nlarge == 0 && nblk_all == 0) break;
         c->st_levels++;
-        // the last level (blocks only): the round's other leaves are all
-        // listed, and when they are many they run on the side stream
-        // beside the blocks (not when profiling, whose events time the
-        // main stream; for few leaves the fork costs more than it hides)
-        const uint32_t nt = c->h_cnt[C_TINY + rp] - done->tiny, nr = c->h_cnt[C_RUN + rp] - done->run;
-        if (nlarge == 0 && !c->profile && div_up(nt, kWaves) + nr >= kForkLeafGroups) {
-            HIPCHK(hipEventRecord(c->ev_fork, st));
-            HIPCHK(hipStreamWaitEvent(c->side, c->ev_fork, 0));
-            launch_leaves(c, B, rp, nsink, *done, false, leaf_tiny_grid(nt), leaf_run_grid(nr), nt, nr, c->side);
-            HIPCHK(hipEventRecord(c->ev_join, c->side));
-            *leaves_forked = true;
-        }
         const Sink sink = make_sink(c, nx_large, nx_ci, rp);
         const uint64_t seed = c->seed ^ ((uint64_t)round << 40) ^ ((uint64_t)level << 32);
         // a level without large segments, in a round whose equal-key
@@ -3585,26 +3711,57 @@ int host_levels(ps5_ctx* c, const Bufs& B, uint32_t round, uint32_t level, int c
         // last work: its blocks finish every string themselves (tail mode)
         // and no further round is needed
         const bool tail = c->tail_blocks && nlarge == 0 && c->h_cnt[C_RUNCONT + rp] == 0;
-        auto sort_blocks = [&] {
+        auto sort_blocks = [&]() -> int {
+            uint32_t blk[kBlkClasses], nt = 0, nr = 0;
+            std::copy(nblk, nblk + kBlkClasses, blk);
+            if (nlarge == 0) {     // the last level: the round's other leaves are all listed
+                nt = c->h_cnt[C_TINY + rp] - done->tiny;
+                nr = c->h_cnt[C_RUN + rp] - done->run;
+            }
+            const uint32_t nt0 = nt, nr0 = nr;
+            const FewLeaves few = take_few_leaves(c, rp, blk_done, blk, *done, &nt, &nr);
+            // beside many blocks, what is few runs on the side stream, and so
+            // do many leaves (not when profiling, whose events time the main
+            // stream; with less beside it the fork costs more than it hides)
+            uint32_t many = 0;
+            for (int cls = 0; cls < kBlkClasses; ++cls) many += blk[cls];
+            if (nlarge == 0 && !c->profile && ((few.grid && many >= (uint32_t)c->cus * kFewLeavesPerCu) ||
+                                               div_up(nt, kWaves) + nr >= kForkLeafGroups)) {
+                HIPCHK(hipEventRecord(c->ev_fork, st));
+                HIPCHK(hipStreamWaitEvent(c->side, c->ev_fork, 0));
+                launch_few_leaves(c, B, few, nsink, tail, c->side);
+                LeavesDone d = *done;
+                d.tiny += nt0 - nt;
+                d.run += nr0 - nr;
+                launch_leaves(c, B, rp, nsink, d, false, leaf_tiny_grid(nt), leaf_run_grid(nr), nt, nr, c->side);
+                HIPCHK(hipEventRecord(c->ev_join, c->side));
+                *leaves_forked = true;
+            } else {
+                launch_few_leaves(c, B, few, nsink, tail, st);
+            }
+            done->tiny += nt0 - nt;
+            done->run += nr0 - nr;
             int bflags = 0;     // the first class waits for the level; the others may run beside it
             for (int cls = 0; cls < kBlkClasses; ++cls) {
-                if (!nblk[cls]) continue;
-                launch_block_class(c, B, rp, cls, blk_done[cls], nblk[cls], false, nblk[cls], nsink, tail, bflags);
-                if (!c->profile) bflags = hipExtAnyOrderLaunch;
-                *after_blocks = nlarge == 0;
-                sum_sizes(c, c->w.l_block[rp] + (uint64_t)cls * c->w.cap_block, blk_done[cls],
-                          c->d_cnt + C_BLOCK + 2 * cls + rp, blk_done[cls] + nblk[cls], S_BLOCK);
+                if (blk[cls]) {
+                    launch_block_class(c, B, rp, cls, blk_done[cls], blk[cls], false, blk[cls], nsink, tail, bflags);
+                    if (!c->profile) bflags = hipExtAnyOrderLaunch;
+                    *after_blocks = nlarge == 0;
+                    sum_sizes(c, c->w.l_block[rp] + (uint64_t)cls * c->w.cap_block, blk_done[cls],
+                              c->d_cnt + C_BLOCK + 2 * cls + rp, blk_done[cls] + blk[cls], S_BLOCK);
+                }
                 blk_done[cls] += nblk[cls];
             }
+            return PS5_OK;
         };
         // from level 2 on, the step overwrites the buffer and the run tables
         // of the level before the last: what was listed from them goes first
-        if (level >= 2 || nlarge == 0) sort_blocks();
+        if ((level >= 2 || nlarge == 0) && (rc = sort_blocks())) return rc;
         if (nlarge) {
             if (level >= 2) finish_known_leaves(c, B, rp, nsink, done);
             const int src = level > 0 ? kFromRuns : round > 0 ? kFromPerm : B.lut ? kRootPack : kRootPlain;
             if ((rc = large_step(c, B, nlarge, sink, seed, src, level & 1))) return rc;
-            if (level < 2) sort_blocks();
+            if (level < 2 && (rc = sort_blocks())) return rc;
         }
         HIPCHK(hipGetLastError());
         // blocks only append to the next round's lists: after a level

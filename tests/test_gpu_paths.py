@@ -162,3 +162,32 @@ def test_runs_with_long_common_prefixes(ps5, oracle, shared, planning):
         check(c, oracle, *pack([strs[i] for i in order]))
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("leaf_keys", [3, 8])
+@pytest.mark.parametrize("groups", [
+    {40: 3, 2048: 1}, {64: 9, 65: 1}, {256: 2, 257: 2, 512: 2, 513: 2, 1024: 2, 1025: 2},
+    {20: 200, 700: 9, 5000: 2}, {200: 700, 400: 700, 900: 700}, {100: 2500, 30: 17, 1500: 3}])
+def test_leaves_of_all_kinds_together(ps5, oracle, groups, leaf_keys):
+    """leaves of every kind, few of each in one launch, many in their own
+    kernels; every fourth group repeats one string, so that it is one run"""
+    rng = np.random.default_rng(len(groups) + sum(groups))
+    strs = []
+    for size, count in groups.items():
+        for g in range(count):
+            stem = rng.integers(97, 123, 6).astype(np.uint8).tobytes()
+            if g % 4 == 3:
+                strs += [stem] * size
+            else:
+                tails = rng.integers(97, 123, (size, 12)).astype(np.uint8)
+                cut = rng.integers(0, 13, size)
+                strs += [stem + t[:k].tobytes() for t, k in zip(tails, cut)]
+    order = rng.permutation(len(strs))
+    c = ps5.Context(0)
+    try:
+        c.set_shape(leaf_keys=leaf_keys)
+        arena, offs = pack([strs[i] for i in order])
+        check(c, oracle, arena, offs)
+        check(c, oracle, arena, offs, with_lcp=False)
+    finally:
+        c.close()
