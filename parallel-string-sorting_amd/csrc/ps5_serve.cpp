@@ -10,9 +10,10 @@
 // batch (ps5_sort_batch_device: every request is its own set) and reports
 // the bytes it releases.  Slots run concurrently, so requests that arrive
 // while others are on the GPU are admitted as soon as a slot and memory free
-// up.  Each request's result depends only on its own strings.  Requests are
-// copied between their host arrays and the slot's device buffers directly;
-// device buffers only grow.
+// up.  Each request's result depends only on its own strings.  Large requests
+// are copied between their host arrays and the slot's device buffers directly,
+// small ones together through the slot's pinned staging memory; device buffers
+// only grow.
 //
 // Failure isolation (the role of psstest's fork-per-run status
 // classification, src/psstest.cpp:310-370): a malformed request is rejected
@@ -115,7 +116,17 @@ int grow(T** p, uint64_t* cap, uint64_t need)
     return PS5_OK;
 }
 
+// A copy from or to pageable memory costs 25 to 40 us of the slot's time
+// however small it is, and a request has two to four of them: requests whose
+// arrays are at most kStageSmall bytes are packed into the slot's pinned staging
+// memory, neighbours in the batch with one copy each way.  A burst of 16
+// requests of 10 KB to 4 MB: 1.79 ms without, 1.68 with requests up to 64 KB
+// staged, 1.61 up to 256 KB, 1.50 up to 1 MB and up to 4 MB.
+constexpr uint64_t kStageSmall = 1 << 20;
+constexpr uint64_t kStageBytes = 16 << 20;
+
 struct SlotBuffers {
+    uint8_t* stage = nullptr;        // kStageBytes of pinned host memory, or nullptr: every copy is direct
     uint8_t* arena = nullptr;
     uint64_t arena_cap = 0;
     uint32_t* offs32 = nullptr;
@@ -146,6 +157,8 @@ struct SlotBuffers {
         for (void* q : { (void*)arena, (void*)offs32, (void*)offs64, (void*)perm, (void*)lcp, (void*)first,
                          (void*)base })
             if (q) (void)hipFree(q);
+        if (stage) (void)hipHostFree(stage);
+        stage = nullptr;
     }
 };
 
@@ -178,9 +191,9 @@ void fail_all_locked(ps5_server* s)
     s->cv_space.notify_all();
 }
 
-// Stage the requests of `batch` straight from their host arrays into the
-// slot's device buffers (no host-side packing), sort them as one batch, copy
-// each request's results straight back.  Returns the status of the whole.
+// Stage the requests of `batch` into the slot's device buffers, sort them as
+// one batch, copy each request's results back.  Returns the status of the
+// whole.
 int sort_batch(ps5_ctx* ctx, SlotBuffers& D, const std::vector<Request*>& batch, std::vector<uint64_t>& set_first,
                std::vector<uint64_t>& set_base, std::string* why)
 {
@@ -210,13 +223,52 @@ int sort_batch(ps5_ctx* ctx, SlotBuffers& D, const std::vector<Request*>& batch,
     }
     hipError_t he = hipSuccess;
     auto ok = [&](hipError_t e) { if (e != hipSuccess && he == hipSuccess) he = e; };
-    for (uint32_t i = 0; i < nsets; ++i) {
+    // requests [i, end) that share one copy from or to the `room` bytes of
+    // staging memory left (end == i: request i is copied on its own)
+    auto staged_end = [&](uint32_t i, uint64_t room, auto bytes) {
+        uint32_t j = i;
+        for (uint64_t sum = 0; D.stage && j < nsets; ++j) {
+            if (std::max(batch[j]->arena_bytes, batch[j]->n * 4) > kStageSmall) break;
+            sum += bytes(j);
+            if (sum > room) break;
+        }
+        return j;
+    };
+    struct Staged { uint32_t i, j; uint8_t* perm; uint8_t* lcp; };     // results of requests [i, j)
+    std::vector<Staged> results;
+    uint64_t used = 0;     // bytes of the staging memory
+    auto take = [&](uint64_t bytes) {
+        uint8_t* q = D.stage + used;
+        used += (bytes + 7) & ~7ull;
+        return q;
+    };
+    for (uint32_t i = 0; i < nsets;) {
         const Request* r = batch[i];
-        const uint64_t pad = ((r->arena_bytes + 8) & ~7ull) - r->arena_bytes;
-        if (r->arena_bytes)
-            ok(hipMemcpyAsync(D.arena + set_base[i], r->arena, r->arena_bytes, hipMemcpyHostToDevice, st));
-        ok(hipMemsetAsync(D.arena + set_base[i] + r->arena_bytes, 0, pad, st));
-        if (r->n) ok(hipMemcpyAsync(D.offs32 + set_first[i], r->offs, r->n * 4, hipMemcpyHostToDevice, st));
+        const uint64_t len = (r->arena_bytes + 8) & ~7ull;
+        const uint32_t j = staged_end(i, kStageBytes - used, [&](uint32_t q) {
+            return ((batch[q]->arena_bytes + 8) & ~7ull) + ((batch[q]->n * 4 + 7) & ~7ull);
+        });
+        if (j == i) {
+            if (r->arena_bytes)
+                ok(hipMemcpyAsync(D.arena + set_base[i], r->arena, r->arena_bytes, hipMemcpyHostToDevice, st));
+            ok(hipMemsetAsync(D.arena + set_base[i] + r->arena_bytes, 0, len - r->arena_bytes, st));
+            if (r->n) ok(hipMemcpyAsync(D.offs32 + set_first[i], r->offs, r->n * 4, hipMemcpyHostToDevice, st));
+            ++i;
+            continue;
+        }
+        const uint64_t ab = (j < nsets ? set_base[j] : abytes) - set_base[i], nb = (set_first[j] - set_first[i]) * 4;
+        uint8_t* a = take(ab);
+        uint8_t* o = take(nb);
+        for (uint32_t q = i; q < j; ++q) {
+            const Request* x = batch[q];
+            uint8_t* dst = a + (set_base[q] - set_base[i]);
+            if (x->arena_bytes) std::memcpy(dst, x->arena, x->arena_bytes);
+            std::memset(dst + x->arena_bytes, 0, ((x->arena_bytes + 8) & ~7ull) - x->arena_bytes);
+            if (x->n) std::memcpy(o + (set_first[q] - set_first[i]) * 4, x->offs, x->n * 4);
+        }
+        ok(hipMemcpyAsync(D.arena + set_base[i], a, ab, hipMemcpyHostToDevice, st));
+        if (nb) ok(hipMemcpyAsync(D.offs32 + set_first[i], o, nb, hipMemcpyHostToDevice, st));
+        i = j;
     }
     ok(hipMemsetAsync(D.arena + abytes, 0, 16, st));
     ok(hipMemcpyAsync(D.first, set_first.data(), (nsets + 1) * 8, hipMemcpyHostToDevice, st));
@@ -234,17 +286,41 @@ int sort_batch(ps5_ctx* ctx, SlotBuffers& D, const std::vector<Request*>& batch,
             (void)hipStreamSynchronize(st);
             return rc;
         }
-        for (uint32_t i = 0; i < nsets; ++i) {
+        // (the sort has ended, and with it the uploads: the staging memory is free again)
+        used = 0;
+        for (uint32_t i = 0; i < nsets;) {
             const Request* r = batch[i];
-            if (r->n) ok(hipMemcpyAsync(r->perm, D.perm + set_first[i], r->n * 4, hipMemcpyDeviceToHost, st));
-            if (r->lcp && r->n > 1)
-                ok(hipMemcpyAsync(r->lcp + 1, D.lcp + set_first[i] + 1, (r->n - 1) * 4, hipMemcpyDeviceToHost, st));
+            const uint32_t j = staged_end(i, kStageBytes - used, [&](uint32_t q) { return (batch[q]->n * 4 + 7) / 8 * 16; });
+            if (j == i) {
+                if (r->n) ok(hipMemcpyAsync(r->perm, D.perm + set_first[i], r->n * 4, hipMemcpyDeviceToHost, st));
+                if (r->lcp && r->n > 1)
+                    ok(hipMemcpyAsync(r->lcp + 1, D.lcp + set_first[i] + 1, (r->n - 1) * 4, hipMemcpyDeviceToHost, st));
+                ++i;
+                continue;
+            }
+            const uint64_t nb = (set_first[j] - set_first[i]) * 4;
+            Staged x = { i, j, take(nb), nullptr };
+            if (nb) ok(hipMemcpyAsync(x.perm, D.perm + set_first[i], nb, hipMemcpyDeviceToHost, st));
+            if (std::any_of(batch.begin() + i, batch.begin() + j, [](const Request* q) { return q->lcp && q->n > 1; })) {
+                x.lcp = take(nb);
+                ok(hipMemcpyAsync(x.lcp, D.lcp + set_first[i], nb, hipMemcpyDeviceToHost, st));
+            }
+            results.push_back(x);
+            i = j;
         }
     }
     ok(hipStreamSynchronize(st));
     if (he != hipSuccess) {
         *why = std::string("results: ") + hipGetErrorString(he);
         return PS5_ERR_HIP;
+    }
+    for (const Staged& x : results) {
+        for (uint32_t q = x.i; q < x.j; ++q) {
+            const Request* r = batch[q];
+            const uint64_t at = (set_first[q] - set_first[x.i]) * 4;
+            if (r->n) std::memcpy(r->perm, x.perm + at, r->n * 4);
+            if (r->lcp && r->n > 1) std::memcpy(r->lcp + 1, x.lcp + at + 4, (r->n - 1) * 4);
+        }
     }
     return PS5_OK;
 }
@@ -274,6 +350,10 @@ void run_slot(ps5_server* s, uint32_t slot)
     hipStream_t st = (hipStream_t)ps5_ctx_stream(ctx);
     volatile ps5::AdmitSlot* box = s->aslot + slot;
     SlotBuffers D;
+    if (hipHostMalloc(reinterpret_cast<void**>(&D.stage), kStageBytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        D.stage = nullptr;
+    }
     // warm start: buffers for one batch of the configured size, so that the
     // first requests do not pay for device allocations
     if (s->warm_strings) {

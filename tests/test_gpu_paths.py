@@ -191,3 +191,22 @@ def test_leaves_of_all_kinds_together(ps5, oracle, groups, leaf_keys):
         check(c, oracle, arena, offs, with_lcp=False)
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("bytes_each, count", [(2000, 9), ((1 << 20) - 8, 24), (1 << 20, 3), ((1 << 20) + 1, 3)])
+def test_served_requests_staged_and_direct(ps5, oracle, bytes_each, count):
+    """requests at the size where they are no longer packed together, in
+    batches that need more staging memory than a slot has, beside empty ones
+    and ones without LCPs"""
+    reqs = [ps5.gen_uniform(900 + i, bytes_each, 3, 40, ps5.ALPHA_ASCII94) for i in range(count)]
+    reqs.insert(1, (np.zeros(16, np.uint8), np.zeros(0, np.uint32)))
+    reqs.insert(2, (np.zeros(16, np.uint8), np.zeros(1, np.uint32)))
+    srv = ps5.Server(0, hbm_budget=4 << 30, slots=2, max_batch_strings=16 << 20)
+    try:
+        ids = [srv.submit(a, o, with_lcp=i % 3 != 2) for i, (a, o) in enumerate(reqs)]
+        out = [srv.wait(i) for i in ids]
+    finally:
+        srv.close()
+    for i, ((a, o), (p, l, _)) in enumerate(zip(reqs, out)):
+        if len(o):
+            assert oracle.verify(a, o, p, l)[0] == 0 if i % 3 != 2 else oracle.verify(a, o, p)[0] == 0
