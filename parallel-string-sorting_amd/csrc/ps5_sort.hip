@@ -2399,7 +2399,10 @@ __device__ __forceinline__ bool str_leq_from(const uint8_t* arena, uint64_t alen
 // extracted in input order by one streaming pass (a gather of 8 bytes per
 // string instead of an offset and an arena window); every round writes them
 // beside its outputs for the next.
-constexpr uint32_t kMergeE = 8;                    // outputs per thread
+// (outputs per thread: a thread's co-rank and LCP chain are serial, and the
+// tile's LDS sets how many workgroups hide them.  8 runs of 2 M strings: 977 us
+// with 8, 851 with 4, 974 with 2)
+constexpr uint32_t kMergeE = 4;
 constexpr uint32_t kMergeT = kWG * kMergeE;        // outputs per tile
 
 // a <= b for strings a, b (input indices) whose first 8 characters are ka, kb
@@ -2441,30 +2444,46 @@ __device__ __forceinline__ uint32_t merge_pair(const uint64_t* tstart, uint32_t 
     return lo;
 }
 
-// co[g] = strings of A (of g's pair) that precede the first output of tile g
+// co[g] = strings of A (of g's pair) that precede the first output of tile g.
+// kMergeLanes lanes search together, each testing one of as many positions
+// evenly spread over what is left: a test is a chain of dependent gathers,
+// and halving the range takes 21 of them one after another for runs of 2 M
+// strings (48 to 60 us a round for 16 M strings; with 16 lanes 19 to 37 us, of
+// which more and more are the gathers' own traffic: 8 runs of 2 M, three
+// rounds, take 1009 us with 32 lanes, 977 with 16 and 960 with 8).
+constexpr uint32_t kMergeLanes = 8;
 __global__ __launch_bounds__(kWG) void k_merge_part(Bufs B, const uint32_t* src_idx, const key64* src_key,
                                                     const key64* in_key,
                                                     const uint64_t* first, const uint64_t* mid,
                                                     const uint64_t* tstart, uint32_t npairs, uint32_t* co)
 {
-    const uint64_t g = (uint64_t)blockIdx.x * kWG + tid_x();
+    const uint64_t g = ((uint64_t)blockIdx.x * kWG + tid_x()) / kMergeLanes;
     if (g >= tstart[npairs]) return;
     const uint32_t p = merge_pair(tstart, npairs, g);
     const uint64_t a0 = first[p], b0 = mid[p];
     const uint64_t la = b0 - a0, lb = first[p + 1] - b0;
     const uint64_t diag = (g - tstart[p]) * kMergeT;
     uint64_t i0 = diag > lb ? diag - lb : 0, i1 = min(diag, la);
-    while (i0 < i1) {
-        const uint64_t mi = (i0 + i1) / 2;
-        const uint64_t pa = a0 + mi, pb = b0 + diag - 1 - mi;
-        uint32_t l;
-        if (merge_leq(B, src_idx[pa], src_idx[pb], merge_key(B, src_idx, src_key, in_key, pa),
-                      merge_key(B, src_idx, src_key, in_key, pb), &l))
-            i0 = mi + 1;
-        else
-            i1 = mi;
+    const uint32_t lane = lane_id(), l = lane % kMergeLanes;
+    while (i0 < i1) {     // (the same for the tile's lanes)
+        // A[mi] precedes this tile up to some mi in [i0, i1), and none from there on
+        const uint64_t step = (i1 - i0 + kMergeLanes - 1) / kMergeLanes;
+        const uint64_t mi = i0 + (l + 1) * step - 1;
+        bool before = false;
+        if (mi < i1) {
+            const uint64_t pa = a0 + mi, pb = b0 + diag - 1 - mi;
+            const key64 ka = merge_key(B, src_idx, src_key, in_key, pa), kb = merge_key(B, src_idx, src_key, in_key, pb);
+            uint32_t lcp;
+            // (indices are needed only where the keys do not decide)
+            before = ka != kb || (ka & 0xFFull) == 0 ? ka <= kb
+                                                     : merge_leq(B, src_idx[pa], src_idx[pb], ka, kb, &lcp);
+        }
+        const uint64_t ones = (__ballot(before) >> (lane - l)) & ((1ull << kMergeLanes) - 1);
+        const uint32_t t = (uint32_t)__popcll(ones);
+        i0 += t * step;
+        i1 = min(i1, i0 + step - 1);     // (lane t's position, if it is in the range, does not precede)
     }
-    co[g] = (uint32_t)i0;
+    if (l == 0) co[g] = (uint32_t)i0;
 }
 
 __global__ __launch_bounds__(kWG) void k_merge_tile(Bufs B, const uint32_t* src_idx, const uint32_t* src_lcp,
@@ -4400,51 +4419,60 @@ int ps5_merge_device(ps5_ctx* c, const uint8_t* d_arena, uint64_t arena_bytes, c
     key64* ik = tk[1];
     hipLaunchKernelGGL(k_init, dim3(div_up(n, kWG)), dim3(kWG), 0, st, B, ik, (uint32_t)n);
     HIPCHK(hipGetLastError());
-    const key64* sk = nullptr;
-    int cur = 0;
+    // every round's plan, uploaded at once: first[np + 1], mid[np], tstart[np + 1]
+    struct Round { uint64_t at; uint32_t np; uint64_t tiles; };
+    std::vector<Round> rounds;
+    std::vector<uint64_t> plan;
+    uint64_t most = 0;     // tiles of a round
     while (bounds.size() > 2) {
         const uint32_t nr = (uint32_t)bounds.size() - 1, np = (nr + 1) / 2;
-        std::vector<uint64_t> plan(3 * (np + 1), 0);   // first[np+1], mid[np], tstart[np+1]
-        uint64_t* f = plan.data();
+        const uint64_t at = plan.size();
+        plan.resize(at + 3 * ((uint64_t)np + 1), 0);
+        uint64_t* f = plan.data() + at;
         uint64_t* mdl = f + (np + 1);
         uint64_t* ts = mdl + (np + 1);
+        std::vector<uint64_t> nb(np + 1);
         for (uint32_t p = 0; p < np; ++p) {
             f[p] = bounds[2 * p];
             mdl[p] = bounds[2 * p + 1];
             const uint64_t e = 2 * p + 2 <= nr ? bounds[2 * p + 2] : bounds[2 * p + 1];
             ts[p + 1] = ts[p] + (e - f[p] + kMergeT - 1) / kMergeT;
+            nb[p] = f[p];
         }
-        f[np] = bounds[nr];
-        const uint64_t tiles = ts[np];
-        const bool last = np == 1;
+        f[np] = nb[np] = bounds[nr];
+        rounds.push_back(Round{ at, np, ts[np] });
+        most = std::max(most, ts[np]);
+        bounds.swap(nb);
+    }
+    const uint64_t words = plan.size() + (most + 1) / 2;    // the plans, then co[tiles] as uint32
+    if (words > c->merge_cap) {
+        if (c->d_merge) (void)hipFree(c->d_merge);
+        c->d_merge = nullptr;
+        c->merge_cap = 0;
+        HIPCHK(hipMalloc(&c->d_merge, words * sizeof(uint64_t)));
+        c->merge_cap = words;
+    }
+    // (the vector outlives the copy: the call ends with a read-back)
+    HIPCHK(hipMemcpyAsync(c->d_merge, plan.data(), plan.size() * sizeof(uint64_t), hipMemcpyHostToDevice, st));
+    uint32_t* co = reinterpret_cast<uint32_t*>(c->d_merge + plan.size());
+    const key64* sk = nullptr;
+    int cur = 0;
+    for (const Round& R : rounds) {
+        const bool last = R.np == 1;
         uint32_t* di = last ? d_idx_out : ti[cur];
         uint32_t* dl = last ? d_lcp_out : tl[cur];
         key64* dk = last ? nullptr : tk[cur];
-        const uint64_t words = plan.size() + (tiles + 1) / 2;    // plan, then co[tiles] as uint32
-        if (words > c->merge_cap) {
-            if (c->d_merge) (void)hipFree(c->d_merge);
-            c->d_merge = nullptr;
-            c->merge_cap = 0;
-            HIPCHK(hipMalloc(&c->d_merge, words * sizeof(uint64_t)));
-            c->merge_cap = words;
-        }
-        HIPCHK(hipMemcpyAsync(c->d_merge, plan.data(), plan.size() * sizeof(uint64_t), hipMemcpyHostToDevice, st));
-        if (tiles) {
-            const uint64_t* pf = c->d_merge;
-            const uint64_t* pm = pf + (np + 1);
-            const uint64_t* pt = pm + (np + 1);
-            uint32_t* co = reinterpret_cast<uint32_t*>(c->d_merge + plan.size());
-            hipLaunchKernelGGL(k_merge_part, dim3(div_up(tiles, kWG)), dim3(kWG), 0, st, B, si, sk, ik, pf, pm, pt, np,
-                               co);
+        const uint64_t* pf = c->d_merge + R.at;
+        const uint64_t* pm = pf + (R.np + 1);
+        const uint64_t* pt = pm + (R.np + 1);
+        if (R.tiles) {
+            hipLaunchKernelGGL(k_merge_part, dim3(div_up(R.tiles, kWG / kMergeLanes)), dim3(kWG), 0, st, B, si, sk, ik, pf,
+                               pm, pt, R.np, co);
             HIPCHK(hipGetLastError());
-            hipLaunchKernelGGL(k_merge_tile, dim3(tiles), dim3(kWG), 0, st, B, si, sl, sk, ik, di, dl, dk, pf, pm, pt,
-                               np, co);
+            hipLaunchKernelGGL(k_merge_tile, dim3(R.tiles), dim3(kWG), 0, st, B, si, sl, sk, ik, di, dl, dk, pf, pm, pt,
+                               R.np, co);
             HIPCHK(hipGetLastError());
         }
-        HIPCHK(hipStreamSynchronize(st));     // the plan buffer is rewritten next round
-        std::vector<uint64_t> nb(np + 1);
-        for (uint32_t p = 0; p <= np; ++p) nb[p] = f[p];
-        bounds.swap(nb);
         si = di;
         sl = dl;
         sk = dk;

@@ -210,3 +210,27 @@ def test_served_requests_staged_and_direct(ps5, oracle, bytes_each, count):
     for i, ((a, o), (p, l, _)) in enumerate(zip(reqs, out)):
         if len(o):
             assert oracle.verify(a, o, p, l)[0] == 0 if i % 3 != 2 else oracle.verify(a, o, p)[0] == 0
+
+
+@pytest.mark.parametrize("sizes", [(1, 1), (1023, 1), (1024, 1024), (1, 3000), (4095, 4097, 2), (20000, 7, 0, 20001),
+                                   (9000,) * 9])
+@pytest.mark.parametrize("kind", ["ascii", "equal", "deep"])
+def test_merge_tile_edges(ps5, ctx, oracle, sizes, kind):
+    """tile remainders, runs much shorter than others, empty runs; runs whose
+    strings are all equal or differ past their first 8 characters only"""
+    rng = np.random.default_rng(sum(sizes) + len(kind))
+    n = sum(sizes)
+    stem = {"ascii": b"", "equal": b"same", "deep": b"a-common-prefix-"}[kind]
+    strs = [stem if kind == "equal" else stem + rng.integers(97, 105, rng.integers(0, 9)).astype(np.uint8).tobytes()
+            for _ in range(n)]
+    arena, offs = pack(strs)
+    bounds = np.concatenate([[0], np.cumsum(sizes)]).astype(np.uint64)
+    idx, lcp = np.zeros(n, np.uint32), np.zeros(n, np.uint32)
+    for b, e in zip(bounds[:-1].astype(int), bounds[1:].astype(int)):
+        if e > b:
+            p, l = oracle.brute_sort(arena, offs[b:e])
+            idx[b:e] = p + b
+            lcp[b:e] = l
+    mi, ml = ctx.merge(arena, offs, bounds, idx, lcp)
+    r, msg = oracle.verify(arena, offs, mi, ml)
+    assert r == 0, msg
