@@ -2198,8 +2198,6 @@ __global__ __launch_bounds__(kLeavesWG) __attribute__((amdgpu_waves_per_eu(5))) 
     union Lds {
         BlockLds<kBlkT, kBlkE3, TAIL> b3;
         BlockLds<1024, kBlkE2, TAIL> b2;
-        BlockLds<512, kBlkE1, TAIL> b1;
-        BlockLds<256, kBlkE0, TAIL> b0;
         RunMap<kRunChunk> m;
         struct { key64 k[kLeavesTiny][64]; uint32_t i[kLeavesTiny][64], r[kLeavesTiny][64]; } t;
     };
@@ -2215,8 +2213,10 @@ __global__ __launch_bounds__(kLeavesWG) __attribute__((amdgpu_waves_per_eu(5))) 
     i -= Q.r[J].count;
     PS5_LEAVES_BLOCK(4, kBlkT, kBlkE3, S.b3)
     PS5_LEAVES_BLOCK(3, 1024, kBlkE2, S.b2)
-    PS5_LEAVES_BLOCK(2, 512, kBlkE1, S.b1)
-    PS5_LEAVES_BLOCK(1, 256, kBlkE0, S.b0)
+    // (smaller blocks have as many waves: their LDS is reserved anyway, and a
+    // block's runs of equal keys are finished a wave each)
+    PS5_LEAVES_BLOCK(2, 1024, kBlkE2, S.b2)
+    PS5_LEAVES_BLOCK(1, 1024, kBlkE2, S.b2)
 #undef PS5_LEAVES_BLOCK
     if (i < Q.r[5].count) {
         if (tid_x() < kWG) run_chunk(load_uniform(Q.r[5].list + Q.r[5].first + i), B, nxt, S.m);
@@ -3438,6 +3438,9 @@ void launch_block_class(ps5_ctx* c, const Bufs& B, int rp, int cls, uint32_t fir
     const uint32_t* cnt = c->d_cnt + C_BLOCK + 2 * cls + rp;
     const uint32_t* pf = dev_first ? c->d_cnt + C_BDONE + cls : nullptr;
     const uint32_t cap = c->w.cap_block;
+    // no more blocks than CUs: small ones are given more waves, which finish
+    // more of their runs of equal keys at a time (167 URL-like strings: 40 -> 26 us)
+    if (!dev_first && count <= (uint32_t)c->cus) cls = std::max(cls, 2);
     Launch L(c, K_BLOCK, 0);
     // the default key width (8 keys) has its own instances; others share one
 #define PS5_BLOCK_LAUNCH(M, E, LOOP, TAIL)                                                                         \
@@ -3690,9 +3693,10 @@ int dev_level_kmax(const ps5_ctx* c, uint64_t m, uint32_t level)
 // level are sorted in it (blk_done: blocks already sorted per size class;
 // done: leaves already finished).  Level l of a round writes buffer l & 1.
 int host_levels(ps5_ctx* c, const Bufs& B, uint32_t round, uint32_t level, int cur_ci, uint32_t* blk_done,
-                LeavesDone* done, bool* leaves_forked, uint32_t reset_mask, bool* after_blocks)
+                LeavesDone* done, bool* leaves_forked, uint32_t reset_mask, bool* after_blocks, bool* split)
 {
     *after_blocks = false;     // set when the stream's last packets are the last level's block kernels
+    *split = false;            // set when a segment of the round is split
     hipStream_t st = c->stream;
     const int rp = round & 1, np = rp ^ 1;
     const Sink nsink = make_sink(c, c->w.l_round[np], C_LROUND + np, np);
@@ -3777,6 +3781,7 @@ int host_levels(ps5_ctx* c, const Bufs& B, uint32_t round, uint32_t level, int c
         // of the level before the last: what was listed from them goes first
         if ((level >= 2 || nlarge == 0) && (rc = sort_blocks())) return rc;
         if (nlarge) {
+            *split = true;
             if (level >= 2) finish_known_leaves(c, B, rp, nsink, done);
             const int src = level > 0 ? kFromRuns : round > 0 ? kFromPerm : B.lut ? kRootPack : kRootPlain;
             if ((rc = large_step(c, B, nlarge, sink, seed, src, level & 1))) return rc;
@@ -3826,7 +3831,8 @@ int host_levels(ps5_ctx* c, const Bufs& B, uint32_t round, uint32_t level, int c
 
 // Leaves and leaf boundaries of a round planned on the host (h_cnt holds
 // the round's final counts), then the read-back of the next round's lists.
-int host_round_end(ps5_ctx* c, const Bufs& B, uint32_t round, LeavesDone done, bool leaves_forked, bool after_blocks)
+int host_round_end(ps5_ctx* c, const Bufs& B, uint32_t round, LeavesDone done, bool leaves_forked, bool after_blocks,
+                   bool split)
 {
     hipStream_t st = c->stream;
     const int rp = round & 1, np = rp ^ 1;
@@ -3846,7 +3852,9 @@ int host_round_end(ps5_ctx* c, const Bufs& B, uint32_t round, LeavesDone done, b
     // boundaries below wait for all of them
     else launch_leaves(c, B, rp, nsink, done, false, leaf_tiny_grid(nt - done.tiny), leaf_run_grid(nr - done.run),
                        nt - done.tiny, nr - done.run, st, after_blocks && !c->profile ? hipExtAnyOrderLaunch : 0);
-    if (nt + nb + nr && B.lcp) launch_leafbound(c, B, rp, div_up((uint64_t)nt + nb + nr, kWG), nt + nb + nr);
+    // (a segment that was not split is one leaf, without a boundary to another:
+    // 5 us of a small sort's 55)
+    if (split && nt + nb + nr && B.lcp) launch_leafbound(c, B, rp, div_up((uint64_t)nt + nb + nr, kWG), nt + nb + nr);
     HIPCHK(hipGetLastError());
     return readback(c, c->w.l_round[np], C_LROUND + np);
 }
@@ -3899,12 +3907,12 @@ int sort_round(ps5_ctx* c, SortRun& R, uint32_t round, bool dev, bool* done)
     const Sink nsink = make_sink(c, c->w.l_round[np], C_LROUND + np, np);
     uint32_t blk_done[kBlkClasses] = {};
     LeavesDone done_leaves;
-    bool leaves_forked = false, after_blocks = false;
+    bool leaves_forked = false, after_blocks = false, split = false;
     if (!dev) {
         if ((rc = host_levels(c, B, round, 0, C_LROUND + rp, blk_done, &done_leaves, &leaves_forked, round_mask,
-                              &after_blocks)))
+                              &after_blocks, &split)))
             return rc;
-        if ((rc = host_round_end(c, B, round, done_leaves, leaves_forked, after_blocks))) return rc;
+        if ((rc = host_round_end(c, B, round, done_leaves, leaves_forked, after_blocks, split))) return rc;
     } else {
         // every level of the round without a host synchronisation.  The
         // host knows the round's lists (read back with the previous
@@ -3927,9 +3935,9 @@ int sort_round(ps5_ctx* c, SortRun& R, uint32_t round, bool dev, bool* done)
         const uint32_t L = nl0 ? dev_levels_for(c, mmax) : 0;
         if (L == 0) {
             if ((rc = host_levels(c, B, round, 0, C_LROUND + rp, blk_done, &done_leaves, &leaves_forked, 0u,
-                                  &after_blocks)))
+                                  &after_blocks, &split)))
                 return rc;
-            if ((rc = host_round_end(c, B, round, done_leaves, leaves_forked, after_blocks))) return rc;
+            if ((rc = host_round_end(c, B, round, done_leaves, leaves_forked, after_blocks, split))) return rc;
         } else {
             int in_ci = C_LROUND + rp;
             const Item* in_list = c->w.l_round[rp];
@@ -3987,9 +3995,9 @@ int sort_round(ps5_ctx* c, SortRun& R, uint32_t round, bool dev, bool* done)
                 for (int cls = 0; cls < kBlkClasses; ++cls) blk_done[cls] = c->h_cnt[C_BLOCK + 2 * cls + rp];
                 if ((rc = readback(c, in_list, in_ci))) return rc;
                 done_leaves = LeavesDone{ c->h_cnt[C_TDONE], c->h_cnt[C_RDONE] };
-                if ((rc = host_levels(c, B, round, L, in_ci, blk_done, &done_leaves, &leaves_forked, 0u, &after_blocks)))
+                if ((rc = host_levels(c, B, round, L, in_ci, blk_done, &done_leaves, &leaves_forked, 0u, &after_blocks, &split)))
                     return rc;
-                if ((rc = host_round_end(c, B, round, done_leaves, leaves_forked, after_blocks))) return rc;
+                if ((rc = host_round_end(c, B, round, done_leaves, leaves_forked, after_blocks, split))) return rc;
             } else {
                 uint32_t nb = 0;
                 for (int cls = 0; cls < kBlkClasses; ++cls) nb += c->h_cnt[C_BLOCK + 2 * cls + rp];

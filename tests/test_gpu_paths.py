@@ -234,3 +234,11 @@ def test_merge_tile_edges(ps5, ctx, oracle, sizes, kind):
     mi, ml = ctx.merge(arena, offs, bounds, idx, lcp)
     r, msg = oracle.verify(arena, offs, mi, ml)
     assert r == 0, msg
+
+
+@pytest.mark.parametrize("n", [2, 64, 65, 255, 256, 257, 512, 513, 1025, 2048])
+@pytest.mark.parametrize("with_lcp", [True, False])
+def test_sorts_of_one_block(ps5, ctx, oracle, n, with_lcp):
+    """a sort that is one block of each size class, with deep common prefixes"""
+    strs = [b"http://host%d/" % (i % 3) + s for i, s in enumerate(random_strings(n, 0, 30, b"ab/", n))]
+    check(ctx, oracle, *pack(strs), with_lcp=with_lcp)
