@@ -1059,7 +1059,16 @@ __device__ __forceinline__ void emit_children(const LargeDesc& D, uint32_t start
 // (gsum), and the children.  A segment of one group of chunks sums its bucket
 // counts here, of more it scans the groups' sums, a thread per bucket.  dst:
 // the buffer the level wrote.
-__global__ __launch_bounds__(kBigWG) void k_children(Plan P, Bufs B, const key64* trees, Sink s, uint32_t dst)
+//
+// fused (a level planned on the host whose segments all are of one group and
+// few entries): the segments' run tables are written here, after the bucket
+// starts, and k_hist_runs is not launched.  It takes 5 to 9 us on its own for
+// so little (40 K strings of ACGT: 121 -> 118 us, a burst of 16 served
+// requests 1.45 -> 1.40 ms); a thread writes a bucket's row, which for the
+// hundreds of segments of a level planned on the device is slower than
+// k_hist_runs's turned tiles (64 M strings: 2.12 ms fused, 2.09 not).
+constexpr uint32_t kFusedRuns = 16384;     // entries of a segment
+__global__ __launch_bounds__(kBigWG) void k_children(Plan P, Bufs B, const key64* trees, Sink s, uint32_t dst, int fused)
 {
     __shared__ uint32_t s_sz[kMaxBkt + 1];
     __shared__ uint32_t s_tmp[kBigWaves * kChildLists + 8];     // the scans' scratch, then the lists' bases
@@ -1112,10 +1121,27 @@ __global__ __launch_bounds__(kBigWG) void k_children(Plan P, Bufs B, const key64
             for (int j = 0; j < kChildPer; ++j) {
                 const uint32_t b = tid_x() * kChildPer + j;
                 if (b < nbs) {
-                    g[b] = at;
-                    if (G == 1) g[nbs + b] = 0;
+                    if (fused) s_sz[b] = at;
+                    else g[b] = at;
+                    if (G == 1 && !fused) g[nbs + b] = 0;
                 }
                 at += sz[j];
+            }
+            if (fused) {     // (uniform)
+                __syncthreads();     // the starts are written
+                const uint32_t* h = B.hist + D.hist_base;
+                uint32_t* V = B.vpos + (dst ? B.cap_h : 0ull) + D.hist_base;
+                uint32_t* S = B.src + (dst ? B.cap_h : 0ull) + D.hist_base;
+                for (uint32_t b = tid_x(); b + 1 < nbs; b += kBigWG) {
+                    uint32_t first = s_sz[b];
+#pragma unroll 8
+                    for (uint32_t c = 0; c < D.nch; ++c) {
+                        const uint32_t x = h[c * nbs + b];
+                        V[b * D.nch + c] = first;
+                        S[b * D.nch + c] = D.seg.begin + c * D.chunk + (x >> 16);
+                        first += x & 0xFFFFu;
+                    }
+                }
             }
             emit_children(D, start, sz, dst, trees + (uint64_t)si * kTreeSlots + 1024, s,
                           B.sdepth_out, s_tmp);
@@ -3221,7 +3247,7 @@ uint64_t part_bytes(int src)
 
 // What follows a level's partition: bucket sizes, children, run tables.
 void launch_hist(ps5_ctx* c, const Bufs& B, Plan P, const Sink& sink, uint32_t dst, int kmax, uint32_t g_sum,
-                 uint32_t g_children, uint32_t g_runs, uint64_t hl)
+                 uint32_t g_children, uint32_t g_runs, uint64_t hl, bool fused)
 {
     const uint32_t nbs = 2u << kmax;
     if (g_sum) {     // (segments of more than one group of chunks)
@@ -3230,9 +3256,9 @@ void launch_hist(ps5_ctx* c, const Bufs& B, Plan P, const Sink& sink, uint32_t d
     }
     {
         Launch L(c, K_CHILDREN, g_sum ? hl * 8 / kHistGroup : hl * 4);
-        hipLaunchKernelGGL(k_children, dim3(g_children), dim3(kBigWG), 0, c->stream, P, B, c->w.trees, sink, dst);
+        hipLaunchKernelGGL(k_children, dim3(g_children), dim3(kBigWG), 0, c->stream, P, B, c->w.trees, sink, dst, (int)fused);
     }
-    {
+    if (!fused) {
         Launch L(c, K_HIST, hl * 12);
         hipLaunchKernelGGL(k_hist_runs, dim3(g_runs, div_up(nbs, 64)), dim3(kWG), 0, c->stream, P, B, (int)dst);
     }
@@ -3246,6 +3272,7 @@ int large_step(ps5_ctx* c, const Bufs& B, uint32_t nlarge, const Sink& sink, uin
     hipStream_t st = c->stream;
     uint64_t ntiles = 0, ngroups = 0, hl = 0, gs = 0, elems = 0;
     int kmax = 1;
+    bool fused = true;
     if (nlarge > c->w.cap_large) return set_err(PS5_ERR_CAPACITY, "large list overflow");
     LevelHdr* h_hdr = reinterpret_cast<LevelHdr*>(c->w.h_plan);
     LargeDesc* h_descs = reinterpret_cast<LargeDesc*>(c->w.h_plan + sizeof(LevelHdr));
@@ -3268,6 +3295,7 @@ int large_step(ps5_ctx* c, const Bufs& B, uint32_t nlarge, const Sink& sink, uin
         const uint32_t nspl = (1u << D.k) - 1;
         kmax = std::max(kmax, (int)D.k);
         D.oversample = std::max<uint32_t>(2, std::min<uint32_t>(c->max_oversample, (kMaxSamples / nspl) & ~1u));
+        fused = fused && G == 1 && (uint64_t)T * (2u << D.k) <= kFusedRuns;
         if (ntiles + T > c->w.tiles_cap || ngroups + G > c->w.groups_cap)
             return set_err(PS5_ERR_CAPACITY, "chunk table capacity");
         for (uint32_t t = 0; t < T; ++t) h_tiles[ntiles + t] = TileRef{ i, t };
@@ -3306,7 +3334,7 @@ int large_step(ps5_ctx* c, const Bufs& B, uint32_t nlarge, const Sink& sink, uin
         Launch L(c, K_PART, elems * part_bytes(src) + hl * 4);
         launch_part(c, B, P, div_up(ntiles, kXcds) * kXcds, kmax, src, (uint32_t)ntiles, nlarge == 1);
     }
-    launch_hist(c, B, P, sink, dst, kmax, ngroups > nlarge ? (uint32_t)ngroups : 0u, nlarge, (uint32_t)ngroups, hl);
+    launch_hist(c, B, P, sink, dst, kmax, ngroups > nlarge ? (uint32_t)ngroups : 0u, nlarge, (uint32_t)ngroups, hl, fused);
     c->st_segments += nlarge;
     return PS5_OK;
 }
@@ -3642,7 +3670,7 @@ void dev_level(ps5_ctx* c, const Bufs& B, const Item* list, int ci, uint32_t bou
                     false);
     }
     const uint32_t groups_bound = (uint32_t)std::min<uint64_t>(kDevHistWgs, tiles_bound / kHistGroup + gl);
-    launch_hist(c, B, P, sink, dst, kmax, groups_bound, std::min(gl, kDevChildWgs), groups_bound, 0);
+    launch_hist(c, B, P, sink, dst, kmax, groups_bound, std::min(gl, kDevChildWgs), groups_bound, 0, false);
 }
 
 // Bound on the buckets of a level over segments of at most m strings (its
