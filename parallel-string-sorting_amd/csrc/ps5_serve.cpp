@@ -99,8 +99,8 @@ struct ps5_server {
 namespace {
 
 // device bytes a request occupies while it runs: its characters, uint32 and
-// uint64 offsets, results, and the sort context's work buffers (~72 B per string)
-uint64_t request_bytes(uint64_t arena_bytes, uint64_t n) { return arena_bytes + 16 + n * (4 + 8 + 8 + 72) + 4096; }
+// uint64 offsets, results, and the sort context's work buffers (~88 B per string)
+uint64_t request_bytes(uint64_t arena_bytes, uint64_t n) { return arena_bytes + 16 + n * (4 + 8 + 8 + 88) + 4096; }
 
 // device buffer that only grows, at least by half each time
 template <class T>
