@@ -3418,12 +3418,13 @@ constexpr uint32_t kForkLeafGroups = 8192;    // leaf workgroups worth a side st
 // block classes and 0.4 K others: 363 us apart, 329 with the others together,
 // 316 with those on the side stream, 338 with one of the classes as well.
 constexpr uint32_t kFewLeavesPerCu = 8;
-// Strings of the largest root from which on roots may pack their keys.  The
-// kernels that can pack take about 11 us more (digits, which do not pack,
-// 0.5 M strings: 221 -> 233 us), and smaller roots of a small alphabet have
-// little to gain (40 K strings of ACGT: 161 us plain, 171 packed); 4 M
-// suffixes of ACGT text take 1.36 ms against 1.58, 20 M windows 1.94 against
-// 2.88, a batch of 192 sets (a third of them ACGT) 3.01 against 3.24.
+// Strings of the largest root from which on roots may pack their keys.
+// Packing saves rounds and levels where keys repeat: 4.2 M suffixes of an ACGT
+// text take 0.73 ms against 1.08 plain, 20 M windows 1.47 against 3.03, a batch
+// of 192 sets (a third of them ACGT) 2.21 against 2.59.  Smaller roots of a
+// small alphabet have little to gain (40 K strings of ACGT: 119 us plain, 116
+// packed), and the kernels that can pack cost others a little (0.5 M digits,
+// which do not pack: 163 and 165 us).
 constexpr uint64_t kPackMin = 1u << 20;
 constexpr uint64_t kChainMin = 1u << 22;       // strings of a level whose successor is chained on the device
 // Automatic planning plans a single sort of fewer strings on the device.
