@@ -3427,12 +3427,12 @@ constexpr uint32_t kFewLeavesPerCu = 8;
 // which do not pack: 163 and 165 us).
 constexpr uint64_t kPackMin = 1u << 20;
 constexpr uint64_t kChainMin = 1u << 22;       // strings of a level whose successor is chained on the device
-// Automatic planning plans a single sort of fewer strings on the device.
-// From about 4 M strings on the device plan's bounded grids cost more than
-// the host's synchronisations (0.489 vs 0.50 ms on 4 M strings); below, the
-// two are within a few percent either way, depending on the input (device
-// planning 6-9% faster on 0.13 M digit strings and 0.64 M ASCII strings, 4-7%
-// slower on 0.32 M ASCII strings and on high-LCP windows).
+// Automatic planning plans a single sort of fewer strings on the device, as
+// its callers are told: one synchronisation per round.  The line was drawn
+// where the two modes took the same time; the host now sees which leaves are
+// few and launches them together, and is ahead at every size (39 K strings of
+// ACGT: 115 us, 152 planned on the device; 0.5 M digits: 162 and 214; 4 M
+// ASCII strings: 365 and 375).
 constexpr uint64_t kAutoDevMax = 1u << 22;
 
 // Largest grids of the device-planned levels: their kernels loop over the
