@@ -1376,10 +1376,10 @@ __device__ __forceinline__ void tiny_leaf(const Item& L, const Bufs& B, key64* s
     wave_finish_leaf<NK>(B, L.begin + lane, L.size, k, id, depth, key_fmt(L.flags), true, 0u, s_k, s_i, s_r);
 }
 
-// The tiny leaves from *p_first (first, if null) on of a list, a wave each.
+// The tiny leaves from *p_first (first, if null) to entry `end` of a list, a wave each.
 template <int NK>
 __global__ __launch_bounds__(kWG) void k_leaf_tiny(const Item* items, const uint32_t* p_first, uint32_t first,
-                                                   const uint32_t* cnt_items, uint32_t cap, Bufs B)
+                                                   const uint32_t* cnt_items, uint32_t end, Bufs B)
 {
     __shared__ key64 s_k[kWaves][64];
     __shared__ uint32_t s_i[kWaves][64];
@@ -1389,7 +1389,7 @@ __global__ __launch_bounds__(kWG) void k_leaf_tiny(const Item* items, const uint
         if (B.pending_err && tid_x() == 0) flag_error(B.cnt, ERR_LEVELS);
         return;
     }
-    const uint32_t nitems = min(*cnt_items, cap);     // (an overflow has been flagged)
+    const uint32_t nitems = min(*cnt_items, end);     // (an overflow of the list has been flagged)
     if (p_first) first = *p_first;
     // each wave takes leaves it, it + stride, ... (no workgroup barriers below)
     for (uint32_t it = first + blockIdx.x * kWaves + w; it < nitems; it += gridDim.x * kWaves) {
@@ -2180,16 +2180,16 @@ __device__ __forceinline__ void run_chunk(const Item& L, const Bufs& B, const Si
     }
 }
 
-// The chunks of equal-key leaves from *p_first (first, if null) on of a list.
+// The chunks of equal-key leaves from *p_first (first, if null) to entry `end` of a list.
 __global__ __launch_bounds__(kWG) void k_leaf_run(const Item* items, const uint32_t* p_first, uint32_t first,
-                                                  const uint32_t* cnt_items, uint32_t cap, Bufs B, Sink nxt)
+                                                  const uint32_t* cnt_items, uint32_t end, Bufs B, Sink nxt)
 {
     __shared__ RunMap<kRunChunk> M;
     if (B.pending && *B.pending) {      // the round's levels are not finished
         if (B.pending_err && tid_x() == 0) flag_error(B.cnt, ERR_LEVELS);
         return;
     }
-    const uint32_t nitems = min(*cnt_items, cap);     // (an overflow has been flagged)
+    const uint32_t nitems = min(*cnt_items, end);     // (an overflow of the list has been flagged)
     if (p_first) first = *p_first;
     for (uint32_t ii = first + blockIdx.x; ii < nitems; ii += gridDim.x) {
         __syncthreads();     // the previous chunk's map is no longer read
@@ -3500,29 +3500,33 @@ void launch_block_class(ps5_ctx* c, const Bufs& B, int rp, int cls, uint32_t fir
 #undef PS5_BLOCK_LAUNCH
 }
 
-// Tiny leaves and equal-key chunks of round parity rp on stream s, from the
-// entries done.tiny and done.run on (from the counters C_TDONE and C_RDONE on
-// with dev_first), in grids of g_tiny and g_run workgroups (0 skips a list).
+// Tiny leaves and equal-key chunks of round parity rp on stream s: n_tiny and
+// n_run of them from the entries done.tiny and done.run on, and no more, since
+// what is queued before may have listed leaves that the host does not count
+// yet (with dev_first: from the counters C_TDONE and C_RDONE on, all that are
+// listed), in grids of g_tiny and g_run workgroups (0 skips a list).
 struct LeavesDone { uint32_t tiny = 0, run = 0; };
 void launch_leaves(ps5_ctx* c, const Bufs& B, int rp, const Sink& nsink, LeavesDone done, bool dev_first,
                    uint32_t g_tiny, uint32_t g_run, uint64_t n_tiny, uint64_t n_run, hipStream_t s, int flags = 0)
 {
     if (g_tiny) {
         const uint32_t* first = dev_first ? c->d_cnt + C_TDONE : nullptr;
+        const uint32_t end = dev_first ? c->w.cap_tiny[rp] : (uint32_t)std::min<uint64_t>(c->w.cap_tiny[rp], done.tiny + n_tiny);
         {
             Launch L(c, K_LEAF_TINY, 0);
             const auto f = c->leaf_keys == 8 ? k_leaf_tiny<8> : k_leaf_tiny<0>;
             hipExtLaunchKernelGGL(f, dim3(g_tiny), dim3(kWG), 0, s, nullptr, nullptr, flags, c->w.l_tiny[rp], first,
-                                  done.tiny, c->d_cnt + C_TINY + rp, c->w.cap_tiny[rp], B);
+                                  done.tiny, c->d_cnt + C_TINY + rp, end, B);
         }
         sum_sizes(c, c->w.l_tiny[rp], done.tiny, c->d_cnt + C_TINY + rp, (uint32_t)n_tiny, S_TINY);
     }
     if (g_run) {
         const uint32_t* first = dev_first ? c->d_cnt + C_RDONE : nullptr;
+        const uint32_t end = dev_first ? c->w.cap_run : (uint32_t)std::min<uint64_t>(c->w.cap_run, done.run + n_run);
         {
             Launch L(c, K_LEAF_RUN, 0);
             hipExtLaunchKernelGGL(k_leaf_run, dim3(g_run), dim3(kWG), 0, s, nullptr, nullptr, flags, c->w.l_run[rp], first,
-                                  done.run, c->d_cnt + C_RUN + rp, c->w.cap_run, B, nsink);
+                                  done.run, c->d_cnt + C_RUN + rp, end, B, nsink);
         }
         sum_sizes(c, c->w.l_run[rp], done.run, c->d_cnt + C_RUN + rp, (uint32_t)n_run, S_RUN);
     }

@@ -242,3 +242,61 @@ def test_sorts_of_one_block(ps5, ctx, oracle, n, with_lcp):
     """a sort that is one block of each size class, with deep common prefixes"""
     strs = [b"http://host%d/" % (i % 3) + s for i, s in enumerate(random_strings(n, 0, 30, b"ab/", n))]
     check(ctx, oracle, *pack(strs), with_lcp=with_lcp)
+
+
+def mix64(z):
+    """the sampler's hash (uint64 arrays)"""
+    with np.errstate(over="ignore"):
+        z = z + np.uint64(0x9E3779B97F4A7C15)
+        z = (z ^ (z >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+        z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+        return z ^ (z >> np.uint64(31))
+
+
+def unlucky_sets(nsets, m, samples, seed):
+    """sets of m strings of which the root level's samples show the smallest
+    ones only: all others, half of them in groups that share 8 characters and
+    more, end in one bucket; every other sampled string starts alike"""
+    rng = np.random.default_rng(seed)
+    n, width = nsets * m, 20
+    rows = np.zeros((n, width), np.uint8)
+    rows[:, :width - 1] = rng.integers(98, 123, (n, width - 1))
+    for s in range(nsets):
+        b = s * m
+        stems = rng.integers(98, 123, (40, 8)).astype(np.uint8)
+        rows[b:b + m // 2, :8] = stems[rng.integers(0, 40, m // 2)]
+        rows[b:b + m] = rows[b + rng.permutation(m)]
+        h = mix64(np.uint64(0x5EED5EED) ^ (np.uint64(b) << np.uint64(21)) ^ np.arange(samples, dtype=np.uint64))
+        at = b + ((h >> np.uint64(32)) * np.uint64(m) >> np.uint64(32)).astype(np.int64)
+        rows[at, 0] = 97
+        rows[at[::2], :8] = 97
+    cut = rng.integers(0, 10, n)      # strings of 10 to 19 characters
+    rows[np.arange(width)[None, :] >= width - 1 - cut[:, None]] = 0
+    arena = np.concatenate([rows.reshape(-1), np.zeros(16, np.uint8)])
+    return arena, np.arange(n, dtype=np.uint64) * np.uint64(width), np.arange(nsets + 1, dtype=np.uint64) * np.uint64(m)
+
+
+def test_host_finishes_a_round_with_a_chained_level(ps5, oracle, monkeypatch):
+    """one level planned on the device leaves 4 M strings and more in large
+    segments: the host's next level chains the one after it, while leaves of
+    both earlier levels are listed, each of which is finished once"""
+    nsets, m, leaf_target, oversample = 112, 45000, 64, 2
+    samples = 1023 * oversample       # 2^10 buckets, the depth that 45000 / 64 asks for
+    arena, offs, first = unlucky_sets(nsets, m, samples, 5)
+    stats = {}
+    for chain in ("1", "0"):
+        monkeypatch.setenv("PS5_CHAIN_LEVELS", chain)
+        c = ps5.Context(0)
+        try:
+            c.set_planning(1)
+            c.set_tuning(leaf_target, 10, oversample)
+            perm, lcp = c.sort_batch(arena, offs, first)
+            stats[chain] = c.work_stats()
+        finally:
+            c.close()
+        for k in range(nsets):
+            b, e = int(first[k]), int(first[k + 1])
+            r, msg = oracle.verify(arena, offs[b:e].astype(np.uint32), perm[b:e], lcp[b:e])
+            assert r == 0, (chain, k, msg)
+    # (the host chains a level where it finds, without chaining, none left)
+    assert stats["1"]["levels"] == stats["0"]["levels"] + 1, stats
