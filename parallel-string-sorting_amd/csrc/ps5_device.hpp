@@ -161,12 +161,13 @@ __device__ __forceinline__ uint32_t chars_before_nul(const Chars24& c)
 }
 
 // The packed key of c under the code table lut (LDS: 0 for the NUL, 1.. for
-// the alphabet, 0x81 for anything else).  *bad is set when a character of
-// the key is outside the alphabet.  BITS code bits, BITS * 7 or more of them
-// per 32-bit word, so that a character costs a byte extract, a table read
-// and a shift-or.
+// the alphabet, 0x81 for anything else).  A character of the key outside the
+// alphabet goes into the bitmap *unknown (global memory, shared with other
+// workgroups) and sets *bad.  BITS code bits, BITS * 7 or more of them per
+// 32-bit word, so that a character costs a byte extract, a table read and a
+// shift-or.
 template <int BITS>
-__device__ __forceinline__ key64 pack_key(const Chars24& c, const uint8_t* lut, bool* bad)
+__device__ __forceinline__ key64 pack_key(const Chars24& c, const uint8_t* lut, uint32_t* unknown, bool* bad)
 {
     constexpr int kPerWord = BITS == 3 ? 10 : BITS == 4 ? 8 : 6;
     constexpr int kChars = BITS == 3 ? 21 : BITS == 4 ? 16 : 12;
@@ -186,8 +187,13 @@ __device__ __forceinline__ key64 pack_key(const Chars24& c, const uint8_t* lut, 
         k = 0;
         for (int i = 0; i < kChars && i < (int)len; ++i) {
             const uint64_t w = i < 8 ? c.w[0] : i < 16 ? c.w[1] : c.w[2];
-            const uint32_t code = lut[(uint32_t)(w >> (8 * (i & 7))) & 0xFFu];
-            if (code & 0x80u) *bad = true;
+            const uint32_t ch = (uint32_t)(w >> (8 * (i & 7))) & 0xFFu, code = lut[ch];
+            if (code & 0x80u) {
+                *bad = true;
+                uint32_t* word = unknown + (ch >> 5);
+                const uint32_t bit = 1u << (ch & 31);
+                if (!(__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit)) atomicOr(word, bit);
+            }
             k |= (key64)(code & 0x1Fu) << (64 - (i + 1) * BITS);
         }
         return k;
@@ -195,9 +201,10 @@ __device__ __forceinline__ key64 pack_key(const Chars24& c, const uint8_t* lut, 
     if (len < (uint32_t)kChars) k = len ? k & (~0ull << (64 - len * BITS)) : 0ull;
     return k;
 }
-__device__ __forceinline__ key64 pack_key_fmt(const Chars24& c, uint32_t fmt, const uint8_t* lut, bool* bad)
+__device__ __forceinline__ key64 pack_key_fmt(const Chars24& c, uint32_t fmt, const uint8_t* lut, uint32_t* unknown, bool* bad)
 {
-    return fmt == 1 ? pack_key<3>(c, lut, bad) : fmt == 2 ? pack_key<4>(c, lut, bad) : pack_key<5>(c, lut, bad);
+    return fmt == 1 ? pack_key<3>(c, lut, unknown, bad)
+         : fmt == 2 ? pack_key<4>(c, lut, unknown, bad) : pack_key<5>(c, lut, unknown, bad);
 }
 
 // tid_x() through an opaque move: values derived from it are recomputed

@@ -122,6 +122,7 @@ constexpr uint32_t ERR_CAP = 1u, ERR_LCP = 2u, ERR_BOUNDS = 4u;
 constexpr uint32_t ERR_LEVELS = 8u;          // a captured round had more levels than it was built with
 constexpr uint32_t ERR_ALPHA = 16u;          // a packed root holds a character outside the alphabet its samples showed
 constexpr uint32_t kLutBytes = 256;          // code table of one packed root
+constexpr uint32_t kRootCode = kLutBytes + 32;     // the table, then the alphabet as a bitmap
 
 // Formats of a key.  Format 0: 8 characters of 8 bits.  Formats 1..3: codes
 // of 3, 4 or 5 bits, 21, 16 or 12 characters (code 0 is the NUL, the
@@ -206,7 +207,9 @@ struct Bufs {
     uint32_t pending_err;      // ... and that is an error (ERR_LEVELS: a captured graph cannot continue the round)
     const uint32_t* sdepth_in; // depths of this round's segments (null in round 0: depth 0)
     uint32_t* sdepth_out;      // depths of the next round's segments
-    uint8_t* lut;              // code tables of packed roots, kLutBytes per large segment; null: every key has format 0
+    uint8_t* lut;              // code tables and alphabets of packed roots, kRootCode bytes per large segment; null: every
+                               // key has format 0
+    uint32_t widen;            // non-zero: a root's alphabet is the one in lut, not that of its samples
     uint32_t leaf_keys;        // keys (8 characters each) a leaf pass fetches per string at a time, 1..8
 };
 

@@ -301,11 +301,14 @@ __global__ __launch_bounds__(kBigWG) void k_plan(PlanArgs A, uint32_t* cnt)
 // strings again.  When the samples say that a key would be shared by
 // kPackRun strings or more beside its own (d equal neighbours among s sorted
 // samples of n strings: 2 d n / s^2 strings for each key, one of them the
-// string itself, drawn twice) and the
-// characters of a second sample form an alphabet of at most 31, the root's
-// keys hold 21, 16 or 12 packed characters instead.  A character the sample
-// missed is found by the extraction (ERR_ALPHA) and the sort starts over
-// unpacked.
+// string itself, drawn twice) and the sampled strings' first 24 characters
+// form an alphabet of at most 31, the root's keys hold 21, 16 or 12 packed
+// characters instead.  A character that the samples do not show is found by
+// the extraction (ERR_ALPHA), which adds it to the root's alphabet in B.lut;
+// no children are listed then, and the sort starts over with the alphabets
+// found (B.widen; plain keys where one has more than 31 characters).  20 M
+// windows of 100 characters: 1.48 ms, with an N in 10^6 characters 2.00 (4.0 when
+// the whole sort started over with plain keys, 2.97 with plain keys alone).
 
 // what the kernels of a level know of its segments' strings: buckets of the
 // level before, roots with plain keys, roots that may pack theirs, or
@@ -314,35 +317,12 @@ constexpr int kFromRuns = 0, kRootPlain = 1, kRootPack = 2, kFromPerm = 3;
 
 struct TreeLds {
     key64 samp[kMaxSamples + 1];      // + 1: a merge step reads the slot after the one it takes
-    uint32_t alpha[8];                // characters of the sample
+    uint32_t alpha[8];                // the alphabet
     uint32_t dups;                    // equal neighbours among the sorted samples
-    uint8_t lut[kLutBytes];           // code table
+    uint8_t lut[kLutBytes];           // characters seen, then the code table
 };
 constexpr float kPackRun = 1.0f;
-constexpr uint32_t kAlphaSamples = 256;
-
-// the alphabet of one string per thread, as a bitmap in S.alpha (cleared by the caller)
-__device__ __forceinline__ void sample_alphabet(const Item& seg, const Bufs& B, uint64_t seed, uint32_t* alpha)
-{
-    const uint64_t h = mix64(seed ^ 0xA1FABE7ull ^ ((uint64_t)seg.begin << 21) ^ ((uint64_t)tid_x() << 40));
-    const uint32_t pos = seg.begin + (uint32_t)(((h >> 32) * (uint64_t)seg.size) >> 32);
-    const Chars24 c = load_chars24(B.arena, B.alen, str_off(B, pos));
-    const uint32_t len = chars_before_nul(c);
-    uint32_t m[8] = {};
-#pragma unroll
-    for (int i = 0; i < 24; ++i) {
-        const uint32_t ch = (uint32_t)(c.w[i / 8] >> (8 * (i & 7))) & 0xFFu;
-        const uint32_t bit = (uint32_t)i < len ? 1u << (ch & 31) : 0u;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) m[j] |= (ch >> 5) == (uint32_t)j ? bit : 0u;
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) m[j] |= (uint32_t)__shfl_xor((int)m[j], d, 64);
-        if (lane_id() == 0 && m[j]) atomicOr(&alpha[j], m[j]);
-    }
-}
+constexpr uint32_t kMaxAlphabet = 31;       // five code bits
 
 template <int SRC>
 __device__ __forceinline__ void tree_of_segment(LargeDesc* Dp, uint32_t si, const Bufs& B, uint64_t seed, key64* tree,
@@ -374,8 +354,8 @@ __device__ __forceinline__ void tree_of_segment(LargeDesc* Dp, uint32_t si, cons
     const bool act = o < P;
     constexpr bool may_pack = SRC == kRootPack;
     if (may_pack) {     // (cleared before the merge rounds' barriers)
-        if (tid_x() < 8) S.alpha[tid_x()] = 0;
-        if (tid_x() == 8) S.dups = 0;
+        if (tid_x() < kLutBytes / 4) reinterpret_cast<uint32_t*>(S.lut)[tid_x()] = 0;
+        if (tid_x() == kLutBytes / 4) S.dups = 0;
     }
     auto sample = [&](uint32_t j) {
         const uint64_t h = mix64(seed ^ ((uint64_t)seg.begin << 21) ^ (uint64_t)j);
@@ -477,12 +457,31 @@ __device__ __forceinline__ void tree_of_segment(LargeDesc* Dp, uint32_t si, cons
         __syncthreads();
         const uint32_t dups = S.dups;
         if (dups < 16 || 2.0f * (float)dups * (float)seg.size < (1.0f + kPackRun) * (float)ss * (float)ss) break;     // (uniform)
-        if (tid_x() < kAlphaSamples) sample_alphabet(seg, B, seed, S.alpha);     // (whole waves)
+        uint8_t* code_out = B.lut + (uint64_t)si * kRootCode;
+        uint32_t* alpha_out = reinterpret_cast<uint32_t*>(code_out + kLutBytes);
+        if (B.widen) {     // (uniform)
+            if (tid_x() < kLutBytes) S.lut[tid_x()] = (uint8_t)((alpha_out[tid_x() / 32] >> (tid_x() & 31)) & 1u);
+        } else if (act) {
+#pragma unroll 1
+            for (uint32_t j = o; j < o + kPer && j < ss; ++j) {
+                const Chars24 c = load_chars24(B.arena, B.alen, str_off(B, sample(j)));
+                const uint32_t len = chars_before_nul(c);
+#pragma unroll
+                for (int i = 0; i < 24; ++i)
+                    if ((uint32_t)i < len) S.lut[(uint32_t)(c.w[i / 8] >> (8 * (i & 7))) & 0xFFu] = 1;
+            }
+        }
         __syncthreads();
+        if (tid_x() < kLutBytes) {     // (whole waves)
+            const uint64_t seen = __ballot(S.lut[tid_x()] != 0);
+            if ((tid_x() & 31) == 0) S.alpha[tid_x() / 32] = (uint32_t)(seen >> (tid_x() & 32));
+        }
+        __syncthreads();
+        if (tid_x() < 8) alpha_out[tid_x()] = S.alpha[tid_x()];
         uint32_t sigma = 0;
 #pragma unroll
         for (int j = 0; j < 8; ++j) sigma += (uint32_t)__popc(S.alpha[j]);
-        fmt = sigma <= 7 ? 1u : sigma <= 15 ? 2u : sigma <= 31 ? 3u : 0u;
+        fmt = sigma <= 7 ? 1u : sigma <= 15 ? 2u : sigma <= kMaxAlphabet ? 3u : 0u;
         if (fmt == 0) break;     // (uniform)
         if (tid_x() < kLutBytes) {
             const uint32_t c = tid_x();
@@ -491,7 +490,7 @@ __device__ __forceinline__ void tree_of_segment(LargeDesc* Dp, uint32_t si, cons
             rank += (uint32_t)__popc(S.alpha[c / 32] & ((1u << (c & 31)) - 1));
             const uint32_t code = c == 0 ? 0u : (S.alpha[c / 32] >> (c & 31)) & 1u ? rank : 0x81u;
             S.lut[c] = (uint8_t)code;
-            B.lut[(uint64_t)si * kLutBytes + c] = (uint8_t)code;
+            code_out[c] = (uint8_t)code;
         }
         __syncthreads();
         // the same samples with packed keys (a rolled loop: this code runs in
@@ -499,8 +498,9 @@ __device__ __forceinline__ void tree_of_segment(LargeDesc* Dp, uint32_t si, cons
         if (act) {
 #pragma unroll 1
             for (uint32_t j = o; j < o + kPer; ++j) {
-                bool bad = false;     // (the extraction flags it; any splitters do)
-                s_samp[j] = j < ss ? pack_key_fmt(load_chars24(B.arena, B.alen, str_off(B, sample(j))), fmt, S.lut, &bad)
+                bool bad = false;     // (the alphabet holds the samples' characters)
+                s_samp[j] = j < ss ? pack_key_fmt(load_chars24(B.arena, B.alen, str_off(B, sample(j))), fmt, S.lut,
+                                                  alpha_out, &bad)
                                    : ~0ull;
             }
 #pragma unroll
@@ -747,8 +747,24 @@ __device__ __forceinline__ void part_chunk(uint32_t ti, const Plan& P, const Buf
         static_assert(kPartWaves * kH * 64 * 8 <= L::kCntOff && kE % kH == 0, "the groups' keys fit the stage");
         key64* s_w = reinterpret_cast<key64*>(smem + L::kStageOff) + w * kH * 64;
         __syncthreads();
-        if (tid < kLutBytes) s_lut[tid] = B.lut[(uint64_t)tr.seg * kLutBytes + tid];
+        uint8_t* code = B.lut + (uint64_t)tr.seg * kRootCode;
+        uint32_t* unknown = reinterpret_cast<uint32_t*>(code + kLutBytes);
+        if (tid < kLutBytes) s_lut[tid] = code[tid];
+        // once a character is missing, the sort starts over: the other chunks
+        // only complete the alphabet, or do nothing when it is already too
+        // large to pack
+        if (tid == 0) {
+            uint32_t over = __hip_atomic_load(&B.cnt[C_ERR], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ERR_ALPHA;
+            if (over) {
+                uint32_t sigma = 0;
+                for (int j = 0; j < 8; ++j)
+                    sigma += (uint32_t)__popc(__hip_atomic_load(unknown + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                if (sigma > kMaxAlphabet) over = ~0u;
+            }
+            s_tmp[15] = over;
+        }
         __syncthreads();
+        if (s_tmp[15] == ~0u) return;     // (uniform)
         bool bad = false;
 #pragma unroll
         for (int e0 = 0; e0 < kE; e0 += kH) {
@@ -760,13 +776,14 @@ __device__ __forceinline__ void part_chunk(uint32_t ti, const Plan& P, const Buf
 #pragma unroll 2
             for (int j = 0; j < kH; ++j) {
                 const uint32_t q = min(wb + (e0 + j) * 64 + lane, m - 1);
-                s_w[j * 64 + lane] =
-                    pack_key_fmt(load_chars24(B.arena, B.alen, str_off(B, seg.begin + cb + q)), fmt, s_lut, &bad);
+                s_w[j * 64 + lane] = pack_key_fmt(load_chars24(B.arena, B.alen, str_off(B, seg.begin + cb + q)), fmt,
+                                                  s_lut, unknown, &bad);
             }
 #pragma unroll
             for (int j = 0; j < kH; ++j) kv[e0 + j] = s_w[j * 64 + lane];
         }
         if (bad) flag_error(B.cnt, ERR_ALPHA);
+        if (s_tmp[15]) return;     // (uniform)
         __syncthreads();     // the table is read
         if (tid < kLutBytes / 4) reinterpret_cast<uint32_t*>(s_cnt)[tid] = 0;
     }
@@ -906,10 +923,18 @@ __global__ __launch_bounds__(kPartThreads, 4) void k_part(Plan P, Bufs B, const 
     }
 }
 
+// a packed root met a character outside its alphabet: nothing of the level is
+// of use, and without children no later one finds any work
+__device__ __forceinline__ bool starts_over(const Bufs& B)
+{
+    return B.lut && (load_uniform(B.cnt + C_ERR) & ERR_ALPHA);
+}
+
 // Bucket counts summed over groups of kHistGroup chunks (segments of more
 // than one group): row 1 + g of the segment's gsum.
 __global__ __launch_bounds__(kWG) void k_hist_sum(Plan P, Bufs B)
 {
+    if (starts_over(B)) return;
     const uint32_t ng = P.hdr->ngroups;
     for (uint32_t gi = blockIdx.x; gi < ng; gi += gridDim.x) {
         const TileRef gr = load_uniform(P.groups + gi);
@@ -922,7 +947,7 @@ __global__ __launch_bounds__(kWG) void k_hist_sum(Plan P, Bufs B)
             uint32_t s = 0;
 #pragma unroll 8
             for (uint32_t c = c0; c < c1; ++c) s += h[(uint64_t)c * nbs + b] & 0xFFFFu;
-                B.gsum[D.gbase + (1 + gr.t) * nbs + b] = s;
+            B.gsum[D.gbase + (1 + gr.t) * nbs + b] = s;
         }
     }
 }
@@ -935,6 +960,7 @@ __global__ __launch_bounds__(kWG) void k_hist_runs(Plan P, Bufs B, int buf)
 {
     __shared__ uint32_t s_h[64][65];
     static_assert(kHistGroup == 64, "a lane per chunk of a group");
+    if (starts_over(B)) return;
     const uint32_t ng = P.hdr->ngroups;
     uint32_t* V = B.vpos + (buf ? B.cap_h : 0ull);
     uint32_t* S = B.src + (buf ? B.cap_h : 0ull);
@@ -1072,6 +1098,7 @@ __global__ __launch_bounds__(kBigWG) void k_children(Plan P, Bufs B, const key64
 {
     __shared__ uint32_t s_sz[kMaxBkt + 1];
     __shared__ uint32_t s_tmp[kBigWaves * kChildLists + 8];     // the scans' scratch, then the lists' bases
+    if (starts_over(B)) return;
     const uint32_t nlarge = P.hdr->nlarge;
     for (uint32_t si = blockIdx.x; si < nlarge; si += gridDim.x) {
         const LargeDesc D = load_uniform(P.desc + si);
@@ -2714,7 +2741,7 @@ struct WorkBuffers {
     uint64_t tiles_cap = 0, groups_cap = 0;
     key64* trees = nullptr;          // kTreeSlots splitter slots per large segment
     uint64_t trees_cap = 0;
-    uint8_t* lut = nullptr;          // kLutBytes per large segment (trees_cap of them)
+    uint8_t* lut = nullptr;          // kRootCode bytes per large segment (trees_cap of them)
     // bucket counts of a level (hist_cap entries), their group sums, and the
     // run tables (hist_cap entries for each of the two buffers)
     uint32_t* hist = nullptr;
@@ -2892,7 +2919,7 @@ int ensure_tables(ps5_ctx* c)
         c->w.lut = nullptr;
         c->w.trees_cap = 0;
         HIPCHK(hipMalloc(&c->w.trees, (uint64_t)c->w.cap_large * kTreeSlots * sizeof(key64)));
-        HIPCHK(hipMalloc(&c->w.lut, (uint64_t)c->w.cap_large * kLutBytes));
+        HIPCHK(hipMalloc(&c->w.lut, (uint64_t)c->w.cap_large * kRootCode));
         c->w.trees_cap = c->w.cap_large;
         c->w_gen++;
     }
@@ -2984,7 +3011,7 @@ constexpr ScratchLayout scratch_layout(uint64_t cap)
     L.desc = take(plan_bytes_of(cap));
     L.trees_cap = cl;
     L.trees = take(L.trees_cap * kTreeSlots * sizeof(key64));
-    L.lut = take(L.trees_cap * kLutBytes);
+    L.lut = take(L.trees_cap * kRootCode);
     L.hist_cap = hist_cap_of(cap, kChunkMin, kMinTiles);
     L.hist = take(L.hist_cap * sizeof(uint32_t));
     L.vpos = take(2 * L.hist_cap * sizeof(uint32_t));
@@ -3155,8 +3182,8 @@ int wait_stage(ps5_ctx* c, uint32_t seq)
 }
 
 // (not a status of the ABI) the sort's packed keys met a character outside
-// their alphabet: run_sort starts over with plain keys
-constexpr int kUnpack = -1;
+// their alphabet: run_sort starts over
+constexpr int kStartOver = -1;
 
 int readback(ps5_ctx* c, const Item* list, int ci)
 {
@@ -3169,7 +3196,7 @@ int readback(ps5_ctx* c, const Item* list, int ci)
     if (rc) return rc;
     c->st_syncs++;
     memcpy(c->h_cnt, c->h_stage, C_NCNT * sizeof(uint32_t));
-    if (c->h_cnt[C_ERR] & ERR_ALPHA) return kUnpack;
+    if (c->h_cnt[C_ERR] & ERR_ALPHA) return kStartOver;
     if (c->h_cnt[C_ERR] & ERR_CAP) return set_err(PS5_ERR_CAPACITY, "work list capacity exceeded");
     if (c->h_cnt[C_ERR] & ERR_LCP) return set_err(PS5_ERR_INTERNAL, "equal keys across a leaf boundary");
     if (c->h_cnt[C_ERR] & ERR_BOUNDS) return set_err(PS5_ERR_INTERNAL, "device bounds check failed");
@@ -4090,8 +4117,12 @@ void graph_round(ps5_ctx* c, SortRun& R, uint32_t round, uint32_t L, uint32_t nl
     if (B.lcp) launch_leafbound(c, B, rp, (uint32_t)std::min<uint64_t>(kDevBoundWgs, div_up(n, kWG)), n);
 }
 
+// How a sort's roots choose their keys: plain, packed as their samples say, or
+// packed with the alphabets that a sort with kPackSampled found.
+enum Packing { kPackNone, kPackSampled, kPackWidened };
+
 int run_sort_keys(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_t* offs, const uint64_t* offs64,
-                  uint32_t n, uint32_t* perm, uint32_t* lcp, const uint64_t* set_first, uint32_t nsets, bool pack)
+                  uint32_t n, uint32_t* perm, uint32_t* lcp, const uint64_t* set_first, uint32_t nsets, Packing pack)
 {
     int rc = ensure_capacity(c, n);
     if (!rc) rc = ensure_tables(c);
@@ -4123,6 +4154,7 @@ int run_sort_keys(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_
     B.leaf_keys = c->leaf_keys;
     set_depths(c, B, 0);
     B.lut = nullptr;
+    B.widen = pack == kPackWidened;
 
     // the roots (one, or a batch's sets) and their sizes
     uint32_t root_kmax = 1;                     // largest treebits of a large root
@@ -4156,7 +4188,7 @@ int run_sort_keys(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_
     } else if ((rc = setup_roots(c, n, set_first, nsets))) {
         return rc;
     }
-    if (pack && root_max >= kPackMin) B.lut = c->w.lut;     // large roots may pack their keys
+    if (pack != kPackNone && root_max >= kPackMin) B.lut = c->w.lut;     // large roots may pack their keys
     SortRun R{ B, n, alen, root_kmax, root_max, root_sum };
     uint32_t start = 0;
     if (c->graph_rounds && !c->profile) {
@@ -4239,13 +4271,15 @@ int run_sort(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_t* of
              uint32_t n, uint32_t* perm, uint32_t* lcp, const uint64_t* set_first, uint32_t nsets)
 {
     const bool graph = c->graph_rounds && !c->profile;
-    int rc = run_sort_keys(c, arena, alen, offs, offs64, n, perm, lcp, set_first, nsets, !graph);
-    if (rc != kUnpack) return rc;
+    int rc = run_sort_keys(c, arena, alen, offs, offs64, n, perm, lcp, set_first, nsets, graph ? kPackNone : kPackSampled);
+    if (rc != kStartOver) return rc;
     HIPCHK(hipStreamSynchronize(c->side));
     HIPCHK(hipStreamSynchronize(c->stream));
     if (c->profile) collect_events(c);
-    rc = run_sort_keys(c, arena, alen, offs, offs64, n, perm, lcp, set_first, nsets, false);
-    return rc == kUnpack ? set_err(PS5_ERR_INTERNAL, "plain keys flagged as packed") : rc;
+    // (every root's level saw all of its strings, so this finds no other character)
+    if (c->trace) fprintf(stderr, "[ps5] a packed root met a character outside its alphabet: starting over\n");
+    rc = run_sort_keys(c, arena, alen, offs, offs64, n, perm, lcp, set_first, nsets, kPackWidened);
+    return rc == kStartOver ? set_err(PS5_ERR_INTERNAL, "a packed key outside its whole root's alphabet") : rc;
 }
 
 }  // namespace

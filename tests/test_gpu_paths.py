@@ -300,3 +300,27 @@ def test_host_finishes_a_round_with_a_chained_level(ps5, oracle, monkeypatch):
             assert r == 0, (chain, k, msg)
     # (the host chains a level where it finds, without chaining, none left)
     assert stats["1"]["levels"] == stats["0"]["levels"] + 1, stats
+
+
+@pytest.mark.parametrize("known, others, as_sigma", [
+    (4, 1, 5), (4, 3, 7), (4, 4, 8), (7, 1, 8), (4, 11, 15), (4, 12, 16), (15, 1, 16), (20, 11, 31), (4, 28, 32), (31, 1, 32), (4, 200, 204)])
+def test_packed_root_with_a_wider_alphabet(ctx, oracle, known, others, as_sigma):
+    """characters outside the samples' alphabet, each in one string only: the
+    sort starts over with the alphabet of all, and is split as if the samples
+    had shown it (plain keys from 32 characters on)"""
+    n, hi = 1060000, 60
+    arena, offs = packed_case(known, n, 17 * known + others, hi=hi)
+    rng = np.random.default_rng(others)
+    used = np.unique(arena)
+    unused = np.setdiff1d(np.arange(1, 256), used).astype(np.uint8)
+    offs64 = offs.astype(np.int64)
+    long = np.flatnonzero(np.diff(np.append(offs64, arena.size - 16)) > 12)
+    at = offs64[rng.choice(long, others, replace=False)] + rng.integers(0, 9, others)
+    arena[at] = rng.choice(unused, others, replace=False)
+    check(ctx, oracle, arena, offs)
+    rounds = ctx.work_stats()["rounds"]
+    check(ctx, oracle, arena, offs, with_lcp=False)
+    # the same strings' shape where every character is frequent
+    common, common_offs = packed_case(as_sigma, n, 17 * known + others, hi=hi)
+    ctx.sort(common, common_offs)
+    assert rounds == ctx.work_stats()["rounds"], ctx.work_stats()
