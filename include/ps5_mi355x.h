@@ -119,7 +119,7 @@ int ps5_sort_device(ps5_ctx* ctx, const uint8_t* d_arena, uint64_t arena_bytes,
  * it is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Arguments
  * and results are those of ps5_sort_device; the work buffers come from a
- * static device array of 128 MiB that every GPU the library runs on holds
+ * static device array of 104 MiB that every GPU the library runs on holds
  * (one copy per GPU and process) until the process ends, so n is limited to
  * ps5_noalloc_max_strings() (2^20); a larger n is rejected with
  * PS5_ERR_ARG.  The call makes no hipMalloc/hipFree or other allocating call

@@ -288,7 +288,12 @@ __device__ __forceinline__ void flag_error(uint32_t* cnt, uint32_t e) { atomicOr
 // characters the strings of the round segment that starts at rbeg share
 __device__ __forceinline__ uint32_t seg_depth(const Bufs& B, uint32_t rbeg)
 {
-    return B.sdepth_in ? B.sdepth_in[rbeg] : 0u;
+    return B.sdepth_in ? B.sdepth_in[rbeg >> kDepthShift] : 0u;
+}
+// the same of a leaf of at most kTinyT strings
+__device__ __forceinline__ uint32_t tiny_depth(const Bufs& B, const Item& it)
+{
+    return it.flags & F_NEXT ? it.row : seg_depth(B, it.rbeg);
 }
 
 // byte offset of input string i in the arena

@@ -14,8 +14,8 @@
 //              first sorted position and the place in rec of the bucket's
 //              strings in that chunk (its run), bucket-major
 //   bkey[n]    uint64 scratch: depth key of the first/last position of a leaf
-//   sdepth[2][n] uint32 by round parity: characters the strings of the round
-//              segment starting at a position are known to share
+//   sdepth[2][n / 64] uint32 by round parity: characters the strings of the
+//              round segment starting at a position are known to share
 //   perm[n], lcp[n]  results (caller memory); between rounds perm holds the
 //              input indices of the strings that continue
 //
@@ -49,7 +49,8 @@ constexpr int kMaxTreebits = 10;             // reference DefaultTreebits
 constexpr int kMaxSpl = (1 << kMaxTreebits) - 1;    // 1023 splitters
 constexpr int kMaxBkt = 2 * kMaxSpl + 1;            // 2047 buckets
 constexpr int kMaxSamples = 4096;            // sample keys of one splitter tree
-constexpr uint32_t kTreeSlots = 2048;        // per segment: level-order tree [0,1024), sorted splitters [1024,2048)
+// A segment's splitters in `trees`, from its gbase on: the level-order tree in
+// [0, 1 << k), the sorted splitters in [1 << k, 2 << k).
 // A large segment is cut into the fewest equal chunks of at most a per-level
 // limit of keys: kPartMax, unless the level is too small to give min_tiles
 // chunks that way; then the limit shrinks (not below kChunkMin) so small
@@ -72,6 +73,8 @@ constexpr uint32_t kHistGroup = 64;          // chunks whose bucket counts are s
 constexpr uint32_t kShapeChunkMax = 9216, kShapeChunkMaxRoot = 12032;
 constexpr uint32_t kMinTiles = 512;
 constexpr uint32_t kTinyT = 64;              // leaves sorted by one wave
+constexpr uint32_t kDepthShift = 6;          // a slot of sdepth per kTinyT positions
+static_assert(1u << kDepthShift == kTinyT, "segments of more than kTinyT strings start in slots of their own");
 constexpr uint32_t kBlkT = 2048;             // leaves sorted on chip by one workgroup
 constexpr uint32_t kMaxLeafTarget = 1024;    // largest leaf size the fan-out aims at
 constexpr uint32_t kRunChunk = 4096;         // equal-key leaves are processed in chunks
@@ -90,7 +93,8 @@ struct Item {            // a segment or a leaf
     uint32_t size;       // number of positions
     uint32_t rbeg;       // first position of the round segment it belongs to
     uint32_t flags;      // F_* | key format << kFmtShift | chunk index << kFlagShift
-    uint32_t row, nch;   // a bucket: its first entry in vpos/src and its runs (one per chunk of its segment)
+    uint32_t row, nch;   // a bucket: its first entry in vpos/src and its runs (one per chunk of its segment); row of a
+                         // tiny F_NEXT segment: its depth
 };
 // Where a segment's strings are found: F_IDENT (a root: the string at position
 // p is input string p) and F_NEXT (a segment of an earlier round: perm[p]) say
@@ -149,7 +153,8 @@ struct LargeDesc {       // one segment of the multi-workgroup sample-sort step
     uint32_t chunk;      // keys per chunk (the last one may be short), <= kPartMax
     uint32_t hist_base;  // first entry of this segment's bucket counts (chunk-major, 2 << k per chunk) and of
                          // its vpos/src rows (bucket-major, nch per bucket)
-    uint32_t gbase;      // first entry of its group sums: a row of 2 << k first positions, then a row per group
+    uint32_t gbase;      // first entry of its group sums: a row of 2 << k first positions, then a row per group; and
+                         // of its splitters
     uint32_t k;          // treebits
     uint32_t oversample; // sample keys per splitter
 };
@@ -205,8 +210,11 @@ struct Bufs {
     uint32_t* gsum;      // their sums over groups of chunks
     const uint32_t* pending;   // non-null and non-zero: large segments remain, the round's leaves wait
     uint32_t pending_err;      // ... and that is an error (ERR_LEVELS: a captured graph cannot continue the round)
-    const uint32_t* sdepth_in; // depths of this round's segments (null in round 0: depth 0)
-    uint32_t* sdepth_out;      // depths of the next round's segments
+    // depths of the segments of more than kTinyT strings that start in each
+    // kTinyT positions (at most one does): this round's (null in round 0:
+    // depth 0) and the next round's
+    const uint32_t* sdepth_in;
+    uint32_t* sdepth_out;
     uint8_t* lut;              // code tables and alphabets of packed roots, kRootCode bytes per large segment; null: every
                                // key has format 0
     uint32_t widen;            // non-zero: a root's alphabet is the one in lut, not that of its samples

@@ -183,7 +183,7 @@ struct PlanArgs {
     int ci;                  // their counter
     uint32_t cap_large;      // capacity of that list
     unsigned char* plan;     // header, descriptors, tables (at tiles_off and groups_off)
-    uint64_t tiles_off, tiles_cap, groups_off, groups_cap, hist_cap, gsum_cap, trees_cap;
+    uint64_t tiles_off, tiles_cap, groups_off, groups_cap, hist_cap, gsum_cap;
     uint32_t leaf_target, max_treebits, max_oversample;
     uint32_t chunk_max, chunk_max_root, min_tiles;    // chunk shapes (ps5_ctx_set_shape)
     uint32_t kmax;           // bound of the level's launches (treebits are clamped to it)
@@ -282,7 +282,7 @@ __global__ __launch_bounds__(kBigWG) void k_plan(PlanArgs A, uint32_t* cnt)
         scarry += stot;
     }
     const bool fits = tcarry <= A.tiles_cap && gcarry <= A.groups_cap && hcarry <= A.hist_cap && scarry <= A.gsum_cap &&
-                      hcarry <= 0xFFFFFFFFull && nl <= A.trees_cap;
+                      hcarry <= 0xFFFFFFFFull;
     if (!fits && tid == 0) flag_error(cnt, ERR_CAP);
     if (tid == 0) *hdr = LevelHdr{ fits ? nl : 0u, fits ? tcarry : 0u, fits ? gcarry : 0u, s_kmax, { 0u, 0u, 0u, 0u } };
 }
@@ -292,8 +292,8 @@ __global__ __launch_bounds__(kBigWG) void k_plan(PlanArgs A, uint32_t* cnt)
 // sorting network, then merge-path rounds in LDS); splitter i is sample
 // oversample/2 + oversample*i (the reference's choice for oversample factor 2,
 // bingmann-sample_sort_tree_builder.hpp:44-58) and the tree is stored in
-// level order: trees[seg*2048 + t], t = 1..nspl, followed by the splitters in
-// sorted order at trees[seg*2048 + 1024 + i], i < nspl.
+// level order: trees[gbase + t], t = 1..nspl, followed by the splitters in
+// sorted order at trees[gbase + (1 << k) + i], i < nspl.
 //
 // A root's samples also choose the format of its keys (KeyFmt).  Eight
 // characters of a small alphabet leave many strings equal: 20 M windows of
@@ -510,7 +510,7 @@ __device__ __forceinline__ void tree_of_segment(LargeDesc* Dp, uint32_t si, cons
     if (fmt && tid_x() == 0) Dp->seg.flags = seg.flags | (fmt << kFmtShift);
     const key64* sorted = s_samp;
     for (int t = tid_x() + 1; t <= nspl; t += kBigWG) tree[t] = sorted[a / 2 + a * inorder_of(t, k)];
-    for (int i = tid_x(); i < nspl; i += kBigWG) tree[1024 + i] = sorted[a / 2 + a * i];
+    for (int i = tid_x(); i < nspl; i += kBigWG) tree[nspl + 1 + i] = sorted[a / 2 + a * i];
 }
 
 template <int SRC>
@@ -520,7 +520,7 @@ __global__ __launch_bounds__(kBigWG) void k_tree(Plan P, Bufs B, uint64_t seed, 
     const uint32_t nlarge = P.hdr->nlarge;
     for (uint32_t si = blockIdx.x; si < nlarge; si += gridDim.x) {
         __syncthreads();     // the previous segment's samples are consumed
-        tree_of_segment<SRC>(P.desc + si, si, B, seed, trees + (uint64_t)si * kTreeSlots, S);
+        tree_of_segment<SRC>(P.desc + si, si, B, seed, trees + P.desc[si].gbase, S);
     }
 }
 
@@ -700,7 +700,7 @@ __device__ __forceinline__ void part_chunk(uint32_t ti, const Plan& P, const Buf
     const uint32_t per = ((m + kPartWaves - 1) / kPartWaves + 63) & ~63u;     // positions per wave
     const uint32_t wb = w * per;
     const uint32_t nspl = (1u << k) - 1, nbs = 2u << k;
-    const key64* tree = trees + (uint64_t)tr.seg * kTreeSlots;
+    const key64* tree = trees + D.gbase;
     const uint32_t fmt = SRC == kRootPack ? (seg.flags & kFmtMask) >> kFmtShift : 0u;
     key64 kv[kE];
     uint32_t iv[kE];        // (indices; a root's are its positions)
@@ -1066,7 +1066,7 @@ __device__ __forceinline__ void emit_children(const LargeDesc& D, uint32_t start
             put_item(s.tiny, s.cap_tiny, o_t++, it, s.cnt);
         } else if (b & 1) {
             const uint32_t nch = (m + kRunChunk - 1) / kRunChunk;
-            sdepth_out[it.begin] = 0xFFFFFFFFu;     // (k_leaf_run's chunks lower it)
+            sdepth_out[it.begin >> kDepthShift] = 0xFFFFFFFFu;     // (k_leaf_run's chunks lower it)
             for (uint32_t c = 0; c < nch; ++c) {
                 Item r = it;
                 r.flags = base_flags | F_SORTED | (c << kFlagShift);
@@ -1170,8 +1170,7 @@ __global__ __launch_bounds__(kBigWG) void k_children(Plan P, Bufs B, const key64
                     }
                 }
             }
-            emit_children(D, start, sz, dst, trees + (uint64_t)si * kTreeSlots + 1024, s,
-                          B.sdepth_out, s_tmp);
+            emit_children(D, start, sz, dst, trees + D.gbase + (1u << D.k), s, B.sdepth_out, s_tmp);
         }
         __syncthreads();     // the LDS is reused by the next segment
     }
@@ -1398,7 +1397,7 @@ __device__ __forceinline__ void tiny_leaf(const Item& L, const Bufs& B, key64* s
     }
     key64 k = ~0ull;
     uint32_t id = 0;
-    const uint32_t depth = seg_depth(B, L.rbeg);
+    const uint32_t depth = tiny_depth(B, L);
     load_tiny(B, L, depth, &k, &id);
     wave_finish_leaf<NK>(B, L.begin + lane, L.size, k, id, depth, key_fmt(L.flags), true, 0u, s_k, s_i, s_r);
 }
@@ -2032,8 +2031,8 @@ __device__ __forceinline__ void block_one(const Item L, const Bufs& B, const Sin
                 }
             }
         } else {
-            Item ni = { beg + i, rl, beg + i, F_NEXT, 0u, 0u };
-            if (nr && !keep) B.sdepth_out[beg + i] = depth + F.cpk;
+            Item ni = { beg + i, rl, beg + i, F_NEXT, depth + F.cpk, 0u };
+            if (nr && !small) B.sdepth_out[(beg + i) >> kDepthShift] = depth + F.cpk;
             wave_append_segment(nr && !keep, ni, nxt);
         }
     }
@@ -2194,7 +2193,7 @@ __device__ __forceinline__ void run_chunk(const Item& L, const Bufs& B, const Si
             for (int d = 32; d >= 1; d >>= 1) e = min(e, (uint32_t)__shfl_xor((int)e, d, 64));
             ext = e;     // (of this wave's strings)
         }
-        if (lane == 0) atomicMin(&B.sdepth_out[L.begin], next + ext);
+        if (lane == 0) atomicMin(&B.sdepth_out[L.begin >> kDepthShift], next + ext);
     }
     if (tid_x() < 64) {
         const bool nr = tid_x() == 0 && c == 0 && !term && !single;
@@ -2739,16 +2738,16 @@ struct WorkBuffers {
     unsigned char* h_plan = nullptr;     // pinned, mapped: the host's plans are pulled by k_fetch
     unsigned char* h_plan_dev = nullptr; // its device address
     uint64_t tiles_cap = 0, groups_cap = 0;
-    key64* trees = nullptr;          // kTreeSlots splitter slots per large segment
-    uint64_t trees_cap = 0;
-    uint8_t* lut = nullptr;          // kRootCode bytes per large segment (trees_cap of them)
-    // bucket counts of a level (hist_cap entries), their group sums, and the
-    // run tables (hist_cap entries for each of the two buffers)
+    uint8_t* lut = nullptr;          // kRootCode bytes per large segment (cap_large of them)
+    // bucket counts of a level (hist_cap entries), their group sums and the
+    // segments' splitters (gsum_cap entries each), and the run tables
+    // (hist_cap entries for each of the two buffers)
     uint32_t* hist = nullptr;
     uint32_t* vpos = nullptr;
     uint32_t* src = nullptr;
     uint64_t hist_cap = 0;
     uint32_t* gsum = nullptr;
+    key64* trees = nullptr;
     uint64_t gsum_cap = 0;
 };
 
@@ -2776,6 +2775,7 @@ constexpr uint64_t hist_cap_of(uint64_t cap, uint64_t chunk_max, uint64_t min_ti
     const uint64_t few = cap < kChunkMin * min_tiles ? cap : kChunkMin * min_tiles, many = cap * 2048 / limit;
     return (few > many ? few : many) + cap / 16 + 4096;
 }
+constexpr uint64_t sdepth_cap_of(uint64_t cap) { return (cap >> kDepthShift) + 1; }
 // per bucket its first position and one sum per group of chunks
 constexpr uint64_t gsum_cap_of(uint64_t cap, uint64_t hist_cap) { return hist_cap / kHistGroup + cap / 8 + 8192; }
 // a plan: the level header, cap_large descriptors, the tables of chunks and groups
@@ -2874,6 +2874,8 @@ void free_tables(ps5_ctx* c)
         if (*q) (void)hipFree(*q);
         *q = nullptr;
     }
+    if (c->w.trees) (void)hipFree(c->w.trees);
+    c->w.trees = nullptr;
     c->w.hist_cap = c->w.gsum_cap = 0;
 }
 
@@ -2891,15 +2893,14 @@ void free_buffers(ps5_ctx* c)
         c->w.l_tiny[i] = nullptr; c->w.l_block[i] = nullptr; c->w.l_run[i] = nullptr;
         c->w.sdepth[i] = nullptr;
     }
-    f(c->w.rec); f(c->w.bkey); f(c->w.trees); f(c->w.lut); f(c->w.d_plan);
-    c->w.rec = nullptr; c->w.bkey = nullptr; c->w.trees = nullptr; c->w.lut = nullptr; c->w.d_plan = nullptr;
+    f(c->w.rec); f(c->w.bkey); f(c->w.lut); f(c->w.d_plan);
+    c->w.rec = nullptr; c->w.bkey = nullptr; c->w.lut = nullptr; c->w.d_plan = nullptr;
     free_tables(c);
     if (c->w.h_large) (void)hipHostFree(c->w.h_large);
     if (c->w.h_plan) (void)hipHostFree(c->w.h_plan);
     c->w.h_large = nullptr; c->w.h_plan = nullptr; c->w.h_plan_dev = nullptr;
     c->w.cap = 0;
     c->w.tiles_cap = c->w.groups_cap = 0;
-    c->w.trees_cap = 0;
 }
 
 // The splitter trees, bucket counts and run tables of any level of a sort of
@@ -2910,29 +2911,17 @@ int ensure_tables(ps5_ctx* c)
 {
     const uint64_t hist = hist_cap_of(c->w.cap, std::min(c->chunk_max, c->chunk_max_root), c->min_tiles);
     const uint64_t gsum = gsum_cap_of(c->w.cap, hist);
-    if (c->w.cap_large <= c->w.trees_cap && hist <= c->w.hist_cap && gsum <= c->w.gsum_cap) return PS5_OK;
+    if (hist <= c->w.hist_cap && gsum <= c->w.gsum_cap) return PS5_OK;
     if (c->w.fixed) return set_err(PS5_ERR_CAPACITY, "the scratch holds no tables of this shape");
-    if (c->w.cap_large > c->w.trees_cap) {
-        if (c->w.trees) (void)hipFree(c->w.trees);
-        if (c->w.lut) (void)hipFree(c->w.lut);
-        c->w.trees = nullptr;
-        c->w.lut = nullptr;
-        c->w.trees_cap = 0;
-        HIPCHK(hipMalloc(&c->w.trees, (uint64_t)c->w.cap_large * kTreeSlots * sizeof(key64)));
-        HIPCHK(hipMalloc(&c->w.lut, (uint64_t)c->w.cap_large * kRootCode));
-        c->w.trees_cap = c->w.cap_large;
-        c->w_gen++;
-    }
-    if (hist > c->w.hist_cap || gsum > c->w.gsum_cap) {
-        free_tables(c);
-        HIPCHK(hipMalloc(&c->w.hist, hist * sizeof(uint32_t)));
-        HIPCHK(hipMalloc(&c->w.gsum, gsum * sizeof(uint32_t)));
-        HIPCHK(hipMalloc(&c->w.vpos, 2 * hist * sizeof(uint32_t)));
-        HIPCHK(hipMalloc(&c->w.src, 2 * hist * sizeof(uint32_t)));
-        c->w.hist_cap = hist;
-        c->w.gsum_cap = gsum;
-        c->w_gen++;
-    }
+    free_tables(c);
+    HIPCHK(hipMalloc(&c->w.hist, hist * sizeof(uint32_t)));
+    HIPCHK(hipMalloc(&c->w.gsum, gsum * sizeof(uint32_t)));
+    HIPCHK(hipMalloc(&c->w.trees, gsum * sizeof(key64)));
+    HIPCHK(hipMalloc(&c->w.vpos, 2 * hist * sizeof(uint32_t)));
+    HIPCHK(hipMalloc(&c->w.src, 2 * hist * sizeof(uint32_t)));
+    c->w.hist_cap = hist;
+    c->w.gsum_cap = gsum;
+    c->w_gen++;
     return PS5_OK;
 }
 
@@ -2948,7 +2937,7 @@ int ensure_capacity(ps5_ctx* c, uint64_t n)
     free_buffers(c);
     HIPCHK(hipMalloc(&c->w.rec, 2 * cap * kRecWords * sizeof(uint32_t)));
     HIPCHK(hipMalloc(&c->w.bkey, cap * sizeof(key64)));
-    for (int i = 0; i < 2; ++i) HIPCHK(hipMalloc(&c->w.sdepth[i], cap * sizeof(uint32_t)));
+    for (int i = 0; i < 2; ++i) HIPCHK(hipMalloc(&c->w.sdepth[i], sdepth_cap_of(cap) * sizeof(uint32_t)));
     c->w.cap_large = cap_large_of(cap);
     c->w.cap_block = cap_block_of(cap);
     for (int i = 0; i < 2; ++i) c->w.cap_tiny[i] = cap_tiny_of(cap, i);
@@ -2960,6 +2949,7 @@ int ensure_capacity(ps5_ctx* c, uint64_t n)
         HIPCHK(hipMalloc(&c->w.l_block[i], (uint64_t)kBlkClasses * c->w.cap_block * sizeof(Item)));
         HIPCHK(hipMalloc(&c->w.l_run[i], (uint64_t)c->w.cap_run * sizeof(Item)));
     }
+    HIPCHK(hipMalloc(&c->w.lut, (uint64_t)c->w.cap_large * kRootCode));
     c->w.tiles_cap = tiles_cap_of(cap);
     c->w.groups_cap = groups_cap_of(cap);
     const uint64_t plan_bytes = plan_bytes_of(cap);
@@ -2980,27 +2970,27 @@ int ensure_capacity(ps5_ctx* c, uint64_t n)
 // loaded until the process ends.  Host code never uses the array's name as a
 // device address; the address is resolved once per device with
 // hipGetSymbolAddress (scratch_address) and kept in the context.
-constexpr uint64_t kScratchBytes = 128ull << 20;
+constexpr uint64_t kScratchBytes = 104ull << 20;
 constexpr uint64_t kNoAllocMaxStrings = 1ull << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
-// Byte offsets of the work buffers of a sort of up to `cap` strings inside
-// the scratch, its tables sized for any shape (chunks of kChunkMin keys).
-struct ScratchLayout {
+// Byte offsets of the work buffers of a sort of up to `cap` strings of the
+// given shape in one piece of memory, and their sum.
+struct WorkLayout {
     uint64_t rec, bkey, sdepth[2], lut, l_round[2], l_lvl[2], l_tiny[2], l_block[2], l_run[2];
     uint64_t desc, trees, hist, gsum, vpos, src, total;
-    uint64_t trees_cap, hist_cap, gsum_cap;
+    uint64_t hist_cap, gsum_cap;
 };
 constexpr uint64_t align256(uint64_t x) { return (x + 255) / 256 * 256; }
-constexpr ScratchLayout scratch_layout(uint64_t cap)
+constexpr WorkLayout work_layout(uint64_t cap, uint64_t chunk_max, uint64_t min_tiles)
 {
-    ScratchLayout L{};
+    WorkLayout L{};
     uint64_t o = 0;
     auto take = [&o](uint64_t bytes) { const uint64_t at = o; o = align256(o + bytes); return at; };
     const uint64_t cl = cap_large_of(cap), cb = cap_block_of(cap), cr = cap_run_of(cap);
     L.rec = take(2 * cap * kRecWords * sizeof(uint32_t));
     L.bkey = take(cap * sizeof(key64));
-    for (int i = 0; i < 2; ++i) L.sdepth[i] = take(cap * sizeof(uint32_t));
+    for (int i = 0; i < 2; ++i) L.sdepth[i] = take(sdepth_cap_of(cap) * sizeof(uint32_t));
     for (int i = 0; i < 2; ++i) {
         L.l_round[i] = take(cl * sizeof(Item));
         L.l_lvl[i] = take(cl * sizeof(Item));
@@ -3009,20 +2999,20 @@ constexpr ScratchLayout scratch_layout(uint64_t cap)
         L.l_run[i] = take(cr * sizeof(Item));
     }
     L.desc = take(plan_bytes_of(cap));
-    L.trees_cap = cl;
-    L.trees = take(L.trees_cap * kTreeSlots * sizeof(key64));
-    L.lut = take(L.trees_cap * kRootCode);
-    L.hist_cap = hist_cap_of(cap, kChunkMin, kMinTiles);
+    L.lut = take(cl * kRootCode);
+    L.hist_cap = hist_cap_of(cap, chunk_max, min_tiles);
     L.hist = take(L.hist_cap * sizeof(uint32_t));
     L.vpos = take(2 * L.hist_cap * sizeof(uint32_t));
     L.src = take(2 * L.hist_cap * sizeof(uint32_t));
     L.gsum_cap = gsum_cap_of(cap, L.hist_cap);
     L.gsum = take(L.gsum_cap * sizeof(uint32_t));
+    L.trees = take(L.gsum_cap * sizeof(key64));
     L.total = o;
     return L;
 }
-static_assert(scratch_layout(kNoAllocMaxStrings).total <= kScratchBytes,
-              "the scratch holds the work buffers of its largest sort");
+// the scratch's layout: tables for any shape (chunks of kChunkMin keys)
+constexpr WorkLayout scratch_layout() { return work_layout(kNoAllocMaxStrings, kChunkMin, kMinTiles); }
+static_assert(scratch_layout().total <= kScratchBytes, "the scratch holds the work buffers of its largest sort");
 
 // Device address of `scratch` on `device` (the caller has made it current):
 // resolved on the first call per device and remembered.
@@ -3057,7 +3047,7 @@ std::mutex& scratch_mutex(int device)
 // buffers.  Nothing is allocated.
 WorkBuffers scratch_buffers(unsigned char* base, Item* h_large, unsigned char* h_plan, unsigned char* h_plan_dev)
 {
-    constexpr ScratchLayout L = scratch_layout(kNoAllocMaxStrings);
+    constexpr WorkLayout L = scratch_layout();
     const uint64_t cap = kNoAllocMaxStrings;
     WorkBuffers w;
     w.fixed = true;
@@ -3085,7 +3075,6 @@ WorkBuffers scratch_buffers(unsigned char* base, Item* h_large, unsigned char* h
     w.tiles_cap = tiles_cap_of(cap);
     w.groups_cap = groups_cap_of(cap);
     w.trees = reinterpret_cast<key64*>(base + L.trees);
-    w.trees_cap = L.trees_cap;
     w.lut = base + L.lut;
     w.hist = reinterpret_cast<uint32_t*>(base + L.hist);
     w.hist_cap = L.hist_cap;
@@ -3675,7 +3664,6 @@ void dev_level(ps5_ctx* c, const Bufs& B, const Item* list, int ci, uint32_t bou
     A.groups_cap = c->w.groups_cap;
     A.hist_cap = c->w.hist_cap;
     A.gsum_cap = c->w.gsum_cap;
-    A.trees_cap = c->w.trees_cap;
     A.leaf_target = c->leaf_target;
     A.max_treebits = c->max_treebits;
     A.max_oversample = c->max_oversample;
@@ -4200,7 +4188,7 @@ int run_sort_keys(ps5_ctx* c, const uint8_t* arena, uint64_t alen, const uint32_
         std::vector<uint64_t> key = { (uint64_t)(uintptr_t)arena, alen, (uint64_t)(uintptr_t)offs,
                                       (uint64_t)(uintptr_t)offs64, n, (uint64_t)(uintptr_t)perm,
                                       (uint64_t)(uintptr_t)lcp, nsets, (uint64_t)(uintptr_t)c->w.rec, c->w.cap,
-                                      (uint64_t)(uintptr_t)c->w.trees, c->w.trees_cap, c->leaf_target,
+                                      (uint64_t)(uintptr_t)c->w.trees, c->w.gsum_cap, c->leaf_target,
                                       c->max_treebits, c->max_oversample, c->graph_rounds, c->seed,
                                       c->w_gen, c->w.fixed ? 1u : 0u, c->graph_levels, c->chunk_max,
                                       c->chunk_max_root, c->min_tiles, c->leaf_keys };

@@ -1,5 +1,7 @@
 """GPU tests of single paths of the sort, each at the sizes where it can go
 wrong, bit-exact against the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -324,3 +326,50 @@ def test_packed_root_with_a_wider_alphabet(ctx, oracle, known, others, as_sigma)
     common, common_offs = packed_case(as_sigma, n, 17 * known + others, hi=hi)
     ctx.sort(common, common_offs)
     assert rounds == ctx.work_stats()["rounds"], ctx.work_stats()
+
+
+def device_bytes_free():
+    """free memory of the current device, asked of the HIP runtime that the library uses"""
+    path = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l)
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert ctypes.CDLL(path).hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_work_buffers_of_a_large_context(ps5, oracle):
+    """a context for 40 M strings takes 86 bytes a string (and what the
+    allocator rounds up to): splitters and depths take room for what a level
+    can have, not for every string and segment"""
+    n, slack = 40_000_000, 64 << 20
+    arena, offs = pack(random_strings(5000, 0, 40, b"ab", 3))
+    c = ps5.Context(0)
+    try:
+        before = device_bytes_free()
+        ps5._check(ps5.load().ps5_ctx_reserve(c.h, n), "ps5_ctx_reserve")
+        check(c, oracle, arena, offs)
+        used = before - device_bytes_free()
+        assert used <= 86 * n + slack, used / n
+    finally:
+        c.close()
+
+
+@pytest.mark.parametrize("planning", [0, 1])
+@pytest.mark.parametrize("target, oversample", [(64, 2), (64, 32), (1024, 32)])
+def test_runs_of_every_length_continue(ps5, oracle, planning, target, oversample):
+    """blocks with more short runs of equal keys than they finish themselves
+    (the rest are tiny leaves of the next round, whose depth is their own),
+    between runs at the edge of a tiny leaf and of a block"""
+    rng = np.random.default_rng(target + oversample)
+    strs = []
+    for g, size in enumerate([2] * 3000 + [3] * 900 + [63, 64, 65, 66] * 20 + [2047, 2048, 2049, 5000]):
+        stem = b"%c%07d" % (97 + g % 5, g // 5)
+        tails = rng.integers(97, 100, (size, 20)).astype(np.uint8)
+        strs += [stem + t[:k].tobytes() for t, k in zip(tails, rng.integers(0, 21, size))]
+    order = rng.permutation(len(strs))
+    c = ps5.Context(0)
+    try:
+        c.set_planning(planning)
+        c.set_tuning(target, 10, oversample)
+        check(c, oracle, *pack([strs[i] for i in order]))
+    finally:
+        c.close()
