@@ -4370,7 +4370,8 @@ int ps5_ctx_reserve(ps5_ctx* c, uint64_t n)
     if (!c) return set_err(PS5_ERR_ARG, "ctx is NULL");
     if (n >= 0xFFFFFF00ull) return set_err(PS5_ERR_ARG, "n too large (limit 2^32-256 strings)");
     HIPCHK(hipSetDevice(c->device));
-    return ensure_capacity(c, n);
+    const int rc = ensure_capacity(c, n);
+    return rc ? rc : ensure_tables(c);
 }
 
 void* ps5_ctx_stream(ps5_ctx* c) { return c ? (void*)c->stream : nullptr; }
