@@ -298,8 +298,11 @@ typedef struct ps5_server ps5_server;
  * and released bytes kept in device memory.  With max_batch_strings > 0
  * every slot allocates its device buffers for such a batch at creation (up to
  * min(hbm_budget / slots, 64 * max_batch_strings) characters), so that the
- * first requests do not wait for allocations.  No counterpart in the
- * reference (it sorts one set per call). */
+ * first requests do not wait for allocations.  A request counts with its
+ * characters, offsets, results and a context's work buffers for its strings.
+ * Every slot also holds 16 MiB of pinned host memory, through which requests
+ * whose arrays are at most 1 MiB are copied (directly, if that allocation
+ * fails).  No counterpart in the reference (it sorts one set per call). */
 int ps5_server_create(ps5_server** out, int device, uint64_t hbm_budget, uint32_t slots,
                       uint64_t max_batch_strings);
 void ps5_server_destroy(ps5_server* srv);

@@ -10,6 +10,14 @@ namespace ps5 {
 // Record the calling thread's last error (ps5_last_error) and return code.
 int set_error(int code, const char* fmt, ...);
 
+// Device bytes of the work buffers that a context of the default shape holds
+// for n strings (what the allocator rounds up to comes on top).
+uint64_t work_bytes(uint64_t n);
+
+// Device bytes a served request occupies while it runs: its characters,
+// uint32 and uint64 offsets, results, and its share of a context's work buffers.
+uint64_t request_bytes(uint64_t arena_bytes, uint64_t n);
+
 // Absolute uint64 offsets of a batch staged set by set: for string i of set s
 // (set_first[s] <= i < set_first[s+1]), offs64[i] = set_base[s] + offs32[i].
 // d_first / d_base are device arrays of nsets+1 / nsets entries.  Enqueued on

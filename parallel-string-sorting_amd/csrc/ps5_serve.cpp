@@ -98,10 +98,6 @@ struct ps5_server {
 
 namespace {
 
-// device bytes a request occupies while it runs: its characters, uint32 and
-// uint64 offsets, results, and the sort context's work buffers (~88 B per string)
-uint64_t request_bytes(uint64_t arena_bytes, uint64_t n) { return arena_bytes + 16 + n * (4 + 8 + 8 + 88) + 4096; }
-
 // device buffer that only grows, at least by half each time
 template <class T>
 int grow(T** p, uint64_t* cap, uint64_t need)
@@ -449,6 +445,11 @@ void free_admission(ps5_server* s)
 
 }  // namespace
 
+uint64_t ps5::request_bytes(uint64_t arena_bytes, uint64_t n)
+{
+    return arena_bytes + 16 + n * (4 + 8 + 8) + (work_bytes(n) - work_bytes(0)) + 4096;
+}
+
 extern "C" {
 
 int ps5_server_create(ps5_server** out, int device, uint64_t hbm_budget, uint32_t slots, uint64_t max_batch_strings)
@@ -541,7 +542,7 @@ uint64_t ps5_server_submit(ps5_server* s, const uint8_t* arena, uint64_t arena_b
     r->n = n;
     r->perm = perm;
     r->lcp = lcp;
-    r->dev_bytes = request_bytes(arena_bytes, n);
+    r->dev_bytes = ps5::request_bytes(arena_bytes, n);
     r->t_submit = Clock::now();
     {
         std::unique_lock<std::mutex> lk(s->mu);

@@ -4795,6 +4795,11 @@ int set_error(int code, const char* fmt, ...)
     return code;
 }
 
+uint64_t work_bytes(uint64_t n)
+{
+    return work_layout(n, std::min(kShapeChunkMax, kShapeChunkMaxRoot), kMinTiles).total;
+}
+
 int widen_offsets(ps5_ctx* c, const uint32_t* d_offs32, const uint64_t* d_first, const uint64_t* d_base,
                   uint32_t nsets, uint64_t n, uint64_t* d_offs64)
 {

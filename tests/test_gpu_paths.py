@@ -379,6 +379,16 @@ def test_reserved_context_allocates_nothing(ps5, oracle):
     assert reserved > 0 and first == 0, (reserved, first)
 
 
+@pytest.mark.parametrize("n", [200_000, 1 << 20, 5_000_000, 20_000_000])
+def test_work_bytes_are_what_a_context_holds(ps5, oracle, n):
+    """the bytes that a server charges for work buffers are those that
+    contexts allocate, up to what the allocator rounds up to"""
+    work_bytes = ps5.load()._ZN3ps510work_bytesEm
+    work_bytes.restype, work_bytes.argtypes = ctypes.c_uint64, [ctypes.c_uint64]
+    reserved, first = reserve_and_sort(ps5, oracle, n)
+    assert work_bytes(n) - (1 << 20) <= reserved + first <= work_bytes(n) + (64 << 20)
+
+
 @pytest.mark.parametrize("planning", [0, 1])
 @pytest.mark.parametrize("target, oversample", [(64, 2), (64, 32), (1024, 32)])
 def test_runs_of_every_length_continue(ps5, oracle, planning, target, oversample):

@@ -3,6 +3,8 @@ none of whose slots can start completes every request with an error instead
 of leaving its waiter blocked, and malformed requests are rejected at submit,
 before they could share a batch.  The slots here ask for a device index that
 does not exist, so the same failure is forced on any machine."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -52,3 +54,19 @@ def test_server_rejects_malformed_requests(ps5):
             srv.inject_fault(1)
     finally:
         srv.close()
+
+
+@pytest.mark.parametrize("n", [1, 100, 5000, 1 << 20, 3_000_000, 1 << 28])
+def test_server_charges_what_a_request_holds(ps5, n):
+    """a request's share of the budget: characters, offsets of both widths,
+    results and the work buffers of a context for its strings"""
+    lib = ps5.load()
+    work_bytes, request_bytes = lib._ZN3ps510work_bytesEm, lib._ZN3ps513request_bytesEmm
+    for f, k in ((work_bytes, 1), (request_bytes, 2)):
+        f.restype, f.argtypes = ctypes.c_uint64, [ctypes.c_uint64] * k
+    per_string = 24 + 8 + 42 if n > 1 << 20 else 24 + 8 + 42 + 5 * 4
+    assert work_bytes(n) >= per_string * n
+    chars = 60 * n
+    assert chars + 20 * n + work_bytes(n) - work_bytes(0) <= request_bytes(chars, n) <= chars + 20 * n + work_bytes(n) + 8192
+    # requests batched together are charged no less than one context for all of them
+    assert 16 * request_bytes(chars, n) >= 16 * (chars + 20 * n) + work_bytes(16 * n) - work_bytes(0)
