@@ -461,26 +461,34 @@ __device__ __forceinline__ void tree_of_segment(LargeDesc* Dp, uint32_t si, cons
         uint32_t* alpha_out = reinterpret_cast<uint32_t*>(code_out + kLutBytes);
         if (B.widen) {     // (uniform)
             if (tid_x() < kLutBytes) S.lut[tid_x()] = (uint8_t)((alpha_out[tid_x() / 32] >> (tid_x() & 31)) & 1u);
-        } else if (act) {
-#pragma unroll 1
-            for (uint32_t j = o; j < o + kPer && j < ss; ++j) {
-                const Chars24 c = load_chars24(B.arena, B.alen, str_off(B, sample(j)));
-                const uint32_t len = chars_before_nul(c);
-#pragma unroll
-                for (int i = 0; i < 24; ++i)
-                    if ((uint32_t)i < len) S.lut[(uint32_t)(c.w[i / 8] >> (8 * (i & 7))) & 0xFFu] = 1;
-            }
         }
-        __syncthreads();
-        if (tid_x() < kLutBytes) {     // (whole waves)
-            const uint64_t seen = __ballot(S.lut[tid_x()] != 0);
-            if ((tid_x() & 31) == 0) S.alpha[tid_x() / 32] = (uint32_t)(seen >> (tid_x() & 32));
-        }
-        __syncthreads();
-        if (tid_x() < 8) alpha_out[tid_x()] = S.alpha[tid_x()];
         uint32_t sigma = 0;
+        // (a thread's first sample alone shows most alphabets that are too
+        // large; all four take 10 us)
+#pragma unroll 1
+        for (uint32_t part = 0; part < 2; ++part) {
+            if (!B.widen && act) {
+#pragma unroll 1
+                for (uint32_t j = o + part; j < (part ? o + kPer : o + 1) && j < ss; ++j) {
+                    const Chars24 c = load_chars24(B.arena, B.alen, str_off(B, sample(j)));
+                    const uint32_t len = chars_before_nul(c);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) sigma += (uint32_t)__popc(S.alpha[j]);
+                    for (int i = 0; i < 24; ++i)
+                        if ((uint32_t)i < len) S.lut[(uint32_t)(c.w[i / 8] >> (8 * (i & 7))) & 0xFFu] = 1;
+                }
+            }
+            __syncthreads();
+            if (tid_x() < kLutBytes) {     // (whole waves)
+                const uint64_t seen = __ballot(S.lut[tid_x()] != 0);
+                if ((tid_x() & 31) == 0) S.alpha[tid_x() / 32] = (uint32_t)(seen >> (tid_x() & 32));
+            }
+            __syncthreads();
+            sigma = 0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) sigma += (uint32_t)__popc(S.alpha[j]);
+            if (B.widen || sigma > kMaxAlphabet) break;     // (uniform)
+        }
+        if (tid_x() < 8) alpha_out[tid_x()] = S.alpha[tid_x()];
         fmt = sigma <= 7 ? 1u : sigma <= 15 ? 2u : sigma <= kMaxAlphabet ? 3u : 0u;
         if (fmt == 0) break;     // (uniform)
         if (tid_x() < kLutBytes) {
@@ -3436,11 +3444,16 @@ constexpr uint32_t kForkLeafGroups = 8192;    // leaf workgroups worth a side st
 constexpr uint32_t kFewLeavesPerCu = 8;
 // Strings of the largest root from which on roots may pack their keys.
 // Packing saves rounds and levels where keys repeat: 4.2 M suffixes of an ACGT
-// text take 0.73 ms against 1.08 plain, 20 M windows 1.47 against 3.03, a batch
-// of 192 sets (a third of them ACGT) 2.21 against 2.59.  Smaller roots of a
-// small alphabet have little to gain (40 K strings of ACGT: 119 us plain, 116
-// packed), and the kernels that can pack cost others a little (0.5 M digits,
-// which do not pack: 163 and 165 us).
+// text take 0.70 ms against 1.07 plain, 20 M windows 1.48 against 3.03.  The
+// kernels that can pack cost those that do not a little: 0.5 to 1 M digits or
+// ASCII strings 2-3%, URL-like ones 1-2%, less the larger they are (4.2 M: 0-1%).
+// From 2^20 on packing gains 13-25% and more where it is of use (1 M suffixes
+// 0.63 -> 0.55 ms, 1 M ACGT strings 0.31 -> 0.25); between 2^19 and 2^20 from
+// nothing (0.64 and 0.9 M suffixes, 0.64 M ACGT strings) to 29% (0.75 M, where
+// plain keys need one more level), below 2^19 from -8% (16 K suffixes) to 14%
+// (0.25 M).  The smaller roots of a batch pack with its largest: the line drawn
+// for each root took 2.37 ms for 192 sets of 1 K to 2 M strings (a third ACGT)
+// instead of 2.21, since the plain ones then keep the batch's rounds going.
 constexpr uint64_t kPackMin = 1u << 20;
 constexpr uint64_t kChainMin = 1u << 22;       // strings of a level whose successor is chained on the device
 // Automatic planning plans a single sort of fewer strings on the device, as
