@@ -10,6 +10,13 @@ namespace ps5 {
 // Record the calling thread's last error (ps5_last_error) and return code.
 int set_error(int code, const char* fmt, ...);
 
+// Strings of a chunk at most: larger chunk limits of ps5_ctx_set_shape act as this.
+constexpr uint32_t kChunkLimit = 8192;
+
+// The autotuner's candidates for parameter `param` beside its current value:
+// settings that sort differently.  Returns how many (at most 8) are in out.
+int tune_candidates(int param, uint32_t current, uint32_t* out);
+
 // Device bytes of the work buffers that a context of the default shape holds
 // for n strings (what the allocator rounds up to comes on top).
 uint64_t work_bytes(uint64_t n);

@@ -2703,6 +2703,8 @@ int set_err(int code, const char* fmt, ...)
     return code;
 }
 
+static_assert(kChunkLimit == kPartMax, "the largest chunk");
+
 #define HIPCHK(x)                                                                  \
     do {                                                                           \
         hipError_t _e = (x);                                                       \

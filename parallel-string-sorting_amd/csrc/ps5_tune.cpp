@@ -7,10 +7,10 @@
 //     on-chip blocks are), the splitter-tree depth limit of one level
 //     (max_treebits: fan-out per level, histogram size) and the oversampling
 //     factor (max_oversample: splitter quality against tree-build cost);
-//   - tile shapes: the keys per wave chunk of ordinary levels and of levels
-//     of roots (the unit of stable ranks and of the scatter's LDS reorder:
-//     longer chunks give longer write runs per bucket, shorter ones more
-//     tiles), and the tiles a small level is spread over at least;
+//   - chunk shapes: the keys per chunk of ordinary levels and of levels of
+//     roots (the unit that one workgroup ranks and reorders in LDS: longer
+//     chunks give longer runs per bucket, shorter ones more workgroups), and
+//     the chunks a small level is spread over at least;
 //   - key width: the keys (8 characters each) a leaf pass fetches per string
 //     at a time (wide fetches pay on long shared prefixes, narrow ones save
 //     bandwidth on short strings).
@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "../../include/ps5_mi355x.h"
+#include "ps5_internal.hpp"
 
 namespace {
 
@@ -59,22 +60,14 @@ int autotune(ps5_ctx* ctx, const std::function<int()>& sort_once, uint32_t* leaf
     };
     double best_t = 0;
     if ((rc = time_of(best, &best_t))) return rc;
-    static const std::vector<uint32_t> cands[kParams] = {
-        { 96, 128, 192, 256, 384, 512, 768, 1024 },     // leaf_target
-        { 7, 8, 9, 10 },                                 // max_treebits
-        { 4, 8, 16, 32 },                                // max_oversample
-        { 4096, 6144, 8192, 9216 },                      // chunk_max
-        { 6144, 9216, 12032 },                           // chunk_max_root
-        { 256, 512, 1024, 2048 },                        // min_tiles
-        { 1, 2, 4, 8 },                                  // leaf_keys
-    };
     for (int pass = 0; pass < 2; ++pass) {
         for (int param = 0; param < kParams; ++param) {
             Tuning round_best = best;
-            for (uint32_t c : cands[param]) {
-                if (c == best.v[param]) continue;
+            uint32_t cands[8];
+            const int n = ps5::tune_candidates(param, best.v[param], cands);
+            for (int i = 0; i < n; ++i) {
                 Tuning t = best;
-                t.v[param] = c;
+                t.v[param] = cands[i];
                 double ms = 0;
                 if ((rc = time_of(t, &ms))) return rc;
                 if (ms < best_t) { best_t = ms; round_best = t; }
@@ -91,6 +84,24 @@ int autotune(ps5_ctx* ctx, const std::function<int()>& sort_once, uint32_t* leaf
 }
 
 }  // namespace
+
+int ps5::tune_candidates(int param, uint32_t current, uint32_t* out)
+{
+    static const std::vector<uint32_t> cands[kParams] = {
+        { 96, 128, 192, 256, 384, 512, 768, 1024 },     // leaf_target
+        { 7, 8, 9, 10 },                                 // max_treebits
+        { 4, 8, 16, 32 },                                // max_oversample
+        { 4096, 6144, 8192 },                            // chunk_max
+        { 4096, 6144, 8192 },                            // chunk_max_root
+        { 256, 512, 1024, 2048 },                        // min_tiles
+        { 1, 2, 4, 8 },                                  // leaf_keys
+    };
+    const bool chunk = param == 3 || param == 4;
+    int n = 0;
+    for (uint32_t c : cands[param])
+        if (c != (chunk ? std::min(current, kChunkLimit) : current)) out[n++] = c;
+    return n;
+}
 
 extern "C" int ps5_autotune_device(ps5_ctx* ctx, const uint8_t* d_arena, uint64_t arena_bytes, const uint32_t* d_offs,
                                    uint64_t n, uint32_t* d_perm, uint32_t* d_lcp, uint32_t* leaf_target,

@@ -1,5 +1,6 @@
 """CPU checks of the C ABI library: it loads without a GPU and exports every
 function include/ps5_mi355x.h declares; the product has no CPU fallback."""
+import ctypes
 import os
 import re
 import subprocess
@@ -93,3 +94,17 @@ def test_batch_generator_layout(ps5):
         assert np.all(tail == 0) and end - (o[-1] + lens[-1] + 1) < 8
     again = ps5.gen_batch(0x5EED0004, 64, 1000, 20000, 4, 48)
     assert np.array_equal(again[0], arena) and np.array_equal(again[1], offs)
+
+
+@pytest.mark.parametrize("param, current", [(0, 768), (0, 100), (1, 10), (2, 32), (3, 9216), (3, 8192), (3, 2048), (3, 6144), (4, 12032),
+                                            (4, 9216), (4, 6144), (5, 512), (6, 8)])
+def test_autotuner_times_settings_that_differ(ps5, param, current):
+    """no two candidates of a parameter, nor a candidate and the current
+    value, sort the same way: chunk limits above 8192 act as 8192"""
+    f = ps5.load()._ZN3ps515tune_candidatesEijPj
+    f.restype, f.argtypes = ctypes.c_int, [ctypes.c_int, ctypes.c_uint32, ctypes.POINTER(ctypes.c_uint32)]
+    out = (ctypes.c_uint32 * 8)()
+    n = f(param, current, out)
+    cands = list(out)[:n]
+    acts = [min(v, 8192) if param in (3, 4) else v for v in cands + [current]]
+    assert len(cands) >= 2 and len(set(acts)) == len(acts), cands
