@@ -227,40 +227,11 @@ __device__ __forceinline__ bool kp_less(key64 ka, uint32_t pa, key64 kb, uint32_
     return ka < kb || (ka == kb && pa < pb);
 }
 
-// Workgroups are dispatched to the 8 XCDs round-robin (workgroup i runs on
-// XCD i % 8), and every XCD has its own L2.  This bijection of [0, G) gives
-// each XCD one contiguous range of work items, so neighbouring tiles -- whose
-// histogram entries and bucket output ranges share cache lines -- meet in the
-// same L2.
-__device__ __forceinline__ uint32_t xcd_contiguous(uint32_t bid, uint32_t G)
-{
-    const uint32_t x = bid % kXcds, y = bid / kXcds, q = G / kXcds, r = G % kXcds;
-    return x * q + min(x, r) + y;
-}
-
-// lanes holding the same 11-bit bucket id (all 64 lanes must execute this)
-template <int NB = 11>
-__device__ __forceinline__ uint64_t match_bucket(uint32_t b)
-{
-    const uint64_t act = __ballot(1);
-    uint32_t lo = (uint32_t)act, hi = (uint32_t)(act >> 32);
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-        // m: all ones if bit i of b is set, else zero; lanes agreeing with
-        // this lane on bit i are ~(ballot ^ m), computed as (~ballot) ^ m
-        const uint32_t m = (uint32_t)((int32_t)(b << (31 - i)) >> 31);
-        const uint64_t nbal = ~(uint64_t)__ballot(m != 0u);
-        lo &= (uint32_t)nbal ^ m;
-        hi &= (uint32_t)(nbal >> 32) ^ m;
-    }
-    return ((uint64_t)hi << 32) | lo;
-}
-
-// The same lanes for NB-bit ids with fewer vector instructions (all 64 lanes
-// must execute this): every lane ORs its bit (lanebit) into this wave's table
-// of 64-bit lane masks at the id's low TB bits, reads the entry back -- the
-// lanes agreeing on those bits -- and clears it, and ballots on the NB - TB
-// high bits keep the lanes agreeing on the whole id.  tab holds 1 << TB
+// The lanes holding the same NB-bit bucket id, with few vector instructions
+// (all 64 lanes must execute this): every lane ORs its bit (lanebit) into this
+// wave's table of 64-bit lane masks at the id's low TB bits, reads the entry
+// back -- the lanes agreeing on those bits -- and clears it, and ballots on the
+// NB - TB high bits keep the lanes agreeing on the whole id.  tab holds 1 << TB
 // entries, zero on entry and zero again on return.  The OR of the lanes' bits
 // does not depend on the order the LDS applies them in, and a wave's LDS
 // operations complete in issue order, so every read sees all of the ORs.

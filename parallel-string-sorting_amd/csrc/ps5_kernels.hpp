@@ -85,8 +85,6 @@ __host__ __device__ constexpr int block_class(uint32_t m)
 {
     return m <= 256 ? 0 : m <= 512 ? 1 : m <= 1024 ? 2 : 3;
 }
-constexpr int kRankBits = 21;
-constexpr uint32_t kRankMask = (1u << kRankBits) - 1;
 
 struct Item {            // a segment or a leaf
     uint32_t begin;      // first position

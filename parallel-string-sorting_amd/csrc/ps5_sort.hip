@@ -2714,11 +2714,11 @@ static_assert(kChunkLimit == kPartMax, "the largest chunk");
     } while (0)
 
 enum KernelId {
-    K_INIT, K_TREE, K_PART, K_HIST, K_CHILDREN, K_BLOCK,
+    K_TREE, K_PART, K_HIST, K_CHILDREN, K_BLOCK,
     K_LEAF_TINY, K_LEAF_RUN, K_LEAFBOUND, K_MISC, K_NUM
 };
 const char* kKernelNames[K_NUM] = {
-    "k_init", "k_tree", "k_part", "k_hist", "k_children", "k_block",
+    "k_tree", "k_part", "k_hist", "k_children", "k_block",
     "k_leaf_tiny", "k_leaf_run", "k_leafbound", "k_misc"
 };
 
