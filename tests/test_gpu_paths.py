@@ -409,3 +409,74 @@ def test_runs_of_every_length_continue(ps5, oracle, planning, target, oversample
         check(c, oracle, *pack([strs[i] for i in order]))
     finally:
         c.close()
+
+
+def test_rows_of_many_runs(ps5, oracle):
+    """67 M strings in chunks of 2048: buckets of 32861 runs, more than 64 of
+    them to each sampled one where a chunk or an equal-key leaf is mapped, and
+    longer rows than a tree, a block or a leaf looks at in LDS"""
+    n, width, chunk = 67_300_000, 12, 2048
+    assert -(-n // chunk) > 64 * 512
+    rng = np.random.default_rng(9)
+    rows = rng.integers(48, 89, (n, width), dtype=np.uint8)
+    stems = rng.integers(48, 89, (500, 8), dtype=np.uint8)
+    rows[:n // 4, :8] = stems[rng.integers(0, 500, n // 4)]
+    rows[n // 4:, 5] = 0                     # strings of up to 5 characters
+    rows[:n // 4, width - 1] = 0             # and of 8 to 11
+    cut = rng.integers(0, 4, n, dtype=np.uint8)
+    for k in range(1, 4):
+        rows[:n // 4, width - 1 - k][cut[:n // 4] >= k] = 0
+        rows[n // 4:, 5 - k][cut[n // 4:] >= k] = 0
+    rows = rows.reshape(-1)
+    arena = np.concatenate([rows, np.zeros(16, np.uint8)])
+    del rows
+    order = np.arange(n, dtype=np.uint32).reshape(100, -1).T.reshape(-1)     # (both kinds in every chunk)
+    offs = order * np.uint32(width)
+    c = ps5.Context(0)
+    try:
+        c.set_shape(chunk, chunk, 512, 8)
+        check(c, oracle, arena, offs)
+    finally:
+        c.close()
+
+
+@pytest.mark.parametrize("sigma, stem, tail, rare, packed", [
+    (4, 16, 4, 0, True), (7, 16, 4, 0, True), (15, 11, 4, 0, True), (31, 8, 3, 0, True), (32, 8, 3, 0, False),
+    (4, 16, 4, 1, True), (4, 16, 4, 3, True), (7, 11, 4, 8, True), (15, 8, 3, 16, True), (31, 8, 3, 1, False), (4, 16, 4, 28, False)])
+def test_roots_pack_their_keys(ctx, oracle, sigma, stem, tail, rare, packed):
+    """strings that a packed key of their alphabet holds whole are sorted in
+    one round, in plain keys (which groups of them share) in more; so too when
+    `rare` characters are in one string each, where the samples miss them"""
+    n = 1_060_000
+    rng = np.random.default_rng(sigma + rare)
+    chars = np.sort(rng.choice(np.arange(1, 256), sigma + rare, replace=False)).astype(np.uint8)
+    chars = rng.permutation(chars)
+    alpha = chars[:sigma]
+    width = stem + tail + 1
+    rows = np.zeros((n, width), np.uint8)
+    rows[:, :stem] = alpha[rng.integers(0, sigma, (300, stem))][rng.integers(0, 300, n)]
+    rows[:, stem:-1] = alpha[rng.integers(0, sigma, (n, tail))]
+    rows[rng.choice(n, rare, replace=False), rng.integers(0, width - 1, rare)] = chars[sigma:]
+    arena = np.concatenate([rows.reshape(-1), np.zeros(16, np.uint8)])
+    offs = (np.arange(n, dtype=np.uint32) * np.uint32(width))
+    check(ctx, oracle, arena, offs)
+    rounds = ctx.work_stats()["rounds"]
+    assert (rounds == 1) == packed, rounds
+
+
+def test_noalloc_sort_starts_over(ps5, ctx, oracle):
+    """the largest allocation-free sort packs its keys and meets a character
+    that its samples do not show"""
+    n = int(ps5.load().ps5_noalloc_max_strings())
+    arena, offs = packed_case(4, n, 8, rare=5)
+    bufs = [ps5.DeviceBuffer(arena.size)] + [ps5.DeviceBuffer(4 * n) for _ in range(3)]
+    da, do, dp, dl = bufs
+    try:
+        da.upload(arena)
+        do.upload(offs)
+        ps5._check(ps5.load().ps5_sort_device_noalloc(ctx.h, da.ptr, int(arena.size), do.ptr, n, dp.ptr, dl.ptr), "noalloc")
+        r, msg = oracle.verify(arena, offs, dp.download(np.uint32, n), dl.download(np.uint32, n))
+        assert r == 0, msg
+    finally:
+        for b in bufs:
+            b.free()
