@@ -2134,11 +2134,13 @@ __device__ __forceinline__ uint32_t common_chars(const Bufs& B, const key64 (&re
 // strings are known to share.  Strings with a common prefix (URLs of one host)
 // share more than one key: without looking ahead, every 8 characters of the
 // prefix cost a round of tree, partition and host round trips that split
-// nothing.  64 strings of the chunk say how far looking ahead can go; if
-// anywhere, every string of the chunk is compared with the run's first one
-// over 64 characters, and the run continues after what they all share.
-// 4.4 M URL-like strings (prefixes of 8 to 40 characters, 256 MB): 3.07 -> 1.50
-// ms, 2 instead of 5 rounds with large segments.
+// nothing.  If 64 strings of the chunk agree in their next character, every
+// string of it is compared with the run's first one over 64 characters, and
+// the run continues after what they all share.  4.4 M URL-like strings
+// (prefixes of 8 to 40 characters, 256 MB): 3.07 -> 1.40 ms, 2 instead of 5
+// rounds with large segments.  The sample looks at one key only: most runs of a
+// text share nothing more, and over 64 characters it took half as long as the
+// rest (20 M windows in plain keys, 65 K runs of 300 strings: 850 -> 549 us).
 __device__ __forceinline__ void run_chunk(const Item& L, const Bufs& B, const Sink& nxt, RunMap<kRunChunk>& M)
 {
     const uint32_t c = L.flags >> kFlagShift;
@@ -2182,24 +2184,24 @@ __device__ __forceinline__ void run_chunk(const Item& L, const Bufs& B, const Si
     if (!term) {     // (uniform)
         const uint32_t next = depth + F.cpk;
         const uint32_t id0 = R.R[run_place(B, R, L.begin)].id;
-        key64 ref[kExtKeys];
-        load_keys<kExtKeys>(B.arena, B.alen, str_off(B, min(id0, B.n - 1)) + next, ref);
+        key64 ref[kExtKeys];     // (in vector registers: the scalar ones are short)
+        uint32_t zero;
+        asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+        load_keys<kExtKeys>(B.arena, B.alen, str_off(B, min(id0, B.n - 1)) + next + zero, ref);
         // all waves take the same sample
         const uint32_t lane = lane_id();
         const uint32_t sp = (uint32_t)(((uint64_t)lane * m) >> 6);
-        const uint32_t sid = R.R[place(sp)].id;
-        uint32_t ext = common_chars(B, ref, str_off(B, min(sid, B.n - 1)) + next);
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) ext = min(ext, (uint32_t)__shfl_xor((int)ext, d, 64));
-        if (ext) {     // (uniform)
-            uint32_t e = ext;
+        const key64 ks = string_key(B, R.R[place(sp)].id, next);
+        uint32_t ext = 0;
+        if (__ballot((ref[0] ^ ks) >> 56 != 0 || (ks >> 56) == 0) == 0) {     // (uniform) a character at least
+            ext = 8 * kExtKeys;
+#pragma unroll 4     // (1: 549 -> 577 us, the URL-like strings' runs 220 -> 236)
             for (uint32_t p = tid_x(); p < m; p += kWG) {
                 const uint32_t id = R.R[place(p)].id;
-                e = min(e, common_chars(B, ref, str_off(B, min(id, B.n - 1)) + next));
+                ext = min(ext, common_chars(B, ref, str_off(B, min(id, B.n - 1)) + next));
             }
 #pragma unroll
-            for (int d = 32; d >= 1; d >>= 1) e = min(e, (uint32_t)__shfl_xor((int)e, d, 64));
-            ext = e;     // (of this wave's strings)
+            for (int d = 32; d >= 1; d >>= 1) ext = min(ext, (uint32_t)__shfl_xor((int)ext, d, 64));     // (this wave's strings)
         }
         if (lane == 0) atomicMin(&B.sdepth_out[L.begin >> kDepthShift], next + ext);
     }
