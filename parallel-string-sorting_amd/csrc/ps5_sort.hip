@@ -2507,29 +2507,35 @@ __device__ __forceinline__ uint32_t merge_pair(const uint64_t* tstart, uint32_t 
 }
 
 // co[g] = strings of A (of g's pair) that precede the first output of tile g.
-// kMergeLanes lanes search together, each testing one of as many positions
-// evenly spread over what is left: a test is a chain of dependent gathers,
-// and halving the range takes 21 of them one after another for runs of 2 M
-// strings (48 to 60 us a round for 16 M strings; with 16 lanes 19 to 37 us, of
-// which more and more are the gathers' own traffic: 8 runs of 2 M, three
-// rounds, take 1009 us with 32 lanes, 977 with 16 and 960 with 8).
-constexpr uint32_t kMergeLanes = 8;
+// LANES lanes search together, each testing one of as many positions evenly
+// spread over what is left.  A test is a chain of dependent gathers, and
+// halving the range takes 21 of them one after another for runs of 2 M strings;
+// more lanes take fewer steps and more gathers, which is what counts when the
+// tiles are many.  A round of less than kMergeFew tiles takes 8 lanes, of more
+// 4, of kMergeMany or more one.  8 runs, us:
+//   strings        8 lanes   4      2      1
+//   1 M (ASCII)       98    103    116    129
+//   4 M              224    231    242    262
+//   16 M             835    814    822    852
+//   64 M            3340   3233   3178   3136
+constexpr uint64_t kMergeFew = 8192, kMergeMany = 32768;
+template <uint32_t LANES>
 __global__ __launch_bounds__(kWG) void k_merge_part(Bufs B, const uint32_t* src_idx, const key64* src_key,
                                                     const key64* in_key,
                                                     const uint64_t* first, const uint64_t* mid,
                                                     const uint64_t* tstart, uint32_t npairs, uint32_t* co)
 {
-    const uint64_t g = ((uint64_t)blockIdx.x * kWG + tid_x()) / kMergeLanes;
+    const uint64_t g = ((uint64_t)blockIdx.x * kWG + tid_x()) / LANES;
     if (g >= tstart[npairs]) return;
     const uint32_t p = merge_pair(tstart, npairs, g);
     const uint64_t a0 = first[p], b0 = mid[p];
     const uint64_t la = b0 - a0, lb = first[p + 1] - b0;
     const uint64_t diag = (g - tstart[p]) * kMergeT;
     uint64_t i0 = diag > lb ? diag - lb : 0, i1 = min(diag, la);
-    const uint32_t lane = lane_id(), l = lane % kMergeLanes;
+    const uint32_t lane = lane_id(), l = lane % LANES;
     while (i0 < i1) {     // (the same for the tile's lanes)
         // A[mi] precedes this tile up to some mi in [i0, i1), and none from there on
-        const uint64_t step = (i1 - i0 + kMergeLanes - 1) / kMergeLanes;
+        const uint64_t step = (i1 - i0 + 1 + LANES) / (LANES + 1);
         const uint64_t mi = i0 + (l + 1) * step - 1;
         bool before = false;
         if (mi < i1) {
@@ -2540,7 +2546,7 @@ __global__ __launch_bounds__(kWG) void k_merge_part(Bufs B, const uint32_t* src_
             before = ka != kb || (ka & 0xFFull) == 0 ? ka <= kb
                                                      : merge_leq(B, src_idx[pa], src_idx[pb], ka, kb, &lcp);
         }
-        const uint64_t ones = (__ballot(before) >> (lane - l)) & ((1ull << kMergeLanes) - 1);
+        const uint64_t ones = (__ballot(before) >> (lane - l)) & ((1ull << LANES) - 1);
         const uint32_t t = (uint32_t)__popcll(ones);
         i0 += t * step;
         i1 = min(i1, i0 + step - 1);     // (lane t's position, if it is in the range, does not precede)
@@ -2548,11 +2554,23 @@ __global__ __launch_bounds__(kWG) void k_merge_part(Bufs B, const uint32_t* src_
     if (l == 0) co[g] = (uint32_t)i0;
 }
 
+// Where keys do not decide, every comparison is a chain of gathers from the
+// arena.  A thread finds its first output by ten comparisons, and knows from
+// them what its heads share with the output before it, but at the tile's
+// ends.  With half, every second thread searches between its neighbours' places
+// only: a chain of 12 comparisons, but 6 or 7 for each thread on average.  In a
+// round of kMergeHalf tiles or more, which the gathers' traffic bounds, that
+// is less (16 M strings of ACGT in 8 runs 5.01 ms, 6.08 without half, 7.56 when
+// every thread also compared its heads with the output before it; 16 M of
+// ASCII, whose keys decide, 0.81, 0.80 and 0.82); below, the chain counts
+// (0.3 M of ACGT 160 us with half, 151 without).
+constexpr uint64_t kMergeHalf = 1024;
 __global__ __launch_bounds__(kWG) void k_merge_tile(Bufs B, const uint32_t* src_idx, const uint32_t* src_lcp,
                                                     const key64* src_key, const key64* in_key,
                                                     uint32_t* dst_idx, uint32_t* dst_lcp,
                                                     key64* dst_key, const uint64_t* first, const uint64_t* mid,
-                                                    const uint64_t* tstart, uint32_t npairs, const uint32_t* co)
+                                                    const uint64_t* tstart, uint32_t npairs, const uint32_t* co,
+                                                    bool half)
 {
     // slots [0, na+1): A[ia0-1 .. ia1), slots [na+1, na+nb+2): B[jb0-1 .. jb1);
     // slot 0 of a part is unused when the part starts its run
@@ -2588,36 +2606,73 @@ __global__ __launch_bounds__(kWG) void k_merge_tile(Bufs B, const uint32_t* src_
         }
     }
     __syncthreads();
-    const uint32_t d = tid_x() * kMergeE;
-    if (d < len) {
-        auto leq = [&](uint32_t x, uint32_t y, uint32_t* l) {
-            return merge_leq(B, s_idx[x], s_idx[y], s_key[x], s_key[y], l);
-        };
-        uint32_t i0 = d > nb ? d - nb : 0, i1 = min(d, na);
+    auto leq = [&](uint32_t x, uint32_t y, uint32_t* l) {
+        return merge_leq(B, s_idx[x], s_idx[y], s_key[x], s_key[y], l);
+    };
+    // strings of A among the tile's first d outputs, known to be in [i0, i1];
+    // l1: the LCP of A[i-1] and B[j], l2: of B[j-1] and A[i], where the search
+    // compared them
+    constexpr uint32_t kNoLcp = 0xFFFFFFFFu;
+    auto corank = [&](uint32_t d, uint32_t i0, uint32_t i1, uint32_t* l1, uint32_t* l2) {
+        *l1 = *l2 = kNoLcp;
         while (i0 < i1) {
             const uint32_t mi = (i0 + i1) / 2;
             uint32_t l;
-            if (leq(1 + mi, sb + d - mi, &l)) i0 = mi + 1;     // A[mi] <= B[d-1-mi]
-            else i1 = mi;
-        }
-        uint32_t i = i0, j = d - i0;
-        // LCPs of the next A and B string with the previous output
-        uint32_t lcpa = 0, lcpb = 0;
-        const bool hasa = ia0 + i > 0, hasb = jb0 + j > 0;
-        if (hasa || hasb) {
-            bool prev_is_a;
-            uint32_t l;
-            if (!hasb) prev_is_a = true;
-            else if (!hasa) prev_is_a = false;
-            else prev_is_a = !leq(i, sb + j, &l);
-            const uint32_t prev = prev_is_a ? i : sb + j;
-            if (i < na) {
-                if (prev_is_a) lcpa = s_lcp[1 + i];
-                else leq(prev, 1 + i, &lcpa);
+            if (leq(1 + mi, sb + d - mi, &l)) {     // A[mi] <= B[d-1-mi]
+                i0 = mi + 1;
+                *l1 = l;
+            } else {
+                i1 = mi;
+                *l2 = l;
             }
-            if (j < nb) {
-                if (!prev_is_a) lcpb = s_lcp[sb + 1 + j];
-                else leq(prev, sb + 1 + j, &lcpb);
+        }
+        return i0;
+    };
+    const uint32_t d = tid_x() * kMergeE;
+    uint32_t i = 0, j = 0, l1 = kNoLcp, l2 = kNoLcp;
+    uint32_t lo = d > nb ? d - nb : 0, hi = min(d, na);
+    bool found = false;
+    if (half) {     // (uniform) every second thread's first output is searched
+                    // in the whole tile, by half of the threads; the others'
+                    // lie between their neighbours'
+        uint32_t* s_co = s_olcp;       // co-rank, l1, l2 of kWG / 2 threads
+        static_assert(3 * (kWG / 2) <= kMergeT, "they fit the outputs' memory");
+        const uint32_t t = tid_x(), d2 = 2 * d;
+        if (t < kWG / 2 && d2 < len) {
+            s_co[t] = corank(d2, d2 > nb ? d2 - nb : 0, min(d2, na), &l1, &l2);
+            s_co[kWG / 2 + t] = l1;
+            s_co[kWG + t] = l2;
+        }
+        __syncthreads();
+        if (d < len) {
+            i = s_co[t / 2];
+            l1 = s_co[kWG / 2 + t / 2];
+            l2 = s_co[kWG + t / 2];
+            found = t % 2 == 0;
+            lo = max(lo, i);
+            hi = min(hi, min(d + kMergeE < len ? s_co[t / 2 + 1] : na, i + kMergeE));
+        }
+        __syncthreads();     // (their memory takes the outputs)
+    }
+    uint32_t lcpa = 0, lcpb = 0;       // LCPs of the next A and B string with the previous output
+    if (d < len) {
+        if (!found) i = corank(d, lo, hi, &l1, &l2);
+        j = d - i;
+        // the previous output is the larger one of A[i-1] and B[j-1], and of two
+        // strings before a third the larger shares at least as much with it
+        const bool hasa = ia0 + i > 0, hasb = jb0 + j > 0;
+        if (i < na) {
+            if (hasa) lcpa = s_lcp[1 + i];
+            if (hasb) {
+                if (l2 == kNoLcp) leq(sb + j, 1 + i, &l2);
+                lcpa = max(lcpa, l2);
+            }
+        }
+        if (j < nb) {
+            if (hasb) lcpb = s_lcp[sb + 1 + j];
+            if (hasa) {
+                if (l1 == kNoLcp) leq(i, sb + 1 + j, &l1);
+                lcpb = max(lcpb, l1);
             }
         }
         const uint32_t nout = min(kMergeE, len - d);
@@ -4547,11 +4602,13 @@ int ps5_merge_device(ps5_ctx* c, const uint8_t* d_arena, uint64_t arena_bytes, c
         const uint64_t* pm = pf + (R.np + 1);
         const uint64_t* pt = pm + (R.np + 1);
         if (R.tiles) {
-            hipLaunchKernelGGL(k_merge_part, dim3(div_up(R.tiles, kWG / kMergeLanes)), dim3(kWG), 0, st, B, si, sk, ik, pf,
-                               pm, pt, R.np, co);
+            const uint32_t lanes = R.tiles < kMergeFew ? 8 : R.tiles < kMergeMany ? 4 : 1;
+            const auto part = lanes == 8 ? k_merge_part<8> : lanes == 4 ? k_merge_part<4> : k_merge_part<1>;
+            hipLaunchKernelGGL(part, dim3(div_up(R.tiles, kWG / lanes)), dim3(kWG), 0, st, B, si, sk, ik, pf, pm, pt, R.np,
+                               co);
             HIPCHK(hipGetLastError());
             hipLaunchKernelGGL(k_merge_tile, dim3(R.tiles), dim3(kWG), 0, st, B, si, sl, sk, ik, di, dl, dk, pf, pm, pt,
-                               R.np, co);
+                               R.np, co, R.tiles >= kMergeHalf);
             HIPCHK(hipGetLastError());
         }
         si = di;

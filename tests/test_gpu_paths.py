@@ -480,3 +480,31 @@ def test_noalloc_sort_starts_over(ps5, ctx, oracle):
     finally:
         for b in bufs:
             b.free()
+
+
+def sorted_runs(ctx, ps5, arena, offs, bounds):
+    """(idx, lcp) of contiguous ranges sorted on their own"""
+    idx, lcp = np.zeros(len(offs), np.uint32), np.zeros(len(offs), np.uint32)
+    for b, e in zip(bounds[:-1].astype(int), bounds[1:].astype(int)):
+        if e > b:
+            p, l = ctx.sort(arena, offs[b:e])
+            idx[b:e] = p + np.uint32(b)
+            lcp[b:e] = l
+    return idx, lcp
+
+
+@pytest.mark.parametrize("n, runs", [(60_000, 3), (8_400_000, 2), (8_400_000, 5), (33_600_000, 2), (33_600_000, 7)])
+@pytest.mark.parametrize("alphabet, lo, hi", [(b"ACGT", 4, 24), (b"ab", 0, 14), (bytes(range(33, 127)), 1, 20)])
+def test_merges_of_every_size_class(ps5, ctx, oracle, n, runs, alphabet, lo, hi):
+    """rounds whose tiles are searched by eight lanes, four and one; strings
+    that their first 8 characters decide and that they do not, identical ones"""
+    if n > 10_000_000 and hi > 20:
+        n, lo, hi = 33_600_000, 4, 14
+    arena, offs = ps5.gen_uniform(n + runs, n * (hi + 1), lo, hi, alphabet)
+    offs = offs[:n]
+    rng = np.random.default_rng(runs)
+    bounds = np.concatenate([[0], np.sort(rng.integers(0, n, runs - 1)), [n]]).astype(np.uint64)
+    idx, lcp = sorted_runs(ctx, ps5, arena, offs, bounds)
+    mi, ml = ctx.merge(arena, offs, bounds, idx, lcp)
+    r, msg = oracle.verify(arena, offs, mi, ml)
+    assert r == 0, msg
