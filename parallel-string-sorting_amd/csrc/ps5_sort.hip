@@ -2563,8 +2563,12 @@ __global__ __launch_bounds__(kWG) void k_merge_part(Bufs B, const uint32_t* src_
 // is less (16 M strings of ACGT in 8 runs 5.01 ms, 6.08 without half, 7.56 when
 // every thread also compared its heads with the output before it; 16 M of
 // ASCII, whose keys decide, 0.81, 0.80 and 0.82); below, the chain counts
-// (0.3 M of ACGT 160 us with half, 151 without).
-constexpr uint64_t kMergeHalf = 1024;
+// (8 runs of 0.3 M strings: ACGT 171 us with half, 155 without, URL-like ones
+// 353 and 308).  The line lies where 8 runs of URL-like strings, whose
+// comparisons are the longest, begin to gain (0.5 M 385 and 360 us, 0.7 M 412
+// and 524, 1 M 534 and 782); windows gain later (1 M 484 and 431), ASCII, digits
+// and ACGT lose 1 to 2% between.
+constexpr uint64_t kMergeHalf = 768;
 __global__ __launch_bounds__(kWG) void k_merge_tile(Bufs B, const uint32_t* src_idx, const uint32_t* src_lcp,
                                                     const key64* src_key, const key64* in_key,
                                                     uint32_t* dst_idx, uint32_t* dst_lcp,

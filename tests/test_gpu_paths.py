@@ -508,3 +508,20 @@ def test_merges_of_every_size_class(ps5, ctx, oracle, n, runs, alphabet, lo, hi)
     mi, ml = ctx.merge(arena, offs, bounds, idx, lcp)
     r, msg = oracle.verify(arena, offs, mi, ml)
     assert r == 0, msg
+
+
+@pytest.mark.parametrize("n", [785_407, 785_408, 786_433])
+@pytest.mark.parametrize("runs", [2, 6])
+def test_merges_where_threads_begin_to_search_in_pairs(ps5, ctx, oracle, n, runs):
+    """rounds of 767, 768 and 769 tiles of strings with long common prefixes,
+    some identical"""
+    rng = np.random.default_rng(n)
+    stems = [b"http://%d/" % i * (1 + i % 4) for i in range(40)]
+    pool = [stems[i % 40] + s for i, s in enumerate(random_strings(6000, 0, 9, b"ab", 3))]
+    arena, where = pack(pool)
+    offs = where[rng.integers(0, len(pool), n)]
+    bounds = np.concatenate([[0], np.sort(rng.integers(0, n, runs - 1)), [n]]).astype(np.uint64)
+    idx, lcp = sorted_runs(ctx, ps5, arena, offs, bounds)
+    mi, ml = ctx.merge(arena, offs, bounds, idx, lcp)
+    r, msg = oracle.verify(arena, offs, mi, ml)
+    assert r == 0, msg
