@@ -196,7 +196,7 @@ struct PlanArgs {
 // (ERR_CAP) and planned empty.
 __global__ __launch_bounds__(kBigWG) void k_plan(PlanArgs A, uint32_t* cnt)
 {
-    __shared__ uint32_t s_tmp[kBigWaves];
+    __shared__ uint32_t s_tmp[4 * kBigWaves];
     __shared__ uint32_t s_tb[kBigWG], s_gb[kBigWG];   // chunk and group offsets of a block of segments, for the tables
     __shared__ unsigned long long s_tot;
     __shared__ uint32_t s_ident, s_kmax;
@@ -249,11 +249,11 @@ __global__ __launch_bounds__(kBigWG) void k_plan(PlanArgs A, uint32_t* cnt)
             sc = (2u << D.k) * (G + 1);
             atomicMax(&s_kmax, D.k);
         }
-        uint32_t ttot, gtot, htot, stot;
-        const uint32_t tex = block_excl_scan<kBigWaves>(T, &ttot, s_tmp);
-        const uint32_t gex = block_excl_scan<kBigWaves>(G, &gtot, s_tmp);
-        const uint32_t hex = block_excl_scan<kBigWaves>(hc, &htot, s_tmp);
-        const uint32_t sex = block_excl_scan<kBigWaves>(sc, &stot, s_tmp);
+        const uint32_t each[4] = { T, G, hc, sc };
+        uint32_t ex[4], total[4];
+        block_excl_scan_k<kBigWaves, 4>(each, ex, total, s_tmp);
+        const uint32_t tex = ex[0], gex = ex[1], hex = ex[2], sex = ex[3];
+        const uint32_t ttot = total[0], gtot = total[1], htot = total[2], stot = total[3];
         if (i < nl) {
             D.hist_base = (uint32_t)(hcarry + hex);
             D.gbase = (uint32_t)(scarry + sex);
@@ -1095,12 +1095,13 @@ __device__ __forceinline__ void emit_children(const LargeDesc& D, uint32_t start
 // the buffer the level wrote.
 //
 // fused (a level planned on the host whose segments all are of one group and
-// few entries): the segments' run tables are written here, after the bucket
-// starts, and k_hist_runs is not launched.  It takes 5 to 9 us on its own for
-// so little (40 K strings of ACGT: 121 -> 118 us, a burst of 16 served
-// requests 1.45 -> 1.40 ms); a thread writes a bucket's row, which for the
-// hundreds of segments of a level planned on the device is slower than
-// k_hist_runs's turned tiles (64 M strings: 2.12 ms fused, 2.09 not).
+// few entries, or on the device for one such segment): the segments' run
+// tables are written here, after the bucket starts, and k_hist_runs is not
+// launched.  It takes 5 to 9 us on its own for so little (40 K strings of ACGT:
+// 121 -> 118 us, a burst of 16 served requests 1.45 -> 1.40 ms); a thread
+// writes a bucket's row, which for the hundreds of segments of a level planned
+// on the device is slower than k_hist_runs's turned tiles (64 M strings: 2.12
+// ms fused, 2.09 not).
 constexpr uint32_t kFusedRuns = 16384;     // entries of a segment
 __global__ __launch_bounds__(kBigWG) void k_children(Plan P, Bufs B, const key64* trees, Sink s, uint32_t dst, int fused)
 {
@@ -3766,7 +3767,13 @@ void dev_level(ps5_ctx* c, const Bufs& B, const Item* list, int ci, uint32_t bou
                     false);
     }
     const uint32_t groups_bound = (uint32_t)std::min<uint64_t>(kDevHistWgs, tiles_bound / kHistGroup + gl);
-    launch_hist(c, B, P, sink, dst, kmax, groups_bound, std::min(gl, kDevChildWgs), groups_bound, 0, false);
+    // no segment of so few strings has more than one group of chunks, and the
+    // tables of a single one are k_children's to write if they are short: two
+    // kernels fewer (a sort of 5 K strings 113 -> 105 us, 108 with separate
+    // count, scan and scatter passes; 40 K 117 -> 108)
+    const bool one_group = S <= (uint64_t)kHistGroup * kChunkMin;
+    const bool fused = one_group && gl == 1 && (tiles_bound << (kmax + 1)) <= kFusedRuns;
+    launch_hist(c, B, P, sink, dst, kmax, one_group ? 0u : groups_bound, std::min(gl, kDevChildWgs), groups_bound, 0, fused);
 }
 
 // Bound on the buckets of a level over segments of at most m strings (its

@@ -525,3 +525,29 @@ def test_merges_where_threads_begin_to_search_in_pairs(ps5, ctx, oracle, n, runs
     mi, ml = ctx.merge(arena, offs, bounds, idx, lcp)
     r, msg = oracle.verify(arena, offs, mi, ml)
     assert r == 0, msg
+
+
+@pytest.mark.parametrize("planning, rounds", [(1, 0), (0, 2)])
+@pytest.mark.parametrize("n", [2049, 4097, 30011, 65536, 131071, 131072, 131073, 133121])
+def test_small_levels_planned_on_the_device(ps5, oracle, n, planning, rounds):
+    """single roots whose run tables k_children writes, roots of one group of
+    chunks that have longer ones, and roots of two groups; the same strings in
+    several sets"""
+    rng = np.random.default_rng(n)
+    strs = random_strings(n, 0, 14, b"abcdefgh", n)
+    arena, offs = pack(strs)
+    first = np.concatenate([[0], np.sort(rng.integers(0, n, 2)), [n]]).astype(np.uint64)
+    c = ps5.Context(0)
+    try:
+        c.set_planning(planning)
+        c.set_graph_rounds(rounds)
+        check(c, oracle, arena, offs)
+        c.set_tuning(64, 10, 4)
+        check(c, oracle, arena, offs)
+        perm, lcp = c.sort_batch(arena, offs.astype(np.uint64), first)
+    finally:
+        c.close()
+    for b, e in zip(first[:-1].astype(int), first[1:].astype(int)):
+        if e > b:
+            r, msg = oracle.verify(arena, offs[b:e], perm[b:e], lcp[b:e])
+            assert r == 0, msg
