@@ -141,15 +141,16 @@ uint64_t ps5_noalloc_max_strings(void);
  * round of levels runs without any host synchronisation (one per round, to
  * learn whether another round is needed).  2 (auto): device planning for a
  * single sort of fewer than 4M strings, host planning for larger sorts,
- * batches and profiled sorts.  The default is 0.  All modes give the same
- * results.  No counterpart in the reference (its levels are recursion on
+ * batches and profiled sorts: one synchronisation per round of a small sort,
+ * though host planning is as fast or faster at every size.  The default is 0.
+ * All modes give the same results.  No counterpart in the reference (its levels are recursion on
  * the CPU).  The environment variable PS5_DEV_LEVELS=0/1/2 sets a new
  * context's mode.  Returns PS5_ERR_ARG for any other mode. */
 int ps5_ctx_set_planning(ps5_ctx* ctx, int mode);
 /* The current planning mode (0, 1 or 2), -1 for a NULL context. */
 int ps5_ctx_get_planning(ps5_ctx* ctx);
 
-/* Capture the first `rounds` rounds of a sort (8 characters of depth each)
+/* Capture the first `rounds` rounds of a sort (8 characters of depth or more each)
  * as one HIP graph, planned on the device, and replay it for later sorts with
  * the same buffers, string count, set boundaries and settings (0, the
  * default: off; at most 64).  A sort then needs one host synchronisation for
@@ -207,13 +208,16 @@ int ps5_sort_batch_device(ps5_ctx* ctx, const uint8_t* d_arena, uint64_t arena_b
 
 /* Per-kernel accounting of the last ps5_sort_device call when profiling is
  * on (ps5_ctx_set_profile(ctx, 1)): each launch is bracketed by HIP events on
- * the context's stream. */
+ * the context's stream.  So that each kernel has a time of its own, a profiled
+ * sort runs every kind of leaf in its own kernel and everything one after
+ * another, plans every level on the host and captures nothing: its kernels
+ * together take longer than an ordinary sort. */
 int ps5_ctx_set_profile(ps5_ctx* ctx, int on);
 int ps5_ctx_kernel_count(ps5_ctx* ctx);
 /* name (static string), summed milliseconds, launches, algorithmic bytes */
 int ps5_ctx_kernel_stat(ps5_ctx* ctx, int i, const char** name, double* ms,
                         uint64_t* launches, uint64_t* alg_bytes);
-/* Work statistics of the last sort: rounds (8-byte depth steps), levels,
+/* Work statistics of the last sort: rounds (of 8 characters or more), levels,
  * sample-sort segments, leaves, and the number of host synchronisations. */
 int ps5_ctx_work_stats(ps5_ctx* ctx, uint64_t* rounds, uint64_t* levels,
                        uint64_t* segments, uint64_t* leaves, uint64_t* syncs);
