@@ -143,9 +143,9 @@ uint64_t ps5_noalloc_max_strings(void);
  * single sort of fewer than 4M strings, host planning for larger sorts,
  * batches and profiled sorts: one synchronisation per round of a small sort,
  * though host planning is as fast or faster at every size.  The default is 0.
- * All modes give the same results.  No counterpart in the reference (its levels are recursion on
- * the CPU).  The environment variable PS5_DEV_LEVELS=0/1/2 sets a new
- * context's mode.  Returns PS5_ERR_ARG for any other mode. */
+ * All modes give the same results.  No counterpart in the reference (its levels
+ * are recursion on the CPU).  The environment variable PS5_DEV_LEVELS=0/1/2
+ * sets a new context's mode.  Returns PS5_ERR_ARG for any other mode. */
 int ps5_ctx_set_planning(ps5_ctx* ctx, int mode);
 /* The current planning mode (0, 1 or 2), -1 for a NULL context. */
 int ps5_ctx_get_planning(ps5_ctx* ctx);
